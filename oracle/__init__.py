@@ -291,6 +291,6 @@ def ref_quants():
 
 
 def build_ref():
-    """Compile oracle/_ref from the reference's source tree (only where that tree exists)."""
-    if os.path.isdir("/root/reference"):
+    """Compile oracle/_ref from the reference's source tree (only where its quantiser source is)."""
+    if os.path.isfile("/root/reference/src/minfer/kernels/torch_ext/csrc/quants/impl.cpp"):
         subprocess.run(["make", "-C", _HERE, "ref"], check=True, stdout=subprocess.DEVNULL)
