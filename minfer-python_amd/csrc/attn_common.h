@@ -202,6 +202,12 @@ MA_DEV float sum_across_quads(float x) {
     return sum_across_halves(__builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]));
 }
 
+// x of lane (l ^ M), M = 1 or 2: inside groups of four lanes, one instruction
+template <int M> MA_DEV uint32_t quad_swap(uint32_t x) {
+    static_assert(M == 1 || M == 2, "lanes of one group of four");
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, M == 1 ? 0xb1 : 0x4e, 0xf, 0xf, true);   // quad_perm [1,0,3,2] / [2,3,0,1]
+}
+
 MA_DEV float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Inclusive prefix sum of x over the lanes of a wave.

@@ -37,91 +37,82 @@ enum : uint32_t { TILE_NONE = 0, TILE_ALL = 1, TILE_MIXED = 2 };
 constexpr int kMaxKeyTiles = 2048;  // active-tile list capacity (L <= 131072)
 
 // ------------------------------------------------------------------------------------------
-// Mask classification: cls[b][qt][kt] for 64x64 tiles.  grid (ceil(NKT/16), NQT, B), 256 threads.
+// Mask bytes.  Rows of the mask are L bytes apart and L is any number, so a row starts at any byte; global loads of 4 and
+// 16 bytes need no alignment on this chip, and aligned or not they are one instruction.  MaskCols is a lane's 16 columns,
+// col0 .. col0 + 15 as far as they exist.  Where they cross the end of the row the load ends with the row instead, so nothing
+// past the mask is read; the columns in front of col0 that it brings lie in the same 64-column tile, except where the last
+// tile has fewer than 16 columns (`split`): there they are taken out.  A row shorter than 16 is read byte by byte.
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void classify_mask_kernel(const uint8_t* __restrict__ mask,
-                                                            uint8_t* __restrict__ cls, int L, int NQT,
-                                                            int NKT, int vec) {
-    __shared__ uint32_t any_s[16], all_s[16];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int strip = blockIdx.x, qt = blockIdx.y, b = blockIdx.z;
-    if (tid < 16) { any_s[tid] = 0u; all_s[tid] = 0x01010101u; }
-    __syncthreads();
-    const uint8_t* mb = mask + (size_t)b * L * L;
-    const int col0 = strip * 1024 + lane * 16;  // this lane's 16 key columns
-    uint32_t any_acc = 0u, all_acc = 0x01010101u;
-    if (vec) {
-        if (col0 < L) {
-            // all 16 row segments of this lane are requested before any is used (rows past the end
-            // re-read the last row, which changes neither the OR nor the AND)
-            uint4 x[16];
+typedef u32x4 __attribute__((aligned(1))) u32x4_any;
+typedef uint32_t __attribute__((aligned(1))) u32_any;
+
+struct MaskCols {
+    int first;    // first column that is read
+    int extra;    // columns in front of the lane's own that a load brings
+    bool on;      // the lane has columns
+    bool split;   // (the same for all lanes) a lane's extra columns belong to another tile
+    MA_DEV MaskCols(int col0, int L) {
+        first = L >= 16 ? min(col0, L - 16) : col0;
+        extra = col0 - first;
+        on = col0 < L;
+        split = L >= 16 && (L & 63) > 0 && (L & 63) < 16;
+    }
+    MA_DEV u32x4 load(const uint8_t* row) const { return *reinterpret_cast<const u32x4_any*>(row + first); }   // L >= 16
+    MA_DEV u32x4 load_bytes(const uint8_t* row, int L) const {   // L < 16: the last column again in the bytes past the end
+        u32x4 x = {0u, 0u, 0u, 0u};
+        for (int e = 0; e < 16; ++e) {
+            const uint32_t byte = (uint32_t)row[min(e, L - 1)] << (8 * (e & 3));
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int row = min(qt * 64 + w + 4 * i, L - 1);
-                x[i] = *reinterpret_cast<const uint4*>(mb + (size_t)row * L + col0);
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                any_acc |= x[i].x | x[i].y | x[i].z | x[i].w;
-                all_acc &= x[i].x & x[i].y & x[i].z & x[i].w;
-            }
+            for (int i = 0; i < 4; ++i) x[i] |= (e >> 2) == i ? byte : 0u;
         }
-    } else {
-        for (int r = w; r < 64; r += 4) {
-            const int row = qt * 64 + r;
-            if (row >= L) break;
-            for (int e = 0; e < 16; ++e) {
-                const int col = col0 + e;
-                if (col < L) {
-                    const uint32_t x = mb[(size_t)row * L + col] ? 1u : 0u;
-                    any_acc |= x;
-                    all_acc &= x * 0x01010101u;
+        return x;
+    }
+    // loaded pieces of N rows into the OR and the AND over rows and columns
+    template <int N> MA_DEV void add(const u32x4 (&x)[N], uint32_t& any_acc, uint32_t& all_acc) const {
+        if (!split) {
+#pragma unroll
+            for (int r = 0; r < N; ++r) {
+                any_acc |= x[r][0] | x[r][1] | x[r][2] | x[r][3];
+                all_acc &= x[r][0] & x[r][1] & x[r][2] & x[r][3];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t gone = (uint32_t)((1ull << (8 * min(max(extra - 4 * i, 0), 4))) - 1);
+#pragma unroll
+                for (int r = 0; r < N; ++r) {
+                    any_acc |= x[r][i] & ~gone;
+                    all_acc &= x[r][i] | gone;
                 }
             }
         }
     }
-    // lanes 4t..4t+3 of each wave cover key tile (strip*16 + t)
-    any_acc |= __shfl_xor(any_acc, 1); any_acc |= __shfl_xor(any_acc, 2);
-    all_acc &= __shfl_xor(all_acc, 1); all_acc &= __shfl_xor(all_acc, 2);
-    if ((lane & 3) == 0) {
-        atomicOr(&any_s[lane >> 2], any_acc);
-        atomicAnd(&all_s[lane >> 2], all_acc);
-    }
-    __syncthreads();
-    if (tid < 16) {
-        const int kt = strip * 16 + tid;
-        if (kt < NKT) {
-            const uint32_t c = any_s[tid] == 0u ? TILE_NONE : (all_s[tid] == 0x01010101u ? TILE_ALL : TILE_MIXED);
-            cls[((size_t)b * NQT + qt) * NKT + kt] = (uint8_t)c;
-        }
-    }
-}
+};
 
-// The same for masks whose rows can be read in aligned 16-byte pieces, 64 rows x 256 columns (4 key tiles) per workgroup:
-// a lane takes 16 bytes of one row, the workgroup 16 rows per pass, 4 passes, all requested before any is used.  Four times
-// the workgroups of the general kernel and a quarter of the loads per lane: the pass is latency-bound, not byte-bound
-// (16 MiB at S=4096: 4.4 us instead of 5.1).  grid (ceil(NKT/4), NQT, B).
-__global__ __launch_bounds__(256) void classify_mask_kernel_256(const uint8_t* __restrict__ mask, uint8_t* __restrict__ cls,
-                                                                int L, int NQT, int NKT) {
+// ------------------------------------------------------------------------------------------
+// Mask classification: cls[b][qt][kt] for 64x64 tiles.  64 rows x 256 columns (4 key tiles) per workgroup: a lane takes 16
+// bytes of one row, the workgroup 16 rows per pass, 4 passes, all requested before any is used.  The pass is latency-bound,
+// not byte-bound, so it is spread over as many workgroups as that gives (16 MiB at S=4096: 4.4 us; strips of 1024 columns
+// 5.1).  Rows at any alignment take the same loads: B=4 L=1003 28.6 us read byte by byte -> 4.3 us.
+// grid (ceil(NKT/4), NQT, B).
+// ------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void classify_mask_kernel(const uint8_t* __restrict__ mask, uint8_t* __restrict__ cls,
+                                                            int L, int NQT, int NKT) {
     __shared__ uint32_t any_s[4][4], all_s[4][4];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int strip = blockIdx.x, qt = blockIdx.y, b = blockIdx.z;
     const uint8_t* mb = mask + (size_t)b * L * L;
-    const int col0 = strip * 256 + (tid & 15) * 16;     // this lane's 16 key columns
+    const MaskCols cols(strip * 256 + (tid & 15) * 16, L);
     const int r0 = tid >> 4;                            // row inside a pass of 16 rows
     uint32_t any_acc = 0u, all_acc = 0x01010101u;
-    if (col0 < L) {
-        uint4 x[4];
+    if (cols.on) {
+        u32x4 x[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int row = min(qt * 64 + 16 * i + r0, L - 1);
-            x[i] = *reinterpret_cast<const uint4*>(mb + (size_t)row * L + col0);
+            const uint8_t* row = mb + (size_t)min(qt * 64 + 16 * i + r0, L - 1) * L;
+            x[i] = L >= 16 ? cols.load(row) : cols.load_bytes(row, L);
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            any_acc |= x[i].x | x[i].y | x[i].z | x[i].w;
-            all_acc &= x[i].x & x[i].y & x[i].z & x[i].w;
-        }
+        cols.add(x, any_acc, all_acc);
     }
     // lanes 4t..4t+3 (mod 16) cover key tile t of the strip; rows differ across lane / 16 and across waves
     any_acc |= __shfl_xor(any_acc, 1); any_acc |= __shfl_xor(any_acc, 2);
@@ -157,13 +148,12 @@ struct PrefillParams {
     int NQ;                // workgroup-level query tiles (dense: exact; varlen: upper bound)
     int n_seqs;
     int max_len;           // varlen: rows of a sequence past this many are not computed (>= every length for a valid call)
-    int mask_vec;          // dense: mask rows may be read as aligned 32-bit words
     float scale_log2;      // softmax scale * log2(e)
 };
 
 // MODE_DENSE: dense bool mask, tile classes from the pre-pass.  MODE_VARLEN: packed sequences, causal by index.
-// MODE_DENSE_SELF: dense bool mask of a short problem (L <= 1024, rows readable in 16-byte pieces): every workgroup
-// classifies its own rows of the mask in its prologue, one wave-wide load per row, and no pre-pass is launched.
+// MODE_DENSE_SELF: dense bool mask of a short problem (16 <= L <= 1024): every workgroup classifies its own rows of the
+// mask in its prologue, one wave-wide load per row, and no pre-pass is launched.
 enum { MODE_DENSE = 0, MODE_VARLEN = 1, MODE_DENSE_SELF = 2 };
 constexpr int kSelfClassifyMaxGrid = 512;
 constexpr int kSelfClassifyMaxL = 1024;   // 16 key tiles: lane l of a wave-wide load holds columns 16l .. 16l+15 of one row
@@ -323,21 +313,18 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
         const int rpw = 32 >> p.hpw_log2;
         const int row_first = q_row0 + (w & (HPW - 1)) * rpw;
         uint32_t any_acc = 0u, all_acc = 0x01010101u;
-        if (16 * lane < p.L) {
-            const uint8_t* mb = p.mask + (size_t)b * p.L * p.L + 16 * lane;
+        const MaskCols cols(16 * lane, p.L);
+        if (cols.on) {
+            const uint8_t* mb = p.mask + (size_t)b * p.L * p.L;
             for (int r0 = 0; r0 < rpw; r0 += 8) {
-                uint4 x[8];
+                u32x4 x[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) x[i] = *reinterpret_cast<const uint4*>(mb + (size_t)min(row_first + r0 + i, last_row) * p.L);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    any_acc |= x[i].x | x[i].y | x[i].z | x[i].w;
-                    all_acc &= x[i].x & x[i].y & x[i].z & x[i].w;
-                }
+                for (int i = 0; i < 8; ++i) x[i] = cols.load(mb + (size_t)min(row_first + r0 + i, last_row) * p.L);
+                cols.add(x, any_acc, all_acc);
             }
         }
-        any_acc |= __shfl_xor(any_acc, 1); any_acc |= __shfl_xor(any_acc, 2);
-        all_acc &= __shfl_xor(all_acc, 1); all_acc &= __shfl_xor(all_acc, 2);
+        any_acc |= quad_swap<1>(any_acc); any_acc |= quad_swap<2>(any_acc);
+        all_acc &= quad_swap<1>(all_acc); all_acc &= quad_swap<2>(all_acc);
         if ((lane & 3) == 0) { any_s[w][lane >> 2] = any_acc; all_s[w][lane >> 2] = all_acc; }
         __syncthreads();
         if (w == 0) {
@@ -478,13 +465,13 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
     uint32_t mw[2][4] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
     auto fetch_mask = [&](int kt) {
         const int key0 = kt * 64;
-        if (p.mask_vec && key0 + 64 <= seq_len) {
+        if (key0 + 64 <= seq_len) {
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb)
-                    mw[qb][kb] = *reinterpret_cast<const uint32_t*>(mrow[qb] + key0 + 16 * kb + 4 * quad);
-        } else {  // unaligned rows or a tile crossing the end: bytes, clamped (the range test comes later)
+                    mw[qb][kb] = *reinterpret_cast<const u32_any*>(mrow[qb] + key0 + 16 * kb + 4 * quad);
+        } else {  // a tile crossing the end: bytes, clamped (the range test comes later)
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
@@ -678,8 +665,14 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
         wait_vmcnt<0>();       // this wave's share of tile `it` (and its mask words) has landed
         __syncthreads();       // everyone's has; stage STAGE^1 is no longer being read
         if (it + 1 < n_active) issue_tile(ktn, STAGE ^ 1);
+        // The next tile's mask words are requested after this tile's were used; with 4 waves already in front of a tile that
+        // uses none (a short problem's few tiles wait for everything they request late: L=256 9.0 -> 8.6 us; with 8 waves the
+        // second copy of the requests costs as much as it gives, S=4096 134.4 -> 135.7).
+        const bool fetch = kDense && it + 1 < n_active && cn == TILE_MIXED;
+        const bool early = NW == kWavesSmall && cls_w != TILE_MIXED;
+        if (fetch && early) fetch_mask(ktn);
         if (cls_w != TILE_NONE) process_tile(stage_tag, kt, cls_w);
-        if (kDense && it + 1 < n_active && cn == TILE_MIXED) fetch_mask(ktn);   // after this tile's words were used
+        if (fetch && !early) fetch_mask(ktn);
         e_cur = e_next; e_next = e_after;
     };
     for (int it = 0; it < n_active; it += 2) {
@@ -840,23 +833,18 @@ MINFER_ATTN_EXPORT int minfer_flash_attn(int dtype, const void* q, const void* k
     const int rows_per_wg = 32 * (kWaves >> p.hpw_log2);
     p.NQ = (int)((L + rows_per_wg - 1) / rows_per_wg);
     p.n_seqs = 0;
-    p.mask_vec = ((L & 15) == 0 && aligned16(mask)) ? 1 : 0;
     const int64_t grid = (int64_t)p.NQ * B * Hkv * p.n_hg;
     if (grid > 0x7fffffffLL) return fail(MINFER_ATTN_EINVAL, "flash_attn: problem too large for one launch");
 
-    // A short problem whose mask rows can be read in 16-byte pieces and whose workgroups all fit on the chip at once
-    // (2 per CU, 256 CUs) needs no pre-pass: its workgroups classify their own rows, which takes 2-3 us off a call of
-    // 9-28 us.  With more workgroups than that the pre-pass is cheaper than every head re-reading the mask rows.
-    if (p.mask_vec && L <= kSelfClassifyMaxL && kWaves == kWavesSmall && grid <= kSelfClassifyMaxGrid) {
+    // A short problem whose workgroups all fit on the chip at once (2 per CU, 256 CUs) needs no pre-pass: its workgroups
+    // classify their own rows, which takes 2-3 us off a call of 9-28 us.  With more workgroups than that the pre-pass is
+    // cheaper than every head re-reading the mask rows.
+    if (L >= 16 && L <= kSelfClassifyMaxL && kWaves == kWavesSmall && grid <= kSelfClassifyMaxGrid) {
         p.cls = nullptr;
         return dispatch_prefill_nw<MODE_DENSE_SELF, kWavesSmall>(dtype, D, p, (int)grid, stream);
     }
-    if (p.mask_vec)
-        hipLaunchKernelGGL(classify_mask_kernel_256, dim3((p.NKT + 3) / 4, p.NQT, (unsigned)B), dim3(256), 0, stream,
-                           mask, (uint8_t*)workspace, p.L, p.NQT, p.NKT);
-    else
-        hipLaunchKernelGGL(classify_mask_kernel, dim3((p.NKT + 15) / 16, p.NQT, (unsigned)B), dim3(256), 0, stream,
-                           mask, (uint8_t*)workspace, p.L, p.NQT, p.NKT, p.mask_vec);
+    hipLaunchKernelGGL(classify_mask_kernel, dim3((p.NKT + 3) / 4, p.NQT, (unsigned)B), dim3(256), 0, stream,
+                       mask, (uint8_t*)workspace, p.L, p.NQT, p.NKT);
     if (int rc = check_launch("classify_mask_kernel")) return rc;
     return dispatch_prefill<MODE_DENSE>(dtype, D, p, kWaves, (int)grid, stream);
 }

@@ -128,6 +128,23 @@ def test_dense_matches_oracle(dtype, B, Hq, Hkv, L, D, kind, views):
     assert max_err(out, want) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("offset", [0, 5])
+@pytest.mark.parametrize("B,L,D", [(2, 1, 64), (3, 2, 128), (2, 3, 64), (2, 4, 128), (2, 5, 64), (2, 15, 128), (2, 16, 64), (3, 17, 128),
+                                   (2, 63, 64), (2, 65, 128), (1, 129, 128), (2, 255, 64), (1, 1023, 64), (1, 1025, 128), (1, 1103, 64)])
+def test_mask_rows_at_any_byte(B, L, D, offset):
+    """Rows of the mask start at any byte (L odd, base address odd) and end inside a 16-column piece or a 4-column word; the
+    bytes around the mask are True, so a column read past a row's end would show.  Self-classifying workgroups up to 1024
+    rows, the pre-pass above.  Tolerance: the one every fp16 attention result here has."""
+    gen = torch.Generator().manual_seed(L)
+    q, k, v = workloads.dense_prefill(B, 4, 2, L, D, torch.float16, seed=L, scale=1.0, device=DEV)
+    mask = make_mask("random", B, L, gen)
+    buf = torch.ones(B * L * L + offset + 64, dtype=torch.bool, device=DEV)
+    m = buf[offset:offset + B * L * L].view(B, 1, L, L)
+    m.copy_(mask)
+    out = run_prefill(q, k, v, m)
+    assert max_err(out, oracle.flash_attn(q, k, v, mask)) <= TOL[torch.float16]
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,L,D,kind", [
     (1, 4, 4, 16, 128, "random"),      # n_rep = 1: four query blocks per workgroup, of which one has rows
     (2, 4, 2, 48, 64, "full"),         # n_rep = 2
