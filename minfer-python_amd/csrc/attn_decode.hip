@@ -193,35 +193,27 @@ template <int D> struct DecodeGeom {
     static MA_DEV int swz_k(int row) { return D == 128 ? (row & 15) : ((row >> 1) & 7); }
 };
 
+// What a wave has accumulated over the rows it streamed: lane (l16, quad) holds head l16, O at d = 16db + 4 quad + 0..3
+// (un-normalised, fp32), the head's reference (largest score so far, within the laziness of its updates) and sum.
+template <int D> struct DecodeAcc {
+    f32x4 o[D / 16];
+    float m, l;
+};
+
+// Streams groups of 16 cache rows, rows row_lo .. row_hi - 1 (at least one) of (sequence b, KV head g), for the heads of head
+// group hg; my_k and my_v are the wave's own 16-row LDS areas.
 template <class T, int D>
-__global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode_split_kernel(const DecodeParams p) {
+MA_DEV void stream_rows(const DecodeParams& p, int b, int g, int hg, int row_lo, int row_hi, int n_groups, char* my_k, char* my_v, DecodeAcc<D>& acc) {
     using GEO = DecodeGeom<D>;
     constexpr int RB = GEO::RB, G = GEO::G, RPI = GEO::RPI, NI = GEO::NI;
     constexpr int KC = D / 32;   // 32-wide contraction chunks of K Q^T
     constexpr int DB = D / 16;   // 16-row blocks of O^T
     constexpr int NS = kDecodeStages;
-
-    __shared__ __attribute__((aligned(1024))) char v_lds[kDecodeWaves][kGroupRows * RB];
-    __shared__ __attribute__((aligned(1024))) char k_lds[kDecodeWaves][kGroupRows * RB];
-
-    const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
-    const int l16 = lane & 15, quad = lane >> 4;
-    SegmentWalk walk;
-    if (!walk.start(p, lane, w)) return;   // no share of the work
-    while (walk.next(p)) {
-    const int b = walk.b, split = walk.slot;
-    const int g = walk.pair % p.Hkv, hg = walk.pair / p.Hkv;
-    const int ctx = walk.ctx;
-    const int row_lo = walk.g0 * kGroupRows;
-    const int row_hi = min(walk.g1 * kGroupRows, ctx);
-    const int n_groups = walk.g1 - walk.g0;
-
+    const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
     const int heads_here = min(16, p.n_rep - hg * 16);
     const int head0 = g * p.n_rep + hg * 16;
     const short* Kb = (const short*)p.k + (int64_t)b * p.kv0 + (int64_t)g * p.kv1;
     const short* Vb = (const short*)p.v + (int64_t)b * p.kv0 + (int64_t)g * p.kv1;
-    char* my_v = v_lds[w];
-    char* my_k = k_lds[w];
 
     // ---- Q^T fragments (B operand): column = head l16, k = d = 32c + 8*quad + 0..7 ------------
     s16x8 qf[KC];
@@ -258,7 +250,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode
 #pragma unroll
     for (int s = 0; s < NS; ++s) load_group(s, kr[s], vr[s]);
 
-    f32x4 o_acc[DB];
+    f32x4 (&o_acc)[DB] = acc.o;
 #pragma unroll
     for (int db = 0; db < DB; ++db) o_acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_ref = -INFINITY, l_sum = 0.f;
@@ -331,17 +323,37 @@ __global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode
             load_group(t0 + s + NS, kr[s], vr[s]);
         }
     }
-
-    // ---- the segment's partial result: un-normalised O, reference max and sum of every head -------------
     l_sum += __shfl_xor(l_sum, 16);
     l_sum += __shfl_xor(l_sum, 32);
-    if (l16 < heads_here) {
-        const int64_t slot = ((int64_t)b * p.Hq + head0 + l16) * p.S + split;
+    acc.m = m_ref;
+    acc.l = l_sum;
+}
+
+// The segment's partial result of every head, into the workspace.
+template <int D>
+MA_DEV void store_segment(const DecodeParams& p, int b, int g, int hg, int split, const DecodeAcc<D>& acc) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
+    if (l16 < min(16, p.n_rep - hg * 16)) {
+        const int64_t slot = ((int64_t)b * p.Hq + g * p.n_rep + hg * 16 + l16) * p.S + split;
         float* dst = p.part_o + slot * D + 4 * quad;
 #pragma unroll
-        for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4*>(dst + 16 * db) = o_acc[db];
-        if (quad == 0) { p.part_ml[slot * 2] = m_ref; p.part_ml[slot * 2 + 1] = l_sum; }
+        for (int db = 0; db < D / 16; ++db) *reinterpret_cast<f32x4*>(dst + 16 * db) = acc.o[db];
+        if (quad == 0) { p.part_ml[slot * 2] = acc.m; p.part_ml[slot * 2 + 1] = acc.l; }
     }
+}
+
+template <class T, int D>
+__global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode_split_kernel(const DecodeParams p) {
+    __shared__ __attribute__((aligned(1024))) char v_lds[kDecodeWaves][kGroupRows * D * 2];
+    __shared__ __attribute__((aligned(1024))) char k_lds[kDecodeWaves][kGroupRows * D * 2];
+    const int lane = threadIdx.x & 63, w = wave_id();
+    SegmentWalk walk;
+    if (!walk.start(p, lane, w)) return;   // no share of the work
+    while (walk.next(p)) {
+        const int g = walk.pair % p.Hkv, hg = walk.pair / p.Hkv;
+        DecodeAcc<D> acc;
+        stream_rows<T, D>(p, walk.b, g, hg, walk.g0 * kGroupRows, min(walk.g1 * kGroupRows, walk.ctx), walk.g1 - walk.g0, k_lds[w], v_lds[w], acc);
+        store_segment<D>(p, walk.b, g, hg, walk.slot, acc);
     }
 }
 
@@ -362,9 +374,10 @@ template <int D> struct DecodeGeomQ8 {
     static constexpr int WAVE_LDS = RAW_LDS + PARK;
 };
 
-// kv0/kv1 of DecodeParams are byte strides here; q and out are fp16.
+// stream_rows over rows of Q8_0 blocks, in groups of 32 rows; kv0/kv1 of DecodeParams are byte strides here, q is fp16 and
+// row_lo a multiple of 32.  `area` is the wave's own LDS (DecodeGeomQ8::WAVE_LDS bytes).
 template <int D>
-__global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode_split_q8_kernel(const DecodeParams p) {
+MA_DEV void stream_rows_q8(const DecodeParams& p, int b, int g, int hg, int row_lo, int row_hi, int n_groups, char* area, DecodeAcc<D>& acc) {
     using T = F16;
     using GEO = DecodeGeom<D>;
     using Q = DecodeGeomQ8<D>;
@@ -373,26 +386,12 @@ __global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode
     constexpr int DB = D / 16;   // 16-row blocks of O^T
     constexpr int NS = kDecodeStagesQ8;
     constexpr int GR = kGroupRowsQ8;
-
-    __shared__ __attribute__((aligned(1024))) char lds[kDecodeWaves][(Q::WAVE_LDS + 1023) / 1024 * 1024];
-
-    const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
-    const int l16 = lane & 15, quad = lane >> 4;
-    SegmentWalk walk;
-    if (!walk.start(p, lane, w)) return;   // no share of the work
-    while (walk.next(p)) {
-    const int b = walk.b, split = walk.slot;
-    const int g = walk.pair % p.Hkv, hg = walk.pair / p.Hkv;
-    const int ctx = walk.ctx;
-    const int row_lo = walk.g0 * GR;                         // a multiple of 32
-    const int row_hi = min(walk.g1 * GR, ctx);
-    const int n_groups = walk.g1 - walk.g0;
-
+    const int lane = threadIdx.x & 63, l16 = lane & 15, quad = lane >> 4;
     const int heads_here = min(16, p.n_rep - hg * 16);
     const int head0 = g * p.n_rep + hg * 16;
-    char* raw_k = lds[w];
-    char* raw_v = lds[w];                    // after K's blocks have been read (a wave's LDS operations execute in order)
-    char* park_v = lds[w] + Q::RAW_LDS;
+    char* raw_k = area;
+    char* raw_v = area;                    // after K's blocks have been read (a wave's LDS operations execute in order)
+    char* park_v = area + Q::RAW_LDS;
 
     // The (sequence, KV head)'s rows start at kb; pieces are counted from the 16-byte boundary at or below it.
     // (plain pointer arithmetic, so that the loads below stay global-memory loads)
@@ -467,7 +466,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode
 #pragma unroll
     for (int s = 0; s < NS; ++s) { load_k(general_tag, s, ring[s]); load_v(general_tag, s, ring[s]); }
 
-    f32x4 o_acc[DB];
+    f32x4 (&o_acc)[DB] = acc.o;
 #pragma unroll
     for (int db = 0; db < DB; ++db) o_acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_ref = -INFINITY, l_sum = 0.f;
@@ -600,17 +599,23 @@ __global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode
         for (int s = 0; s < NS; ++s)
             if (t0 + s < n_groups) consume(general_tag, general_tag, t0 + s, ring[s]);
     }
-
-    // ---- the segment's partial result: un-normalised O, reference max and sum of every head -------------
     l_sum += __shfl_xor(l_sum, 16);
     l_sum += __shfl_xor(l_sum, 32);
-    if (l16 < heads_here) {
-        const int64_t slot = ((int64_t)b * p.Hq + head0 + l16) * p.S + split;
-        float* dst = p.part_o + slot * D + 4 * quad;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4*>(dst + 16 * db) = o_acc[db];
-        if (quad == 0) { p.part_ml[slot * 2] = m_ref; p.part_ml[slot * 2 + 1] = l_sum; }
-    }
+    acc.m = m_ref;
+    acc.l = l_sum;
+}
+
+template <int D>
+__global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode_split_q8_kernel(const DecodeParams p) {
+    __shared__ __attribute__((aligned(1024))) char lds[kDecodeWaves][(DecodeGeomQ8<D>::WAVE_LDS + 1023) / 1024 * 1024];
+    const int lane = threadIdx.x & 63, w = wave_id();
+    SegmentWalk walk;
+    if (!walk.start(p, lane, w)) return;   // no share of the work
+    while (walk.next(p)) {
+        const int g = walk.pair % p.Hkv, hg = walk.pair / p.Hkv;
+        DecodeAcc<D> acc;
+        stream_rows_q8<D>(p, walk.b, g, hg, walk.g0 * kGroupRowsQ8, min(walk.g1 * kGroupRowsQ8, walk.ctx), walk.g1 - walk.g0, lds[w], acc);
+        store_segment<D>(p, walk.b, g, hg, walk.slot, acc);
     }
 }
 
@@ -685,6 +690,178 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecodeParams 
     }
 }
 
+// ---- few or short sequences ------------------------------------------------------------------------
+// What the line of equal shares costs a small problem is latency: a wave streams 256 rows one group after the other
+// (0.65 us a group), and a second launch merges.  Here a workgroup of eight waves takes one chunk of p.chunk consecutive
+// rows of one (sequence, KV head, head group), two groups or a few per wave, and merges its waves' results in LDS.  A pair
+// that is one chunk long is done with that; otherwise the chunk's result goes to the workspace and the workgroup that comes
+// last (a counter per pair) merges the pair's chunks, so that there is no second launch.  Results cross from one XCD's L2
+// to another's: they are written and read with device-scope accesses, and a workgroup counts itself only when its own have
+// arrived.  Without counters (p.done null: a stream that is being captured, see stream_counters) decode_merge_kernel does
+// the merging, with the same code and so the same result.
+constexpr int kChunkWaves = 8;
+
+struct ChunkParams {
+    DecodeParams d;
+    void* out;
+    int64_t o0, o1;
+    int chunk;          // rows of a chunk, a multiple of the group
+    uint32_t* done;     // zeroed counters, one per (sequence, head group, KV head); left zero
+};
+
+MA_DEV void store_shared(float* p, float x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+MA_DEV float load_shared(const float* p) { return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// Weights and denominator of one head's partial results 0 .. n-1 whose (max, sum) are read by ml(i): out gets the weight
+// of each over the denominator's reciprocal.  Called by one thread per head.
+struct MergedHead { float m, l; };
+template <class F> MA_DEV MergedHead merge_ml(int n, float scale_log2, F ml) {
+    MergedHead r{-INFINITY, 0.f};
+    for (int i = 0; i < n; ++i) r.m = fmaxf(r.m, ml(i, 0));
+    if (r.m > -INFINITY)
+        for (int i = 0; i < n; ++i) r.l += ml(i, 1) * fast_exp2((ml(i, 0) - r.m) * scale_log2);   // a part without keys has sum 0
+    return r;
+}
+
+// Merges the n chunks of the pair's heads from the workspace and stores the output rows; all threads of the workgroup.
+// The order of the sums depends on nothing but n.
+template <class T, int D>
+MA_DEV void merge_chunks(const ChunkParams& c, int b, int head0, int heads, int n, float* lds_w /* [64][16] */, float* lds_inv /* [16] */) {
+    const DecodeParams& p = c.d;
+    const int tid = threadIdx.x;
+    const int64_t slot0 = ((int64_t)b * p.Hq + head0) * p.S;
+    for (int i = tid; i < n * heads; i += kChunkWaves * 64) {
+        const int h = i / n, s = i - h * n;
+        lds_w[s * 16 + h] = load_shared(p.part_ml + (slot0 + (int64_t)h * p.S + s) * 2);
+        lds_w[(64 + s) * 16 + h] = load_shared(p.part_ml + (slot0 + (int64_t)h * p.S + s) * 2 + 1);
+    }
+    // an output element's parts are requested while the weights are made, eight at a time
+    constexpr int PER = 16 * D / (kChunkWaves * 64);   // elements per thread for 16 heads
+    float x[PER][8];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        const int idx = tid + e * kChunkWaves * 64;
+        if (idx < heads * D) {
+            const float* src = p.part_o + (slot0 + (int64_t)(idx / D) * p.S) * D + idx % D;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) x[e][u] = load_shared(src + (int64_t)min(u, n - 1) * D);
+        }
+    }
+    __syncthreads();
+    if (tid < heads) {
+        const MergedHead r = merge_ml(n, p.scale_log2, [&](int i, int what) { return lds_w[(64 * what + i) * 16 + tid]; });
+        for (int i = 0; i < n; ++i) {
+            const float m = lds_w[i * 16 + tid];
+            lds_w[i * 16 + tid] = m > -INFINITY ? fast_exp2((m - r.m) * p.scale_log2) : 0.f;
+        }
+        lds_inv[tid] = r.l > 0.f ? 1.f / r.l : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        const int idx = tid + e * kChunkWaves * 64;
+        if (idx >= heads * D) break;
+        const int h = idx / D, d = idx % D;
+        const float* src = p.part_o + (slot0 + (int64_t)h * p.S) * D + d;
+        float sum = 0.f;
+        for (int s0 = 0; s0 < n; s0 += 8) {
+            if (s0 > 0) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) x[e][u] = load_shared(src + (int64_t)min(s0 + u, n - 1) * D);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (s0 + u < n) sum += x[e][u] * lds_w[(s0 + u) * 16 + h];
+        }
+        const uint32_t pk = T::pack2(sum * lds_inv[h], 0.f);
+        reinterpret_cast<uint16_t*>(c.out)[(int64_t)b * c.o0 + (int64_t)(head0 + h) * c.o1 + d] = (uint16_t)(pk & 0xffffu);
+    }
+}
+
+// grid (head groups x KV heads, sequences, chunks)
+template <class T, int D, bool Q8>
+__global__ __launch_bounds__(kChunkWaves * 64, 2) void decode_chunk_kernel(const ChunkParams c) {
+    const DecodeParams& p = c.d;
+    constexpr int NW = kChunkWaves, DB = D / 16, GR = Q8 ? kGroupRowsQ8 : kGroupRows;
+    constexpr int WAVE_LDS = Q8 ? (DecodeGeomQ8<D>::WAVE_LDS + 1023) / 1024 * 1024 : 2 * kGroupRows * D * 2;
+    constexpr int ORS = D + 4;   // floats between two heads' rows of a wave's result: their 16-byte pieces start in different banks
+    constexpr int MERGE_LDS = NW * 16 * ORS * 4;
+    constexpr int LDS = NW * WAVE_LDS > MERGE_LDS ? NW * WAVE_LDS : MERGE_LDS;
+    __shared__ __attribute__((aligned(1024))) char lds[LDS];   // the waves' row areas, then their results
+    __shared__ float ml_s[128 * 16], inv_s[16];
+    __shared__ int last_s;
+    const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
+    const int l16 = lane & 15, quad = lane >> 4;
+    const int b = blockIdx.y, split = blockIdx.z;
+    const int hg = p.n_hg == 1 ? 0 : (int)blockIdx.x / p.Hkv, g = (int)blockIdx.x - hg * p.Hkv;
+    const int heads = min(16, p.n_rep - hg * 16), head0 = g * p.n_rep + hg * 16;
+    const int ctx = min(max(p.ctx[b], 0), p.Lmax);
+    const int n = (ctx + c.chunk - 1) / c.chunk;   // chunks of this sequence
+    if (split >= max(n, 1)) return;
+    const int row0 = split * c.chunk, row1 = min(row0 + c.chunk, ctx);
+    const int groups = (row1 - row0 + GR - 1) / GR, per = (groups + NW - 1) / NW;
+    const int g_lo = min(w * per, groups), g_hi = min(g_lo + per, groups);
+    DecodeAcc<D> acc;
+    acc.m = -INFINITY; acc.l = 0.f;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) acc.o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (g_hi > g_lo) {
+        const int lo = row0 + g_lo * GR, hi = min(row0 + g_hi * GR, row1);
+        if constexpr (Q8) stream_rows_q8<D>(p, b, g, hg, lo, hi, g_hi - g_lo, lds + w * WAVE_LDS, acc);
+        else stream_rows<T, D>(p, b, g, hg, lo, hi, g_hi - g_lo, lds + w * WAVE_LDS, lds + w * WAVE_LDS + WAVE_LDS / 2, acc);
+    }
+    __syncthreads();   // every wave is done with its row area
+    float* o_s = reinterpret_cast<float*>(lds);   // [wave][head][ORS]
+    if (l16 < heads) {
+        float* dst = o_s + (w * 16 + l16) * ORS + 4 * quad;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4*>(dst + 16 * db) = acc.o[db];
+        if (quad == 0) { ml_s[w * 16 + l16] = acc.m; ml_s[(64 + w) * 16 + l16] = acc.l; }
+    }
+    __syncthreads();
+    const bool whole = n <= 1;   // the chunk is the whole context: its result is the output
+    const int64_t slot0 = ((int64_t)b * p.Hq + head0) * p.S + split;
+    for (int idx = tid; idx < heads * D; idx += NW * 64) {
+        const int h = idx / D, d = idx % D;
+        const MergedHead r = merge_ml(NW, p.scale_log2, [&](int i, int what) { return ml_s[(64 * what + i) * 16 + h]; });
+        float sum = 0.f;
+        if (r.m > -INFINITY) {
+#pragma unroll
+            for (int i = 0; i < NW; ++i) sum += o_s[(i * 16 + h) * ORS + d] * fast_exp2((ml_s[i * 16 + h] - r.m) * p.scale_log2);
+        }
+        if (whole) {
+            const float inv = r.l > 0.f ? 1.f / r.l : 0.f;
+            reinterpret_cast<uint16_t*>(c.out)[(int64_t)b * c.o0 + (int64_t)(head0 + h) * c.o1 + d] = (uint16_t)(T::pack2(sum * inv, 0.f) & 0xffffu);
+        } else {
+            store_shared(p.part_o + (slot0 + (int64_t)h * p.S) * D + d, sum);
+            if (d == 0) {
+                store_shared(p.part_ml + (slot0 + (int64_t)h * p.S) * 2, r.m);
+                store_shared(p.part_ml + (slot0 + (int64_t)h * p.S) * 2 + 1, r.l);
+            }
+        }
+    }
+    if (whole || !c.done) return;
+    wait_vmcnt<0>();   // the thread's stores have arrived
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t* done = c.done + (size_t)b * gridDim.x + blockIdx.x;
+        const uint32_t before = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last_s = before == (uint32_t)(n - 1);
+        if (last_s) __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (last_s) merge_chunks<T, D>(c, b, head0, heads, n, ml_s, inv_s);
+}
+
+template <class T, int D>
+__global__ __launch_bounds__(kChunkWaves * 64) void decode_merge_kernel(const ChunkParams c) {
+    const DecodeParams& p = c.d;
+    __shared__ float ml_s[128 * 16], inv_s[16];
+    const int b = blockIdx.y, hg = (int)blockIdx.x / p.Hkv, g = (int)blockIdx.x - hg * p.Hkv;
+    const int n = (min(max(p.ctx[b], 0), p.Lmax) + c.chunk - 1) / c.chunk;
+    if (n > 1) merge_chunks<T, D>(c, b, g * p.n_rep + hg * 16, min(16, p.n_rep - hg * 16), n, ml_s, inv_s);
+}
+
 // Smallest share of the work a workgroup takes, in cache rows: 256, or more for very long caches, so that a
 // (sequence, head) never has more than 64 partial results, which is what one wave of the combine kernel merges.
 static int decode_min_share_rows(int64_t Lmax) {
@@ -717,8 +894,46 @@ static int decode_workgroups() {
     return n;
 }
 
+// Rows of a chunk when the problem is one for decode_chunk_kernel, 0 when it is one for the line of equal shares.  The host
+// knows the pairs and the caches' capacity, not the contexts.  Chunks are sized so that their workgroups fill the compute
+// units once (one workgroup each: registers), 256 rows at least.  What the line has over that is balance, whatever the
+// number of pairs and the spread of the contexts, so chunks are taken where a call is mostly fixed cost or where they come
+// out even (us, line / chunks, contexts uniform from a sixteenth of the capacity up unless one number):
+//   up to 1536 rows: 8 pairs of 100 / 1500 rows 17.7 / 7.4 and 16.9 / 10.1; 24 pairs to 3000, Q8_0 19.8 / 12.7; 168 to 1500 21.0 / 20.1
+//   up to 2048 that occupy 9 of 10 units: 128 pairs to 4000 39.8 / 31.6, 256 to 2000 39.5 / 30.4 (96 to 4000, Q8_0, three
+//     quarters of the units: 22.0 / 25.5)
+//   longer ones that occupy 9 of 10 units, four to a pair or more: 32 pairs of 30000 85.5 / 77.4, 40 to 16000 49.5 / 40.9
+//     (three to a pair: 72 to 16000 56.9 / 65.5; two: 120 to 8000 50.4 / 53.8)
+//   short ones in two rounds: 512 pairs to 300 25.9 / 14.9, 400 to 800 24.4 / 21.7 (320 of 1100, Q8_0: 31.6 / 33.7)
+static int decode_chunk_rows(const DecodeParams& p) {
+    const int64_t pairs = (int64_t)p.B * p.Hkv * p.n_hg, units = decode_workgroups() / kDecodeWgPerCu;
+    const int64_t unit_rows = kChunkWaves * p.group_rows;
+    int64_t n = units / pairs;
+    n = n < 1 ? 1 : (n > 64 ? 64 : n);   // merge_chunks holds 64 parts of a head
+    n = n > p.S ? p.S : n;               // the workspace's slots of a row
+    int64_t chunk = (p.Lmax + n - 1) / n;
+    chunk = chunk < 256 ? 256 : (chunk + unit_rows - 1) / unit_rows * unit_rows;
+    n = p.Lmax > 0 ? (p.Lmax + chunk - 1) / chunk : 1;
+    if (pairs > kStreamCounters || chunk > (1 << 24)) return 0;
+    if (pairs * n > units) return pairs * n <= 2 * units && chunk <= 896 ? (int)chunk : 0;
+    const bool full = 10 * pairs * n >= 9 * units;
+    return chunk <= 1536 || (full && (chunk <= 2048 || n >= 4)) ? (int)chunk : 0;
+}
+
+template <class T, int D, bool Q8>
+static int launch_chunks(const DecodeParams& p, int chunk, void* out, int64_t o0, int64_t o1, hipStream_t stream) {
+    const unsigned n = (unsigned)((p.Lmax + chunk - 1) / chunk);
+    const ChunkParams c{p, out, o0, o1, chunk, n > 1 ? stream_counters(stream) : nullptr};
+    hipLaunchKernelGGL((decode_chunk_kernel<T, D, Q8>), dim3((unsigned)(p.Hkv * p.n_hg), (unsigned)p.B, n > 0 ? n : 1), dim3(kChunkWaves * 64), 0, stream, c);
+    if (int rc = check_launch("decode_chunk_kernel")) return rc;
+    if (n <= 1 || c.done) return MINFER_ATTN_OK;
+    hipLaunchKernelGGL((decode_merge_kernel<T, D>), dim3((unsigned)(p.Hkv * p.n_hg), (unsigned)p.B), dim3(kChunkWaves * 64), 0, stream, c);
+    return check_launch("decode_merge_kernel");
+}
+
 template <class T, int D>
 static int launch_decode(const DecodeParams& p, void* out, int64_t o0, int64_t o1, hipStream_t stream) {
+    if (const int chunk = decode_chunk_rows(p)) return launch_chunks<T, D, false>(p, chunk, out, o0, o1, stream);
     hipLaunchKernelGGL((decode_split_kernel<T, D>), dim3((unsigned)p.n_wg), dim3(kDecodeWaves * 64), 0, stream, p);
     if (int rc = check_launch("decode_split_kernel")) return rc;
     hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((p.B * p.Hq + 3) / 4), dim3(256), 0, stream, p, out, o0, o1);
@@ -727,6 +942,7 @@ static int launch_decode(const DecodeParams& p, void* out, int64_t o0, int64_t o
 
 template <int D>
 static int launch_decode_q8(const DecodeParams& p, void* out, int64_t o0, int64_t o1, hipStream_t stream) {
+    if (const int chunk = decode_chunk_rows(p)) return launch_chunks<F16, D, true>(p, chunk, out, o0, o1, stream);
     hipLaunchKernelGGL((decode_split_q8_kernel<D>), dim3((unsigned)p.n_wg), dim3(kDecodeWaves * 64), 0, stream, p);
     if (int rc = check_launch("decode_split_q8_kernel")) return rc;
     hipLaunchKernelGGL((decode_combine_kernel<F16, D>), dim3((p.B * p.Hq + 3) / 4), dim3(256), 0, stream, p, out, o0, o1);

@@ -63,6 +63,15 @@ inline int check_common(int dtype, const void* q, const void* k, const void* v, 
     return MINFER_ATTN_OK;
 }
 
+// Zeroed 32-bit counters for a launch on `stream` whose workgroups count their arrivals in them and leave them zero again,
+// or null when there are none to give (the launch then does without).  Launches on one stream run one after the other, so
+// they can share; every stream gets its own kStreamCounters of them, from a fixed array in the library's code object
+// (kCounterStreams streams per device; later ones get none).  A stream that is being captured gets none either: the captured
+// launch runs wherever and whenever the graph is replayed, possibly next to another launch on the capture's stream.
+constexpr int kStreamCounters = 2048;
+constexpr int kCounterStreams = 64;
+uint32_t* stream_counters(hipStream_t stream);
+
 // Dequantises K and V rows of Q8_0 blocks ([B, Hkv, L] rows of D/32 blocks; byte strides s0, s1 between batch
 // entries and heads; rows dense) into contiguous fp16 [B, Hkv, L, D] (csrc/quant.hip).
 int launch_dequant_q8_0_kv(const void* k, const void* v, void* k_out, void* v_out, int64_t B, int64_t Hkv, int64_t L,

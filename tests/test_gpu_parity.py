@@ -128,6 +128,41 @@ def test_dense_matches_oracle(dtype, B, Hq, Hkv, L, D, kind, views):
     assert max_err(out, want) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("Hq,Hkv,Lmax,D", [
+    (8, 2, 200, 128),     # one chunk: the workgroup's result is the output
+    (4, 4, 257, 64),      # a second chunk of one row
+    (40, 2, 1030, 128),   # 20 heads per KV head: two head groups; several chunks
+    (8, 1, 16400, 64),    # as many chunks as a head's merge holds
+    (64, 8, 3000, 128),   # 6 sequences: every unit has a chunk
+])
+def test_decode_chunks(Hq, Hkv, Lmax, D):
+    """Decode problems small enough to be cut into one chunk of rows per workgroup, at contexts around a wave's, a group's and a
+    chunk's edges: against the oracle, the same again on two streams at once (the arrival counters are the stream's own and
+    end as they began), and bit-equal under graph capture, where a second launch merges.  Tolerance: that of every fp16
+    attention result here."""
+    edges = [0, 1, 16, 17, Lmax // 2 + 1, Lmax]
+    q, kc, vc, _ = workloads.decode_cache(seed=Lmax, device=DEV, B=len(edges), Hq=Hq, Hkv=Hkv, Lmax=Lmax, D=D, ctx_lo=1, ctx_hi=1)
+    ctx = torch.tensor(edges, dtype=torch.int32, device=DEV)
+    streams = [torch.cuda.current_stream(), torch.cuda.Stream()]
+    outs = [torch.full(q.shape, float("nan"), dtype=q.dtype, device=DEV) for _ in range(6)]
+    torch.cuda.synchronize()
+    for i, out in enumerate(outs):
+        with torch.cuda.stream(streams[i % 2]):
+            assert capi.flash_attn_decode(q, kc, vc, ctx, out) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    assert max_err(outs[0], oracle.flash_attn_decode(q, kc, vc, ctx)) <= TOL[torch.float16]
+    assert all(torch.equal(o, outs[0]) for o in outs)
+    out, ws = torch.empty_like(outs[0]), torch.empty(capi.lib().minfer_flash_attn_decode_workspace_bytes(len(edges), Hq, Lmax, D), dtype=torch.uint8, device=DEV)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert capi.flash_attn_decode(q, kc, vc, ctx, out, ws) == capi.OK, capi.last_error()
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, outs[0])
+
+
 @pytest.mark.parametrize("offset", [0, 5])
 @pytest.mark.parametrize("B,L,D", [(2, 1, 64), (3, 2, 128), (2, 3, 64), (2, 4, 128), (2, 5, 64), (2, 15, 128), (2, 16, 64), (3, 17, 128),
                                    (2, 63, 64), (2, 65, 128), (1, 129, 128), (2, 255, 64), (1, 1023, 64), (1, 1025, 128), (1, 1103, 64)])
