@@ -208,8 +208,9 @@ int minfer_gemm(int dtype, int b_layout, const void* A, const void* B, const voi
  * minfer_gemm with a workspace.  A problem of a few dozen rows against a wide weight (a batch of decode steps, a short
  * prefill chunk) has too few output tiles to occupy the chip; given minfer_gemm_workspace_bytes(M, N, K) bytes of
  * device memory (16-byte aligned; 0 = this shape does not use any), the K dimension is cut into slices that run as
- * separate workgroups and meet in the workspace as fp32 partial sums, which a second kernel adds up (alpha, beta and
- * C applied there, one rounding): slices of the 128 x 128 tiles, or, up to 64 rows against an [N, K] weight of fewer
+ * separate workgroups and meet in the workspace as fp32 partial sums, which the last workgroup of a tile or a second
+ * kernel adds up (alpha, beta and C applied there, one rounding): slices of the 128 x 128 tiles, or, up to 64 rows,
+ * of 128-column tiles of a [K, N] weight, or of an [N, K] weight of fewer
  * than 12288 columns, of 64-column stripes (where two launches pay: from 9 rows on below 6144 columns, from 2 on rows
  * of 8192 values and more of at most 1536 columns, from 33 between 6144 and 12288 columns).  With a null workspace the
  * call is minfer_gemm; a workspace smaller than minfer_gemm_workspace_bytes is used only by a path whose slices fit

@@ -73,6 +73,7 @@ struct GemmParams {
     int tiles_m, tiles_n, per_xcd;
     int splits;                   // SPLIT instantiations: K is cut into this many slices, one workgroup per (tile, slice)
     float* part;                  // their fp32 partial products, [splits][M][N]
+    uint32_t* done;               // zeroed arrival counters, one per tile (stripe), left zero; null: gemm_reduce_kernel adds the slices up
     GemmGroup grp;                // used by the GROUPED instantiations only
 };
 // Which weight column unit `c` (a tile column or a column group) belongs to, and its index inside that weight.
@@ -80,6 +81,83 @@ MA_DEV int group_of_unit(const GemmGroup& g, int c, int& local) {
     const int s = c < g.end[0] ? 0 : (c < g.end[1] ? 1 : 2);
     local = c - (s == 0 ? 0 : (s == 1 ? g.end[0] : g.end[1]));
     return s;
+}
+
+// Four consecutive columns of D from the sums in fp32: alpha, beta and C, one rounding.
+template <class T> MA_DEV void store_result(const GemmParams& p, int m, int n, f32x4 sum) {
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = p.alpha * sum[e];
+    if (p.beta != 0.f) {
+        const s16x4 c = *reinterpret_cast<const s16x4*>((const short*)p.C + (int64_t)m * p.ldc + n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += p.beta * T::to_float(c[e]);
+    }
+    uint2 pk;
+    pk.x = T::pack2(v[0], v[1]);
+    pk.y = T::pack2(v[2], v[3]);
+    *reinterpret_cast<uint2*>((short*)p.D + (int64_t)m * p.ldd + n) = pk;
+}
+
+// ---- K slices that meet inside the launch -------------------------------------------------------------------
+// A slice's sums go to the workspace; the workgroup of a tile that comes last (a counter per tile) adds the tile's slices up
+// and stores D: no second launch, which costs the host 2.7 us and the chip 4, as much as many of these products take
+// themselves.  The sums pass from one XCD's L2 to another's, so they are written and read with device-scope accesses, and a
+// workgroup counts itself only when its own have arrived.  Slices are added in their order whoever comes last, as
+// gemm_reduce_kernel adds them, which takes over where there are no counters (stream_counters: a stream under capture).
+MA_DEV void store_slice4(const GemmParams& p, int slice, int m, int n, f32x4 v) {
+    float* at = p.part + ((int64_t)slice * p.M + m) * p.N + n;
+    if (!p.done) { *reinterpret_cast<f32x4*>(at) = v; return; }
+    uint64_t* dst = reinterpret_cast<uint64_t*>(at);
+    const u32x4 b = __builtin_bit_cast(u32x4, v);
+    __hip_atomic_store(dst, ((uint64_t)b[1] << 32) | b[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(dst + 1, ((uint64_t)b[3] << 32) | b[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+MA_DEV f32x4 load_slice4(const GemmParams& p, int slice, int m, int n) {
+    uint64_t* src = reinterpret_cast<uint64_t*>(p.part + ((int64_t)slice * p.M + m) * p.N + n);
+    const uint64_t lo = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint64_t hi = __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_bit_cast(f32x4, u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)});
+}
+// Called by all THREADS threads of a slice's workgroup after their store_slice4: columns n0 .. n1 - 1 (multiples of 4, four
+// at least) of rows m0 .. m1 - 1; `flag`: a shared word.
+template <class T, int THREADS>
+MA_DEV void finish_slices(const GemmParams& p, int tile, int m0, int m1, int n0, int n1, int* flag) {
+    if (!p.done) return;
+    wait_vmcnt<0>();   // the thread's sums have arrived
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t before = __hip_atomic_fetch_add(p.done + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *flag = before == (uint32_t)(p.splits - 1);
+        if (*flag) __hip_atomic_store(p.done + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!*flag) return;
+    const int n4 = (n1 - n0) >> 2, total = (m1 - m0) * n4;
+    // two pieces of four columns and eight slices at a time, so that sixteen loads of a thread are in flight
+    for (int i0 = threadIdx.x; i0 < total; i0 += 2 * THREADS) {
+        int m[2], n[2];
+        f32x4 sum[2], x[2][8];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int i = min(i0 + e * THREADS, total - 1), r = i / n4;
+            m[e] = m0 + r; n[e] = n0 + 4 * (i - r * n4);
+            sum[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        for (int s0 = 0; s0 < p.splits; s0 += 8) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int u = 0; u < 8; ++u) x[e][u] = load_slice4(p, min(s0 + u, p.splits - 1), m[e], n[e]);
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (s0 + u < p.splits) sum[e] = s0 + u == 0 ? x[e][u] : sum[e] + x[e][u];
+        }
+        store_result<T>(p, m[0], n[0], sum[0]);
+        if (i0 + THREADS < total) store_result<T>(p, m[1], n[1], sum[1]);
+    }
 }
 
 // swizzles: granule index of a row XORed with a function of the row (see the attention kernel's TileGeom)
@@ -342,8 +420,8 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
             }
             const int n = nb0 + 4 * quad;
             if (!CONCAT && n >= N) continue;
-            if (SPLIT) {   // the slice's raw sums; gemm_reduce_kernel adds the slices up and applies alpha, beta and C
-                *reinterpret_cast<f32x4*>(p.part + ((int64_t)slice * p.M + m) * N + n) = acc[nb][mb];
+            if (SPLIT) {   // the slice's raw sums
+                store_slice4(p, slice, m, n, acc[nb][mb]);
                 continue;
             }
             float v[4];
@@ -359,6 +437,126 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
             pk.y = T::pack2(v[2], v[3]);
             *reinterpret_cast<uint2*>(Dg + (int64_t)m * ldd + n) = pk;
         }
+    }
+    if constexpr (SPLIT) {
+        __shared__ int last_s;
+        finish_slices<T, SH::WAVES * 64>(p, t, m0, min(m0 + kBM, p.M), n0, min(n0 + kBN, N), &last_s);
+    }
+}
+
+// Up to 64 rows against a weight stored [K, N] (what a square weight is taken for): the work is reading the weight once.  A
+// workgroup of four waves owns 128 columns over a slice of K; 64 k rows of its columns (16 KiB, 256 consecutive bytes of each
+// row) and the activations' 64 values are a stage, copied global -> LDS, and a ring of six or seven stages fills the LDS: the
+// whole slice of a 4096 x 4096 weight is in flight at once.  A wave multiplies all rows with its 32 columns, the weight
+// fragments through transpose reads as in gemm_kernel.  The 128-row tiles that took these calls before copied 16 KiB of
+// activation rows per stage whatever M is, with two stages in flight (one row of 4096 x 4096 13.1 -> 9.5 us, with the slices
+// added up inside the launch).
+template <int MB> struct KnRowsGeom {
+    static constexpr int CA = (2 * MB + 3) / 4, CB = 4, NC = CA + CB;   // wave-wide copies per wave and stage (8 activation rows, 4 k rows each)
+    static constexpr int A_BYTES = 4096 * CA, B_BYTES = 16384;         // (the activation copies past 16 MB rows land behind them)
+    static constexpr int NS = MB <= 2 ? 7 : 6;                          // 140 / 144 KiB
+};
+template <class T, int MB>
+__global__ __launch_bounds__(4 * 64) void gemm_kn_rows_kernel(const GemmParams p) {
+    using G = KnRowsGeom<MB>;
+    constexpr int NS = G::NS;
+    __shared__ __attribute__((aligned(1024))) char b_lds[NS][G::B_BYTES];
+    __shared__ __attribute__((aligned(1024))) char a_lds[NS][G::A_BYTES];
+    const int lane = threadIdx.x & 63, w = wave_id(), l16 = lane & 15, quad = lane >> 4;
+    const int tile = (int)blockIdx.x / p.splits, slice = (int)blockIdx.x - tile * p.splits;
+    const int n0 = tile * 128;
+    const int kt_all = p.K / kBK, kt_first = slice * kt_all / p.splits, KT = (slice + 1) * kt_all / p.splits - kt_first;
+
+    uint32_t a_off[G::CA], b_off[G::CB];
+#pragma unroll
+    for (int j = 0; j < G::CA; ++j) {
+        const int row = 8 * (4 * j + w) + (lane >> 3);
+        a_off[j] = (uint32_t)((int64_t)min(row, p.M - 1) * p.lda + 8 * ((lane & 7) ^ swz_row_tile(row & 63))) * 2u;
+    }
+#pragma unroll
+    for (int j = 0; j < G::CB; ++j) {
+        const int row = 4 * (4 * j + w) + (lane >> 4);
+        b_off[j] = (uint32_t)((int64_t)row * p.ldb + min(n0 + 8 * ((lane & 15) ^ swz_col_tile(row)), p.N - 8)) * 2u;
+    }
+    auto issue = [&](int t, int st) {
+        const int64_t k0 = (int64_t)(kt_first + t) * kBK;
+        const short* ab = (const short*)p.A + k0;
+        const short* bb = (const short*)p.B + k0 * p.ldb;
+#pragma unroll
+        for (int j = 0; j < G::CB; ++j) copy16_global_to_lds<true>(bb, b_off[j], &b_lds[st][1024 * (4 * j + w)]);
+#pragma unroll
+        for (int j = 0; j < G::CA; ++j) copy16_global_to_lds<true>(ab, a_off[j], &a_lds[st][1024 * (4 * j + w)]);
+    };
+    // fragment addresses in stage 0 (see gemm_kernel)
+    uint32_t m_rd[2], n_rd[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) m_rd[ks] = lds_addr(&a_lds[0][0]) + l16 * 128 + 16 * ((4 * ks + quad) ^ swz_row_tile(l16));
+    {
+        const int krow = 8 * quad + (l16 >> 2);
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+            const int col = 32 * w + 16 * nb + 4 * (l16 & 3);
+            n_rd[nb] = lds_addr(&b_lds[0][0]) + krow * 256 + 16 * ((col >> 3) ^ swz_col_tile(krow)) + 2 * (col & 7);
+        }
+    }
+    f32x4 acc[2][MB];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // this wave's copies of all but the `later` most recently issued stages have landed (copies retire in order)
+    auto wait_later = [&](int later) {
+        if (later >= 5) wait_vmcnt<5 * G::NC>();
+        else if (later == 4) wait_vmcnt<4 * G::NC>();
+        else if (later == 3) wait_vmcnt<3 * G::NC>();
+        else if (later == 2) wait_vmcnt<2 * G::NC>();
+        else if (later == 1) wait_vmcnt<G::NC>();
+        else wait_vmcnt<0>();
+    };
+#pragma unroll
+    for (int t = 0; t < NS - 1; ++t)
+        if (t < KT) issue(t, t);
+    int st = 0;
+    for (int t = 0; t < KT; ++t) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // step t - 1 has been read
+        wait_later(min(NS - 2, KT - 1 - t));
+        __syncthreads();                                     // ... by every wave, and step t has landed for every wave
+        if (t + NS - 1 < KT) issue(t + NS - 1, st == 0 ? NS - 1 : st - 1);
+        const uint32_t ao = st * G::A_BYTES, bo = st * G::B_BYTES;
+        st = st == NS - 1 ? 0 : st + 1;
+        s16x8 nf[2][2], mf[2][MB];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                const s16x4 t0 = lds_read_tr16(n_rd[nb] + bo, 32 * ks * 256), t1 = lds_read_tr16(n_rd[nb] + bo, (32 * ks + 4) * 256);
+                nf[ks][nb] = s16x8{t0[0], t0[1], t0[2], t0[3], t1[0], t1[1], t1[2], t1[3]};
+            }
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) mf[ks][mb] = lds_read_b128(m_rd[ks] + ao, mb * (kRowTile / 4));
+        }
+        __builtin_amdgcn_sched_barrier(0);   // all reads first
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = T::mfma16(nf[ks][nb], mf[ks][mb], acc[nb][mb]);
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        const int m = 16 * mb + l16;
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+            const int n = n0 + 32 * w + 16 * nb + 4 * quad;
+            if (m >= p.M || n >= p.N) continue;
+            if (p.splits > 1) store_slice4(p, slice, m, n, acc[nb][mb]);
+            else store_result<T>(p, m, n, acc[nb][mb]);
+        }
+    }
+    if (p.splits > 1) {
+        __shared__ int last_s;
+        finish_slices<T, 4 * 64>(p, tile, 0, p.M, n0, min(n0 + 128, p.N), &last_s);
     }
 }
 
@@ -578,7 +776,7 @@ template <int MB> struct StripeGeom {
     static constexpr int CW = 8, CX = 2 * MB;                  // copies per wave and segment
 };
 // SLICED: p.splits workgroups per stripe, each over its share of the segments; they leave raw fp32 sums in p.part
-// ([slice][M][N]) for gemm_reduce_kernel.
+// ([slice][M][N]) for finish_slices.
 // GROUPED: the stripes of up to three weights numbered through (p.grp.end in stripes), alpha = 1 and no C.
 template <class T, int MB, bool SLICED = false, bool GROUPED = false>
 __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p) {
@@ -724,7 +922,7 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
 #pragma unroll
         for (int u = 1; u < 4; ++u) sum += red[((u * 4 + w) * MB + mb) * 64 + lane];
         if (SLICED) {
-            *reinterpret_cast<f32x4*>(p.part + ((int64_t)slice * p.M + m) * p.N + n) = sum;
+            store_slice4(p, slice, m, n, sum);
             continue;
         }
         float v[4];
@@ -742,6 +940,10 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
     }
     cb += nb;
     if (cb < blk_last) __syncthreads();                        // the sums have been read: the next chunk's copies may land there
+    }
+    if constexpr (SLICED) {
+        __shared__ int last_s;
+        finish_slices<T, 4 * 64>(p, (int)blockIdx.x / p.splits, 0, p.M, 16 * blk_first, min(16 * blk_last, p.N), &last_s);
     }
 }
 // Which widths it takes (in stripes of 64 columns; weights coming from memory): from 96 on every row count that reaches
@@ -1170,7 +1372,7 @@ static int launch_skinny_q8(const GemmParams& p, hipStream_t stream) {
 constexpr int kQ8SegBytes = 272;
 constexpr int kQ8Stage = 22 * 1024;                            // 17 KiB of row segments, 3 KiB the extra copies land in; three stages hold the 64 KiB of partial sums
 // SLICED: p.splits workgroups per chunk of four blocks, each over its share of the segments; raw fp32 sums into p.part
-// ([slice][M][N]) for gemm_reduce_kernel (a narrow weight with a workspace, as gemm_stripe_kernel has it).
+// ([slice][M][N]) for finish_slices (a narrow weight with a workspace, as gemm_stripe_kernel has it).
 template <int MB, bool SLICED = false>
 __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams p) {
     using T = F16;
@@ -1283,7 +1485,7 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams
 #pragma unroll
         for (int u = 1; u < 4; ++u) sum += red[((u * 4 + w) * MB + mb) * 64 + lane];
         if (SLICED) {
-            *reinterpret_cast<f32x4*>(p.part + ((int64_t)slice * p.M + m) * p.N + n) = sum;
+            store_slice4(p, slice, m, n, sum);
             continue;
         }
         float v[4];
@@ -1301,6 +1503,10 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams
     }
     cb += nb;
     if (cb < blk_last) __syncthreads();
+    }
+    if constexpr (SLICED) {
+        __shared__ int last_s;
+        finish_slices<T, 4 * 64>(p, (int)blockIdx.x / p.splits, 0, p.M, 16 * blk_first, min(16 * blk_last, p.N), &last_s);
     }
 }
 // Which calls it takes: 2-64 rows, whole segments of 8 blocks, rows that start on 16-byte boundaries, and a weight wide
@@ -1362,26 +1568,30 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmParams p) {
         const int m = (int)(i / n4), n = 4 * (int)(i % n4);
         f32x4 sum = *reinterpret_cast<const f32x4*>(p.part + (int64_t)m * p.N + n);
         for (int sl = 1; sl < p.splits; ++sl) sum += *reinterpret_cast<const f32x4*>(p.part + ((int64_t)sl * p.M + m) * p.N + n);
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = p.alpha * sum[e];
-        if (p.beta != 0.f) {
-            const s16x4 c = *reinterpret_cast<const s16x4*>((const short*)p.C + (int64_t)m * p.ldc + n);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += p.beta * T::to_float(c[e]);
-        }
-        uint2 pk;
-        pk.x = T::pack2(v[0], v[1]);
-        pk.y = T::pack2(v[2], v[3]);
-        *reinterpret_cast<uint2*>((short*)p.D + (int64_t)m * p.ldd + n) = pk;
+        store_result<T>(p, m, n, sum);
     }
 }
 
-static int launch_stripe_q8_slices(GemmParams& p, hipStream_t stream) {
-    if (int rc = launch_stripe_q8<true>(p, stream)) return rc;
+// The counters of a sliced launch, when its workgroups are to add the slices up themselves: up to 2 MiB of sums.  Written
+// through to where every XCD sees them they pass at about a microsecond per MiB, so larger ones are left to a second launch
+// (fused / two launches: 1 MiB 12.2 / 13.4 us, 1.9 MiB 23.7 / 25.3, 2.4 MiB 18.0 / 15.0, 5 MiB 16.7 / 13.7).  At most 256 tiles.
+static uint32_t* slice_counters(const GemmParams& p, hipStream_t stream) {
+    return (int64_t)p.splits * p.M * p.N * 4 <= (2 << 20) ? stream_counters(stream) : nullptr;
+}
+
+// After a sliced launch: nothing where its workgroups have added the slices up themselves.
+template <class T>
+static int launch_reduce(const GemmParams& p, hipStream_t stream) {
+    if (p.done) return MINFER_ATTN_OK;
     const int grid = (int)std::min<int64_t>(((int64_t)p.M * (p.N / 4) + 255) / 256, 256 * 8);
-    hipLaunchKernelGGL((gemm_reduce_kernel<F16>), dim3(grid), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((gemm_reduce_kernel<T>), dim3(grid), dim3(256), 0, stream, p);
     return check_launch("gemm_reduce_kernel");
+}
+
+static int launch_stripe_q8_slices(GemmParams& p, hipStream_t stream) {
+    p.done = slice_counters(p, stream);
+    if (int rc = launch_stripe_q8<true>(p, stream)) return rc;
+    return launch_reduce<F16>(p, stream);
 }
 
 // How many K slices a problem is cut into when a workspace is at hand: problems whose 128 x 128 tiles would leave most
@@ -1405,10 +1615,29 @@ static int gemm_splits(int64_t M, int64_t N, int64_t K) {
 
 template <class T>
 static int launch_stripe_slices(GemmParams& p, hipStream_t stream) {
+    p.done = slice_counters(p, stream);
     if (int rc = launch_stripe<T, true>(p, (p.N + 15) / 16, stream)) return rc;
-    const int grid = (int)std::min<int64_t>(((int64_t)p.M * (p.N / 4) + 255) / 256, 256 * 8);
-    hipLaunchKernelGGL((gemm_reduce_kernel<T>), dim3(grid), dim3(256), 0, stream, p);
-    return check_launch("gemm_reduce_kernel");
+    return launch_reduce<T>(p, stream);
+}
+
+// [K, N] weights of up to 64 rows: slices of K bring the column tiles up to the chip's 256 compute units, every slice two
+// steps of 64 at least.
+constexpr int64_t kKnRows = 64;
+static int kn_slices(int64_t M, int64_t N, int64_t K) {
+    if (M < 1 || M > kKnRows || K % kBK != 0 || K < 8 * kBK || N % 8 != 0) return 1;
+    const int64_t tiles = (N + 127) / 128;
+    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, K / kBK / 2), 64));
+}
+template <class T>
+static int launch_kn_rows(GemmParams& p, hipStream_t stream) {
+    const dim3 grid((unsigned)((p.N + 127) / 128 * p.splits)), block(4 * 64);
+    p.done = p.splits > 1 ? slice_counters(p, stream) : nullptr;
+    if (p.M <= 16) hipLaunchKernelGGL((gemm_kn_rows_kernel<T, 1>), grid, block, 0, stream, p);
+    else if (p.M <= 32) hipLaunchKernelGGL((gemm_kn_rows_kernel<T, 2>), grid, block, 0, stream, p);
+    else if (p.M <= 48) hipLaunchKernelGGL((gemm_kn_rows_kernel<T, 3>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((gemm_kn_rows_kernel<T, 4>), grid, block, 0, stream, p);
+    if (int rc = check_launch("gemm_kn_rows_kernel")) return rc;
+    return p.splits > 1 ? launch_reduce<T>(p, stream) : MINFER_ATTN_OK;
 }
 
 template <class T, bool NT>
@@ -1418,12 +1647,11 @@ static int launch_split(GemmParams& p, hipStream_t stream) {
     p.tiles_n = (p.N + SH::BN - 1) / SH::BN;
     p.per_xcd = 0;
     const int64_t wgs = (int64_t)p.tiles_m * p.tiles_n * p.splits;
+    p.done = slice_counters(p, stream);
     if (one_workgroup_per_unit(wgs)) hipLaunchKernelGGL((gemm_kernel<T, NT, GemmSmall3, false, true>), dim3((unsigned)wgs), dim3(SH::WAVES * 64), 0, stream, p);
     else hipLaunchKernelGGL((gemm_kernel<T, NT, SH, false, true>), dim3((unsigned)wgs), dim3(SH::WAVES * 64), 0, stream, p);
     if (int rc = check_launch("gemm_kernel (K slices)")) return rc;
-    const int grid = (int)std::min<int64_t>(((int64_t)p.M * (p.N / 4) + 255) / 256, 256 * 8);
-    hipLaunchKernelGGL((gemm_reduce_kernel<T>), dim3(grid), dim3(256), 0, stream, p);
-    return check_launch("gemm_reduce_kernel");
+    return launch_reduce<T>(p, stream);
 }
 
 template <class T, bool NT, class SH>
@@ -1672,6 +1900,12 @@ static int gemm_impl(int dtype, int b_layout, const void* A, const void* B, cons
         return dtype == MINFER_ATTN_F16 ? launch_gemv<F16>(p, p.N, stream) : launch_gemv<BF16>(p, p.N, stream);
     if (fast && nt && (M <= 16 || (!can_split && (M <= 32 || (M <= 64 && N * K <= (INT64_C(1) << 25))))))
         return dtype == MINFER_ATTN_F16 ? launch_skinny<F16>(p, stream) : launch_skinny<BF16>(p, stream);
+    if (fast && !nt && M <= kKnRows) {
+        const int kn = workspace && aligned16(workspace) ? kn_slices(M, N, K) : 1;
+        p.splits = workspace_bytes >= (size_t)kn * (size_t)M * (size_t)N * sizeof(float) ? kn : 1;
+        p.part = (float*)workspace;
+        return dtype == MINFER_ATTN_F16 ? launch_kn_rows<F16>(p, stream) : launch_kn_rows<BF16>(p, stream);
+    }
     if (can_split) {
         p.splits = splits; p.part = (float*)workspace;
         if (dtype == MINFER_ATTN_F16) return nt ? launch_split<F16, true>(p, stream) : launch_split<F16, false>(p, stream);
@@ -1689,7 +1923,7 @@ MINFER_ATTN_EXPORT int minfer_gemm(int dtype, int b_layout, const void* A, const
 
 MINFER_ATTN_EXPORT size_t minfer_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
-    const int splits = std::max(gemm_splits(M, N, K), stripe_slices(M, N, K));
+    const int splits = std::max(std::max(gemm_splits(M, N, K), stripe_slices(M, N, K)), kn_slices(M, N, K));
     return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 

@@ -281,6 +281,46 @@ def test_gemm_k_slices_against_oracle(layout, dtype, M, N, K, alpha, beta):
     assert_close(d2, exact, dtype, "fallback")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 8, 64),          # one K step, one column block half a wave wide
+    (16, 128, 128),      # one tile
+    (17, 136, 512),      # a second tile of 8 columns; four slices of two steps
+    (32, 264, 576),      # nine steps
+    (33, 4096, 4096),    # eight slices of as many steps as the ring has stages
+    (48, 1000, 3072),
+    (49, 520, 5120),     # slices longer than the ring
+    (64, 4104, 2048),
+    (64, 33000, 128),    # more tiles than compute units
+])
+def test_few_rows_against_a_kn_weight(dtype, M, N, K):
+    """The [K, N] kernel of up to 64 rows: edges of its row blocks, column tiles, K slices and ring, with slices that meet inside
+    the launch (twice on one stream: the arrival counters end as they began), in a second launch (under graph capture, same
+    bits) and without a workspace; the bound is this file's."""
+    a, b, c = make(M, N, K, KN, dtype, seed=M + N + K)
+    exact = oracle.gemm(a.float().numpy(), b.float().numpy(), c.float().numpy(), 2.0, 3.0, KN)
+    da, db, dc = a.to(DEV), b.to(DEV), c.to(DEV)
+    need = capi.lib().minfer_gemm_workspace_bytes(M, N, K)
+    ws = torch.full((max(need, 16),), 0xFF, dtype=torch.uint8, device=DEV)
+    outs = [torch.full((M, N), float("nan"), dtype=dtype, device=DEV) for _ in range(4)]
+    for d in outs[:2]:
+        assert capi.gemm_ws(da, db, dc, d, 2.0, 3.0, ws, KN) == capi.OK, capi.last_error()
+    assert capi.gemm(da, db, dc, outs[2], 2.0, 3.0, KN) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert capi.gemm_ws(da, db, dc, outs[3], 2.0, 3.0, ws, KN) == capi.OK, capi.last_error()
+    for _ in range(2):
+        outs[3].fill_(float("nan"))
+        ws.fill_(0xFF)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(outs[3], outs[0])
+    assert torch.equal(outs[1], outs[0])
+    assert_close(outs[0], exact, dtype, "slices")
+    assert_close(outs[2], exact, dtype, "no workspace")
+
+
 def test_gemm_workspace_bytes_is_zero_where_tiles_fill_the_chip():
     L = capi.lib()
     assert L.minfer_gemm_workspace_bytes(4096, 4096, 4096) == 0
