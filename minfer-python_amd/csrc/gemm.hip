@@ -28,32 +28,46 @@ namespace minfer_attn {
 
 
 constexpr int kBK = 64;
-// Two tile shapes: 8 waves (2 x 4) on 256 x 256 for problems that fill the chip with such tiles, 4 waves (2 x 2) on
-// 128 x 128 otherwise.  A wave owns 32*MB rows x 32*NB columns (as blocks of 16 x 16); OCC waves per SIMD.
-template <int MB_, int NB_, int WAVES_N_, int OCC_, int WAVES_M_ = 2, int NS_ = 2> struct GemmShape {
-    static constexpr int MB = MB_, NB = NB_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, WAVES = WAVES_M * WAVES_N, OCC = OCC_;
+// Tile shapes: 8 waves (2 x 4) on 256 x 256 where the problem fills the chip with such tiles, smaller ones where it does not
+// (pick_tile).  A wave owns M16 x N16 blocks of 16 x 16; OCC waves per SIMD.
+template <int M16_, int N16_, int WAVES_N_, int OCC_, int WAVES_M_ = 2, int NS_ = 2> struct GemmShape {
+    static constexpr int M16 = M16_, N16 = N16_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, WAVES = WAVES_M * WAVES_N, OCC = OCC_;
     static constexpr int NS = NS_;   // stages of the K ring in LDS: NS - 1 steps in flight while one is multiplied
-    static constexpr int BM = 32 * MB * WAVES_M, BN = 32 * NB * WAVES_N;
+    static constexpr int BM = 16 * M16 * WAVES_M, BN = 16 * N16 * WAVES_N;
     static constexpr int A_PANEL = BM * 128, B_PANEL = BN * 128;   // bytes of one K step
-    static constexpr int A_COPIES = A_PANEL / 1024 / WAVES, B_COPIES = B_PANEL / 1024 / WAVES;   // wave-wide copies per wave
+    // wave-wide copies (1 KiB) per wave and K step; every wave makes the same number, so that they can be counted: where the A
+    // panel's do not come out even the last waves copy a piece again (the same bytes to the same place)
+    static constexpr int A_PIECES = A_PANEL / 1024, A_COPIES = (A_PIECES + WAVES - 1) / WAVES, B_COPIES = B_PANEL / 1024 / WAVES;
+    static_assert(B_PANEL % (1024 * WAVES) == 0 && A_PIECES >= WAVES, "whole copies");
 };
 // (4 waves with 128 x 128 each, GemmShape<4, 4, 2, 1>, read a third fewer LDS bytes per flop.  Compiled as it stands
 // that shape spills: its 256 accumulators leave the allocator no register to move anything with.  On 32 x 32 blocks,
 // with 14 of the 16 accumulator blocks pinned to the accumulation registers and 2 to the vector registers by inline
 // assembly, it was spill-free and ended level with the 8-wave shape at 4096^3 and 4 % behind at 8192^3.)
-using GemmBig = GemmShape<4, 2, 4, 2>;
-using GemmSmall = GemmShape<2, 2, 2, 2>;
+using GemmBig = GemmShape<8, 4, 4, 2>;
+using GemmSmall = GemmShape<4, 4, 2, 2>;
 // The same tile with three stages (96 KiB of LDS: one workgroup per compute unit) for launches of at most one workgroup per
 // compute unit anyway: two steps in flight instead of one (clocks settled, 512 x 6144 x 4096 as 192 tiles 43.6 -> 36.6 us,
 // 1024 x 4096 x 4096 as 256 tiles 44.9 -> 40.1, 256 x 14336 x 4096 44.9 -> 38.5; with more workgroups than compute units
 // two resident workgroups of two stages are ahead, 2048 x 4096 x 4096 66.9 against 78.6; four stages lose to three throughout).
-using GemmSmall3 = GemmShape<2, 2, 2, 2, 2, 3>;
+using GemmSmall3 = GemmShape<4, 4, 2, 2, 2, 3>;
 static bool one_workgroup_per_unit(int64_t workgroups) { return workgroups <= 256; }
-// 256 x 192 (8 waves as 4 x 2, a wave owns 64 x 96): for widths that are multiples of 192 whose 256 x 256 tiles would
-// leave half the chip idle in their last round (4096 x 6144 is 384 large tiles, one and a half rounds on 256 compute
-// units, but 512 of these, two full rounds of three quarters the work each).  [N, K] weights only: its 192 columns are
-// three 64-row sub-tiles of such a weight, but one and a half of the 128-column sub-tiles of a [K, N] one.
-using GemmWide = GemmShape<2, 3, 2, 2, 4>;
+// Sizes in between, for problems whose 256 x 256 tiles would leave much of the chip idle in their only or last round.  All run
+// at what the LDS and the barrier of a K step leave, 5-20 % below the large tile's rate per flop, so they pay where they save a
+// half-empty round.
+// 256 x 192 (8 waves as 4 x 2, a wave owns 64 x 96), [N, K] weights only: its 192 columns are three 64-row sub-tiles of such a
+// weight, but one and a half of the 128-column sub-tiles of a [K, N] one (4096 x 6144 x 4096: 512 tiles, two full rounds,
+// where the large ones take one and a half; 1200 x 28672 x 4096 294 -> 268 us).
+using GemmWide = GemmShape<4, 6, 2, 2, 4>;
+// 192 x 256, for [K, N] weights in its place (2500 x 4096 x 4096: 160 large tiles 87 us, 224 of these 77).
+using GemmRows192 = GemmShape<6, 4, 4, 2>;
+// 160 x 256, [N, K] weights: the odd row counts (600 x 14336 x 4096: 168 large tiles 97-99 us, 224 of these 75-78).  156 KiB of LDS
+// hold three stages, which a weight that comes from memory needs at this size of step (two stages: 82-83 us; a [K, N]
+// weight gains nothing over 192 x 256).
+using GemmRows160 = GemmShape<5, 4, 4, 2, 2, 3>;
+// 128 x 256, three stages: half the large tile as one workgroup instead of two of 128 x 128, a quarter fewer bytes copied per flop
+// (300 x 14336 x 4096 67 -> 58 us, [K, N] 900 x 8192 x 8192 142 -> 132, 1777 x 4096 x 4096 64 -> 61).
+using GemmFlat = GemmShape<4, 4, 4, 2, 2, 3>;
 constexpr int kRowTile = 8192;              // sub-tile [64 rows][64 k], 128-byte rows (A, and B as [N, K])
 constexpr int kColTile = 16384;             // sub-tile [64 k][128 n], 256-byte rows (B as [K, N])
 
@@ -165,13 +179,13 @@ MA_DEV int swz_row_tile(int row) { return (row >> 1) & 7; }        // 128-byte r
 MA_DEV int swz_col_tile(int row) { return ((row & 3) << 2) | ((row >> 2) & 2); }   // 256-byte rows, transposing reads of 4 rows x 32 bytes by each of two 16-lane groups 8 rows apart
 
 // CONCAT (with GROUPED, [N, K] weights whose widths are multiples of 64): the weights' columns are numbered through as
-// one wide matrix and tiled without regard to where one weight ends, so a tile may hold columns of two weights; every
+// one wide matrix (p.N columns) and tiled without regard to where one weight ends, so a tile may hold columns of two weights; every
 // 64-column sub-tile of the B panel and every 32-column block of a wave lies inside one weight, which is looked up
 // per copy instruction and per block (grp.end = cumulative column counts).
 template <class T, bool NT, class SH, bool GROUPED = false, bool SPLIT = false, bool CONCAT = false>
 __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const GemmParams p) {
     static_assert(!CONCAT || (GROUPED && NT && !SPLIT && SH::WAVES == 8), "CONCAT: grouped [N, K] weights, one sub-tile per copy index");
-    constexpr int kBM = SH::BM, kBN = SH::BN, NW = SH::WAVES, MB = SH::MB, NB = SH::NB, CA = SH::A_COPIES, CB = SH::B_COPIES;
+    constexpr int kBM = SH::BM, kBN = SH::BN, NW = SH::WAVES, CA = SH::A_COPIES, CB = SH::B_COPIES;
     constexpr int NS = SH::NS;
     static_assert(NS >= 2 && NS <= 4, "two to four stages");
     __shared__ __attribute__((aligned(1024))) char a_lds[NS][SH::A_PANEL];
@@ -179,7 +193,7 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
 
     const int lane = threadIdx.x & 63, w = wave_id();
     const int h = lane >> 5, l32 = lane & 31;
-    const int wm = w % SH::WAVES_M, wn = w / SH::WAVES_M;   // wave's place in the tile: rows 32*MB*wm .., columns 32*NB*wn ..
+    const int wm = w % SH::WAVES_M, wn = w / SH::WAVES_M;   // wave's place in the tile: rows 16*M16*wm .., columns 16*N16*wn ..
     static_assert(NT || SH::BN % 128 == 0, "a [K, N] weight is staged in sub-tiles of 128 columns");
 
     // ---- which tile ----------------------------------------------------------------------------------
@@ -221,7 +235,7 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
     const short* b_src[CONCAT ? CB : 1];   // CONCAT: first weight row of copy j's sub-tile (wave-uniform)
 #pragma unroll
     for (int j = 0; j < CA; ++j) {
-        const int q = j * NW + w;
+        const int q = j * NW + w < SH::A_PIECES ? j * NW + w : (j - 1) * NW + w;
         const int sub = q >> 3, row = 8 * (q & 7) + (lane >> 3), pg = lane & 7;
         const int m = min(m0 + 64 * sub + row, p.M - 1) - m0;
         a_off[j] = (uint32_t)((int64_t)m * p.lda + 8 * (pg ^ swz_row_tile(row))) * 2u;
@@ -233,7 +247,7 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
         if (CONCAT) {   // copy j of every wave lies in sub-tile j, whose 64 weight rows belong to one weight
             const int row = 8 * (q & 7) + (lane >> 3), pg = lane & 7;
             int local;
-            const int sg = group_of_unit(p.grp, n0 + 64 * j, local);
+            const int sg = group_of_unit(p.grp, min(n0 + 64 * j, p.N - 64), local);   // (past the last weight: its last columns)
             const int64_t ldj = sg == 0 ? p.grp.ldb[0] : sg == 1 ? p.grp.ldb[1] : p.grp.ldb[2];
             b_src[j] = (const short*)(sg == 0 ? p.grp.B[0] : sg == 1 ? p.grp.B[1] : p.grp.B[2]) + (int64_t)local * ldj;
             b_off[j] = (uint32_t)((int64_t)row * ldj + 8 * (pg ^ swz_row_tile(row))) * 2u;
@@ -280,7 +294,7 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
     // 32 values; a fragment is 16 rows x 32 k, lane (l16, quad) holding row l16, k = 8 quad + 0..7 of the slice: 16 bytes
     // at granule (4 slice + quad) ^ swizzle of the row.  A 16-row block is a quarter of a 64-row sub-tile; the swizzle of
     // row 16 b + l16 does not depend on b.
-    constexpr int M16 = 2 * MB, N16 = 2 * NB, BLK = kRowTile / 4;
+    constexpr int M16 = SH::M16, N16 = SH::N16, BLK = kRowTile / 4;
     const int l16 = lane & 15, quad = lane >> 4;
     constexpr int NRD = N16 < 4 ? 4 : N16;
     uint32_t m_rd[2], n_rd[NRD];
@@ -412,6 +426,7 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
         for (int nb = 0; nb < N16; ++nb) {
             int nb0 = n0 + 16 * N16 * wn + 16 * nb;   // first column of the block
             if (CONCAT) {                              // ... inside the weight that holds the block
+                if (nb0 >= p.N) continue;
                 int local;
                 const int sg = group_of_unit(p.grp, nb0, local);
                 nb0 = local;
@@ -1678,28 +1693,55 @@ static double rounds_cost(int64_t tiles) {
     const int64_t full = tiles / cus, rest = tiles % cus;
     return (double)full + (rest ? 0.55 + 0.45 * (double)rest / cus : 0.0);
 }
-// A 256 x 192 tile is 0.75 of a 256 x 256 one and runs 5 % below its rate per flop (8192 x 6144 x 4096: 366 against 347 us).
-static bool wide_shape_pays(int64_t big_tiles, int64_t wide_tiles) {
-    return 0.75 * 1.05 * rounds_cost(wide_tiles) < 0.97 * rounds_cost(big_tiles);
+// The tile shape whose rounds of the chip cost least.  A shape's factor is the time of a full round of it, in rounds of the
+// large tile, as measured at K = 4096 and 8192 with both layouts, f16 and bf16, from one round to 28 (its share of the work
+// divided by its rate): 256 x 192 0.75-0.83, 192 x 256 0.78-0.85, 160 x 256 0.68-0.75, 128 x 256 0.57-0.61, two 128 x 128 on a
+// compute unit 0.58-0.65, one with three stages 0.41.  The large tile wins ties.
+enum class Tile { Big, Wide, Rows192, Rows160, Flat, Small, Small3 };
+static int64_t tile_count(int64_t M, int64_t N, int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
+template <bool NT>
+static Tile pick_tile(int64_t M, int64_t N, int64_t big_tiles, int64_t small_tiles) {
+    Tile best = Tile::Big;
+    double cost = rounds_cost(big_tiles);
+    auto consider = [&](Tile t, double c) { if (c < cost) { cost = c; best = t; } };
+    if (NT) {
+        consider(Tile::Wide, 0.81 * rounds_cost(tile_count(M, N, GemmWide::BM, GemmWide::BN)));
+        consider(Tile::Rows160, 0.73 * rounds_cost(tile_count(M, N, GemmRows160::BM, GemmRows160::BN)));
+    } else {
+        consider(Tile::Rows192, 0.81 * rounds_cost(tile_count(M, N, GemmRows192::BM, GemmRows192::BN)));
+    }
+    consider(Tile::Flat, 0.60 * rounds_cost(tile_count(M, N, GemmFlat::BM, GemmFlat::BN)));
+    if (one_workgroup_per_unit(small_tiles)) consider(Tile::Small3, 0.41 * rounds_cost(small_tiles));
+    else consider(Tile::Small, 0.64 * rounds_cost((small_tiles + 1) / 2));
+    return best;
 }
 
 template <class T, bool NT>
 static int launch_gemm(GemmParams& p, bool fast, hipStream_t stream) {
     if (fast) {
-        // large tiles halve the LDS and L2 traffic per flop; they are worth it once they fill most of the chip
-        const int64_t big_tiles = (int64_t)((p.M + GemmBig::BM - 1) / GemmBig::BM) * ((p.N + GemmBig::BN - 1) / GemmBig::BN);
-        if constexpr (NT) {
-            if (big_tiles >= 160 && p.N % GemmWide::BN == 0 &&
-                wide_shape_pays(big_tiles, (int64_t)((p.M + GemmWide::BM - 1) / GemmWide::BM) * (p.N / GemmWide::BN)))
-                return launch_tiled<T, NT, GemmWide>(p, stream);
+        switch (pick_tile<NT>(p.M, p.N, tile_count(p.M, p.N, GemmBig::BM, GemmBig::BN), tile_count(p.M, p.N, GemmSmall::BM, GemmSmall::BN))) {
+        case Tile::Big: return launch_tiled<T, NT, GemmBig>(p, stream);
+        case Tile::Wide: if constexpr (NT) return launch_tiled<T, NT, GemmWide>(p, stream); break;
+        case Tile::Rows160: if constexpr (NT) return launch_tiled<T, NT, GemmRows160>(p, stream); break;
+        case Tile::Rows192: if constexpr (!NT) return launch_tiled<T, NT, GemmRows192>(p, stream); break;
+        case Tile::Flat: return launch_tiled<T, NT, GemmFlat>(p, stream);
+        case Tile::Small: return launch_tiled<T, NT, GemmSmall>(p, stream);
+        case Tile::Small3: return launch_tiled<T, NT, GemmSmall3>(p, stream);
         }
-        if (big_tiles >= 160) return launch_tiled<T, NT, GemmBig>(p, stream);
-        const int64_t small_tiles = (int64_t)((p.M + GemmSmall::BM - 1) / GemmSmall::BM) * ((p.N + GemmSmall::BN - 1) / GemmSmall::BN);
-        return one_workgroup_per_unit(small_tiles) ? launch_tiled<T, NT, GemmSmall3>(p, stream) : launch_tiled<T, NT, GemmSmall>(p, stream);
     }
     const int grid = (int)std::min<int64_t>(((int64_t)p.M * p.N + 255) / 256, 256 * 16);
     hipLaunchKernelGGL((gemm_plain_kernel<T, NT>), dim3(grid), dim3(256), 0, stream, p);
     return check_launch("gemm_plain_kernel");
+}
+
+// [N, K] weights numbered through as one of p.N columns; p.grp.end = cumulative column counts
+template <class T, class SH>
+static int launch_concat(GemmParams& p, hipStream_t stream) {
+    p.tiles_m = (p.M + SH::BM - 1) / SH::BM;
+    p.tiles_n = (p.N + SH::BN - 1) / SH::BN;
+    p.per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
+    hipLaunchKernelGGL((gemm_kernel<T, true, SH, true, false, true>), dim3(p.per_xcd * 8), dim3(SH::WAVES * 64), 0, stream, p);
+    return check_launch("gemm_kernel (grouped, columns numbered through)");
 }
 
 // Up to three weights [N_s, K] against one A in one launch (alpha = 1, no C): the tiled kernel over the concatenated
@@ -1755,27 +1797,26 @@ static int launch_grouped(GemmParams& p, int n_w, hipStream_t stream) {
 #undef MINFER_SKINNY
         return check_launch("gemm_skinny_kernel (grouped)");
     }
-    int64_t big_tiles = 0;
-    for (int s = 0; s < n_w; ++s) big_tiles += (int64_t)((p.M + GemmBig::BM - 1) / GemmBig::BM) * ((p.grp.N[s] + GemmBig::BN - 1) / GemmBig::BN);
-    const bool big = big_tiles >= 160;
-    // 256 x 192 tiles over the weights' columns numbered through, when that fills the chip's rounds better (the Llama-3-8B
-    // QKV projection of 4096 tokens: 384 large tiles, one and a half rounds, or 512 of these, two rounds of 3/4 the work)
-    bool concat = big && n_sum % GemmWide::BN == 0 && n_sum < (INT64_C(1) << 31);
-    for (int s = 0; s < n_w; ++s) concat = concat && p.grp.N[s] % 64 == 0;
-    if (concat) {
-        const int64_t wide_tiles = (int64_t)((p.M + GemmWide::BM - 1) / GemmWide::BM) * (n_sum / GemmWide::BN);
-        concat = wide_shape_pays(big_tiles, wide_tiles);
+    int64_t big_tiles = 0, small_tiles = 0;
+    bool concat = n_sum < (INT64_C(1) << 31);
+    for (int s = 0; s < n_w; ++s) {
+        big_tiles += tile_count(p.M, p.grp.N[s], GemmBig::BM, GemmBig::BN);
+        small_tiles += tile_count(p.M, p.grp.N[s], GemmSmall::BM, GemmSmall::BN);
+        concat = concat && p.grp.N[s] % 64 == 0;
     }
+    // the sizes in between over the weights' columns numbered through, when they fill the chip's rounds better (the Llama-3-8B
+    // QKV projection of 4096 tokens: 384 large tiles, one and a half rounds, or 512 of 256 x 192, two rounds of 3/4 the work)
+    Tile tile = big_tiles >= 160 ? Tile::Big : Tile::Small;
     if (concat) {
+        tile = pick_tile<true>(p.M, n_sum, big_tiles, small_tiles);
         int acc = 0;
         for (int s = 0; s < kMaxGroup; ++s) { if (s < n_w) acc += p.grp.N[s]; p.grp.end[s] = acc; }
-        p.N = (int)n_sum;
-        p.tiles_m = (p.M + GemmWide::BM - 1) / GemmWide::BM;
-        p.tiles_n = (int)(n_sum / GemmWide::BN);
-        p.per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
-        hipLaunchKernelGGL((gemm_kernel<T, true, GemmWide, true, false, true>), dim3(p.per_xcd * 8), dim3(GemmWide::WAVES * 64), 0, stream, p);
-        return check_launch("gemm_kernel (grouped, columns numbered through)");
+        if (tile == Tile::Wide || tile == Tile::Rows160 || tile == Tile::Flat) p.N = (int)n_sum;
+        if (tile == Tile::Wide) return launch_concat<T, GemmWide>(p, stream);
+        if (tile == Tile::Rows160) return launch_concat<T, GemmRows160>(p, stream);
+        if (tile == Tile::Flat) return launch_concat<T, GemmFlat>(p, stream);
     }
+    const bool big = tile == Tile::Big;
     const int bm = big ? GemmBig::BM : GemmSmall::BM, bn = big ? GemmBig::BN : GemmSmall::BN;
     p.tiles_m = (p.M + bm - 1) / bm;
     p.tiles_n = fill_ends(bn);

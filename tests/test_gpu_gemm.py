@@ -112,6 +112,28 @@ def test_gemm_matches_oracle(layout, dtype, M, N, K, alpha, beta):
         assert float((d.float() - ref).abs().max()) <= 2.0 ** -MANT[dtype] * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout,M,N,K,alpha,beta", [
+    (NK, 593, 14344, 64, 1.0, 0.0),      # 160 x 256: one K step of the three stages, a ragged last tile row and column
+    (NK, 470, 16392, 256, 2.0, 3.0),     # four steps
+    (NK, 900, 8200, 320, 1.0, 1.0),      # five steps
+    (NK, 1003, 8200, 192, 2.0, 3.0),     # 256 x 192 over a width that is no multiple of 192
+    (NK, 385, 8200, 128, 1.0, 1.0),      # 128 x 256: two steps; a last tile row of one row
+    (NK, 130, 16392, 448, 2.0, 3.0),
+    (KN, 385, 8200, 192, 1.0, 0.0),
+    (KN, 257, 12296, 64, 2.0, 3.0),
+    (KN, 520, 14344, 64, 1.0, 1.0),      # 192 x 256
+    (KN, 385, 16392, 320, 2.0, 3.0),     # a last tile row of one row, an odd number of steps
+])
+def test_gemm_tiles_between_the_small_and_the_large_one(layout, dtype, M, N, K, alpha, beta):
+    """Every element against torch's product in 64 bits, within the bound of assert_close."""
+    a, b, c = make(M, N, K, layout, dtype, M + N + K)
+    d = torch.full((M, N), float("nan"), dtype=dtype, device=DEV)
+    assert capi.gemm(a.to(DEV), b.to(DEV), c.to(DEV), d, alpha, beta, layout) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    assert_close(d, (alpha * (a.double() @ (b if layout == KN else b.T).double()) + beta * c.double()).numpy(), dtype)
+
+
 def test_gemm_golden_strided_and_in_place():
     z = np.load(os.path.join(os.path.dirname(__file__), "golden", "gemm_small.npz"))
     a, b, c = (torch.from_numpy(z[k]).to(DEV) for k in "abc")
@@ -162,6 +184,9 @@ def test_gemm_op_reference_test_recipe(kerns, S, alpha, beta):
     (4096, 128, 4096, 2048, 2048),     # 8192 columns: no multiple of 192, 256 x 256 tiles per weight
     (512, 6144, 6144, 1024, 1024),     # the reference test's head shape at a smaller batch: 128 x 128 tiles
     (300, 256, 200, 72, 136),          # ragged rows, widths that end inside a tile
+    (593, 128, 12288, 1024, 1088),     # 160 x 256 tiles over the columns numbered through, the last one past the third weight's end
+    (300, 320, 12288, 1024, 1088),     # 128 x 256 ones
+    (1003, 64, 8192, 1024, 1088),      # 256 x 192 ones
     (1, 4096, 4096, 1024, 1024),       # a decode step: whole weight rows per wave, the three weights' rows numbered through
     (1, 8192, 1032, 8, 520),           # the same with the activations in LDS and runs of rows that cross from one weight to the next
     (2, 4096, 4096, 1024, 1024),       # up to 16 rows, K a multiple of 512: the LDS-staged few-row kernel over the three weights' column groups
