@@ -862,12 +862,14 @@ __global__ __launch_bounds__(kChunkWaves * 64) void decode_merge_kernel(const Ch
     if (n > 1) merge_chunks<T, D>(c, b, g * p.n_rep + hg * 16, min(16, p.n_rep - hg * 16), n, ml_s, inv_s);
 }
 
-// Smallest share of the work a workgroup takes, in cache rows: 256, or more for very long caches, so that a
-// (sequence, head) never has more than 64 partial results, which is what one wave of the combine kernel merges.
+// Smallest share of the line a wave takes, in cache rows: 128, or more for very long caches, so that a (sequence, head) never
+// has more than 64 partial results, which is what one wave of the combine kernel merges.  (With 256 a line of 128 to 256 rows
+// a wave left up to half of the waves idle: 40 sequences of 1101 rows over 8 KV heads, Q8_0 31.7 -> 29.5 us, fp16 39.9 -> 36.8;
+// 136 pairs to 4382 39.5 -> 33.7; longer and shorter ones as before.)
 static int decode_min_share_rows(int64_t Lmax) {
     int64_t c = (Lmax + 59) / 60;
     c = (c + 63) / 64 * 64;
-    return (int)(c > 256 ? c : 256);
+    return (int)(c > 128 ? c : 128);
 }
 // Partial results a (sequence, head) can have: a pair's rows overlap at most this many shares.
 static int decode_slots(int64_t Lmax) { return (int)(Lmax / decode_min_share_rows(Lmax)) + 3; }
@@ -904,8 +906,14 @@ static int decode_workgroups() {
 //     quarters of the units: 22.0 / 25.5)
 //   longer ones that occupy 9 of 10 units, four to a pair or more: 32 pairs of 30000 85.5 / 77.4, 40 to 16000 49.5 / 40.9
 //     (three to a pair: 72 to 16000 56.9 / 65.5; two: 120 to 8000 50.4 / 53.8)
-//   short ones in two rounds: 512 pairs to 300 25.9 / 14.9, 400 to 800 24.4 / 21.7 (320 of 1100, Q8_0: 31.6 / 33.7)
-static int decode_chunk_rows(const DecodeParams& p) {
+//   more pairs than units, a workgroup per context (what is in flight on a unit does not change with the rounds):
+//     head_dim 64, 16-bit caches, any number of pairs to 1536: 512 of 1000 28.6 / 21.7, 1024 to 1000 30.3 / 27.6, 320 to
+//       1400 19.1 / 18.0 (320 to 3000 30.7 / 35.1)
+//     head_dim 128, 16-bit, up to two rounds: 512 to 300 25.9 / 14.2, 400 to 800 25.9 / 22.9, and to 1536 where the rounds come
+//       out full: 512 of 1000 49.4 / 43.7, to 1400 41.3 / 39.9 (320 of 1400 43.5 / 45.8; 768 to 1000 41.3 / 42.7)
+//     Q8_0, up to two rounds, where a context is a group or two per wave: head_dim 128 to 512, 512 to 300 18.7 / 15.4, 400 of 450
+//       23.5 / 19.3 (320 of 600 21.9 / 23.7); head_dim 64 to 896 (512 to 1400 19.8 / 21.2)
+static int decode_chunk_rows(const DecodeParams& p, int D, bool q8) {
     const int64_t pairs = (int64_t)p.B * p.Hkv * p.n_hg, units = decode_workgroups() / kDecodeWgPerCu;
     const int64_t unit_rows = kChunkWaves * p.group_rows;
     int64_t n = units / pairs;
@@ -915,7 +923,11 @@ static int decode_chunk_rows(const DecodeParams& p) {
     chunk = chunk < 256 ? 256 : (chunk + unit_rows - 1) / unit_rows * unit_rows;
     n = p.Lmax > 0 ? (p.Lmax + chunk - 1) / chunk : 1;
     if (pairs > kStreamCounters || chunk > (1 << 24)) return 0;
-    if (pairs * n > units) return pairs * n <= 2 * units && chunk <= 896 ? (int)chunk : 0;
+    if (pairs * n > units) {
+        const bool any_rounds = D == 64 && !q8, full_rounds = 10 * pairs * n >= 9 * 2 * units;
+        const int64_t longest = q8 ? (D == 64 ? 896 : 512) : (any_rounds || full_rounds ? 1536 : 896);
+        return (any_rounds || pairs * n <= 2 * units) && chunk <= longest ? (int)chunk : 0;
+    }
     const bool full = 10 * pairs * n >= 9 * units;
     return chunk <= 1536 || (full && (chunk <= 2048 || n >= 4)) ? (int)chunk : 0;
 }
@@ -933,7 +945,7 @@ static int launch_chunks(const DecodeParams& p, int chunk, void* out, int64_t o0
 
 template <class T, int D>
 static int launch_decode(const DecodeParams& p, void* out, int64_t o0, int64_t o1, hipStream_t stream) {
-    if (const int chunk = decode_chunk_rows(p)) return launch_chunks<T, D, false>(p, chunk, out, o0, o1, stream);
+    if (const int chunk = decode_chunk_rows(p, D, false)) return launch_chunks<T, D, false>(p, chunk, out, o0, o1, stream);
     hipLaunchKernelGGL((decode_split_kernel<T, D>), dim3((unsigned)p.n_wg), dim3(kDecodeWaves * 64), 0, stream, p);
     if (int rc = check_launch("decode_split_kernel")) return rc;
     hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((p.B * p.Hq + 3) / 4), dim3(256), 0, stream, p, out, o0, o1);
@@ -942,7 +954,7 @@ static int launch_decode(const DecodeParams& p, void* out, int64_t o0, int64_t o
 
 template <int D>
 static int launch_decode_q8(const DecodeParams& p, void* out, int64_t o0, int64_t o1, hipStream_t stream) {
-    if (const int chunk = decode_chunk_rows(p)) return launch_chunks<F16, D, true>(p, chunk, out, o0, o1, stream);
+    if (const int chunk = decode_chunk_rows(p, D, true)) return launch_chunks<F16, D, true>(p, chunk, out, o0, o1, stream);
     hipLaunchKernelGGL((decode_split_q8_kernel<D>), dim3((unsigned)p.n_wg), dim3(kDecodeWaves * 64), 0, stream, p);
     if (int rc = check_launch("decode_split_q8_kernel")) return rc;
     hipLaunchKernelGGL((decode_combine_kernel<F16, D>), dim3((p.B * p.Hq + 3) / 4), dim3(256), 0, stream, p, out, o0, o1);

@@ -163,6 +163,34 @@ def test_decode_chunks(Hq, Hkv, Lmax, D):
         assert torch.equal(out, outs[0])
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Lmax,D,q8", [
+    (33, 16, 8, 1536, 64, False),    # a workgroup per context, one round and a bit
+    (33, 16, 16, 300, 64, False),    # more than two rounds
+    (33, 16, 8, 890, 128, False),
+    (60, 8, 8, 1500, 128, False),    # two rounds that come out full
+    (33, 16, 8, 512, 128, True),
+    (33, 16, 8, 760, 64, True),
+    (33, 16, 8, 1537, 64, False),    # past those limits: the line of equal shares
+    (40, 16, 8, 1101, 128, True),    # ... its shares between 128 and 256 rows
+    (40, 16, 8, 1101, 128, False),
+])
+def test_decode_more_contexts_than_units(B, Hq, Hkv, Lmax, D, q8):
+    """Contexts from nothing to the capacity, around a group's and a wave's edges, against the oracle.  Tolerance: that of every
+    fp16 attention result here."""
+    lens = [Lmax, 0, 1, 16, 31, 33, 127, 129, 255, 257, Lmax - 1, Lmax // 2 + 1]
+    q, kc, vc, _ = workloads.decode_cache(seed=B + Lmax, device=DEV, B=B, Hq=Hq, Hkv=Hkv, Lmax=Lmax, D=D, ctx_lo=1, ctx_hi=1)
+    ctx = torch.tensor([lens[i % len(lens)] for i in range(B)], dtype=torch.int32, device=DEV)
+    out = torch.full(q.shape, float("nan"), dtype=q.dtype, device=DEV)
+    if q8:
+        kc, vc = workloads.q8_0_rows(kc), workloads.q8_0_rows(vc)
+        assert capi.flash_attn_decode_q8_0(q, kc, vc, ctx, out) == capi.OK, capi.last_error()
+        want = oracle.flash_attn_decode_q8_0(q.cpu(), kc.cpu(), vc.cpu(), ctx.cpu())
+    else:
+        assert capi.flash_attn_decode(q, kc, vc, ctx, out) == capi.OK, capi.last_error()
+        want = oracle.flash_attn_decode(q, kc, vc, ctx)
+    assert max_err(out, want) <= TOL[torch.float16]
+
+
 @pytest.mark.parametrize("offset", [0, 5])
 @pytest.mark.parametrize("B,L,D", [(2, 1, 64), (3, 2, 128), (2, 3, 64), (2, 4, 128), (2, 5, 64), (2, 15, 128), (2, 16, 64), (3, 17, 128),
                                    (2, 63, 64), (2, 65, 128), (1, 129, 128), (2, 255, 64), (1, 1023, 64), (1, 1025, 128), (1, 1103, 64)])
