@@ -771,9 +771,21 @@ static int dispatch_prefill(int dtype, int64_t D, const PrefillParams& p, int wa
 // (clocks settled, 4 / 8 waves: B=8 L=1024 54.6 / 65.2 us, B=4 L=2048 88 / 102, B=1 L=8192 292 / 330, L=16384 1113 / 1267;
 // head_dim 128 for comparison: L=1536 180 / 182, L=2048 151.5 / 149.6, L=4096 143.7 / 134.4, L=8192 506 / 494).
 constexpr int64_t kSmallWorkgroupMaxRows = 1024;
-static int prefill_waves(int64_t longest, int64_t D) {
+// A launch of few workgroups of 8 waves ends with its longest one, on a chip that is half idle by then (under a causal mask a
+// workgroup has half of the longest one's tiles on average): up to one and a half of them per compute unit the small ones, which
+// share out in finer pieces, are ahead (4 / 8 waves, 32 heads over 8: L=1536 39.2 / 46.7 us, 1777 47.6 / 55.3, 3000 86.0 / 90.9,
+// 3500 107.6 / 106.7; 8 over 2: L=2048 44.9 / 57.2, 4096 84.2 / 106.2, B=2 L=8192 275 / 267).  A packed batch is counted by its
+// tokens and has short sequences' workgroups between, so up to one and a quarter (4 sequences to 1600 30.3 / 32.2, 2 of 64
+// heads over 8 27.4 / 26.7); heads that share K and V with no other head make 256-row workgroups of a sequence, whose
+// waves wait for the diagonal's: there up to 1536 rows (32 sequences to 1200, 24 over 8 145 / 159, 16 to 1600 118 / 121).
+static int prefill_waves(int64_t longest, int64_t D, int64_t big_workgroups, int64_t few, bool heads_share) {
     if (MINFER_PREFILL_FORCE_WAVES) return MINFER_PREFILL_FORCE_WAVES;
-    return (D == 64 || longest <= kSmallWorkgroupMaxRows) ? kWavesSmall : kWavesBig;
+    if (D == 64 || longest <= kSmallWorkgroupMaxRows || big_workgroups <= few) return kWavesSmall;
+    return !heads_share && longest <= kSmallWorkgroupMaxRows * 3 / 2 ? kWavesSmall : kWavesBig;
+}
+// log2 of the query heads of one GQA group that a workgroup takes
+static int heads_per_workgroup_log2(int64_t n_rep, int waves) {
+    return n_rep % 8 == 0 && waves >= 8 ? 3 : (n_rep % 4 == 0 ? 2 : (n_rep % 2 == 0 ? 1 : 0));
 }
 
 // The global->LDS copies of K/V tiles and query rows and the output stores address a block's rows with a 32-bit unsigned
@@ -794,7 +806,7 @@ static void fill_common(PrefillParams& p, const void* q, const void* k, const vo
     p.kv0 = st->kv0; p.kv1 = st->kv1; p.kv2 = st->kv2;
     p.o0 = st->o0; p.o1 = st->o1; p.o2 = st->o2;
     p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.n_rep = (int)(Hq / Hkv);
-    p.hpw_log2 = (p.n_rep % 8 == 0 && kWaves >= 8) ? 3 : (p.n_rep % 4 == 0) ? 2 : ((p.n_rep % 2 == 0) ? 1 : 0);
+    p.hpw_log2 = heads_per_workgroup_log2(p.n_rep, kWaves);
     p.n_hg = p.n_rep >> p.hpw_log2;
     p.scale_log2 = (float)(1.4426950408889634 / sqrt((double)D));
 }
@@ -825,7 +837,9 @@ MINFER_ATTN_EXPORT int minfer_flash_attn(int dtype, const void* q, const void* k
     hipStream_t stream = (hipStream_t)stream_v;
 
     PrefillParams p{};
-    const int kWaves = prefill_waves(L, D);
+    const int big_log2 = heads_per_workgroup_log2(Hq / Hkv, kWavesBig);
+    const int64_t big_rows = 32 * (kWavesBig >> big_log2);
+    const int kWaves = prefill_waves(L, D, (L + big_rows - 1) / big_rows * B * (Hq >> big_log2), 384, true);
     fill_common(p, q, k, v, out, Hq, Hkv, D, st, kWaves);
     p.mask = mask; p.cls = (const uint8_t*)workspace; p.cu = nullptr;
     p.L = (int)L; p.B = (int)B;
@@ -866,7 +880,7 @@ MINFER_ATTN_EXPORT int minfer_flash_attn_varlen(int dtype, const void* q, const 
     // must be at least the longest sequence (as in every varlen attention interface).
     const int64_t max_len = (max_seqlen > 0 && max_seqlen < T) ? max_seqlen : T;
     PrefillParams p{};
-    const int kWaves = prefill_waves(max_len, D);
+    const int kWaves = prefill_waves(max_len, D, T * Hq / (32 * kWavesBig), 320, Hq / Hkv % 2 == 0);
     fill_common(p, q, k, v, out, Hq, Hkv, D, st, kWaves);
     p.mask = nullptr; p.cls = nullptr; p.cu = cu_seqlens;
     p.L = (int)T; p.B = 1;
