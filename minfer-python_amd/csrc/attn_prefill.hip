@@ -177,8 +177,12 @@ template <int D, int NW> struct TileGeom {
     static MA_DEV int swz_v(int row) { return D == 128 ? ((row & 7) << 1) : (((row >> 1) & 3) << 1); }
 };
 
-template <class T, int D, int MODE, int NW>
-__global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams p) {
+// TEAMS = 2: two teams of NW waves hold the same query rows and take the even and the odd key tiles of the list, each with stages
+// of its own; the second team's sums go to the first through LDS.  A launch of few workgroups ends with its longest one, whose
+// tiles run one after the other: this halves them.
+template <class T, int D, int MODE, int NW, int TEAMS = 1>
+__global__ __launch_bounds__(NW * TEAMS * 64, 2) void prefill_kernel(const PrefillParams p) {
+    static_assert(TEAMS == 1 || NW == 4, "the teams' stages and the 32 rows of NW waves fill the LDS");
     using GEO = TileGeom<D, NW>;
     constexpr int RB = GEO::RB, G = GEO::G, RPI = GEO::RPI, NLD = GEO::NLD;
     constexpr int KC = D / 32;   // 32-wide contraction chunks of Q K^T
@@ -187,7 +191,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
     constexpr int STAGE_BYTES = 2 * GEO::TILE_BYTES;   // a stage = the K tile followed by the V tile
     constexpr int ROWS_BYTES = 32 * RB;                // a wave's 32 query (or output) rows
 
-    __shared__ __attribute__((aligned(1024))) char kv_lds[2][STAGE_BYTES];
+    __shared__ __attribute__((aligned(1024))) char kv_lds_all[TEAMS][2][STAGE_BYTES];
     constexpr bool kDense = MODE != MODE_VARLEN;
     __shared__ uint32_t tile_list[MODE == MODE_DENSE ? kMaxKeyTiles : (MODE == MODE_DENSE_SELF ? kSelfClassifyMaxL / 64 : 1)];
     __shared__ int n_active_s;
@@ -200,7 +204,9 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
     constexpr bool kAliasRows = NW * ROWS_BYTES <= STAGE_BYTES;
     __shared__ __attribute__((aligned(1024))) char q_lds_own[kAliasRows ? 1 : NW][kAliasRows ? 16 : ROWS_BYTES];
 
-    const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    const int w = TEAMS == 1 ? wave : wave & (NW - 1), team = TEAMS == 1 ? 0 : wave / NW;   // wave of the team
+    char (&kv_lds)[2][STAGE_BYTES] = kv_lds_all[team];
     const int l16 = lane & 15, quad = lane >> 4;
     const int HPW = 1 << p.hpw_log2, QBW = kWaves >> p.hpw_log2;  // heads, 32-row query blocks per workgroup
     char* const q_stage = kAliasRows ? &kv_lds[1][w * ROWS_BYTES] : &q_lds_own[kAliasRows ? 0 : w][0];
@@ -327,7 +333,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
         all_acc &= quad_swap<1>(all_acc); all_acc &= quad_swap<2>(all_acc);
         if ((lane & 3) == 0) { any_s[w][lane >> 2] = any_acc; all_s[w][lane >> 2] = all_acc; }
         __syncthreads();
-        if (w == 0) {
+        if (wave == 0) {
             const int kt = lane;
             uint32_t c = 0;
             if (kt < p.NKT) {
@@ -344,7 +350,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
         __syncthreads();
         n_active = n_active_s;
     } else if (MODE == MODE_DENSE) {
-        if (w == 0) {
+        if (wave == 0) {
             int cnt = 0;
             for (int base = 0; base < p.NKT; base += 64) {
                 const int kt = base + lane;
@@ -387,7 +393,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
     // In this one instantiation the compiler (out of scalar registers) keeps the row bases in vector registers and moves
     // them to scalar ones right in front of every copy, closer than a copy may follow such a move (copy16_global_to_lds);
     // the build's scan of the generated code is what says which instantiations need this.
-    constexpr bool kFreshBases = MODE == MODE_VARLEN && NW == 4 && D == 128;
+    constexpr bool kFreshBases = TEAMS > 1 || (MODE == MODE_VARLEN && NW == 4 && D == 128);
     auto issue_tile = [&](int kt, int stage) {
         const int key0 = kt * 64;
         const short* kbase = Kh + (int64_t)key0 * p.kv2;
@@ -452,14 +458,14 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
             kt = (int)(e & 0xffffu);
             cls_w = (e >> (16 + 2 * my_qt64_slot)) & 3u;
         } else {
-            kt = it;
+            kt = TEAMS * it + team;
             cls_w = (64 * kt + 63 <= q_row0) ? TILE_ALL : ((64 * kt > q_row0 + 31) ? TILE_NONE : TILE_MIXED);
         }
         if (!wave_on) cls_w = TILE_NONE;
     };
     auto list_entry = [&](int it) -> uint32_t {   // wave-uniform
         if (!kDense || n_active <= 0) return 0u;
-        return __builtin_amdgcn_readfirstlane(tile_list[min(it, n_active - 1)]);
+        return __builtin_amdgcn_readfirstlane(tile_list[min(TEAMS * it + team, n_active - 1)]);
     };
     // mask words of a MIXED dense tile: word [qb][kb] covers keys key0 + 16kb + 4 quad + 0..3 of query row qrow[qb]
     uint32_t mw[2][4] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
@@ -635,9 +641,10 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
 
     // ---- main loop: one barrier per tile; the copy of tile t+1 is issued right after the barrier that
     // opens tile t, into the stage tile t-1 has just vacated ---------------------------------------
+    const int n_own = (n_active - team + TEAMS - 1) / TEAMS, n_it = (n_active + TEAMS - 1) / TEAMS;   // the team's tiles, the longer team's
     uint32_t e_cur = list_entry(0), e_next = list_entry(1);
     int kt_first = 0; uint32_t cls_first = TILE_NONE;
-    if (n_active > 0) {
+    if (n_own > 0) {
         tile_of(e_cur, 0, kt_first, cls_first);
         issue_tile(kt_first, 0);
     }
@@ -646,7 +653,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
     // the base-2 exponent of the softmax weight (minus the running reference it is initialised with).
     // The rows were requested before the tile list was built, and the first K/V tile after them: copies retire in
     // order, so the rows have landed once no more than that tile's copies are outstanding.
-    if (n_active > 0) wait_vmcnt<2 * NLD>(); else wait_vmcnt<0>();
+    if (n_own > 0) wait_vmcnt<2 * NLD>(); else wait_vmcnt<0>();
     {
         const uint32_t qa = lds_addr(q_stage) + l16 * RB;
         const int sw = GEO::swz_k(l16);   // the same for row 16 + l16
@@ -655,7 +662,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
 #pragma unroll
             for (int c = 0; c < KC; ++c) qf[qb][c] = T::scale8(lds_read_b128(qa + 16 * ((4 * c + quad) ^ sw), 16 * qb * RB), c2);
     }
-    if (kDense && n_active > 0 && cls_first == TILE_MIXED) fetch_mask(kt_first);
+    if (kDense && n_own > 0 && cls_first == TILE_MIXED) fetch_mask(kt_first);
     auto iteration = [&](auto stage_tag, int it) {
         constexpr int STAGE = decltype(stage_tag)::value;
         int kt, ktn; uint32_t cls_w, cn;
@@ -664,20 +671,45 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
         const uint32_t e_after = list_entry(it + 2);   // read early, used next iteration
         wait_vmcnt<0>();       // this wave's share of tile `it` (and its mask words) has landed
         __syncthreads();       // everyone's has; stage STAGE^1 is no longer being read
-        if (it + 1 < n_active) issue_tile(ktn, STAGE ^ 1);
+        if (it + 1 < n_own) issue_tile(ktn, STAGE ^ 1);
         // The next tile's mask words are requested after this tile's were used; with 4 waves already in front of a tile that
         // uses none (a short problem's few tiles wait for everything they request late: L=256 9.0 -> 8.6 us; with 8 waves the
         // second copy of the requests costs as much as it gives, S=4096 134.4 -> 135.7).
-        const bool fetch = kDense && it + 1 < n_active && cn == TILE_MIXED;
+        const bool fetch = kDense && it + 1 < n_own && cn == TILE_MIXED;
         const bool early = NW == kWavesSmall && cls_w != TILE_MIXED;
         if (fetch && early) fetch_mask(ktn);
-        if (cls_w != TILE_NONE) process_tile(stage_tag, kt, cls_w);
+        if (cls_w != TILE_NONE && (TEAMS == 1 || it < n_own)) process_tile(stage_tag, kt, cls_w);
         if (fetch && !early) fetch_mask(ktn);
         e_cur = e_next; e_next = e_after;
     };
-    for (int it = 0; it < n_active; it += 2) {
+    for (int it = 0; it < n_it; it += 2) {
         iteration(std::integral_constant<int, 0>{}, it);
-        if (it + 1 < n_active) iteration(std::integral_constant<int, 1>{}, it + 1);
+        if (it + 1 < n_it) iteration(std::integral_constant<int, 1>{}, it + 1);
+    }
+    if constexpr (TEAMS > 1) {
+        // the second team's output blocks, references and denominators through its own stages, lane by lane
+        static_assert(NW * DB * 2 * 1024 <= 2 * STAGE_BYTES, "16 bytes per lane and block");
+        __shared__ f32x4 ml_s[NW][64];
+        f32x4* const o_s = reinterpret_cast<f32x4*>(&kv_lds_all[1][0][0]) + w * DB * 2 * 64 + lane;
+        __syncthreads();   // its last tile has been read
+        if (team == 1) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int qb = 0; qb < 2; ++qb) o_s[(2 * db + qb) * 64] = o_acc[db][qb];
+            ml_s[w][lane] = f32x4{m_ref[0], m_ref[1], l_sum[0], l_sum[1]};
+        }
+        __syncthreads();
+        if (team == 1) return;
+        const f32x4 ml = ml_s[w][lane];
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+            const float m = fmaxf(m_ref[qb], ml[qb]);   // a team that has seen no key has sums of zero
+            const float a0 = m_ref[qb] == -INFINITY ? 0.f : fast_exp2(m_ref[qb] - m), a1 = ml[qb] == -INFINITY ? 0.f : fast_exp2(ml[qb] - m);
+            l_sum[qb] = l_sum[qb] * a0 + ml[2 + qb] * a1;
+#pragma unroll
+            for (int db = 0; db < DB; ++db) o_acc[db][qb] = o_acc[db][qb] * a0 + o_s[(2 * db + qb) * 64] * a1;
+        }
     }
 
     // ---- epilogue: normalise, transpose through the wave's staging area, store whole rows ---------------
@@ -693,7 +725,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_kernel(const PrefillParams
         inv[qb] = l > 0.f ? 1.f / l : 0.f;
     }
     {
-        const int free_stage = (n_active & 1);   // the last tile sat in stage (n_active - 1) & 1
+        const int free_stage = n_it & 1;   // the last tile sat in stage (n_it - 1) & 1
         const uint32_t so = kAliasRows ? lds_addr(&kv_lds[0][0]) + free_stage * STAGE_BYTES + w * ROWS_BYTES : lds_addr(q_stage);
         typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
         typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
@@ -738,22 +770,33 @@ static size_t cls_bytes(int64_t B, int64_t L) {
     return (size_t)(B * nt * nt + 255) / 256 * 256;
 }
 
-template <class T, int D, int MODE, int NW>
+template <class T, int D, int MODE, int NW, int TEAMS>
 static int launch_prefill(const PrefillParams& p, int grid, hipStream_t stream) {
-    hipLaunchKernelGGL((prefill_kernel<T, D, MODE, NW>), dim3(grid), dim3(NW * 64), 0, stream, p);
+    hipLaunchKernelGGL((prefill_kernel<T, D, MODE, NW, TEAMS>), dim3(grid), dim3(NW * TEAMS * 64), 0, stream, p);
     return check_launch("prefill_kernel");
 }
 
-template <int MODE, int NW>
+template <int MODE, int NW, int TEAMS = 1>
 static int dispatch_prefill_nw(int dtype, int64_t D, const PrefillParams& p, int grid, hipStream_t stream) {
     if (dtype == MINFER_ATTN_F16) {
-        return D == 128 ? launch_prefill<F16, 128, MODE, NW>(p, grid, stream) : launch_prefill<F16, 64, MODE, NW>(p, grid, stream);
+        return D == 128 ? launch_prefill<F16, 128, MODE, NW, TEAMS>(p, grid, stream) : launch_prefill<F16, 64, MODE, NW, TEAMS>(p, grid, stream);
     }
-    return D == 128 ? launch_prefill<BF16, 128, MODE, NW>(p, grid, stream) : launch_prefill<BF16, 64, MODE, NW>(p, grid, stream);
+    return D == 128 ? launch_prefill<BF16, 128, MODE, NW, TEAMS>(p, grid, stream) : launch_prefill<BF16, 64, MODE, NW, TEAMS>(p, grid, stream);
 }
 
+// Two teams of four waves instead of one where a unit has a single workgroup anyway and its tiles, from eight of them, outweigh
+// the hand-over (us, one team / two): dense, 8 heads over 2 L=512 15.3 / 14.7, 2048 44.7 / 36.9, 4096 84.2 / 68.0, at head_dim
+// 64 62.5 / 44.9; 32 over 8 L=1024 25.8 / 22.7; 16 of 2048 under a window of 256 keys 18.7 / 17.1 (L=256 10.8 / 11.3).  With two
+// workgroups to a unit causal masks still gain (L=1777 48.3 / 40.2) and windows lose (23.3 / 28.3), and which it is stands in the
+// mask; a packed batch is causal, and part of its grid is empty: 2 sequences to 1600, 32 over 8 20.5 / 19.4, 4 to 2500, 16
+// heads 56.7 / 50.5 (4 to 1600, 24 over 8 28.4 / 34.5).
+static bool two_teams_pay(int64_t longest, int64_t grid, bool packed) {
+    return longest >= 512 && grid <= (!packed ? 256 : (longest > 2048 ? 512 : 320));
+}
 template <int MODE>
 static int dispatch_prefill(int dtype, int64_t D, const PrefillParams& p, int waves, int grid, hipStream_t stream) {
+    if (waves == kWavesSmall && two_teams_pay(MODE == MODE_VARLEN ? p.max_len : p.L, grid, MODE == MODE_VARLEN))
+        return dispatch_prefill_nw<MODE, kWavesSmall, 2>(dtype, D, p, grid, stream);
     return waves == kWavesSmall ? dispatch_prefill_nw<MODE, kWavesSmall>(dtype, D, p, grid, stream)
                                 : dispatch_prefill_nw<MODE, kWavesBig>(dtype, D, p, grid, stream);
 }
@@ -855,6 +898,7 @@ MINFER_ATTN_EXPORT int minfer_flash_attn(int dtype, const void* q, const void* k
     // cheaper than every head re-reading the mask rows.
     if (L >= 16 && L <= kSelfClassifyMaxL && kWaves == kWavesSmall && grid <= kSelfClassifyMaxGrid) {
         p.cls = nullptr;
+        if (two_teams_pay(L, grid, false)) return dispatch_prefill_nw<MODE_DENSE_SELF, kWavesSmall, 2>(dtype, D, p, (int)grid, stream);
         return dispatch_prefill_nw<MODE_DENSE_SELF, kWavesSmall>(dtype, D, p, (int)grid, stream);
     }
     hipLaunchKernelGGL(classify_mask_kernel, dim3((p.NKT + 3) / 4, p.NQT, (unsigned)B), dim3(256), 0, stream,

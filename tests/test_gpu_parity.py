@@ -191,6 +191,44 @@ def test_decode_more_contexts_than_units(B, Hq, Hkv, Lmax, D, q8):
     assert max_err(out, want) <= TOL[torch.float16]
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,L,D,kind", [
+    (1, 8, 2, 512, 128, "causal"),     # the shortest; the workgroups classify their own rows
+    (1, 3, 3, 640, 64, "random"),
+    (2, 4, 4, 1000, 128, "window"),
+    (1, 4, 1, 1025, 64, "random"),     # the pre-pass's classes; a last key tile of one row
+    (1, 6, 2, 1111, 128, "causal"),
+    (1, 2, 2, 1500, 128, "empty"),     # rows, whole tiles and one of the two teams without a key
+])
+def test_prefill_two_teams(B, Hq, Hkv, L, D, kind, dtype):
+    """Few workgroups, whose two teams of waves take every other key tile, against the oracle.  Tolerance: that of every
+    attention result here."""
+    gen = torch.Generator().manual_seed(L)
+    q, k, v = workloads.dense_prefill(B, Hq, Hkv, L, D, dtype, seed=L, scale=1.0, device=DEV)
+    if kind == "empty":
+        mask = torch.zeros(B, 1, L, L, dtype=torch.bool)
+        mask[:, :, 64:128, 70:75] = True       # one tile of the list
+        mask[:, :, 200:320, 64:192] = True     # two
+        mask[:, :, 1400:, ::130] = True
+    else:
+        mask = workloads.causal_mask(B, L) if kind == "causal" else workloads.window_mask(B, L, 200) if kind == "window" else make_mask("random", B, L, gen)
+    out = run_prefill(q, k, v, mask.to(DEV))
+    assert max_err(out, oracle.flash_attn(q, k, v, mask)) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,lens", [
+    (8, 2, 128, [1, 0, 65, 700, 64, 513]),
+    (4, 4, 64, [2100, 129, 33]),
+])
+def test_packed_two_teams(Hq, Hkv, D, lens):
+    gen = torch.Generator().manual_seed(sum(lens))
+    q, k, v = (torch.randn(1, H, sum(lens), D, generator=gen).half() for H in (Hq, Hkv, Hkv))
+    cu = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32)
+    out = torch.full(q.shape, float("nan"), dtype=q.dtype, device=DEV)
+    assert capi.flash_attn_varlen(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), max(lens), out) == capi.OK, capi.last_error()
+    assert max_err(out, oracle.flash_attn_varlen(q, k, v, cu)) <= TOL[torch.float16]
+
+
 @pytest.mark.parametrize("offset", [0, 5])
 @pytest.mark.parametrize("B,L,D", [(2, 1, 64), (3, 2, 128), (2, 3, 64), (2, 4, 128), (2, 5, 64), (2, 15, 128), (2, 16, 64), (3, 17, 128),
                                    (2, 63, 64), (2, 65, 128), (1, 129, 128), (2, 255, 64), (1, 1023, 64), (1, 1025, 128), (1, 1103, 64)])
