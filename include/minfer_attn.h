@@ -70,7 +70,8 @@ int minfer_flash_attn(int dtype, const void* q, const void* k, const void* v,
                       const minfer_attn_strides* strides,
                       void* workspace, size_t workspace_bytes, void* stream);
 
-/* Bytes of workspace minfer_flash_attn_decode needs (split-KV partial results). */
+/* Bytes of workspace for minfer_flash_attn_decode (split-KV partial results).  A workspace that holds the partial results of
+ * 256-row shares only (Lmax up to 7680: Lmax / 256 + 3 per head instead of Lmax / 128 + 3) is accepted as well, and used so. */
 size_t minfer_flash_attn_decode_workspace_bytes(int64_t B, int64_t Hq, int64_t Lmax, int64_t D);
 
 /*
@@ -92,7 +93,7 @@ int minfer_flash_attn_decode(int dtype, const void* q, const void* k_cache, cons
  * under HIP graph capture, serving loops and harnesses that forbid hipMalloc.  It has no counterpart in the
  * reference.  The split-KV partial results go to a device array that is part of the library's code object
  * (MINFER_DECODE_NOALLOC_SCRATCH_BYTES bytes on every GPU the library is used on, held until the process ends);
- * a problem whose minfer_flash_attn_decode_workspace_bytes(B, Hq, Lmax, D) exceeds that size is rejected with
+ * a problem whose partial results of 256-row shares exceed that size is rejected with
  * MINFER_ATTN_EWORKSPACE (nothing launched).  The call allocates and frees nothing.  Its first call on a device
  * looks the array's address up (which may load the code object): make that call outside a graph capture.  All calls
  * on one GPU share the array: calls that overlap in time on one GPU (two streams, two threads) race; calls that

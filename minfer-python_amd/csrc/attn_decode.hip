@@ -866,16 +866,19 @@ __global__ __launch_bounds__(kChunkWaves * 64) void decode_merge_kernel(const Ch
 // has more than 64 partial results, which is what one wave of the combine kernel merges.  (With 256 a line of 128 to 256 rows
 // a wave left up to half of the waves idle: 40 sequences of 1101 rows over 8 KV heads, Q8_0 31.7 -> 29.5 us, fp16 39.9 -> 36.8;
 // 136 pairs to 4382 39.5 -> 33.7; longer and shorter ones as before.)
-static int decode_min_share_rows(int64_t Lmax) {
+// The partial results of shares that fine take up to twice the workspace: a caller's that holds those of 256 rows only, and the
+// allocation-free call's fixed one where it does, is enough and gets those.
+constexpr int kFineShare = 128, kCoarseShare = 256;
+static int decode_min_share_rows(int64_t Lmax, int floor_rows) {
     int64_t c = (Lmax + 59) / 60;
     c = (c + 63) / 64 * 64;
-    return (int)(c > 128 ? c : 128);
+    return (int)(c > floor_rows ? c : floor_rows);
 }
 // Partial results a (sequence, head) can have: a pair's rows overlap at most this many shares.
-static int decode_slots(int64_t Lmax) { return (int)(Lmax / decode_min_share_rows(Lmax)) + 3; }
+static int decode_slots(int64_t Lmax, int floor_rows) { return (int)(Lmax / decode_min_share_rows(Lmax, floor_rows)) + 3; }
 
-static size_t decode_ws_bytes(int64_t B, int64_t Hq, int64_t Lmax, int64_t D) {
-    const int64_t S = decode_slots(Lmax);
+static size_t decode_ws_bytes(int64_t B, int64_t Hq, int64_t Lmax, int64_t D, int floor_rows) {
+    const int64_t S = decode_slots(Lmax, floor_rows);
     return (size_t)(B * Hq * S * (D + 2) * 4 + 255) / 256 * 256 + (size_t)((B + 1) * 4 + 255) / 256 * 256 + 256;
 }
 
@@ -904,8 +907,8 @@ static int decode_workgroups() {
 //   up to 1536 rows: 8 pairs of 100 / 1500 rows 17.7 / 7.4 and 16.9 / 10.1; 24 pairs to 3000, Q8_0 19.8 / 12.7; 168 to 1500 21.0 / 20.1
 //   up to 2048 that occupy 9 of 10 units: 128 pairs to 4000 39.8 / 31.6, 256 to 2000 39.5 / 30.4 (96 to 4000, Q8_0, three
 //     quarters of the units: 22.0 / 25.5)
-//   longer ones that occupy 9 of 10 units, four to a pair or more: 32 pairs of 30000 85.5 / 77.4, 40 to 16000 49.5 / 40.9
-//     (three to a pair: 72 to 16000 56.9 / 65.5; two: 120 to 8000 50.4 / 53.8)
+//   longer ones are the line's: contexts that are alike would gain (32 pairs of 30000 85.5 / 77.4), others leave units idle
+//     (32 pairs, 4 sequences of 2254 to 36077, 43.6 / 55.3; 72 to 16000 56.9 / 65.5; 120 to 8000 50.4 / 53.8)
 //   more pairs than units, a workgroup per context (what is in flight on a unit does not change with the rounds):
 //     head_dim 64, 16-bit caches, any number of pairs to 1536: 512 of 1000 28.6 / 21.7, 1024 to 1000 30.3 / 27.6, 320 to
 //       1400 19.1 / 18.0 (320 to 3000 30.7 / 35.1)
@@ -929,7 +932,7 @@ static int decode_chunk_rows(const DecodeParams& p, int D, bool q8) {
         return (any_rounds || pairs * n <= 2 * units) && chunk <= longest ? (int)chunk : 0;
     }
     const bool full = 10 * pairs * n >= 9 * units;
-    return chunk <= 1536 || (full && (chunk <= 2048 || n >= 4)) ? (int)chunk : 0;
+    return chunk <= (full ? 2048 : 1536) ? (int)chunk : 0;
 }
 
 template <class T, int D, bool Q8>
@@ -967,7 +970,7 @@ using namespace minfer_attn;
 
 MINFER_ATTN_EXPORT size_t minfer_flash_attn_decode_workspace_bytes(int64_t B, int64_t Hq, int64_t Lmax, int64_t D) {
     if (B <= 0 || Hq <= 0 || Lmax < 0 || D <= 0) return 256;
-    return decode_ws_bytes(B, Hq, Lmax, D);   // Lmax == 0 (an empty cache) still has its rows' slots: the call writes zeros
+    return decode_ws_bytes(B, Hq, Lmax, D, kFineShare);   // Lmax == 0 (an empty cache) still has its rows' slots: the call writes zeros
 }
 
 // Fills the launch parameters both decode entry points share; returns an error code or MINFER_ATTN_OK.
@@ -979,15 +982,16 @@ static int fill_decode(DecodeParams& p, const void* q, const void* k_cache, cons
     if (B > 65535 || Hq > 65535) return fail(MINFER_ATTN_EINVAL, "flash_attn_decode: B or n_heads > 65535 unsupported");
     if (Lmax > (1 << 30)) return fail(MINFER_ATTN_EINVAL, "flash_attn_decode: Lmax too large");
     if (B == 0) return MINFER_ATTN_OK;
-    if (!workspace || workspace_bytes < decode_ws_bytes(B, Hq, Lmax, D) || !aligned16(workspace))
+    if (!workspace || workspace_bytes < decode_ws_bytes(B, Hq, Lmax, D, kCoarseShare) || !aligned16(workspace))
         return fail(MINFER_ATTN_EWORKSPACE, "flash_attn_decode: workspace too small or misaligned (see minfer_flash_attn_decode_workspace_bytes)");
     p.q = q; p.k = k_cache; p.v = v_cache; p.ctx = ctx_lens;
     p.q0 = st->q0; p.q1 = st->q1; p.kv0 = st->kv0; p.kv1 = st->kv1; p.kv2 = st->kv2;
     p.B = (int)B; p.Hq = (int)Hq; p.Hkv = (int)Hkv; p.n_rep = (int)(Hq / Hkv); p.Lmax = (int)Lmax;
     p.n_hg = (p.n_rep + 15) / 16;
     p.group_rows = group_rows;
-    p.min_quota = decode_min_share_rows(Lmax) / group_rows;
-    p.S = decode_slots(Lmax);
+    const int share = workspace_bytes >= decode_ws_bytes(B, Hq, Lmax, D, kFineShare) ? kFineShare : kCoarseShare;
+    p.min_quota = decode_min_share_rows(Lmax, share) / group_rows;
+    p.S = decode_slots(Lmax, share);
     p.n_wg = decode_workgroups();
     // the line of work is indexed with 32-bit integers
     if ((int64_t)B * Hkv * p.n_hg * ((Lmax + group_rows - 1) / group_rows) > 0x7fffffffLL - 65536)
@@ -1098,10 +1102,10 @@ MINFER_ATTN_EXPORT int minfer_flash_attn_decode_noalloc(int dtype, const void* q
     if (B < 0 || Lmax < 0) return fail(MINFER_ATTN_EINVAL, "flash_attn_decode_noalloc: negative B or Lmax");
     if (B > 65535 || Lmax > (1 << 30)) return fail(MINFER_ATTN_EINVAL, "flash_attn_decode_noalloc: B > 65535 or Lmax > 2^30 unsupported");
     if (B == 0) return MINFER_ATTN_OK;
-    if (decode_ws_bytes(B, Hq, Lmax, D) > (size_t)MINFER_DECODE_NOALLOC_SCRATCH_BYTES) {
+    if (decode_ws_bytes(B, Hq, Lmax, D, kCoarseShare) > (size_t)MINFER_DECODE_NOALLOC_SCRATCH_BYTES) {
         snprintf(error_buf(), 512, "flash_attn_decode_noalloc: B=%lld Hq=%lld Lmax=%lld D=%lld needs %zu bytes of partial results, "
                  "the built-in scratch holds %zu; use minfer_flash_attn_decode with a workspace",
-                 (long long)B, (long long)Hq, (long long)Lmax, (long long)D, decode_ws_bytes(B, Hq, Lmax, D),
+                 (long long)B, (long long)Hq, (long long)Lmax, (long long)D, decode_ws_bytes(B, Hq, Lmax, D, kCoarseShare),
                  (size_t)MINFER_DECODE_NOALLOC_SCRATCH_BYTES);
         return MINFER_ATTN_EWORKSPACE;
     }

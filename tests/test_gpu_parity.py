@@ -191,6 +191,26 @@ def test_decode_more_contexts_than_units(B, Hq, Hkv, Lmax, D, q8):
     assert max_err(out, want) <= TOL[torch.float16]
 
 
+def test_decode_with_the_partial_results_of_coarse_shares():
+    """A workspace that holds the partial results of 256-row shares and no more, one byte less, and the allocation-free call on
+    a problem whose finer shares its scratch does not hold.  Against the oracle."""
+    B, Hq, Hkv, Lmax, D = 64, 64, 1, 5000, 128
+    q, kc, vc, _ = workloads.decode_cache(seed=1, device=DEV, B=B, Hq=Hq, Hkv=Hkv, Lmax=Lmax, D=D, ctx_lo=1, ctx_hi=1)
+    ctx = torch.tensor([[5000, 1, 300, 2047][i % 4] for i in range(B)], dtype=torch.int32, device=DEV)
+    up = lambda n: (n + 255) // 256 * 256
+    need = up(B * Hq * (Lmax // 256 + 3) * (D + 2) * 4) + up((B + 1) * 4) + 256
+    assert need < 64 << 20 < capi.lib().minfer_flash_attn_decode_workspace_bytes(B, Hq, Lmax, D)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    out, out2 = (torch.full(q.shape, float("nan"), dtype=q.dtype, device=DEV) for _ in range(2))
+    assert capi.flash_attn_decode(q, kc, vc, ctx, out, ws[:-1]) == capi.EWORKSPACE
+    assert capi.flash_attn_decode(q, kc, vc, ctx, out, ws) == capi.OK, capi.last_error()
+    assert capi.flash_attn_decode_noalloc(q, kc, vc, ctx, out2) == capi.OK, capi.last_error()
+    some = [0, 1, 2, 3, 61, 62]
+    want = oracle.flash_attn_decode(q[some], kc[some], vc[some], ctx[some])
+    for o in (out, out2):
+        assert not torch.isnan(o).any() and max_err(o[some], want) <= TOL[torch.float16]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,Hq,Hkv,L,D,kind", [
     (1, 8, 2, 512, 128, "causal"),     # the shortest; the workgroups classify their own rows
