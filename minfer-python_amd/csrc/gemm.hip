@@ -436,7 +436,7 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
             const int n = nb0 + 4 * quad;
             if (!CONCAT && n >= N) continue;
             if (SPLIT) {   // the slice's raw sums
-                store_slice4(p, slice, m, n, acc[nb][mb]);
+                *reinterpret_cast<f32x4*>(p.part + ((int64_t)slice * p.M + m) * p.N + n) = acc[nb][mb];
                 continue;
             }
             float v[4];
@@ -452,10 +452,6 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
             pk.y = T::pack2(v[2], v[3]);
             *reinterpret_cast<uint2*>(Dg + (int64_t)m * ldd + n) = pk;
         }
-    }
-    if constexpr (SPLIT) {
-        __shared__ int last_s;
-        finish_slices<T, SH::WAVES * 64>(p, t, m0, min(m0 + kBM, p.M), n0, min(n0 + kBN, N), &last_s);
     }
 }
 
@@ -1587,11 +1583,13 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmParams p) {
     }
 }
 
-// The counters of a sliced launch, when its workgroups are to add the slices up themselves: up to 2 MiB of sums.  Written
-// through to where every XCD sees them they pass at about a microsecond per MiB, so larger ones are left to a second launch
-// (fused / two launches: 1 MiB 12.2 / 13.4 us, 1.9 MiB 23.7 / 25.3, 2.4 MiB 18.0 / 15.0, 5 MiB 16.7 / 13.7).  At most 256 tiles.
+// The counters of a sliced launch, when its workgroups are to add the slices up themselves: up to 16 rows and 2 MiB of sums.
+// Written through to where every XCD sees them they pass at about a microsecond per MiB, so larger ones are left to a second
+// launch (fused / two launches: 1 MiB 12.2 / 13.4 us, 1.9 MiB 23.7 / 25.3, 2.4 MiB 18.0 / 15.0, 5 MiB 16.7 / 13.7), and so are
+// more rows, and so the slices of gemm_kernel, whose tiles' last workgroups add up what a second launch spreads over the chip (17 x 528 x 1152 9.5 / 8.7, 40 x
+// 808 x 1600 13.3 / 9.8, 24 x 3424 x 1408 11.3 / 9.7).  At most 256 tiles.
 static uint32_t* slice_counters(const GemmParams& p, hipStream_t stream) {
-    return (int64_t)p.splits * p.M * p.N * 4 <= (2 << 20) ? stream_counters(stream) : nullptr;
+    return p.M <= 16 && (int64_t)p.splits * p.M * p.N * 4 <= (2 << 20) ? stream_counters(stream) : nullptr;
 }
 
 // After a sliced launch: nothing where its workgroups have added the slices up themselves.
@@ -1636,12 +1634,12 @@ static int launch_stripe_slices(GemmParams& p, hipStream_t stream) {
 }
 
 // [K, N] weights of up to 64 rows: slices of K bring the column tiles up to the chip's 256 compute units, every slice two
-// steps of 64 at least.
+// steps of 64 at least; from 17 rows on four and at most 32 slices, since the sums grow with the rows.
 constexpr int64_t kKnRows = 64;
 static int kn_slices(int64_t M, int64_t N, int64_t K) {
     if (M < 1 || M > kKnRows || K % kBK != 0 || K < 8 * kBK || N % 8 != 0) return 1;
     const int64_t tiles = (N + 127) / 128;
-    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, K / kBK / 2), 64));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, K / kBK / (M <= 16 ? 2 : 4)), M <= 16 ? 64 : 32));
 }
 template <class T>
 static int launch_kn_rows(GemmParams& p, hipStream_t stream) {
@@ -1662,7 +1660,6 @@ static int launch_split(GemmParams& p, hipStream_t stream) {
     p.tiles_n = (p.N + SH::BN - 1) / SH::BN;
     p.per_xcd = 0;
     const int64_t wgs = (int64_t)p.tiles_m * p.tiles_n * p.splits;
-    p.done = slice_counters(p, stream);
     if (one_workgroup_per_unit(wgs)) hipLaunchKernelGGL((gemm_kernel<T, NT, GemmSmall3, false, true>), dim3((unsigned)wgs), dim3(SH::WAVES * 64), 0, stream, p);
     else hipLaunchKernelGGL((gemm_kernel<T, NT, SH, false, true>), dim3((unsigned)wgs), dim3(SH::WAVES * 64), 0, stream, p);
     if (int rc = check_launch("gemm_kernel (K slices)")) return rc;
