@@ -1653,12 +1653,24 @@ static int launch_kn_rows(GemmParams& p, hipStream_t stream) {
     return p.splits > 1 ? launch_reduce<T>(p, stream) : MINFER_ATTN_OK;
 }
 
+static int64_t tile_count(int64_t M, int64_t N, int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
+
 template <class T, bool NT>
 static int launch_split(GemmParams& p, hipStream_t stream) {
     using SH = GemmSmall;
     p.tiles_m = (p.M + SH::BM - 1) / SH::BM;
     p.tiles_n = (p.N + SH::BN - 1) / SH::BN;
     p.per_xcd = 0;
+    // As 128 x 256 tiles with three stages where these in the same slices fill the chip once by themselves: half the copies of A and
+    // two steps in flight instead of one (250 x 8192 x 8192 62.8 -> 54.2 us, 180 x 4136 x 11776 56.0 -> 46.8, 100 x 8192 x 8192 42.7
+    // -> 37.6, 512 x 4096 x 4096 33.0 -> 31.3; half a chip of them 129 x 4096 x 4096 22.0 -> 26.6).
+    const int64_t flat_wgs = tile_count(p.M, p.N, GemmFlat::BM, GemmFlat::BN) * p.splits;
+    if (flat_wgs > 192 && flat_wgs <= 256) {
+        p.tiles_n = (p.N + GemmFlat::BN - 1) / GemmFlat::BN;
+        hipLaunchKernelGGL((gemm_kernel<T, NT, GemmFlat, false, true>), dim3((unsigned)flat_wgs), dim3(GemmFlat::WAVES * 64), 0, stream, p);
+        if (int rc = check_launch("gemm_kernel (K slices, 128 x 256)")) return rc;
+        return launch_reduce<T>(p, stream);
+    }
     const int64_t wgs = (int64_t)p.tiles_m * p.tiles_n * p.splits;
     if (one_workgroup_per_unit(wgs)) hipLaunchKernelGGL((gemm_kernel<T, NT, GemmSmall3, false, true>), dim3((unsigned)wgs), dim3(SH::WAVES * 64), 0, stream, p);
     else hipLaunchKernelGGL((gemm_kernel<T, NT, SH, false, true>), dim3((unsigned)wgs), dim3(SH::WAVES * 64), 0, stream, p);
@@ -1695,7 +1707,6 @@ static double rounds_cost(int64_t tiles) {
 // divided by its rate): 256 x 192 0.75-0.83, 192 x 256 0.78-0.85, 160 x 256 0.68-0.75, 128 x 256 0.57-0.61, two 128 x 128 on a
 // compute unit 0.58-0.65, one with three stages 0.41.  The large tile wins ties.
 enum class Tile { Big, Wide, Rows192, Rows160, Flat, Small, Small3 };
-static int64_t tile_count(int64_t M, int64_t N, int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 template <bool NT>
 static Tile pick_tile(int64_t M, int64_t N, int64_t big_tiles, int64_t small_tiles) {
     Tile best = Tile::Big;

@@ -346,6 +346,23 @@ def test_few_rows_against_a_kn_weight(dtype, M, N, K):
     assert_close(outs[2], exact, dtype, "no workspace")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout,M,N,K", [
+    (NK, 70, 8136, 8256),      # eight slices of 16 and 17 steps; a last tile of 200 columns
+    (KN, 70, 8136, 8256),
+    (NK, 250, 8072, 4160),     # four; a last tile row of 122
+    (KN, 129, 8072, 4160),     # ... of one
+])
+def test_gemm_k_slices_of_wide_tiles(layout, dtype, M, N, K):
+    """Slices of 128 x 256 tiles, every element against torch's product in 64 bits within the bound of assert_close."""
+    a, b, c = make(M, N, K, layout, dtype, M + N + K)
+    ws = torch.full((capi.lib().minfer_gemm_workspace_bytes(M, N, K),), 0xFF, dtype=torch.uint8, device=DEV)
+    d = torch.full((M, N), float("nan"), dtype=dtype, device=DEV)
+    assert capi.gemm_ws(a.to(DEV), b.to(DEV), c.to(DEV), d, 2.0, 3.0, ws, layout) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    assert_close(d, (2.0 * (a.double() @ (b if layout == KN else b.T).double()) + 3.0 * c.double()).numpy(), dtype)
+
+
 def test_gemm_workspace_bytes_is_zero_where_tiles_fill_the_chip():
     L = capi.lib()
     assert L.minfer_gemm_workspace_bytes(4096, 4096, 4096) == 0
