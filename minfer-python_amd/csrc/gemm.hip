@@ -6,7 +6,7 @@
 // ("A x B^T", the layout of its QKV projection, whose launcher is empty in the reference), C and D are [M, N].
 //
 // Design.  A workgroup (8 waves, two per SIMD) owns a 256 x 256 tile of D (128 x 128 with 4 waves for problems
-// too small to fill the chip with large tiles) and walks K in steps of 64; the A and B panels of a step (32 KB
+// too small to fill the chip with large tiles, sizes between the two where they fill it better: pick_tile) and walks K in steps of 64; the A and B panels of a step (32 KB
 // each) are copied global->LDS without passing through registers, double-buffered, one barrier per step
 // (placed inside the step, so that the matrix pipe keeps running across step boundaries).
 // Every wave owns 128 (64) rows (m) x 64 columns (n) as 8 (4) x 4 accumulator blocks of 16x16
