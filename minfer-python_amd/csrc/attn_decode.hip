@@ -712,14 +712,15 @@ struct ChunkParams {
 MA_DEV void store_shared(float* p, float x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 MA_DEV float load_shared(const float* p) { return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// Weights and denominator of one head's partial results 0 .. n-1 whose (max, sum) are read by ml(i): out gets the weight
-// of each over the denominator's reciprocal.  Called by one thread per head.
+// Reference and denominator of one head's partial results 0 .. n-1, whose (max, sum) are read by ml(i, 0) and ml(i, 1), and the
+// weight of a part with reference m.  A part without a reference has no key, and sums of zero, or only scores that are NaN, and
+// sums of NaN: its weight is 0 and multiplies them like any other, so that NaN stays NaN.
 struct MergedHead { float m, l; };
+MA_DEV float merge_weight(float m, float m_all, float scale_log2) { return m > -INFINITY ? fast_exp2((m - m_all) * scale_log2) : 0.f; }
 template <class F> MA_DEV MergedHead merge_ml(int n, float scale_log2, F ml) {
     MergedHead r{-INFINITY, 0.f};
     for (int i = 0; i < n; ++i) r.m = fmaxf(r.m, ml(i, 0));
-    if (r.m > -INFINITY)
-        for (int i = 0; i < n; ++i) r.l += ml(i, 1) * fast_exp2((ml(i, 0) - r.m) * scale_log2);   // a part without keys has sum 0
+    for (int i = 0; i < n; ++i) r.l += ml(i, 1) * merge_weight(ml(i, 0), r.m, scale_log2);
     return r;
 }
 
@@ -750,10 +751,7 @@ MA_DEV void merge_chunks(const ChunkParams& c, int b, int head0, int heads, int 
     __syncthreads();
     if (tid < heads) {
         const MergedHead r = merge_ml(n, p.scale_log2, [&](int i, int what) { return lds_w[(64 * what + i) * 16 + tid]; });
-        for (int i = 0; i < n; ++i) {
-            const float m = lds_w[i * 16 + tid];
-            lds_w[i * 16 + tid] = m > -INFINITY ? fast_exp2((m - r.m) * p.scale_log2) : 0.f;
-        }
+        for (int i = 0; i < n; ++i) lds_w[i * 16 + tid] = merge_weight(lds_w[i * 16 + tid], r.m, p.scale_log2);
         lds_inv[tid] = r.l > 0.f ? 1.f / r.l : 0.f;
     }
     __syncthreads();
@@ -825,10 +823,8 @@ __global__ __launch_bounds__(kChunkWaves * 64, 2) void decode_chunk_kernel(const
         const int h = idx / D, d = idx % D;
         const MergedHead r = merge_ml(NW, p.scale_log2, [&](int i, int what) { return ml_s[(64 * what + i) * 16 + h]; });
         float sum = 0.f;
-        if (r.m > -INFINITY) {
 #pragma unroll
-            for (int i = 0; i < NW; ++i) sum += o_s[(i * 16 + h) * ORS + d] * fast_exp2((ml_s[i * 16 + h] - r.m) * p.scale_log2);
-        }
+        for (int i = 0; i < NW; ++i) sum += o_s[(i * 16 + h) * ORS + d] * merge_weight(ml_s[i * 16 + h], r.m, p.scale_log2);
         if (whole) {
             const float inv = r.l > 0.f ? 1.f / r.l : 0.f;
             reinterpret_cast<uint16_t*>(c.out)[(int64_t)b * c.o0 + (int64_t)(head0 + h) * c.o1 + d] = (uint16_t)(T::pack2(sum * inv, 0.f) & 0xffffu);

@@ -163,6 +163,44 @@ def test_decode_chunks(Hq, Hkv, Lmax, D):
         assert torch.equal(out, outs[0])
 
 
+@pytest.mark.parametrize("Hq,Hkv,Lmax,D,q8", [
+    (8, 2, 200, 128, False),      # one chunk, merged by its workgroup
+    (8, 2, 190, 64, True),
+    (8, 2, 3000, 64, False),      # chunks merged by the last workgroup, a whole one without a number among them
+    (8, 2, 3000, 128, True),
+    (40, 40, 1700, 64, False),    # the line of equal shares
+])
+def test_decode_keeps_nan(Hq, Hkv, Lmax, D, q8):
+    """A query row with a NaN, a KV head whose keys are all NaN and one whose first half of keys is: the rows that attend them
+    are NaN throughout, and no other row changes by a bit.  The same from the merge of a second launch (under graph capture)."""
+    n_rep = Hq // Hkv
+    q, kc, vc, _ = workloads.decode_cache(seed=Lmax, device=DEV, B=4, Hq=Hq, Hkv=Hkv, Lmax=Lmax, D=D, ctx_lo=1, ctx_hi=1)
+    ctx = torch.tensor([Lmax, Lmax, Lmax, Lmax - 7], dtype=torch.int32, device=DEV)
+    call = capi.flash_attn_decode
+    if q8:
+        kc, vc, call = workloads.q8_0_rows(kc), workloads.q8_0_rows(vc), capi.flash_attn_decode_q8_0
+    clean, out, replayed = (torch.zeros(q.shape, dtype=q.dtype, device=DEV) for _ in range(3))
+    assert call(q, kc, vc, ctx, clean) == capi.OK, capi.last_error()
+    assert not torch.isnan(clean).any()
+    q[0, 1, 0, D // 3] = float("nan")
+    nan_keys = kc[1, Hkv - 1], kc[2, 0, :Lmax // 2]
+    for rows in nan_keys:
+        (rows.view(-1, 34)[:, :2].view(torch.float16) if q8 else rows).fill_(float("nan"))   # (Q8_0: the blocks' scales)
+    want_nan = torch.zeros(q.shape, dtype=torch.bool, device=DEV)
+    want_nan[0, 1] = want_nan[1, (Hkv - 1) * n_rep:] = want_nan[2, :n_rep] = True
+    assert call(q, kc, vc, ctx, out) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    ws = torch.empty(capi.lib().minfer_flash_attn_decode_workspace_bytes(4, Hq, Lmax, D), dtype=torch.uint8, device=DEV)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert call(q, kc, vc, ctx, replayed, ws) == capi.OK, capi.last_error()
+    graph.replay()
+    torch.cuda.synchronize()
+    for o in (out, replayed):
+        assert torch.equal(torch.isnan(o), want_nan), [(torch.isnan(o) != want_nan)[b].flatten(1).any(1).nonzero().flatten().tolist() for b in range(4)]
+        assert torch.equal(o[~want_nan], clean[~want_nan])
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,Lmax,D,q8", [
     (33, 16, 8, 1536, 64, False),    # a workgroup per context, one round and a bit
     (33, 16, 16, 300, 64, False),    # more than two rounds
