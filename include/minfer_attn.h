@@ -79,7 +79,9 @@ size_t minfer_flash_attn_decode_workspace_bytes(int64_t B, int64_t Hq, int64_t L
  * (the reference's cache layout, src/minfer/core.py:105-127); ctx_lens int32 [B] on the device;
  * query b attends cache rows 0..ctx_lens[b]-1 (rows beyond are never read into the result;
  * ctx_lens[b] == 0 yields zeros).  The KV range is split across workgroups and merged by a
- * log-sum-exp combine kernel.  No counterpart in the reference (its op requires Lq == Lk,
+ * log-sum-exp combine kernel, or, for few or short sequences on a device's null stream (stream 0), by the last
+ * workgroup of a (sequence, KV head) in the same launch; on every other stream, and so under graph capture, a second
+ * launch does that, with the same result to the bit.  No counterpart in the reference (its op requires Lq == Lk,
  * flash_attn/op.cuh:74-78); strides->q2 and strides->o2 are ignored.
  */
 int minfer_flash_attn_decode(int dtype, const void* q, const void* k_cache, const void* v_cache,
@@ -209,8 +211,9 @@ int minfer_gemm(int dtype, int b_layout, const void* A, const void* B, const voi
  * minfer_gemm with a workspace.  A problem of a few dozen rows against a wide weight (a batch of decode steps, a short
  * prefill chunk) has too few output tiles to occupy the chip; given minfer_gemm_workspace_bytes(M, N, K) bytes of
  * device memory (16-byte aligned; 0 = this shape does not use any), the K dimension is cut into slices that run as
- * separate workgroups and meet in the workspace as fp32 partial sums, which the last workgroup of a tile or a second
- * kernel adds up (alpha, beta and C applied there, one rounding): slices of the 128 x 128 tiles, or, up to 64 rows,
+ * separate workgroups and meet in the workspace as fp32 partial sums, which the last workgroup of a tile (small sums on
+ * a device's null stream, stream 0) or a second kernel adds up, with the same result to the bit (alpha, beta and C
+ * applied there, one rounding): slices of the 128 x 128 tiles, or, up to 64 rows,
  * of 128-column tiles of a [K, N] weight, or of an [N, K] weight of fewer
  * than 12288 columns, of 64-column stripes (where two launches pay: from 9 rows on below 6144 columns, from 2 on rows
  * of 8192 values and more of at most 1536 columns, from 33 between 6144 and 12288 columns).  With a null workspace the

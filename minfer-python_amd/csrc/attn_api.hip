@@ -1,33 +1,24 @@
 // Entry points of the C ABI that are not tied to one operator.
-#include <mutex>
+#include <atomic>
 
 #include "attn_host.h"
 
 namespace minfer_attn {
-static __device__ uint32_t counter_pool[kCounterStreams * kStreamCounters];   // zero when the code object is loaded
+static __device__ uint32_t counter_pool[kStreamCounters];   // zero when the code object is loaded, on every device
 
 uint32_t* stream_counters(hipStream_t stream) {
-    if (stream == hipStreamPerThread) return nullptr;   // one handle, another stream in every thread
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &st) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
-    if (st != hipStreamCaptureStatusNone) return nullptr;
+    if (stream) return nullptr;
+    static std::atomic<uint32_t*> base[64];   // concurrent first calls at worst both look the address up
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
-    struct Device { uint32_t* base = nullptr; int n = 0; hipStream_t stream[kCounterStreams]; };
-    static std::mutex mu;
-    static Device devices[64];
-    std::lock_guard<std::mutex> lock(mu);
-    Device& d = devices[dev];
-    for (int i = 0; i < d.n; ++i)
-        if (d.stream[i] == stream) return d.base + (size_t)i * kStreamCounters;
-    if (d.n == kCounterStreams) return nullptr;
-    if (!d.base) {
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) { (void)hipGetLastError(); return nullptr; }
+    uint32_t* p = base[dev].load(std::memory_order_acquire);
+    if (!p) {
         void* ptr = nullptr;
         if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(counter_pool)) != hipSuccess || !ptr) { (void)hipGetLastError(); return nullptr; }
-        d.base = (uint32_t*)ptr;
+        p = (uint32_t*)ptr;
+        base[dev].store(p, std::memory_order_release);
     }
-    d.stream[d.n] = stream;
-    return d.base + (size_t)d.n++ * kStreamCounters;
+    return p;
 }
 }  // namespace minfer_attn
 

@@ -697,7 +697,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecodeParams 
 // that is one chunk long is done with that; otherwise the chunk's result goes to the workspace and the workgroup that comes
 // last (a counter per pair) merges the pair's chunks, so that there is no second launch.  Results cross from one XCD's L2
 // to another's: they are written and read with device-scope accesses, and a workgroup counts itself only when its own have
-// arrived.  Without counters (p.done null: a stream that is being captured, see stream_counters) decode_merge_kernel does
+// arrived.  Without counters (p.done null: any stream but the null stream, see stream_counters) decode_merge_kernel does
 // the merging, with the same code and so the same result.
 constexpr int kChunkWaves = 8;
 

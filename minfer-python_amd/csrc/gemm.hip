@@ -118,7 +118,7 @@ template <class T> MA_DEV void store_result(const GemmParams& p, int m, int n, f
 // and stores D: no second launch, which costs the host 2.7 us and the chip 4, as much as many of these products take
 // themselves.  The sums pass from one XCD's L2 to another's, so they are written and read with device-scope accesses, and a
 // workgroup counts itself only when its own have arrived.  Slices are added in their order whoever comes last, as
-// gemm_reduce_kernel adds them, which takes over where there are no counters (stream_counters: a stream under capture).
+// gemm_reduce_kernel adds them, which takes over where there are no counters (stream_counters: any stream but the null stream).
 MA_DEV void store_slice4(const GemmParams& p, int slice, int m, int n, f32x4 v) {
     float* at = p.part + ((int64_t)slice * p.M + m) * p.N + n;
     if (!p.done) { *reinterpret_cast<f32x4*>(at) = v; return; }

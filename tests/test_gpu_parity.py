@@ -7,6 +7,7 @@ At the full benchmark sizes the oracle is evaluated on a sample of query rows (i
 program) and the whole output is additionally compared with a plain fp32 torch evaluation of the
 same formula on the GPU.
 """
+import ctypes
 import math
 
 import numpy as np
@@ -161,6 +162,26 @@ def test_decode_chunks(Hq, Hkv, Lmax, D):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, outs[0])
+
+
+def test_merged_parts_on_every_kind_of_stream(monkeypatch):
+    """The null stream, the per-thread one (handle 2) and a created one: whether a launch's last workgroups or a second launch
+    merge the parts of a decode and add up the K slices of a projection, the bits are the same."""
+    q, kc, vc, ctx = workloads.decode_cache(seed=3, device=DEV, B=2, Hq=8, Hkv=2, Lmax=3000, D=128, ctx_lo=2000, ctx_hi=3000)
+    x, w = torch.randn(3, 4096, device=DEV).half(), torch.randn(4096, 1024, device=DEV).half()
+    ws = torch.empty(capi.lib().minfer_gemm_workspace_bytes(3, 1024, 4096), dtype=torch.uint8, device=DEV)
+    created = torch.cuda.Stream()
+    got = []
+    for handle in (0, 2, created.cuda_stream, 0):
+        monkeypatch.setattr(capi, "_stream", lambda: ctypes.c_void_p(handle))
+        out, y = torch.full(q.shape, float("nan"), dtype=q.dtype, device=DEV), torch.full((3, 1024), float("nan"), dtype=q.dtype, device=DEV)
+        torch.cuda.synchronize()
+        assert capi.flash_attn_decode(q, kc, vc, ctx, out) == capi.OK, capi.last_error()
+        assert capi.gemm_ws(x, w, None, y, 1.0, 0.0, ws) == capi.OK, capi.last_error()
+        torch.cuda.synchronize()
+        got.append((out, y))
+    assert not any(torch.isnan(t).any() for t in got[0])
+    assert all(torch.equal(a, b) for g in got[1:] for a, b in zip(g, got[0]))
 
 
 @pytest.mark.parametrize("Hq,Hkv,Lmax,D,q8", [

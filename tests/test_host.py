@@ -3,7 +3,9 @@ argument validation rejects bad calls before anything is launched, and the Pytho
 the reference's names (reference: src/minfer/kernels/__init__.py, torch_ext/ops.py:234-266)."""
 import ctypes
 import inspect
+import os
 import re
+import subprocess
 
 import pytest
 import torch
@@ -385,3 +387,50 @@ def test_build_scan_finds_dependences_too_close_to_an_asm_statement():
     assert len(build.asm_hazards("kernel_b:\n" + cvt + "\tv_pk_mul_f16 v63, v63, v136\n" + mfma)) == 1
     assert build.asm_hazards("kernel_b:\n" + cvt + "\tv_pk_mul_f16 v63, v63, v136\n" * 2 + mfma) == []
     assert build.asm_hazards("kernel_b:\n" + cvt.replace("v51", "v70") + mfma) == []
+
+
+FAKE_HIP = r"""
+#pragma once
+#include <stddef.h>
+#include <stdint.h>
+#define __device__
+typedef int hipError_t; typedef int hipDevice_t; typedef struct fake_stream* hipStream_t;
+enum { hipSuccess = 0 };
+enum hipStreamCaptureStatus { hipStreamCaptureStatusNone = 0, hipStreamCaptureStatusActive = 1 };
+#define hipStreamPerThread ((hipStream_t)2)
+#define HIP_SYMBOL(x) ((const void*)&(x))
+extern "C" { inline int fake_current = 0, fake_owner = 0; }
+inline hipError_t hipGetLastError() { return hipSuccess; }
+inline const char* hipGetErrorString(hipError_t) { return ""; }
+inline hipError_t hipGetDevice(int* d) { *d = fake_current; return hipSuccess; }
+inline hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t* d) { *d = s ? fake_owner : fake_current; return hipSuccess; }
+inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st) { *st = hipStreamCaptureStatusNone; return hipSuccess; }
+inline hipError_t hipGetSymbolAddress(void** p, const void*) { *p = (void*)(uintptr_t)(0x1000000 * (fake_current + 1)); return hipSuccess; }
+"""
+
+
+def test_arrival_counters_go_to_one_stream_of_one_device(tmp_path):
+    """csrc/attn_api.hip compiled for the host against a stand-in for the HIP runtime that says which device is current and which
+    one a stream belongs to.  A handle names neither for good: after hipStreamDestroy, which need not wait for the stream's
+    work, a new stream may have it, and hipStreamPerThread is another stream in every thread.  The null stream of a device is
+    always the same one; it gets that device's counters, and nothing else gets any."""
+    (tmp_path / "hip").mkdir()
+    (tmp_path / "hip" / "hip_runtime.h").write_text(FAKE_HIP)
+    (tmp_path / "probe.cpp").write_text("""
+#include "attn_api.hip"
+extern "C" uintptr_t probe(uintptr_t stream, int current, int owner) {
+    fake_current = current; fake_owner = owner;
+    return (uintptr_t)minfer_attn::stream_counters((hipStream_t)stream);
+}
+""")
+    so = tmp_path / "probe.so"
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I", str(tmp_path), "-I", os.path.join(capi.ROOT, "include"),
+                    "-I", os.path.join(capi.ROOT, "minfer-python_amd", "csrc"), str(tmp_path / "probe.cpp"), "-o", str(so)], check=True)
+    probe = ctypes.CDLL(str(so)).probe
+    probe.restype, probe.argtypes = ctypes.c_size_t, [ctypes.c_size_t, ctypes.c_int, ctypes.c_int]
+    base = [0x1000000 * (dev + 1) for dev in range(3)]
+    assert [probe(0, dev, 0) for dev in (0, 1, 0, 2, 1)] == [base[dev] for dev in (0, 1, 0, 2, 1)]
+    assert probe(2, 0, 0) == 0                      # hipStreamPerThread
+    assert probe(0x7000, 0, 1) == 0                 # another device's stream
+    assert probe(0x7000, 1, 1) == 0                 # a created stream, and the next one at its address
+    assert probe(0, 64, 0) == 0                     # a device past the table
