@@ -26,6 +26,7 @@
 // classifies every 64x64 mask tile as none / all / mixed; the main kernel skips "none" tiles,
 // runs "all" tiles unmasked and reads mask bytes only for "mixed" tiles, which keeps arbitrary
 // masks bit-exact while a causal mask costs one byte-read tile per row of tiles.
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_common.h"
@@ -789,13 +790,16 @@ static int dispatch_prefill_nw(int dtype, int64_t D, const PrefillParams& p, int
 // 64 62.5 / 44.9; 32 over 8 L=1024 25.8 / 22.7; 16 of 2048 under a window of 256 keys 18.7 / 17.1 (L=256 10.8 / 11.3).  With two
 // workgroups to a unit causal masks still gain (L=1777 48.3 / 40.2) and windows lose (23.3 / 28.3), and which it is stands in the
 // mask; a packed batch is causal, and part of its grid is empty: 2 sequences to 1600, 32 over 8 20.5 / 19.4, 4 to 2500, 16
-// heads 56.7 / 50.5 (4 to 1600, 24 over 8 28.4 / 34.5).
+// heads 56.7 / 50.5 (4 to 1600, 24 over 8 28.4 / 34.5).  A packed batch without a bound of its lengths is taken for one of up to
+// three times the mean (32 heads over 8, equal lengths: 8 of 128 8.6 / 10.2, 6 of 160 9.5 / 10.3, 4 of 192 9.4 / 10.0, 4 of 256
+// 10.8 / 10.8, 2 of 400 14.0 / 13.2; uneven ones of such means gain, 511, 333, 0, 20, 64 and 100 16.0 / 14.4, 511, 30 and 20
+// 15.1 / 13.7).
 static bool two_teams_pay(int64_t longest, int64_t grid, bool packed) {
     return longest >= 512 && grid <= (!packed ? 256 : (longest > 2048 ? 512 : 320));
 }
 template <int MODE>
-static int dispatch_prefill(int dtype, int64_t D, const PrefillParams& p, int waves, int grid, hipStream_t stream) {
-    if (waves == kWavesSmall && two_teams_pay(MODE == MODE_VARLEN ? p.max_len : p.L, grid, MODE == MODE_VARLEN))
+static int dispatch_prefill(int dtype, int64_t D, const PrefillParams& p, int waves, int64_t longest, int grid, hipStream_t stream) {
+    if (waves == kWavesSmall && two_teams_pay(longest, grid, MODE == MODE_VARLEN))
         return dispatch_prefill_nw<MODE, kWavesSmall, 2>(dtype, D, p, grid, stream);
     return waves == kWavesSmall ? dispatch_prefill_nw<MODE, kWavesSmall>(dtype, D, p, grid, stream)
                                 : dispatch_prefill_nw<MODE, kWavesBig>(dtype, D, p, grid, stream);
@@ -904,7 +908,7 @@ MINFER_ATTN_EXPORT int minfer_flash_attn(int dtype, const void* q, const void* k
     hipLaunchKernelGGL(classify_mask_kernel, dim3((p.NKT + 3) / 4, p.NQT, (unsigned)B), dim3(256), 0, stream,
                        mask, (uint8_t*)workspace, p.L, p.NQT, p.NKT);
     if (int rc = check_launch("classify_mask_kernel")) return rc;
-    return dispatch_prefill<MODE_DENSE>(dtype, D, p, kWaves, (int)grid, stream);
+    return dispatch_prefill<MODE_DENSE>(dtype, D, p, kWaves, L, (int)grid, stream);
 }
 
 MINFER_ATTN_EXPORT int minfer_flash_attn_varlen(int dtype, const void* q, const void* k, const void* v,
@@ -939,7 +943,8 @@ MINFER_ATTN_EXPORT int minfer_flash_attn_varlen(int dtype, const void* q, const 
     p.max_len = (int)max_len;
     const int64_t grid = (int64_t)p.NQ * Hkv * p.n_hg;
     if (grid > 0x7fffffffLL) return fail(MINFER_ATTN_EINVAL, "flash_attn_varlen: problem too large for one launch");
-    return dispatch_prefill<MODE_VARLEN>(dtype, D, p, kWaves, (int)grid, stream);
+    const int64_t likely = max_len < T ? max_len : std::min<int64_t>(T, 3 * T / n_seqs);   // (see two_teams_pay)
+    return dispatch_prefill<MODE_VARLEN>(dtype, D, p, kWaves, likely, (int)grid, stream);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -308,6 +308,22 @@ def test_packed_two_teams(Hq, Hkv, D, lens):
     assert max_err(out, oracle.flash_attn_varlen(q, k, v, cu)) <= TOL[torch.float16]
 
 
+@pytest.mark.parametrize("D,lens", [(128, [100] * 12), (64, [90, 0, 70, 100, 33] * 5), (128, [513, 0, 700, 65])])
+def test_packed_with_no_bound_of_the_lengths(D, lens):
+    """max_seqlen 0 (not known), or one that says no more than the number of tokens does, does not make a batch of short sequences
+    one for the kernel of two teams, whose sums meet in another order, nor keep a batch of long ones from it: the same bits as
+    with the bound."""
+    gen = torch.Generator().manual_seed(sum(lens))
+    q, k, v = (torch.randn(1, H, sum(lens), D, generator=gen).half().to(DEV) for H in (8, 2, 2))
+    cu = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32, device=DEV)
+    outs = [torch.full(q.shape, float("nan"), dtype=q.dtype, device=DEV) for _ in range(3)]
+    for bound, out in zip((max(lens), 0, sum(lens) + 1), outs):
+        assert capi.flash_attn_varlen(q, k, v, cu, bound, out) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    assert max_err(outs[0], oracle.flash_attn_varlen(q.cpu(), k.cpu(), v.cpu(), cu.cpu())) <= TOL[torch.float16]
+    assert torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
+
+
 @pytest.mark.parametrize("offset", [0, 5])
 @pytest.mark.parametrize("B,L,D", [(2, 1, 64), (3, 2, 128), (2, 3, 64), (2, 4, 128), (2, 5, 64), (2, 15, 128), (2, 16, 64), (3, 17, 128),
                                    (2, 63, 64), (2, 65, 128), (1, 129, 128), (2, 255, 64), (1, 1023, 64), (1, 1025, 128), (1, 1103, 64)])
