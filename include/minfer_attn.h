@@ -218,7 +218,7 @@ int minfer_gemm(int dtype, int b_layout, const void* A, const void* B, const voi
  * than 12288 columns, of 64-column stripes (where two launches pay: from 9 rows on below 6144 columns, from 2 on rows
  * of 8192 values and more of at most 1536 columns, from 33 between 6144 and 12288 columns).  With a null workspace the
  * call is minfer_gemm; a workspace smaller than minfer_gemm_workspace_bytes is used only by a path whose slices fit
- * in it.  No counterpart in the
+ * in it, and up to 64 rows against a [K, N] weight for as many slices as it holds.  No counterpart in the
  * reference, whose gemm_cuda takes no scratch memory (reference: gemm/op.cuh:218-316); same contract for the
  * workspace as the attention entry points (contents need not be initialised; one per stream).
  */

@@ -346,6 +346,26 @@ def test_few_rows_against_a_kn_weight(dtype, M, N, K):
     assert_close(outs[2], exact, dtype, "no workspace")
 
 
+@pytest.mark.parametrize("M,N,K", [(9, 1000, 4096), (40, 4096, 4096), (64, 2056, 2048)])
+def test_few_rows_against_a_kn_weight_in_a_smaller_workspace(M, N, K):
+    """A workspace one byte short of minfer_gemm_workspace_bytes, one of two slices and one of less than two: as many slices as it
+    holds, none past its end; the bound is this file's."""
+    a, b, c = make(M, N, K, KN, torch.float16, seed=M + N)
+    exact = oracle.gemm(a.float().numpy(), b.float().numpy(), c.float().numpy(), 2.0, 3.0, KN)
+    da, db, dc = a.to(DEV), b.to(DEV), c.to(DEV)
+    need = capi.lib().minfer_gemm_workspace_bytes(M, N, K)
+    for size in (need - 1, 2 * 4 * M * N, 2 * 4 * M * N - 1):
+        ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=DEV)
+        d = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
+        assert capi.gemm_ws(da, db, dc, d, 2.0, 3.0, ws[:size], KN) == capi.OK, capi.last_error()
+        torch.cuda.synchronize()
+        assert_close(d, exact, torch.float16, f"{size} bytes")
+        slices = ws[:need // (4 * M * N) * 4 * M * N].view(-1, 4 * M * N)
+        written = [bool((s != 0xFF).any()) for s in slices]
+        fit = size // (4 * M * N)
+        assert written == [i < fit and fit > 1 for i in range(len(written))], (size, written)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("layout,M,N,K", [
     (NK, 70, 8136, 8256),      # eight slices of 16 and 17 steps; a last tile of 200 columns
