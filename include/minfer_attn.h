@@ -218,11 +218,13 @@ int minfer_gemm(int dtype, int b_layout, const void* A, const void* B, const voi
  * than 12288 columns, of 64-column stripes (where two launches pay: from 9 rows on below 6144 columns, from 2 on rows
  * of 8192 values and more of at most 1536 columns, from 33 between 6144 and 12288 columns).  With a null workspace the
  * call is minfer_gemm; a workspace smaller than minfer_gemm_workspace_bytes is used only by a path whose slices fit
- * in it, and up to 64 rows against a [K, N] weight for as many slices as it holds.  No counterpart in the
- * reference, whose gemm_cuda takes no scratch memory (reference: gemm/op.cuh:218-316); same contract for the
+ * in it, and up to 64 rows against a [K, N] weight for as many slices as it holds.
+ * minfer_gemm_workspace_bytes is enough for either layout; minfer_gemm_layout_workspace_bytes is what one of them
+ * (MINFER_GEMM_B_KN, MINFER_GEMM_B_NK) can use, which up to 64 rows is often less.  No counterpart in the reference, whose gemm_cuda takes no scratch memory (reference: gemm/op.cuh:218-316); same contract for the
  * workspace as the attention entry points (contents need not be initialised; one per stream).
  */
 size_t minfer_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+size_t minfer_gemm_layout_workspace_bytes(int b_layout, int64_t M, int64_t N, int64_t K);
 int minfer_gemm_ws(int dtype, int b_layout, const void* A, const void* B, const void* C, void* D,
                    int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int64_t ldd,
                    double alpha, double beta, void* workspace, size_t workspace_bytes, void* stream);

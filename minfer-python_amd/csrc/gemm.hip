@@ -1971,6 +1971,14 @@ MINFER_ATTN_EXPORT int minfer_gemm(int dtype, int b_layout, const void* A, const
     return gemm_impl(dtype, b_layout, A, B, C, D, M, N, K, lda, ldb, ldc, ldd, alpha, beta, nullptr, 0, stream_v);
 }
 
+MINFER_ATTN_EXPORT size_t minfer_gemm_layout_workspace_bytes(int b_layout, int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
+    int splits;   // the most slices that a route of gemm_impl cuts K into for this layout
+    if (b_layout == MINFER_GEMM_B_KN) splits = M <= kKnRows ? kn_slices(M, N, K) : gemm_splits(M, N, K);
+    else splits = std::max(stripe_slices(M, N, K), M > 16 ? gemm_splits(M, N, K) : 1);
+    return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+
 MINFER_ATTN_EXPORT size_t minfer_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
     const int splits = std::max(std::max(gemm_splits(M, N, K), stripe_slices(M, N, K)), kn_slices(M, N, K));
@@ -2003,7 +2011,7 @@ MINFER_ATTN_EXPORT size_t minfer_gemm_q8_0_workspace_bytes(int64_t M, int64_t N,
         const int slices = q8_slices(M, N, K);
         return slices > 1 ? (size_t)slices * (size_t)M * (size_t)N * sizeof(float) : 0;
     }
-    return q8_dequant_bytes(N, K) + minfer_gemm_workspace_bytes(M, N, K);
+    return q8_dequant_bytes(N, K) + minfer_gemm_layout_workspace_bytes(MINFER_GEMM_B_NK, M, N, K);
 }
 
 MINFER_ATTN_EXPORT int minfer_gemm_q8_0(const void* A, const void* Bq, const void* C, void* D, int64_t M, int64_t N, int64_t K,

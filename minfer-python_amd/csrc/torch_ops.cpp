@@ -458,7 +458,7 @@ void gemm_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype_size, double
         // through the dequantised weight like the shapes that kernel does not take
         const auto misaligned = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) != 0; };
         if (ws_bytes == 0 && (misaligned(A.const_data_ptr()) || misaligned(D.const_data_ptr()) || (beta != 0.0 && misaligned(C.const_data_ptr()))))
-            ws_bytes = ((static_cast<size_t>(N) * static_cast<size_t>(K) * 2 + 255) & ~static_cast<size_t>(255)) + minfer_gemm_workspace_bytes(M, N, K);
+            ws_bytes = ((static_cast<size_t>(N) * static_cast<size_t>(K) * 2 + 255) & ~static_cast<size_t>(255)) + minfer_gemm_layout_workspace_bytes(MINFER_GEMM_B_NK, M, N, K);
         Tensor ws = byte_workspace(A, ws_bytes);
         check_rc(minfer_gemm_q8_0(A.const_data_ptr(), B.const_data_ptr(), C.const_data_ptr(), D.mutable_data_ptr(), M, N, K, K, N, N,
                                   alpha, beta, ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, current_stream()),
@@ -479,7 +479,7 @@ void gemm_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype_size, double
     STD_TORCH_CHECK(C.sizes().equals(D.sizes()), "gemm: C and D shapes differ");
     STD_TORCH_CHECK(alpha != 0.0, "gemm: alpha must not be 0");
     // a few dozen rows against a wide weight run as K slices that meet in a workspace
-    const size_t ws_bytes = minfer_gemm_workspace_bytes(M, N, K);
+    const size_t ws_bytes = minfer_gemm_layout_workspace_bytes(kn ? MINFER_GEMM_B_KN : MINFER_GEMM_B_NK, M, N, K);
     Tensor ws = byte_workspace(A, ws_bytes);
     check_rc(minfer_gemm_ws(t == ScalarType::Half ? MINFER_ATTN_F16 : MINFER_ATTN_BF16, kn ? MINFER_GEMM_B_KN : MINFER_GEMM_B_NK,
                             A.const_data_ptr(), B.const_data_ptr(), C.const_data_ptr(), D.mutable_data_ptr(), M, N, K, K,
@@ -520,7 +520,7 @@ void qkv_hip(int64_t q_qtype_int, int64_t k_qtype_int, int64_t v_qtype_int, int6
         size_t ws_max = 0;
         for (int i = 0; i < 3; ++i) {
             const int64_t N = outs[i]->dim() == 3 ? outs[i]->size(-1) : 0;
-            const size_t need = qtypes[i] == MINFER_Q8_0 ? minfer_gemm_q8_0_workspace_bytes(M, N, K) : minfer_gemm_workspace_bytes(M, N, K);
+            const size_t need = qtypes[i] == MINFER_Q8_0 ? minfer_gemm_q8_0_workspace_bytes(M, N, K) : minfer_gemm_layout_workspace_bytes(MINFER_GEMM_B_NK, M, N, K);
             ws_max = need > ws_max ? need : ws_max;
         }
         Tensor wsp = byte_workspace(x, ws_max);

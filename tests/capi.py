@@ -63,6 +63,8 @@ def lib():
         L.minfer_gemm_ws.argtypes = [ctypes.c_int, ctypes.c_int, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, dbl, dbl, vp, ctypes.c_size_t, vp]
         L.minfer_gemm_workspace_bytes.restype = ctypes.c_size_t
         L.minfer_gemm_workspace_bytes.argtypes = [i64, i64, i64]
+        L.minfer_gemm_layout_workspace_bytes.restype = ctypes.c_size_t
+        L.minfer_gemm_layout_workspace_bytes.argtypes = [ctypes.c_int, i64, i64, i64]
         L.minfer_gemm_q8_0.restype = ctypes.c_int
         L.minfer_gemm_q8_0.argtypes = [vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, dbl, dbl, vp, ctypes.c_size_t, vp]
         L.minfer_gemm_q8_0_workspace_bytes.restype = ctypes.c_size_t

@@ -190,6 +190,21 @@ def test_gemm_workspace_sizes():
     assert ws(0, 4096, 4096) == 0 and ws(-1, 4096, 4096) == 0 and ws(64, 4096, 1 << 40) == 0
 
 
+def test_gemm_workspace_sizes_by_layout():
+    """What one layout can use: never more than the size for either, nothing for an [N, K] weight that no route cuts into slices."""
+    L = capi.lib()
+    by = lambda layout, *shape: L.minfer_gemm_layout_workspace_bytes(layout, *shape)
+    kn, nk = capi.GEMM_B_KN, capi.GEMM_B_NK
+    assert by(nk, 16, 1024, 1024) == 0 and by(kn, 16, 1024, 1024) == 8 * 16 * 1024 * 4      # 8 column tiles, slices of two steps
+    assert by(nk, 16, 14336, 4096) == 0 and by(kn, 16, 14336, 4096) == 2 * 16 * 14336 * 4
+    assert by(nk, 16, 4096, 14336) == 4 * 16 * 4096 * 4                                       # 64 stripes
+    assert by(nk, 256, 4096, 4096) == by(kn, 256, 4096, 4096) == 4 * 256 * 4096 * 4         # tiles
+    assert by(nk, 0, 4096, 4096) == by(kn, -1, 4096, 4096) == by(kn, 64, 4096, 1 << 40) == 0
+    for M in (1, 9, 16, 17, 40, 64, 65, 300):
+        for N, K in ((1024, 1024), (1000, 4096), (4096, 4096), (14336, 4096), (4096, 14336), (1536, 8960), (4100, 4096), (512, 100)):
+            assert max(by(kn, M, N, K), by(nk, M, N, K)) <= L.minfer_gemm_workspace_bytes(M, N, K)
+
+
 def test_q8_0_validation_rejects_before_launch():
     L = capi.lib()
     quant = lambda dtype=capi.F32, x=0x1000, y=0x2000, n=4, k=128: L.minfer_quant_q8_0(dtype, x, y, n, k, None)
