@@ -53,9 +53,9 @@ def make(M, N, K, layout, dtype, seed):
     (3000, 4104, 64, 2.0, 0.0),      # the same with ragged edges
     (33, 17, 50, 1.0, 1.0),          # nothing tileable: plain kernel
     (64, 64, 72, 1.0, 0.0),          # K not a multiple of 64: plain kernel
-    (8, 4096, 4096, 1.0, 0.0),       # a decode step's tokens: with an [N, K] weight, the kernel that streams it once
-    (64, 1024, 1792, 2.0, 3.0),      # its largest row count; K steps not a multiple of the eight waves
-    (48, 8192, 8192, 1.0, 0.0),      # more than 32 rows against a large weight: the tiled kernel again
+    (8, 4096, 4096, 1.0, 0.0),       # a decode step's tokens: kernels that stream the weight once
+    (64, 1024, 1792, 2.0, 3.0),      # their largest row count; K steps not a multiple of the eight waves
+    (48, 8192, 8192, 1.0, 0.0),      # more than 32 rows against a large weight
     (2048, 6144, 128, 1.0, 1.0),     # [N, K]: 256 x 192 tiles (one full round instead of three quarters of one)
     (1800, 6144, 64, 2.0, 3.0),      # the same with a ragged last tile row
     (30, 5200, 128, 2.0, 1.0),       # wide enough for two column groups per workgroup, the last one ragged
@@ -124,6 +124,8 @@ def test_gemm_matches_oracle(layout, dtype, M, N, K, alpha, beta):
     (KN, 257, 12296, 64, 2.0, 3.0),
     (KN, 520, 14344, 64, 1.0, 1.0),      # 192 x 256
     (KN, 385, 16392, 320, 2.0, 3.0),     # a last tile row of one row, an odd number of steps
+    (NK, 1545, 4904, 192, 2.0, 3.0),     # 128 x 128, two workgroups per unit: a width that larger tiles would round up
+    (KN, 1545, 4904, 192, 2.0, 3.0),
 ])
 def test_gemm_tiles_between_the_small_and_the_large_one(layout, dtype, M, N, K, alpha, beta):
     """Every element against torch's product in 64 bits, within the bound of assert_close."""
@@ -270,12 +272,12 @@ def test_qkv_op_and_reference_checks(kerns):
 @pytest.mark.parametrize("layout", [KN, NK])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K,alpha,beta", [
-    (64, 4096, 4096, 1.0, 0.0),      # 32 tiles, 8 slices of 8 steps
+    (64, 4096, 4096, 1.0, 0.0),      # [K, N]: 32 tiles of 128 columns, 8 slices of 8 steps; [N, K]: four slices of 64 stripes
     (100, 1032, 2048, 2.0, 3.0),     # ragged rows and columns, C read by the second kernel
     (256, 2048, 1024, 0.5, 1.0),     # two tile rows
     (40, 512, 1984, 1.0, 0.0),       # K steps (31) not a multiple of the slice count
-    (1, 4096, 4096, 1.0, 1.0),       # one row: with [K, N] the sliced tiles, with [N, K] still the few-row kernel
-    (24, 1024, 2048, 1.0, 1.0),      # 17-32 rows: with a workspace the sliced tiles for both layouts
+    (1, 4096, 4096, 1.0, 1.0),       # one row: with [K, N] slices of 128 columns, with [N, K] still the few-row kernel
+    (24, 1024, 2048, 1.0, 1.0),      # 17-32 rows: with a workspace [K, N] slices of 128 columns, [N, K] the sliced tiles
     (256, 8192, 1024, 1.0, 1.0),     # 128 tiles: two slices, so that two workgroups share a compute unit
     # [N, K] weights of fewer than 192 stripes of 64 columns: K slices of the stripe kernel
     (8, 5120, 5120, 2.0, 3.0),       # 80 stripes, three slices of 6, 7 and 7 segments

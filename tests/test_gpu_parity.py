@@ -105,7 +105,7 @@ def test_golden_decode_and_varlen():
     (1, 8, 2, 256, 64, "causal", False),     # benchmark configuration 1 shape
     (2, 8, 2, 320, 128, "causal", True),     # reference-style transposed views
     (2, 6, 2, 200, 128, "window", False),    # n_rep = 3, symmetric window (reference test case B)
-    (2, 4, 4, 333, 128, "random", False),    # L % 4 != 0: byte-wise mask path, per-batch masks
+    (2, 4, 4, 333, 128, "random", False),    # L % 4 != 0: mask rows at any byte, per-batch masks
     (1, 16, 2, 520, 64, "random", True),     # n_rep = 8
     (1, 12, 2, 136, 128, "blocky", False),   # n_rep = 6
     (1, 16, 1, 264, 128, "causal", False),   # n_rep = 16
@@ -113,8 +113,8 @@ def test_golden_decode_and_varlen():
     (1, 4, 2, 63, 64, "causal", False),
     (3, 4, 1, 65, 128, "full", False),
     (1, 4, 1, 1040, 128, "blocky", False),
-    # above 1024 rows the launch uses 8-wave workgroups (4-wave ones below): the same kinds of edges there
-    (1, 6, 2, 1093, 128, "random", False),   # n_rep = 3, byte-wise mask path
+    # above 1024 rows the pre-pass classifies the mask (few workgroups: two teams of four waves; eight waves are in the next test)
+    (1, 6, 2, 1093, 128, "random", False),   # n_rep = 3
     (1, 8, 1, 1100, 64, "window", True),     # n_rep = 8, D = 64, transposed views
     (2, 4, 4, 1029, 128, "causal", False),   # n_rep = 1, a last tile of 5 rows
 ])
@@ -127,6 +127,23 @@ def test_dense_matches_oracle(dtype, B, Hq, Hkv, L, D, kind, views):
     want = oracle.flash_attn(q, k, v, mask)
     assert not torch.isnan(out).any()
     assert max_err(out, want) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,L,kind", [
+    (3, 32, 8, 1093, "random"),    # n_rep = 4: 64 rows per workgroup, a last key tile of 5 rows
+    (3, 32, 4, 1100, "window"),    # n_rep = 8: 32 rows
+    (20, 4, 4, 1029, "causal"),    # n_rep = 1: 256 rows
+    (13, 6, 2, 1111, "blocky"),    # n_rep = 3: 256 rows, key tiles that no row attends
+])
+def test_dense_eight_waves(dtype, B, Hq, Hkv, L, kind):
+    """More than 384 workgroups of eight waves over more than 1024 rows, which is what takes them, at ragged sizes: every element
+    against the fp32 evaluation on the GPU."""
+    gen = torch.Generator().manual_seed(L)
+    q, k, v = workloads.dense_prefill(B, Hq, Hkv, L, 128, dtype, seed=L, scale=0.5, device=DEV)
+    mask = make_mask(kind, B, L, gen).to(DEV)
+    out = run_prefill(q, k, v, mask)
+    assert max_err(out, torch_ref(q, k, v, mask)) <= TOL[dtype]
 
 
 @pytest.mark.parametrize("Hq,Hkv,Lmax,D", [
@@ -352,9 +369,9 @@ def test_mask_rows_at_any_byte(B, L, D, offset):
     (3, 32, 8, 512, 128, "blocky"),    # more workgroups than fit on the chip at once: the pre-pass classifies
 ])
 def test_short_dense_masks_classified_inside_the_kernel(B, Hq, Hkv, L, D, kind):
-    """A short dense problem with 16-byte readable mask rows launches no classification pre-pass: each workgroup
-    classifies its own mask rows.  Checked against the oracle, and bit for bit against the same call with the mask at an
-    odd address, which takes the pre-pass and the byte-wise mask reads."""
+    """A short dense problem launches no classification pre-pass: each workgroup classifies its own mask rows.  Checked against
+    the oracle, bit for bit against the same call with the mask at an odd address and, up to 511 rows (from there on few
+    workgroups take two teams), bit for bit against a batch of copies, too many for the chip, which takes the pre-pass."""
     dtype = torch.float16
     gen = torch.Generator().manual_seed(77 * L + Hq)
     q, k, v = workloads.dense_prefill(B, Hq, Hkv, L, D, dtype, seed=L + Hq + 1, scale=0.5, device=DEV)
@@ -367,6 +384,10 @@ def test_short_dense_masks_classified_inside_the_kernel(B, Hq, Hkv, L, D, kind):
     shifted.copy_(md)
     assert shifted.data_ptr() % 16 == 1
     assert torch.equal(run_prefill(q, k, v, shifted), out)
+    if L < 512:
+        n = 512 // (B * Hkv) + 1                 # a workgroup per (batch entry, KV head) at least
+        many = run_prefill(*(t.repeat(n, 1, 1, 1) for t in (q, k, v, md)))
+        assert torch.equal(many.view(n, *out.shape), out.expand(n, *out.shape))
 
 
 def test_cpu_plumbing_config_on_gpu():
@@ -588,7 +609,7 @@ def test_varlen_matches_oracle_and_dense(dtype, Hq, Hkv, D, lens):
     assert capi.flash_attn_varlen(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), max(lens), out) == capi.OK, capi.last_error()
     torch.cuda.synchronize()
     assert max_err(out, oracle.flash_attn_varlen(q, k, v, cu)) <= TOL[dtype]
-    # max_seqlen chooses the workgroup shape (4 waves up to 1024 rows, 8 above; 0 = not known = T): the same bits either way
+    # max_seqlen sizes the launch and chooses the kernel (0, or one past T: not known): the same bits either way
     out0 = torch.full(q.shape, float("nan"), dtype=dtype, device=DEV)
     assert capi.flash_attn_varlen(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), 0, out0) == capi.OK, capi.last_error()
     out_big = torch.full(q.shape, float("nan"), dtype=dtype, device=DEV)
