@@ -821,7 +821,8 @@ constexpr int64_t kSmallWorkgroupMaxRows = 1024;
 // A launch of few workgroups of 8 waves ends with its longest one, on a chip that is half idle by then (under a causal mask a
 // workgroup has half of the longest one's tiles on average): up to one and a half of them per compute unit the small ones, which
 // share out in finer pieces, are ahead (4 / 8 waves, 32 heads over 8: L=1536 39.2 / 46.7 us, 1777 47.6 / 55.3, 3000 86.0 / 90.9,
-// 3500 107.6 / 106.7; 8 over 2: L=2048 44.9 / 57.2, 4096 84.2 / 106.2, B=2 L=8192 275 / 267).  A packed batch is counted by its
+// 3500 107.6 / 106.7; 8 over 2: L=2048 44.9 / 57.2, 4096 84.2 / 106.2, B=2 L=8192 275 / 267).  The rule cannot see the mask, and
+// windows go either way: 256 keys L=2500 32.8 / 37.6, L=1300 21.2 / 19.9.  A packed batch is counted by its
 // tokens and has short sequences' workgroups between, so up to one and a quarter (4 sequences to 1600 30.3 / 32.2, 2 of 64
 // heads over 8 27.4 / 26.7); heads that share K and V with no other head make 256-row workgroups of a sequence, whose
 // waves wait for the diagonal's: there up to 1536 rows (32 sequences to 1200, 24 over 8 145 / 159, 16 to 1600 118 / 121).

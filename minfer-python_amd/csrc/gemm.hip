@@ -6,8 +6,9 @@
 // ("A x B^T", the layout of its QKV projection, whose launcher is empty in the reference), C and D are [M, N].
 //
 // Design.  A workgroup (8 waves, two per SIMD) owns a 256 x 256 tile of D (128 x 128 with 4 waves for problems
-// too small to fill the chip with large tiles, sizes between the two where they fill it better: pick_tile) and walks K in steps of 64; the A and B panels of a step (32 KB
-// each) are copied global->LDS without passing through registers, double-buffered, one barrier per step
+// too small to fill the chip with large tiles, sizes between the two where they fill it better: pick_tile) and walks K in
+// steps of 64; the A and B panels of a step (32 KB each) are copied global->LDS without passing through registers into a
+// ring of two stages (three where the LDS holds them and a workgroup has its unit to itself), one barrier per step
 // (placed inside the step, so that the matrix pipe keeps running across step boundaries).
 // Every wave owns 128 (64) rows (m) x 64 columns (n) as 8 (4) x 4 accumulator blocks of 16x16
 // (v_mfma_f32_16x16x32) and computes the transposed product D^T = B^T A^T, so that a lane ends up with 4
@@ -116,9 +117,13 @@ template <class T> MA_DEV void store_result(const GemmParams& p, int m, int n, f
 // ---- K slices that meet inside the launch -------------------------------------------------------------------
 // A slice's sums go to the workspace; the workgroup of a tile that comes last (a counter per tile) adds the tile's slices up
 // and stores D: no second launch, which costs the host 2.7 us and the chip 4, as much as many of these products take
-// themselves.  The sums pass from one XCD's L2 to another's, so they are written and read with device-scope accesses, and a
-// workgroup counts itself only when its own have arrived.  Slices are added in their order whoever comes last, as
-// gemm_reduce_kernel adds them, which takes over where there are no counters (stream_counters: any stream but the null stream).
+// themselves.  The sums pass from one XCD's L2 to another's, so they are written and read with device-scope accesses, which
+// go past the L2s on both sides, and a workgroup counts itself only when its own have arrived (each thread waits for its stores,
+// the barrier for the threads).  The reader's loads come after the count: its value decides whether they run at all, thread 0
+// has it before the second barrier, and no load moves up over a barrier in the compiler or in the wave.  In the memory model
+// that is not an order, since nothing here is a release or an acquire; with both on the count it would be, and then every arrival
+// writes back its XCD's L2 and invalidates it (a single user's attention block, whose decode and output projection merge this way,
+// 37.7 -> 40.1 us).  Slices are added in their order whoever comes last, as gemm_reduce_kernel adds them, which takes over where there are no counters (stream_counters: any stream but the null stream).
 MA_DEV void store_slice4(const GemmParams& p, int slice, int m, int n, f32x4 v) {
     float* at = p.part + ((int64_t)slice * p.M + m) * p.N + n;
     if (!p.done) { *reinterpret_cast<f32x4*>(at) = v; return; }
@@ -980,7 +985,8 @@ static int launch_stripe(const GemmParams& p0, int blocks, hipStream_t stream) {
     return check_launch("gemm_stripe_kernel");
 }
 // A weight of fewer than 192 stripes: with a workspace, K slices bring the workgroups up to the chip's 256 compute units
-// (every slice four segments at least); the slices' sums are added up by gemm_reduce_kernel.  1 = no slices.
+// (every slice four segments at least); the slices' sums are added up by finish_slices or gemm_reduce_kernel (slice_counters).
+// 1 = no slices.
 static int stripe_slices(int64_t M, int64_t N, int64_t K) {
     const int64_t stripes = (N + 63) / 64;
     if (M < 1 || M > 64 || K % kStripeSeg != 0 || N % 8 != 0 || stripes >= 192) return 1;
@@ -1618,7 +1624,7 @@ static int gemm_splits(int64_t M, int64_t N, int64_t K) {
     if (tiles > 256 || kt < 8) return 1;
     int64_t s = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, kt / 4), 32));
     // 64-127 tiles get two or three slices that way and fill the chip once; twice as many, while a slice stays 16 steps long,
-    // keep two workgroups on a compute unit ([K,N] 4096 x 14336 at 1-16 rows: 27.5 -> 22 us; 128 rows 37 -> 32).  Tiles that
+    // keep two workgroups on a compute unit (128 rows of [K,N] 4096 x 14336 37 -> 32 us).  Tiles that
     // fill the chip by themselves (129-256) are cut in two only for long rows: the second launch and the partial sums cost
     // what the second workgroup per unit gains at K = 8192 and less (clocks settled, sliced / not: 512 x 8192 x 8192 89.0 /
     // 76.8 us, 1024 x 4096 x 4096 47.0 / 44.7, 256 x 14336 x 4096 47.5 / 44.9; 1024 x 4096 x 14336 134 / 146)
