@@ -3,7 +3,8 @@
 // Work decomposition.  One workgroup = 8 waves (two per SIMD, so one wave's softmax overlaps the
 // other's MFMAs) = one KV head x (HPW query heads of that KV head's GQA group) x (QBW consecutive
 // 32-row query blocks), HPW*QBW = 8, so the K/V tiles a workgroup stages in LDS are shared by
-// every query head of the group.  Each wave owns 32 query rows of one head (two blocks of 16) and keeps
+// every query head of the group.  Short sequences and launches of few workgroups take 4 waves
+// (prefill_waves), where a unit would have one such workgroup two teams of them (two_teams_pay).  Each wave owns 32 query rows of one head (two blocks of 16) and keeps
 // its Q fragments, the 64x32 score tile and the Dx32 output accumulator in registers.
 //
 // Per 64-key tile a wave computes S^T = K Q^T with v_mfma_f32_16x16x32 (K from LDS as the MFMA A operand,
@@ -14,7 +15,8 @@
 // double-buffered: the copy of tile t+1 is issued right after the barrier that opens tile t.  The K
 // fragments of a tile pass through a ring of two register buffers, refilled two chunks ahead.
 //
-// Query rows in, output rows out.  Every wave has a private 8 KiB LDS area.  Its 32 query rows
+// Query rows in, output rows out.  Every wave has a private 8 KiB LDS area (with 4 waves inside the
+// K/V stages).  Its 32 query rows
 // are copied there global->LDS as whole rows (full 128/256-byte lines per request) and read back
 // as MFMA fragments; at the end the normalised output goes through the same area so that the
 // wave stores whole rows as well.  Read straight into fragment layout, a load or store
@@ -22,8 +24,8 @@
 // no barrier is involved.
 //
 // Masking.  The reference operator takes an arbitrary dense bool mask [B,1,L,L]
-// (reference: src/minfer/kernels/torch_ext/csrc/cuda/flash_attn/op.cuh:28).  A pre-pass
-// classifies every 64x64 mask tile as none / all / mixed; the main kernel skips "none" tiles,
+// (reference: src/minfer/kernels/torch_ext/csrc/cuda/flash_attn/op.cuh:28).  A pre-pass, or in short
+// problems every workgroup for its own rows, classifies every 64x64 mask tile as none / all / mixed; the kernel skips "none" tiles,
 // runs "all" tiles unmasked and reads mask bytes only for "mixed" tiles, which keeps arbitrary
 // masks bit-exact while a causal mask costs one byte-read tile per row of tiles.
 #include <algorithm>

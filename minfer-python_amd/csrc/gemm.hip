@@ -123,7 +123,8 @@ template <class T> MA_DEV void store_result(const GemmParams& p, int m, int n, f
 // has it before the second barrier, and no load moves up over a barrier in the compiler or in the wave.  In the memory model
 // that is not an order, since nothing here is a release or an acquire; with both on the count it would be, and then every arrival
 // writes back its XCD's L2 and invalidates it (a single user's attention block, whose decode and output projection merge this way,
-// 37.7 -> 40.1 us).  Slices are added in their order whoever comes last, as gemm_reduce_kernel adds them, which takes over where there are no counters (stream_counters: any stream but the null stream).
+// 37.7 -> 40.1 us).  Slices are added in their order whoever comes last, as gemm_reduce_kernel adds them, which takes over where
+// there are no counters (stream_counters: any stream but the null stream).
 MA_DEV void store_slice4(const GemmParams& p, int slice, int m, int n, f32x4 v) {
     float* at = p.part + ((int64_t)slice * p.M + m) * p.N + n;
     if (!p.done) { *reinterpret_cast<f32x4*>(at) = v; return; }
