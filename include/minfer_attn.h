@@ -213,12 +213,12 @@ int minfer_gemm(int dtype, int b_layout, const void* A, const void* B, const voi
  * bytes of device memory (16-byte aligned; 0 = this shape does not use any), the K dimension is cut into slices
  * that run as separate workgroups and meet in the workspace as fp32 partial sums, which the last workgroup of a
  * tile (small sums on a device's null stream, stream 0) or a second kernel adds up, with the same result to the bit
- * (alpha, beta and C applied there, one rounding): slices of 128 x 128 or 128 x 256 tiles, or, up to 64 rows, of
+ * (alpha, beta and C applied there, one rounding): slices of tiles, or, up to 64 rows, of
  * 128-column tiles of a [K, N] weight, or of an [N, K] weight of fewer than 12288 columns, of 64-column stripes
  * (where two launches pay: from 9 rows on below 6144 columns, from 2 on rows of 8192 values and more of at most
  * 1536 columns, from 33 between 6144 and 12288 columns).  With a null workspace the call is minfer_gemm; a
- * workspace smaller than minfer_gemm_workspace_bytes is used only by a path whose slices fit in it, and up to 64
- * rows against a [K, N] weight for as many slices as it holds.  minfer_gemm_workspace_bytes is enough for either
+ * workspace smaller than minfer_gemm_workspace_bytes is used only by a path whose slices fit in it, and from 65 rows
+ * on, or against a [K, N] weight, for as many slices as it holds.  minfer_gemm_workspace_bytes is enough for either
  * layout; minfer_gemm_layout_workspace_bytes is what one of them (MINFER_GEMM_B_KN, MINFER_GEMM_B_NK) can use,
  * which up to 64 rows is often less.  No counterpart in the reference, whose gemm_cuda takes no scratch memory
  * (reference: gemm/op.cuh:218-316); same contract for the workspace as the attention entry points (contents need

@@ -23,7 +23,7 @@ EXT_SO = os.path.join(EXT_DIR, "_C.so")
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
-KERNEL_SOURCES = ["attn_prefill.hip", "attn_decode.hip", "rope.hip", "rmsnorm.hip", "gemm.hip", "quant.hip", "calib.hip", "attn_api.hip"]
+KERNEL_SOURCES = ["attn_prefill.hip", "attn_decode.hip", "rope.hip", "rmsnorm.hip", "gemm.hip", "gemm_tile_f16.hip", "gemm_tile_bf16.hip", "quant.hip", "calib.hip", "attn_api.hip"]
 
 
 def _run(cmd):
@@ -38,10 +38,18 @@ def asm_hazards(asm_text):
     """Distances the compiler cannot keep because one end is inside an asm statement, looked for in the device code:
     (1) a global->LDS copy (always emitted from asm here) whose scalar address pair was written by a vector instruction
         (readfirstlane / readlane) fewer than five instructions earlier;
-    (2) a matrix instruction that reads a register written inside an asm statement fewer than two instructions earlier.
+    (2) a matrix instruction that reads a register written inside an asm statement fewer than two instructions earlier;
+    (3) an instruction outside asm statements that touches an accumulation register fewer than 18 issue slots after a matrix
+        instruction inside one wrote it (16x16x32: 11 are needed).
     Returns a list of (function, offending instruction, the write it follows too closely)."""
     import re
     found, func, window, in_asm = [], "?", [], False
+
+    def acc_regs(text):
+        regs = set()
+        for m in re.finditer(r"\ba(?:\[(\d+):(\d+)\]|(\d+)\b)", text):
+            regs.update(range(int(m.group(1)), int(m.group(2)) + 1) if m.group(1) else (int(m.group(3)),))
+        return regs
     for raw in asm_text.split("\n"):
         line = raw.strip()
         if line.startswith(";;#ASMSTART"):
@@ -85,9 +93,21 @@ def asm_hazards(asm_text):
                         hi = int(d.group(2)) if d.lastindex and d.lastindex >= 2 else lo
                         if srcs.intersection(range(lo, hi + 1)):
                             found.append((func, line, prev))
+        if not in_asm and window:
+            touched = acc_regs(line)
+            states = 0
+            for prev, prev_in_asm in reversed(window) if touched else ():
+                if states >= 18:
+                    break
+                if prev_in_asm and prev.startswith("v_mfma") and touched.intersection(acc_regs(prev.split(",", 1)[0])):
+                    found.append((func, line, prev))
+                n = re.match(r"s_nop (\d+)", prev)
+                states += int(n.group(1)) + 1 if n else 1
         window.append((line, in_asm))
-        if len(window) > 8:
+        if len(window) > 20:
             window.pop(0)
+        if op in ("s_branch", "s_endpgm"):
+            window = []   # what stands next in the text does not run next
     return found
 
 

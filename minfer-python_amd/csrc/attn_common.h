@@ -138,6 +138,15 @@ MA_DEV void copy16_global_to_lds(const void* uniform_base, uint32_t lane_byte_of
                      : "memory", "m0");
 }
 
+// Same, for a loop that counts its issue slots: the destination as a wave-uniform LDS address plus a compile-time offset (three
+// instructions; from a generic pointer the address costs two to four more).  The base must be a scalar value long before the call.
+template <int LDS_OFFSET> MA_DEV void copy16_global_to_lds_at(const void* uniform_base, uint32_t lane_byte_offset, uint32_t lds_uniform) {
+    asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
+                 :
+                 : "s"(lds_uniform), "i"(LDS_OFFSET), "v"(lane_byte_offset), "s"((uint64_t)(uintptr_t)uniform_base)
+                 : "memory", "m0", "scc");
+}
+
 // 32-bit LDS address of a __shared__ object, and reads at such an address plus a compile-time offset
 // (which the instruction carries as an immediate, so one address register serves many reads).
 MA_DEV uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(lds_void*)p; }

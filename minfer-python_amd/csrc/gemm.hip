@@ -5,114 +5,19 @@
 // dims flattened), B is the weight either as [K, N] ("A x B", what its tuned kernel handles) or as [N, K]
 // ("A x B^T", the layout of its QKV projection, whose launcher is empty in the reference), C and D are [M, N].
 //
-// Design.  A workgroup (8 waves, two per SIMD) owns a 256 x 256 tile of D (128 x 128 with 4 waves for problems
-// too small to fill the chip with large tiles, sizes between the two where they fill it better: pick_tile) and walks K in
-// steps of 64; the A and B panels of a step (32 KB each) are copied global->LDS without passing through registers into a
-// ring of two stages (three where the LDS holds them and a workgroup has its unit to itself), one barrier per step
-// (placed inside the step, so that the matrix pipe keeps running across step boundaries).
-// Every wave owns 128 (64) rows (m) x 64 columns (n) as 8 (4) x 4 accumulator blocks of 16x16
-// (v_mfma_f32_16x16x32) and computes the transposed product D^T = B^T A^T, so that a lane ends up with 4
-// consecutive n of one row m and the epilogue stores 8 bytes per block: B supplies the MFMA A operand (for the
-// [K, N] layout through LDS transpose reads, the same way the attention kernel reads V^T; for [N, K] through
-// plain 16-byte reads) and A supplies the B operand (16-byte reads).  LDS panels are split into sub-tiles
-// with XOR swizzles of the kind the attention kernel's K and V tiles use, so both read patterns are free of bank
-// conflicts.  Workgroup ids are dealt so that one XCD works on consecutive tiles of a tile row (they share the
-// A panel in that XCD's L2).
+// Design.  From 65 rows on a workgroup of four waves owns a tile of D of 128 to 256 rows and columns (gemm_tile.h) and walks K in
+// steps of 64; the A and B panels of a step are copied global->LDS without passing through registers into a ring of two or three
+// stages, one barrier per step.  Which tile, and whether K is cut into slices that meet in a workspace, is what plan_tiles estimates
+// to be quickest.  Up to 64 rows the work is reading the weight once: the kernels of this file.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
+#include <utility>
 
-#include "attn_common.h"
-#include "attn_host.h"
+#include "gemm_common.h"
 #include "quant_q8.h"
 
 namespace minfer_attn {
-
-
-constexpr int kBK = 64;
-// Tile shapes: 8 waves (2 x 4) on 256 x 256 where the problem fills the chip with such tiles, smaller ones where it does not
-// (pick_tile).  A wave owns M16 x N16 blocks of 16 x 16; OCC waves per SIMD.
-template <int M16_, int N16_, int WAVES_N_, int OCC_, int WAVES_M_ = 2, int NS_ = 2> struct GemmShape {
-    static constexpr int M16 = M16_, N16 = N16_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, WAVES = WAVES_M * WAVES_N, OCC = OCC_;
-    static constexpr int NS = NS_;   // stages of the K ring in LDS: NS - 1 steps in flight while one is multiplied
-    static constexpr int BM = 16 * M16 * WAVES_M, BN = 16 * N16 * WAVES_N;
-    static constexpr int A_PANEL = BM * 128, B_PANEL = BN * 128;   // bytes of one K step
-    // wave-wide copies (1 KiB) per wave and K step; every wave makes the same number, so that they can be counted: where the A
-    // panel's do not come out even the last waves copy a piece again (the same bytes to the same place)
-    static constexpr int A_PIECES = A_PANEL / 1024, A_COPIES = (A_PIECES + WAVES - 1) / WAVES, B_COPIES = B_PANEL / 1024 / WAVES;
-    static_assert(B_PANEL % (1024 * WAVES) == 0 && A_PIECES >= WAVES, "whole copies");
-};
-// (4 waves with 128 x 128 each, GemmShape<4, 4, 2, 1>, read a third fewer LDS bytes per flop.  Compiled as it stands
-// that shape spills: its 256 accumulators leave the allocator no register to move anything with.  On 32 x 32 blocks,
-// with 14 of the 16 accumulator blocks pinned to the accumulation registers and 2 to the vector registers by inline
-// assembly, it was spill-free and ended level with the 8-wave shape at 4096^3 and 4 % behind at 8192^3.)
-using GemmBig = GemmShape<8, 4, 4, 2>;
-using GemmSmall = GemmShape<4, 4, 2, 2>;
-// The same tile with three stages (96 KiB of LDS: one workgroup per compute unit) for launches of at most one workgroup per
-// compute unit anyway: two steps in flight instead of one (clocks settled, 512 x 6144 x 4096 as 192 tiles 43.6 -> 36.6 us,
-// 1024 x 4096 x 4096 as 256 tiles 44.9 -> 40.1, 256 x 14336 x 4096 44.9 -> 38.5; with more workgroups than compute units
-// two resident workgroups of two stages are ahead, 2048 x 4096 x 4096 66.9 against 78.6; four stages lose to three throughout).
-using GemmSmall3 = GemmShape<4, 4, 2, 2, 2, 3>;
-static bool one_workgroup_per_unit(int64_t workgroups) { return workgroups <= 256; }
-// Sizes in between, for problems whose 256 x 256 tiles would leave much of the chip idle in their only or last round.  All run
-// at what the LDS and the barrier of a K step leave, 5-20 % below the large tile's rate per flop, so they pay where they save a
-// half-empty round.
-// 256 x 192 (8 waves as 4 x 2, a wave owns 64 x 96), [N, K] weights only: its 192 columns are three 64-row sub-tiles of such a
-// weight, but one and a half of the 128-column sub-tiles of a [K, N] one (4096 x 6144 x 4096: 512 tiles, two full rounds,
-// where the large ones take one and a half; 1200 x 28672 x 4096 294 -> 268 us).
-using GemmWide = GemmShape<4, 6, 2, 2, 4>;
-// 192 x 256, for [K, N] weights in its place (2500 x 4096 x 4096: 160 large tiles 87 us, 224 of these 77).
-using GemmRows192 = GemmShape<6, 4, 4, 2>;
-// 160 x 256, [N, K] weights: the odd row counts (600 x 14336 x 4096: 168 large tiles 97-99 us, 224 of these 75-78).  156 KiB of LDS
-// hold three stages, which a weight that comes from memory needs at this size of step (two stages: 82-83 us; a [K, N]
-// weight gains nothing over 192 x 256).
-using GemmRows160 = GemmShape<5, 4, 4, 2, 2, 3>;
-// 128 x 256, three stages: half the large tile as one workgroup instead of two of 128 x 128, a quarter fewer bytes copied per flop
-// (300 x 14336 x 4096 67 -> 58 us, [K, N] 900 x 8192 x 8192 142 -> 132, 1777 x 4096 x 4096 64 -> 61).
-using GemmFlat = GemmShape<4, 4, 4, 2, 2, 3>;
-constexpr int kRowTile = 8192;              // sub-tile [64 rows][64 k], 128-byte rows (A, and B as [N, K])
-constexpr int kColTile = 16384;             // sub-tile [64 k][128 n], 256-byte rows (B as [K, N])
-
-// Several weights that share A in one launch (the QKV projection): the column tiles (tiled kernel) or column groups
-// (few-row kernel) of weight s follow those of weight s - 1; `end` holds the cumulative counts.  No C operand.
-constexpr int kMaxGroup = 3;
-struct GemmGroup {
-    const void* B[kMaxGroup]; void* D[kMaxGroup];
-    int N[kMaxGroup], end[kMaxGroup];
-    int64_t ldb[kMaxGroup], ldd[kMaxGroup];
-};
-struct GemmParams {
-    const void* A; const void* B; const void* C; void* D;
-    int M, N, K;
-    int64_t lda, ldb, ldc, ldd;   // row strides in elements
-    float alpha, beta;
-    int tiles_m, tiles_n, per_xcd;
-    int splits;                   // SPLIT instantiations: K is cut into this many slices, one workgroup per (tile, slice)
-    float* part;                  // their fp32 partial products, [splits][M][N]
-    uint32_t* done;               // zeroed arrival counters, one per tile (stripe), left zero; null: gemm_reduce_kernel adds the slices up
-    GemmGroup grp;                // used by the GROUPED instantiations only
-};
-// Which weight column unit `c` (a tile column or a column group) belongs to, and its index inside that weight.
-MA_DEV int group_of_unit(const GemmGroup& g, int c, int& local) {
-    const int s = c < g.end[0] ? 0 : (c < g.end[1] ? 1 : 2);
-    local = c - (s == 0 ? 0 : (s == 1 ? g.end[0] : g.end[1]));
-    return s;
-}
-
-// Four consecutive columns of D from the sums in fp32: alpha, beta and C, one rounding.
-template <class T> MA_DEV void store_result(const GemmParams& p, int m, int n, f32x4 sum) {
-    float v[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = p.alpha * sum[e];
-    if (p.beta != 0.f) {
-        const s16x4 c = *reinterpret_cast<const s16x4*>((const short*)p.C + (int64_t)m * p.ldc + n);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += p.beta * T::to_float(c[e]);
-    }
-    uint2 pk;
-    pk.x = T::pack2(v[0], v[1]);
-    pk.y = T::pack2(v[2], v[3]);
-    *reinterpret_cast<uint2*>((short*)p.D + (int64_t)m * p.ldd + n) = pk;
-}
 
 // ---- K slices that meet inside the launch -------------------------------------------------------------------
 // A slice's sums go to the workspace; the workgroup of a tile that comes last (a counter per tile) adds the tile's slices up
@@ -177,287 +82,6 @@ MA_DEV void finish_slices(const GemmParams& p, int tile, int m0, int m1, int n0,
         }
         store_result<T>(p, m[0], n[0], sum[0]);
         if (i0 + THREADS < total) store_result<T>(p, m[1], n[1], sum[1]);
-    }
-}
-
-// swizzles: granule index of a row XORed with a function of the row (see the attention kernel's TileGeom)
-MA_DEV int swz_row_tile(int row) { return (row >> 1) & 7; }        // 128-byte rows, read 32 rows x 16 bytes
-MA_DEV int swz_col_tile(int row) { return ((row & 3) << 2) | ((row >> 2) & 2); }   // 256-byte rows, transposing reads of 4 rows x 32 bytes by each of two 16-lane groups 8 rows apart
-
-// CONCAT (with GROUPED, [N, K] weights whose widths are multiples of 64): the weights' columns are numbered through as
-// one wide matrix (p.N columns) and tiled without regard to where one weight ends, so a tile may hold columns of two weights; every
-// 64-column sub-tile of the B panel and every 32-column block of a wave lies inside one weight, which is looked up
-// per copy instruction and per block (grp.end = cumulative column counts).
-template <class T, bool NT, class SH, bool GROUPED = false, bool SPLIT = false, bool CONCAT = false>
-__global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const GemmParams p) {
-    static_assert(!CONCAT || (GROUPED && NT && !SPLIT && SH::WAVES == 8), "CONCAT: grouped [N, K] weights, one sub-tile per copy index");
-    constexpr int kBM = SH::BM, kBN = SH::BN, NW = SH::WAVES, CA = SH::A_COPIES, CB = SH::B_COPIES;
-    constexpr int NS = SH::NS;
-    static_assert(NS >= 2 && NS <= 4, "two to four stages");
-    __shared__ __attribute__((aligned(1024))) char a_lds[NS][SH::A_PANEL];
-    __shared__ __attribute__((aligned(1024))) char b_lds[NS][SH::B_PANEL];
-
-    const int lane = threadIdx.x & 63, w = wave_id();
-    const int h = lane >> 5, l32 = lane & 31;
-    const int wm = w % SH::WAVES_M, wn = w / SH::WAVES_M;   // wave's place in the tile: rows 16*M16*wm .., columns 16*N16*wn ..
-    static_assert(NT || SH::BN % 128 == 0, "a [K, N] weight is staged in sub-tiles of 128 columns");
-
-    // ---- which tile ----------------------------------------------------------------------------------
-    // (SPLIT: consecutive workgroup ids are the K slices of one tile, so the slices of a tile run on different XCDs)
-    const int unit = SPLIT ? (int)blockIdx.x : (int)(blockIdx.x & 7) * p.per_xcd + (int)(blockIdx.x >> 3);
-    const int slice = SPLIT ? unit % p.splits : 0;
-    const int t = SPLIT ? unit / p.splits : unit;
-    if (t >= p.tiles_m * p.tiles_n) return;
-    // Tiles are numbered down bands of kGroupM tile rows, so that the tiles an XCD runs at one time form a block that
-    // shares A row panels as well as B column panels in its L2 (row-major numbering made every XCD read all of B).
-    constexpr int kGroupM = 4;
-    const int band = t / (kGroupM * p.tiles_n), in_band = t % (kGroupM * p.tiles_n);
-    const int first_m = band * kGroupM, gm = min(kGroupM, p.tiles_m - first_m);
-    const int m0 = (first_m + in_band % gm) * kBM;
-    int n0 = (in_band / gm) * kBN;
-
-    const short* Ag = (const short*)p.A;
-    const short* Bg = (const short*)p.B;
-    short* Dg = (short*)p.D;
-    int N = p.N;
-    int64_t ldb = p.ldb, ldd = p.ldd;
-    if (GROUPED && !CONCAT) {   // the tile column's weight, output and place inside them (all wave-uniform)
-        int local;
-        const int sg = group_of_unit(p.grp, in_band / gm, local);
-        n0 = local * kBN;
-        Bg = (const short*)(sg == 0 ? p.grp.B[0] : sg == 1 ? p.grp.B[1] : p.grp.B[2]);
-        Dg = (short*)(sg == 0 ? p.grp.D[0] : sg == 1 ? p.grp.D[1] : p.grp.D[2]);
-        N = sg == 0 ? p.grp.N[0] : sg == 1 ? p.grp.N[1] : p.grp.N[2];
-        ldb = sg == 0 ? p.grp.ldb[0] : sg == 1 ? p.grp.ldb[1] : p.grp.ldb[2];
-        ldd = sg == 0 ? p.grp.ldd[0] : sg == 1 ? p.grp.ldd[1] : p.grp.ldd[2];
-    }
-
-    // ---- global -> LDS copies: lane offsets (bytes) from the panel's first element ---------------------
-    // Every wave issues 4 wave-wide copies (1 KB each) per panel and K step; copy q = j*NW + w of a panel covers
-    //   A (and B as [N, K]): rows 8*(q%8) .. +7 of sub-tile q/8 (64 rows of 128 bytes each);
-    //   B as [K, N]:         k rows 4*(q%16) .. +3 of sub-tile q/16 (64 k rows of 256 bytes, 128 columns).
-    uint32_t a_off[CA], b_off[CB];
-    int a_dst[CA], b_dst[CB];
-    const short* b_src[CONCAT ? CB : 1];   // CONCAT: first weight row of copy j's sub-tile (wave-uniform)
-#pragma unroll
-    for (int j = 0; j < CA; ++j) {
-        const int q = j * NW + w < SH::A_PIECES ? j * NW + w : (j - 1) * NW + w;
-        const int sub = q >> 3, row = 8 * (q & 7) + (lane >> 3), pg = lane & 7;
-        const int m = min(m0 + 64 * sub + row, p.M - 1) - m0;
-        a_off[j] = (uint32_t)((int64_t)m * p.lda + 8 * (pg ^ swz_row_tile(row))) * 2u;
-        a_dst[j] = sub * kRowTile + 8 * (q & 7) * 128;
-    }
-#pragma unroll
-    for (int j = 0; j < CB; ++j) {
-        const int q = j * NW + w;
-        if (CONCAT) {   // copy j of every wave lies in sub-tile j, whose 64 weight rows belong to one weight
-            const int row = 8 * (q & 7) + (lane >> 3), pg = lane & 7;
-            int local;
-            const int sg = group_of_unit(p.grp, min(n0 + 64 * j, p.N - 64), local);   // (past the last weight: its last columns)
-            const int64_t ldj = sg == 0 ? p.grp.ldb[0] : sg == 1 ? p.grp.ldb[1] : p.grp.ldb[2];
-            b_src[j] = (const short*)(sg == 0 ? p.grp.B[0] : sg == 1 ? p.grp.B[1] : p.grp.B[2]) + (int64_t)local * ldj;
-            b_off[j] = (uint32_t)((int64_t)row * ldj + 8 * (pg ^ swz_row_tile(row))) * 2u;
-            b_dst[j] = j * kRowTile + 8 * (q & 7) * 128;
-        } else if (NT) {
-            const int sub = q >> 3, row = 8 * (q & 7) + (lane >> 3), pg = lane & 7;
-            const int n = min(n0 + 64 * sub + row, N - 1) - n0;
-            b_off[j] = (uint32_t)((int64_t)n * ldb + 8 * (pg ^ swz_row_tile(row))) * 2u;
-            b_dst[j] = sub * kRowTile + 8 * (q & 7) * 128;
-        } else {
-            const int sub = q >> 4, row = 4 * (q & 15) + (lane >> 4), pg = lane & 15;
-            const int col = min(n0 + 128 * sub + 8 * (pg ^ swz_col_tile(row)), N - 8) - n0;
-            b_off[j] = (uint32_t)((int64_t)row * ldb + col) * 2u;
-            b_dst[j] = sub * kColTile + 4 * (q & 15) * 256;
-        }
-    }
-    // K steps of this workgroup: all of them, or its slice
-    const int kt_all = p.K / kBK;
-    const int kt_first = SPLIT ? (int)((int64_t)slice * kt_all / p.splits) : 0;
-    const int KT = SPLIT ? (int)((int64_t)(slice + 1) * kt_all / p.splits) - kt_first : kt_all;
-    // (With three stages the compiler runs out of scalar registers in some instantiations and moves the panel bases from
-    // vector registers right in front of every copy, closer than a copy may follow such a move: those wait the documented
-    // distance inside the copy, see copy16_global_to_lds; the build's scan of the generated code is what finds such cases.)
-    constexpr bool kFreshBases = SH::NS > 2;
-    // copy c of a step (the wave's A copies, then its B copies) into a stage
-    auto copy_one = [&](int kt_rel, int stage, int c) __attribute__((always_inline)) {
-        const int kt = kt_first + kt_rel;
-        if (c < CA) {
-            copy16_global_to_lds<kFreshBases>(Ag + (int64_t)m0 * p.lda + (int64_t)kt * kBK, a_off[c], &a_lds[stage][a_dst[c]]);
-        } else {
-            const int j = c - CA;
-            const short* bbase = NT ? Bg + (int64_t)n0 * ldb + (int64_t)kt * kBK : Bg + (int64_t)kt * kBK * ldb + n0;
-            copy16_global_to_lds<kFreshBases>(CONCAT ? b_src[CONCAT ? j : 0] + (int64_t)kt * kBK : bbase, b_off[j], &b_lds[stage][b_dst[j]]);
-        }
-    };
-    auto issue = [&](int kt_rel, int stage) __attribute__((always_inline)) {
-#pragma unroll
-        for (int c = 0; c < CA + CB; ++c) copy_one(kt_rel, stage, c);
-    };
-
-    // ---- per-lane LDS read addresses (stage 0; stage, sub-tile and block offsets are immediates) ---------
-    // The matrix instruction is v_mfma_f32_16x16x32 (on random fp16 operands the chip sustains 1.80-1.90 PFLOP/s of it and
-    // 1.56-1.62 of v_mfma_f32_32x32x16, and a power-bound GEMM runs at what its matrix instruction sustains).  A K step is two slices of
-    // 32 values; a fragment is 16 rows x 32 k, lane (l16, quad) holding row l16, k = 8 quad + 0..7 of the slice: 16 bytes
-    // at granule (4 slice + quad) ^ swizzle of the row.  A 16-row block is a quarter of a 64-row sub-tile; the swizzle of
-    // row 16 b + l16 does not depend on b.
-    constexpr int M16 = SH::M16, N16 = SH::N16, BLK = kRowTile / 4;
-    const int l16 = lane & 15, quad = lane >> 4;
-    constexpr int NRD = N16 < 4 ? 4 : N16;
-    uint32_t m_rd[2], n_rd[NRD];
-    {
-        const int sw = swz_row_tile(l16);
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const uint32_t o = l16 * 128 + 16 * ((4 * ks + quad) ^ sw);
-            m_rd[ks] = lds_addr(&a_lds[0][0]) + M16 * wm * BLK + o;
-            if (NT) n_rd[ks] = lds_addr(&b_lds[0][0]) + N16 * wn * BLK + o;    // n fragments: as the m fragments
-        }
-        if (!NT) {
-            // n fragments through transpose reads of the [k][n] sub-tile: the 16-lane group `quad` addresses k rows
-            // 8 quad + 0..3 (second read: + 4) of the slice, 16 columns, and lane l16 receives column l16
-            const int krow = 8 * quad + (l16 >> 2);
-            const int swv = swz_col_tile(krow);
-#pragma unroll
-            for (int nb = 0; nb < NRD; ++nb) {
-                const int n = 16 * (N16 * wn + (nb < N16 ? nb : 0)), col = (n & 127) + 4 * (l16 & 3);
-                n_rd[nb] = lds_addr(&b_lds[0][0]) + (n >> 7) * kColTile + krow * 256 + 16 * ((col >> 3) ^ swv) + 2 * (col & 7);
-            }
-        }
-    }
-
-    f32x4 acc[N16][M16];
-#pragma unroll
-    for (int nb = 0; nb < N16; ++nb)
-#pragma unroll
-        for (int mb = 0; mb < M16; ++mb) acc[nb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // n fragment nb / m fragment mb of slice ks of a stage
-    auto read_n = [&](auto stage_tag, int ks, int nb) __attribute__((always_inline)) -> s16x8 {
-        constexpr int BOFF = decltype(stage_tag)::value * SH::B_PANEL;
-        if (NT) return lds_read_b128(n_rd[ks], BOFF + nb * BLK);
-        const s16x4 t0 = lds_read_tr16(n_rd[nb], BOFF + (32 * ks) * 256);
-        const s16x4 t1 = lds_read_tr16(n_rd[nb], BOFF + (32 * ks + 4) * 256);
-        return s16x8{t0[0], t0[1], t0[2], t0[3], t1[0], t1[1], t1[2], t1[3]};
-    };
-    auto read_m = [&](auto stage_tag, int ks, int mb) __attribute__((always_inline)) -> s16x8 {
-        constexpr int AOFF = decltype(stage_tag)::value * SH::A_PANEL;
-        return lds_read_b128(m_rd[ks], AOFF + mb * BLK);
-    };
-    // ---- main loop ---------------------------------------------------------------------------------------
-    // A slice is N16 groups of M16 MFMAs (group nb: n fragment nb against every m fragment).  The n fragments are
-    // double-buffered: the next slice's are read during groups 1 .. N16-2, one read after an MFMA; the m fragments have
-    // one buffer, refilled in the last group, fragment mb right after the last MFMA that uses it.  The workgroup's only
-    // barrier per K step sits after group 0 of the step's second slice: by then every read of the stage has returned
-    // (the last were issued a group earlier) and the wave's share of the next stage's copy, issued a whole step
-    // before, has landed; what follows the barrier reads the next stage and copies the step after next into the stage
-    // just vacated, one copy after an MFMA.  Every MFMA, read and copy is pinned where it is written (scheduling
-    // barriers): left alone the compiler moves reads down to just before their use, where nothing of the wave covers
-    // their latency.
-    s16x8 nf[2][N16], mf[M16];
-    constexpr int NC = CA + CB;
-    constexpr int MID = (N16 - 2) * M16;    // MFMAs of groups 1 .. N16-2
-    auto pin = [&]() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
-    // one slice: MFMAs on nf[buf] and mf; `next_tag`/`ks_next` name the slice read meanwhile (has_next: there is one);
-    // SECOND: the step's second slice, with the barrier after group 0 and, if copy_kt >= 0, that step's copies after it
-    // this wave's copies of all but the `later` most recently issued steps have landed (copies retire in order)
-    auto wait_stages = [&](int later) __attribute__((always_inline)) {
-        if (NS >= 4 && later >= 3) wait_vmcnt<(NS >= 4 ? 3 : 0) * NC>();
-        else if (NS >= 3 && later == 2) wait_vmcnt<(NS >= 3 ? 2 : 0) * NC>();
-        else if (later == 1) wait_vmcnt<NC>();
-        else wait_vmcnt<0>();
-    };
-    auto k_slice = [&](auto next_tag, int ks_next, int buf, bool has_next, auto second_tag, int copy_kt, auto stage_tag, int later = 0) __attribute__((always_inline)) {
-        constexpr bool SECOND = decltype(second_tag)::value;
-        constexpr int STAGE = decltype(stage_tag)::value;
-#pragma unroll
-        for (int nb = 0; nb < N16; ++nb) {
-#pragma unroll
-            for (int mb = 0; mb < M16; ++mb) {
-                acc[nb][mb] = T::mfma16(nf[buf][nb], mf[mb], acc[nb][mb]);
-                pin();
-                if (nb >= 1 && nb <= N16 - 2) {
-                    const int i = (nb - 1) * M16 + mb;   // 0 .. MID-1
-                    if (has_next) {
-#pragma unroll
-                        for (int r = (N16 * i + MID - 1) / MID; r < (N16 * (i + 1) + MID - 1) / MID; ++r) nf[buf ^ 1][r] = read_n(next_tag, ks_next, r);
-                    }
-                    if (SECOND && copy_kt >= 0) {
-#pragma unroll
-                        for (int c = (NC * i + MID - 1) / MID; c < (NC * (i + 1) + MID - 1) / MID; ++c) copy_one(copy_kt, STAGE, c);
-                    }
-                } else if (nb == N16 - 1) {
-                    if (has_next) mf[mb] = read_m(next_tag, ks_next, mb);
-                }
-                pin();
-            }
-            if (SECOND && nb == 0) {
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave has read everything it needs from this stage
-                wait_stages(later);                                    // and its share of the next stage has landed
-                __syncthreads();
-                pin();
-            }
-        }
-    };
-    auto step = [&](auto stage_tag, int kt) __attribute__((always_inline)) {
-        constexpr int STAGE = decltype(stage_tag)::value;
-        using Next = std::integral_constant<int, (STAGE + 1) % NS>;
-        pin();
-        k_slice(stage_tag, 1, 0, true, std::false_type{}, -1, stage_tag);
-        // at the barrier the next step's stage must have landed; the steps after it, up to NS - 2 of them, may be in flight
-        k_slice(Next{}, 0, 1, kt + 1 < KT, std::true_type{}, kt + NS < KT ? kt + NS : -1, stage_tag, min(NS - 2, KT - 2 - kt));
-    };
-#pragma unroll
-    for (int st = 0; st < NS; ++st)
-        if (st < KT) issue(st, st);
-    wait_stages(min(NS, KT) - 1);   // the copies of step 0 retire first
-    __syncthreads();
-#pragma unroll
-    for (int nb = 0; nb < N16; ++nb) nf[0][nb] = read_n(std::integral_constant<int, 0>{}, 0, nb);
-#pragma unroll
-    for (int mb = 0; mb < M16; ++mb) mf[mb] = read_m(std::integral_constant<int, 0>{}, 0, mb);
-    for (int kt = 0; kt < KT; kt += NS) {
-        step(std::integral_constant<int, 0>{}, kt);
-        if (kt + 1 < KT) step(std::integral_constant<int, 1>{}, kt + 1);
-        if constexpr (NS > 2) if (kt + 2 < KT) step(std::integral_constant<int, 2 % NS>{}, kt + 2);
-        if constexpr (NS > 3) if (kt + 3 < KT) step(std::integral_constant<int, 3 % NS>{}, kt + 3);
-    }
-
-    // ---- epilogue: D = alpha * acc + beta * C; register e of a block is n = 4 quad + e, m = l16 ----
-    const short* Cg = (const short*)p.C;
-#pragma unroll
-    for (int mb = 0; mb < M16; ++mb) {
-        const int m = m0 + 16 * M16 * wm + 16 * mb + l16;
-        if (m >= p.M) continue;
-#pragma unroll
-        for (int nb = 0; nb < N16; ++nb) {
-            int nb0 = n0 + 16 * N16 * wn + 16 * nb;   // first column of the block
-            if (CONCAT) {                              // ... inside the weight that holds the block
-                if (nb0 >= p.N) continue;
-                int local;
-                const int sg = group_of_unit(p.grp, nb0, local);
-                nb0 = local;
-                Dg = (short*)(sg == 0 ? p.grp.D[0] : sg == 1 ? p.grp.D[1] : p.grp.D[2]);
-                ldd = sg == 0 ? p.grp.ldd[0] : sg == 1 ? p.grp.ldd[1] : p.grp.ldd[2];
-            }
-            const int n = nb0 + 4 * quad;
-            if (!CONCAT && n >= N) continue;
-            if (SPLIT) {   // the slice's raw sums
-                *reinterpret_cast<f32x4*>(p.part + ((int64_t)slice * p.M + m) * p.N + n) = acc[nb][mb];
-                continue;
-            }
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = p.alpha * acc[nb][mb][e];
-            if (p.beta != 0.f) {
-                const s16x4 c = *reinterpret_cast<const s16x4*>(Cg + (int64_t)m * p.ldc + n);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] += p.beta * T::to_float(c[e]);
-            }
-            uint2 pk;
-            pk.x = T::pack2(v[0], v[1]);
-            pk.y = T::pack2(v[2], v[3]);
-            *reinterpret_cast<uint2*>(Dg + (int64_t)m * ldd + n) = pk;
-        }
     }
 }
 
@@ -1614,25 +1238,6 @@ static int launch_stripe_q8_slices(GemmParams& p, hipStream_t stream) {
     return launch_reduce<F16>(p, stream);
 }
 
-// How many K slices a problem is cut into when a workspace is at hand: problems whose 128 x 128 tiles would leave most
-// of the chip idle (a few dozen rows against a wide weight), every slice at least 4 steps of 64 long.  1 = no split.
-// Up to 256 tiles: one workgroup of these tiles per compute unit leaves its matrix pipes waiting for every K step, two
-// overlap (256 x 8192 x 8192, 128 tiles: 75 -> 52 us; 512 x 8192 x 28672, 256 tiles: 400 -> 317).
-static int gemm_splits(int64_t M, int64_t N, int64_t K) {
-    if (K % kBK != 0 || N % 8 != 0) return 1;
-    const int64_t tiles = ((M + GemmSmall::BM - 1) / GemmSmall::BM) * ((N + GemmSmall::BN - 1) / GemmSmall::BN);
-    const int64_t kt = K / kBK;
-    if (tiles > 256 || kt < 8) return 1;
-    int64_t s = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, kt / 4), 32));
-    // 64-127 tiles get two or three slices that way and fill the chip once; twice as many, while a slice stays 16 steps long,
-    // keep two workgroups on a compute unit (128 rows of [K,N] 4096 x 14336 37 -> 32 us).  Tiles that
-    // fill the chip by themselves (129-256) are cut in two only for long rows: the second launch and the partial sums cost
-    // what the second workgroup per unit gains at K = 8192 and less (clocks settled, sliced / not: 512 x 8192 x 8192 89.0 /
-    // 76.8 us, 1024 x 4096 x 4096 47.0 / 44.7, 256 x 14336 x 4096 47.5 / 44.9; 1024 x 4096 x 14336 134 / 146)
-    if (tiles >= 64 && tiles * s <= 256 && kt / (2 * s) >= 16 && (s >= 2 || kt >= 192)) s *= 2;
-    return (int)s;
-}
-
 template <class T>
 static int launch_stripe_slices(GemmParams& p, hipStream_t stream) {
     p.done = slice_counters(p, stream);
@@ -1660,44 +1265,9 @@ static int launch_kn_rows(GemmParams& p, hipStream_t stream) {
     return p.splits > 1 ? launch_reduce<T>(p, stream) : MINFER_ATTN_OK;
 }
 
+// ---- which tiles, how many K slices --------------------------------------------------------------------------
 static int64_t tile_count(int64_t M, int64_t N, int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
-
-template <class T, bool NT>
-static int launch_split(GemmParams& p, hipStream_t stream) {
-    using SH = GemmSmall;
-    p.tiles_m = (p.M + SH::BM - 1) / SH::BM;
-    p.tiles_n = (p.N + SH::BN - 1) / SH::BN;
-    p.per_xcd = 0;
-    // As 128 x 256 tiles with three stages where these in the same slices fill the chip once by themselves: half the copies of A and
-    // two steps in flight instead of one (250 x 8192 x 8192 62.8 -> 54.2 us, 180 x 4136 x 11776 56.0 -> 46.8, 100 x 8192 x 8192 42.7
-    // -> 37.6, 512 x 4096 x 4096 33.0 -> 31.3; half a chip of them 129 x 4096 x 4096 22.0 -> 26.6).
-    const int64_t flat_wgs = tile_count(p.M, p.N, GemmFlat::BM, GemmFlat::BN) * p.splits;
-    if (flat_wgs > 192 && flat_wgs <= 256) {
-        p.tiles_n = (p.N + GemmFlat::BN - 1) / GemmFlat::BN;
-        hipLaunchKernelGGL((gemm_kernel<T, NT, GemmFlat, false, true>), dim3((unsigned)flat_wgs), dim3(GemmFlat::WAVES * 64), 0, stream, p);
-        if (int rc = check_launch("gemm_kernel (K slices, 128 x 256)")) return rc;
-        return launch_reduce<T>(p, stream);
-    }
-    const int64_t wgs = (int64_t)p.tiles_m * p.tiles_n * p.splits;
-    if (one_workgroup_per_unit(wgs)) hipLaunchKernelGGL((gemm_kernel<T, NT, GemmSmall3, false, true>), dim3((unsigned)wgs), dim3(SH::WAVES * 64), 0, stream, p);
-    else hipLaunchKernelGGL((gemm_kernel<T, NT, SH, false, true>), dim3((unsigned)wgs), dim3(SH::WAVES * 64), 0, stream, p);
-    if (int rc = check_launch("gemm_kernel (K slices)")) return rc;
-    return launch_reduce<T>(p, stream);
-}
-
-template <class T, bool NT, class SH>
-static int launch_tiled(GemmParams& p, hipStream_t stream) {
-    p.tiles_m = (p.M + SH::BM - 1) / SH::BM;
-    p.tiles_n = (p.N + SH::BN - 1) / SH::BN;
-    p.per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
-    hipLaunchKernelGGL((gemm_kernel<T, NT, SH>), dim3(p.per_xcd * 8), dim3(SH::WAVES * 64), 0, stream, p);
-    return check_launch("gemm_kernel");
-}
-
-// Rounds of the chip a launch of `tiles` workgroups (one per compute unit at a time) costs: full rounds count 1; a last
-// round that fills only part of the chip counts 0.55 + 0.45 x that part (its compute units run faster, the chip being
-// less loaded: 4096 x 6144 x 4096 as 384 large tiles takes 1.76 rounds' time, 2048 x 6144 x 4096 as 192 takes 0.87).
-static double rounds_cost(int64_t tiles) {
+static int compute_units() {
     static std::atomic<int> cached[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
@@ -1706,57 +1276,85 @@ static double rounds_cost(int64_t tiles) {
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
         cached[dev].store(cus, std::memory_order_relaxed);
     }
-    const int64_t full = tiles / cus, rest = tiles % cus;
-    return (double)full + (rest ? 0.55 + 0.45 * (double)rest / cus : 0.0);
+    return cus;
 }
-// The tile shape whose rounds of the chip cost least.  A shape's factor is the time of a full round of it, in rounds of the
-// large tile, as measured at K = 4096 and 8192 with both layouts, f16 and bf16, from one round to 28 (its share of the work
-// divided by its rate): 256 x 192 0.75-0.83, 192 x 256 0.78-0.85, 160 x 256 0.68-0.75, 128 x 256 0.57-0.61, two 128 x 128 on a
-// compute unit 0.58-0.65, one with three stages 0.41.  The large tile wins ties.
-enum class Tile { Big, Wide, Rows192, Rows160, Flat, Small, Small3 };
-template <bool NT>
-static Tile pick_tile(int64_t M, int64_t N, int64_t big_tiles, int64_t small_tiles) {
-    Tile best = Tile::Big;
-    double cost = rounds_cost(big_tiles);
-    auto consider = [&](Tile t, double c) { if (c < cost) { cost = c; best = t; } };
-    if (NT) {
-        consider(Tile::Wide, 0.81 * rounds_cost(tile_count(M, N, GemmWide::BM, GemmWide::BN)));
-        consider(Tile::Rows160, 0.73 * rounds_cost(tile_count(M, N, GemmRows160::BM, GemmRows160::BN)));
-    } else {
-        consider(Tile::Rows192, 0.81 * rounds_cost(tile_count(M, N, GemmRows192::BM, GemmRows192::BN)));
+// Microseconds of a launch of `tiles` tiles in `slices` K slices each, weights from memory: whole rounds of the chip, the last,
+// partly filled one at 0.76 + 0.24 of its share (its units run faster), a round its K steps at 20 ns per pair of 16-row blocks (two
+// workgroups on a unit 1.84 of one; with two stages a step that is shorter than the largest tile's does not cover its copies) and
+// 3.8 us of first and last copies and results; the copies of all tiles at 31 TB/s and the weight at 7 TB/s, which are hidden behind
+// that in part: the three add up as their squares; 3.6 us around it, 0.9 more for the launch that adds the slices up, and 0.29 us
+// per MB of sums.  Fitted to 4700 timed calls (150 shapes of 65 to 7000 rows, both layouts, up to 40 choices each): the choice it
+// makes is 1.0 % behind the best one on average, fixed rules for 128 x 128 and 128 x 256 slices and a table of rounds 6 %.
+static double plan_cost(const GemmTile& t, int64_t tiles, int slices, int64_t M, int64_t N, int64_t K, int cus) {
+    const double steps = (double)((K / kBK + slices - 1) / slices), area = t.m16 * t.n16;
+    const double step = (0.0201 * area + 0.0738) * (t.occ == 2 ? 1.84 : 1.0) + (t.ns == 2 && t.occ == 1 ? 0.0147 + 0.0076 * (64 - area) : 0.0);
+    const int64_t wgs = tiles * slices, per = (int64_t)cus * t.occ, full = wgs / per, rest = wgs % per;
+    const double rounds = (double)full + (rest ? 0.76 + 0.24 * (double)rest / (double)per : 0.0);
+    const double compute = rounds * (step * steps + 3.8), weight = (double)N * (double)K * 2 / 7.0e6;
+    const double copies = (double)tiles * (double)(K / kBK) * (t.m16 + t.n16) * 4096 / 31.3e6;
+    const double launch = 3.6 + sqrt(compute * compute + copies * copies + weight * weight);
+    return slices > 1 ? launch + 0.9 + 0.286e-6 * slices * (double)M * (double)N * 4 : launch;
+}
+// The cheapest tile shape and number of slices, up to max_slices of them (what a workspace holds): slices that bring the
+// workgroups to one or two rounds of the chip or just below, 3 steps long at least, with 64 MiB of sums at most.
+struct TilePlan { int tile, slices; };
+static TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, bool nt, int64_t max_slices) {
+    const int cus = compute_units();
+    const int64_t room = std::min<int64_t>(std::min<int64_t>(32, max_slices), std::min<int64_t>(K / kBK / 3, (INT64_C(16) << 20) / (M * N)));
+    TilePlan best{0, 1};
+    double cost = 0;
+    for (int i = 0; i < kGemmTileCount; ++i) {
+        const GemmTile& t = kGemmTiles[i];
+        if (!nt && t.n16 % 4 != 0) continue;
+        const int64_t tiles = tile_count(M, N, 32 * t.m16, 32 * t.n16), fill = (int64_t)cus * t.occ / tiles;
+        if (t.occ == 2 && tiles * std::max<int64_t>(room, 1) <= cus) continue;   // one workgroup to a unit: the other entry's three stages
+        const int64_t options[5] = {1, fill, fill - 1, fill * 3 / 4, 2 * fill};
+        for (int o = 0; o < 5; ++o) {
+            if (options[o] > room && options[o] != 1) continue;
+            if (options[o] < 1 || (o > 0 && options[o] == 1)) continue;
+            const double c = plan_cost(t, tiles, (int)options[o], M, N, K, cus);
+            if (cost == 0 || c < cost) { cost = c; best = {i, (int)options[o]}; }
+        }
     }
-    consider(Tile::Flat, 0.60 * rounds_cost(tile_count(M, N, GemmFlat::BM, GemmFlat::BN)));
-    if (one_workgroup_per_unit(small_tiles)) consider(Tile::Small3, 0.41 * rounds_cost(small_tiles));
-    else consider(Tile::Small, 0.64 * rounds_cost((small_tiles + 1) / 2));
     return best;
+}
+// The plan a shape gets with all the workspace it wants.  A call asks twice (for the workspace and to launch), so the last few
+// are kept; they depend on nothing but the sizes (and the chip's units, which do not differ between the devices of a process).
+static TilePlan full_plan(int64_t M, int64_t N, int64_t K, bool nt) {
+    struct Entry { int64_t M, N, K; bool nt; TilePlan plan; };
+    static thread_local Entry kept[16];
+    Entry& e = kept[(uint64_t)(M * 31 + N * 7 + K + nt) % 16];
+    if (e.M != M || e.N != N || e.K != K || e.nt != nt) e = Entry{M, N, K, nt, plan_tiles(M, N, K, nt, 1 << 20)};
+    return e.plan;
+}
+// Slices that a workspace is sized for: the plan's, and no fewer than bring 128 x 128 tiles to one round of the chip (to two while
+// a slice stays 16 steps long), four steps long at least: the size has been that, and callers may keep a workspace by it.
+static int gemm_slices(int64_t M, int64_t N, int64_t K, bool nt) {
+    if (K <= 0 || K % kBK != 0 || N % 8 != 0) return 1;
+    int64_t s = 1;
+    const int64_t tiles = tile_count(M, N, 128, 128), kt = K / kBK;
+    if (tiles <= 256 && kt >= 8) {
+        s = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, kt / 4), 32));
+        if (tiles >= 64 && tiles * s <= 256 && kt / (2 * s) >= 16 && (s >= 2 || kt >= 192)) s *= 2;
+    }
+    return std::max((int)s, full_plan(M, N, K, nt).slices);
+}
+
+template <class T> static int launch_tile(const GemmParams& p, bool nt, int tile, hipStream_t stream) {
+    return std::is_same<T, F16>::value ? launch_gemm_tile_f16(p, nt, tile, stream) : launch_gemm_tile_bf16(p, nt, tile, stream);
+}
+template <class T>
+static int launch_gemm(GemmParams& p, bool nt, const TilePlan& plan, hipStream_t stream) {
+    p.splits = plan.slices;
+    if (int rc = launch_tile<T>(p, nt, plan.tile, stream)) return rc;
+    return plan.slices > 1 ? launch_reduce<T>(p, stream) : MINFER_ATTN_OK;
 }
 
 template <class T, bool NT>
-static int launch_gemm(GemmParams& p, bool fast, hipStream_t stream) {
-    if (fast) {
-        switch (pick_tile<NT>(p.M, p.N, tile_count(p.M, p.N, GemmBig::BM, GemmBig::BN), tile_count(p.M, p.N, GemmSmall::BM, GemmSmall::BN))) {
-        case Tile::Big: return launch_tiled<T, NT, GemmBig>(p, stream);
-        case Tile::Wide: if constexpr (NT) return launch_tiled<T, NT, GemmWide>(p, stream); break;
-        case Tile::Rows160: if constexpr (NT) return launch_tiled<T, NT, GemmRows160>(p, stream); break;
-        case Tile::Rows192: if constexpr (!NT) return launch_tiled<T, NT, GemmRows192>(p, stream); break;
-        case Tile::Flat: return launch_tiled<T, NT, GemmFlat>(p, stream);
-        case Tile::Small: return launch_tiled<T, NT, GemmSmall>(p, stream);
-        case Tile::Small3: return launch_tiled<T, NT, GemmSmall3>(p, stream);
-        }
-    }
+static int launch_plain(const GemmParams& p, hipStream_t stream) {
     const int grid = (int)std::min<int64_t>(((int64_t)p.M * p.N + 255) / 256, 256 * 16);
     hipLaunchKernelGGL((gemm_plain_kernel<T, NT>), dim3(grid), dim3(256), 0, stream, p);
     return check_launch("gemm_plain_kernel");
-}
-
-// [N, K] weights numbered through as one of p.N columns; p.grp.end = cumulative column counts
-template <class T, class SH>
-static int launch_concat(GemmParams& p, hipStream_t stream) {
-    p.tiles_m = (p.M + SH::BM - 1) / SH::BM;
-    p.tiles_n = (p.N + SH::BN - 1) / SH::BN;
-    p.per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
-    hipLaunchKernelGGL((gemm_kernel<T, true, SH, true, false, true>), dim3(p.per_xcd * 8), dim3(SH::WAVES * 64), 0, stream, p);
-    return check_launch("gemm_kernel (grouped, columns numbered through)");
 }
 
 // Up to three weights [N_s, K] against one A in one launch (alpha = 1, no C): the tiled kernel over the concatenated
@@ -1773,7 +1371,7 @@ static int launch_grouped(GemmParams& p, int n_w, hipStream_t stream) {
         }
         return acc;
     };
-    if (p.M == 1 && p.K <= kGemvMaxKHalfs && (n_sum * p.K >= (INT64_C(1) << 25) || !rows_lds_takes(p.M, p.K)) && n_sum <= 0x7fffffffLL) {   // one row: whole weight rows per wave, numbered through (the rule of gemm_impl)
+    if (p.M == 1 && p.K <= kGemvMaxKHalfs && (n_sum * p.K >= (INT64_C(1) << 25) || !rows_lds_takes(p.M, p.K))) {   // one row: whole weight rows per wave, numbered through (the rule of gemm_impl)
         int acc = 0;
         for (int s = 0; s < kMaxGroup; ++s) { if (s < n_w) acc += p.grp.N[s]; p.grp.end[s] = acc; }
         return launch_gemv<T, true>(p, (int)n_sum, stream);
@@ -1812,34 +1410,9 @@ static int launch_grouped(GemmParams& p, int n_w, hipStream_t stream) {
 #undef MINFER_SKINNY
         return check_launch("gemm_skinny_kernel (grouped)");
     }
-    int64_t big_tiles = 0, small_tiles = 0;
-    bool concat = n_sum < (INT64_C(1) << 31);
-    for (int s = 0; s < n_w; ++s) {
-        big_tiles += tile_count(p.M, p.grp.N[s], GemmBig::BM, GemmBig::BN);
-        small_tiles += tile_count(p.M, p.grp.N[s], GemmSmall::BM, GemmSmall::BN);
-        concat = concat && p.grp.N[s] % 64 == 0;
-    }
-    // the sizes in between over the weights' columns numbered through, when they fill the chip's rounds better (the Llama-3-8B
-    // QKV projection of 4096 tokens: 384 large tiles, one and a half rounds, or 512 of 256 x 192, two rounds of 3/4 the work)
-    Tile tile = big_tiles >= 160 ? Tile::Big : Tile::Small;
-    if (concat) {
-        tile = pick_tile<true>(p.M, n_sum, big_tiles, small_tiles);
-        int acc = 0;
-        for (int s = 0; s < kMaxGroup; ++s) { if (s < n_w) acc += p.grp.N[s]; p.grp.end[s] = acc; }
-        if (tile == Tile::Wide || tile == Tile::Rows160 || tile == Tile::Flat) p.N = (int)n_sum;
-        if (tile == Tile::Wide) return launch_concat<T, GemmWide>(p, stream);
-        if (tile == Tile::Rows160) return launch_concat<T, GemmRows160>(p, stream);
-        if (tile == Tile::Flat) return launch_concat<T, GemmFlat>(p, stream);
-    }
-    const bool big = tile == Tile::Big;
-    const int bm = big ? GemmBig::BM : GemmSmall::BM, bn = big ? GemmBig::BN : GemmSmall::BN;
-    p.tiles_m = (p.M + bm - 1) / bm;
-    p.tiles_n = fill_ends(bn);
-    p.per_xcd = (p.tiles_m * p.tiles_n + 7) / 8;
-    if (big) hipLaunchKernelGGL((gemm_kernel<T, true, GemmBig, true>), dim3(p.per_xcd * 8), dim3(GemmBig::WAVES * 64), 0, stream, p);
-    else if (one_workgroup_per_unit((int64_t)p.per_xcd * 8)) hipLaunchKernelGGL((gemm_kernel<T, true, GemmSmall3, true>), dim3(p.per_xcd * 8), dim3(GemmSmall::WAVES * 64), 0, stream, p);
-    else hipLaunchKernelGGL((gemm_kernel<T, true, GemmSmall, true>), dim3(p.per_xcd * 8), dim3(GemmSmall::WAVES * 64), 0, stream, p);
-    return check_launch("gemm_kernel (grouped)");
+    fill_ends(1);   // the tiled kernel takes the weights' columns numbered through
+    p.N = (int)n_sum;
+    return launch_gemm<T>(p, true, plan_tiles(p.M, n_sum, p.K, true, 1), stream);
 }
 
 }  // namespace minfer_attn
@@ -1858,16 +1431,16 @@ MINFER_ATTN_EXPORT int minfer_qkv(int dtype, const void* x, const void* wq, cons
     void* O[3] = {q_out, k_out, v_out};
     if (M < 0 || K < 0 || M > 0x7fffffffLL || K > 0x7fffffffLL) return fail(MINFER_ATTN_EINVAL, "qkv: bad M or K");
     if (!x || ldx < K) return fail(MINFER_ATTN_EINVAL, "qkv: x is null or its leading dimension is smaller than K");
-    bool fast = K > 0 && K % kBK == 0 && ldx % 8 == 0 && aligned16(x) && (int64_t)GemmBig::BM * ldx < (1LL << 30);
+    bool fast = K > 0 && K % kBK == 0 && ldx % 8 == 0 && aligned16(x) && (int64_t)256 * ldx < (1LL << 30);
     for (int s = 0; s < 3; ++s) {
         if (Ns[s] < 0 || Ns[s] > 0x7fffffffLL) return fail(MINFER_ATTN_EINVAL, "qkv: bad output width");
         if (!W[s] || !O[s]) return fail(MINFER_ATTN_EINVAL, "qkv: null pointer");
         if (ldw[s] < K || ldo[s] < Ns[s]) return fail(MINFER_ATTN_EINVAL, "qkv: a leading dimension is smaller than its row");
         fast = fast && Ns[s] % 8 == 0 && ldw[s] % 8 == 0 && ldo[s] % 4 == 0 && aligned16(W[s]) && ((uintptr_t)O[s] & 7u) == 0 &&
-               (int64_t)std::max<int64_t>(GemmBig::BN, kBK) * ldw[s] < (1LL << 30);
+               (int64_t)256 * ldw[s] < (1LL << 30);
     }
     if (M == 0) return MINFER_ATTN_OK;
-    if (!fast || Nq == 0 || Nk == 0 || Nv == 0) {   // shapes the tiled kernels cannot take: three separate launches
+    if (!fast || Nq == 0 || Nk == 0 || Nv == 0 || Nq + Nk + Nv > 0x7fffffffLL) {   // shapes the tiled kernels cannot take: three separate launches
         for (int s = 0; s < 3; ++s)
             if (int rc = minfer_gemm(dtype, MINFER_GEMM_B_NK, x, W[s], nullptr, O[s], M, Ns[s], K, ldx, ldw[s], Ns[s], ldo[s], 1.0, 0.0, stream_v))
                 return rc;
@@ -1902,14 +1475,14 @@ static int gemm_impl(int dtype, int b_layout, const void* A, const void* B, cons
     // the tiled kernel moves 16-byte pieces and whole 64-wide K steps, and addresses a panel with 32-bit offsets
     const bool fast = K > 0 && K % kBK == 0 && N % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && ldd % 4 == 0 &&
                       aligned16(A) && aligned16(B) && ((uintptr_t)D & 7u) == 0 && ((uintptr_t)C & 7u) == 0 &&
-                      (int64_t)GemmBig::BM * lda < (1LL << 30) && (int64_t)std::max<int64_t>(GemmBig::BN, kBK) * ldb < (1LL << 30);
+                      (int64_t)256 * lda < (1LL << 30) && (int64_t)256 * ldb < (1LL << 30);
     hipStream_t stream = (hipStream_t)stream_v;
     // A decode step's few tokens against an [N, K] weight: stream the weight once.  Which kernel does that best was
     // measured with the calls cycling over copies of the weight, 640 MiB in all: a weight of up to 256 MiB called again
     // and again is served by the chip's last-level cache, where the order of the kernels is a different one (14336 x
     // 4096 at one row: stripes 18.0 us against 19.5 for whole rows per wave from the cache, 24.2 against 21.9 from memory).
-    const int splits = fast && workspace && aligned16(workspace) ? gemm_splits(M, N, K) : 1;
-    const bool can_split = splits > 1 && workspace_bytes >= (size_t)splits * (size_t)M * (size_t)N * sizeof(float);
+    const size_t fit = workspace && aligned16(workspace) ? workspace_bytes / ((size_t)M * (size_t)N * sizeof(float)) : 0;   // slices the workspace holds
+    const bool can_split = fast && fit > 1 && full_plan(M, N, K, nt).slices > 1;
     const int64_t stripes = (N + 63) / 64;
     const bool rows_takes = rows_lds_takes(M, K);
     // one row: whole weight rows per wave (14336 x 4096: 21.9 us, the 16-column kernel 23.6, stripes 24.2; 28672 x 8192:
@@ -1957,19 +1530,19 @@ static int gemm_impl(int dtype, int b_layout, const void* A, const void* B, cons
     if (fast && nt && (M <= 16 || (!can_split && (M <= 32 || (M <= 64 && N * K <= (INT64_C(1) << 25))))))
         return dtype == MINFER_ATTN_F16 ? launch_skinny<F16>(p, stream) : launch_skinny<BF16>(p, stream);
     if (fast && !nt && M <= kKnRows) {
-        const int kn = workspace && aligned16(workspace) ? kn_slices(M, N, K) : 1;
-        const size_t fit = workspace_bytes / ((size_t)M * (size_t)N * sizeof(float));   // a smaller workspace: as many slices as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
+        const int kn = kn_slices(M, N, K);   // a smaller workspace: as many slices as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
         p.splits = fit < (size_t)kn ? std::max((int)fit, 1) : kn;
         p.part = (float*)workspace;
         return dtype == MINFER_ATTN_F16 ? launch_kn_rows<F16>(p, stream) : launch_kn_rows<BF16>(p, stream);
     }
-    if (can_split) {
-        p.splits = splits; p.part = (float*)workspace;
-        if (dtype == MINFER_ATTN_F16) return nt ? launch_split<F16, true>(p, stream) : launch_split<F16, false>(p, stream);
-        return nt ? launch_split<BF16, true>(p, stream) : launch_split<BF16, false>(p, stream);
+    if (fast) {
+        TilePlan plan = full_plan(M, N, K, nt);
+        if ((size_t)plan.slices > std::max<size_t>(fit, 1)) plan = plan_tiles(M, N, K, nt, std::max<int64_t>((int64_t)fit, 1));
+        p.part = (float*)workspace;
+        return dtype == MINFER_ATTN_F16 ? launch_gemm<F16>(p, nt, plan, stream) : launch_gemm<BF16>(p, nt, plan, stream);
     }
-    if (dtype == MINFER_ATTN_F16) return nt ? launch_gemm<F16, true>(p, fast, stream) : launch_gemm<F16, false>(p, fast, stream);
-    return nt ? launch_gemm<BF16, true>(p, fast, stream) : launch_gemm<BF16, false>(p, fast, stream);
+    if (dtype == MINFER_ATTN_F16) return nt ? launch_plain<F16, true>(p, stream) : launch_plain<F16, false>(p, stream);
+    return nt ? launch_plain<BF16, true>(p, stream) : launch_plain<BF16, false>(p, stream);
 }
 
 MINFER_ATTN_EXPORT int minfer_gemm(int dtype, int b_layout, const void* A, const void* B, const void* C, void* D,
@@ -1981,14 +1554,14 @@ MINFER_ATTN_EXPORT int minfer_gemm(int dtype, int b_layout, const void* A, const
 MINFER_ATTN_EXPORT size_t minfer_gemm_layout_workspace_bytes(int b_layout, int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
     int splits;   // the most slices that a route of gemm_impl cuts K into for this layout
-    if (b_layout == MINFER_GEMM_B_KN) splits = M <= kKnRows ? kn_slices(M, N, K) : gemm_splits(M, N, K);
-    else splits = std::max(stripe_slices(M, N, K), M > 16 ? gemm_splits(M, N, K) : 1);
+    if (b_layout == MINFER_GEMM_B_KN) splits = M <= kKnRows ? kn_slices(M, N, K) : gemm_slices(M, N, K, false);
+    else splits = std::max(stripe_slices(M, N, K), M > 16 ? gemm_slices(M, N, K, true) : 1);
     return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
 MINFER_ATTN_EXPORT size_t minfer_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
-    const int splits = std::max(std::max(gemm_splits(M, N, K), stripe_slices(M, N, K)), kn_slices(M, N, K));
+    const int splits = std::max(std::max(gemm_slices(M, N, K, true), gemm_slices(M, N, K, false)), std::max(stripe_slices(M, N, K), kn_slices(M, N, K)));
     return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 

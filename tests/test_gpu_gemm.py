@@ -136,6 +136,45 @@ def test_gemm_tiles_between_the_small_and_the_large_one(layout, dtype, M, N, K, 
     assert_close(d, (alpha * (a.double() @ (b if layout == KN else b.T).double()) + beta * c.double()).numpy(), dtype)
 
 
+@pytest.mark.parametrize("layout,M,N,K", [
+    (KN, 977, 4152, 64),          # 128 x 128, two to a unit
+    (KN, 71, 424, 192),           # 128 x 128
+    (NK, 67, 360, 256),           # 128 x 128
+    (NK, 1147, 3640, 320),        # 128 x 192
+    (KN, 899, 6536, 448),         # 128 x 256
+    (NK, 905, 6568, 640),         # 128 x 256
+    (KN, 137, 1944, 64),          # 160 x 128
+    (NK, 137, 3816, 128),         # 160 x 128
+    (NK, 897, 6632, 192),         # 160 x 224
+    (KN, 1059, 7192, 256),        # 160 x 256
+    (NK, 1349, 6296, 320),        # 160 x 256
+    (KN, 651, 6584, 448),         # 192 x 128
+    (NK, 647, 6568, 640),         # 192 x 128
+    (NK, 903, 3592, 64),          # 192 x 192
+    (KN, 1287, 7176, 128),        # 192 x 256
+    (NK, 1811, 5416, 192),        # 192 x 256
+    (KN, 645, 6200, 256),         # 224 x 128
+    (NK, 657, 6632, 320),         # 224 x 128
+    (NK, 1773, 4904, 448),        # 224 x 192
+    (KN, 1561, 6440, 640),        # 224 x 256
+    (NK, 2119, 4824, 64),         # 224 x 256
+    (NK, 2025, 4888, 128),        # 256 x 224
+    (KN, 2027, 5976, 192),        # 256 x 256
+    (NK, 1807, 7192, 256),        # 256 x 256
+])
+def test_gemm_every_tile_shape(layout, M, N, K):
+    """A shape for which plan_tiles takes each tile (as the comments say; without a workspace, on 256 compute units), the last tile
+    row and column ragged, from one K step (fewer than the ring has stages) to ten: every element against torch's product in 64
+    bits, within the bound of assert_close."""
+    dtype = torch.float16 if (M + K // 64) % 2 else torch.bfloat16
+    alpha, beta = (2.0, 3.0) if K % 128 else (1.0, 0.0)
+    a, b, c = make(M, N, K, layout, dtype, M + N + K)
+    d = torch.full((M, N), float("nan"), dtype=dtype, device=DEV)
+    assert capi.gemm(a.to(DEV), b.to(DEV), c.to(DEV), d, alpha, beta, layout) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    assert_close(d, (alpha * (a.double() @ (b if layout == KN else b.T).double()) + beta * c.double()).numpy(), dtype)
+
+
 def test_gemm_golden_strided_and_in_place():
     z = np.load(os.path.join(os.path.dirname(__file__), "golden", "gemm_small.npz"))
     a, b, c = (torch.from_numpy(z[k]).to(DEV) for k in "abc")
@@ -199,6 +238,8 @@ def test_gemm_op_reference_test_recipe(kerns, S, alpha, beta):
     (33, 50, 17, 17, 9),               # nothing tileable: three plain launches
     # 5-64 rows, K a multiple of 256, 96 stripes of 64 columns or more over the three weights: the stripe kernel, every weight
     # with workgroups of its own in proportion to its width
+    (300, 320, 1000, 72, 136),         # tiles and 16-column blocks that hold columns of two or three weights
+    (1100, 192, 1032, 1000, 8),
     (5, 4096, 4096, 1024, 1024),
     (16, 512, 4096, 1024, 1032),       # a last stripe of 8 columns in the third weight
     (40, 1024, 4104, 1024, 1024),      # ... in the first; three blocks of activation rows

@@ -402,6 +402,12 @@ def test_build_scan_finds_dependences_too_close_to_an_asm_statement():
     assert len(build.asm_hazards("kernel_b:\n" + cvt + "\tv_pk_mul_f16 v63, v63, v136\n" + mfma)) == 1
     assert build.asm_hazards("kernel_b:\n" + cvt + "\tv_pk_mul_f16 v63, v63, v136\n" * 2 + mfma) == []
     assert build.asm_hazards("kernel_b:\n" + cvt.replace("v51", "v70") + mfma) == []
+    acc = "\t;;#ASMSTART\n\tv_mfma_f32_16x16x32_f16 a[4:7], v[50:53], v[58:61], a[4:7]\n\t;;#ASMEND\n"
+    read = "\tv_accvgpr_read_b32 v1, a6\n"
+    assert len(build.asm_hazards("kernel_c:\n" + acc + "\ts_nop 15\n" + read)) == 1       # 16 slots of the 18 that are kept
+    assert build.asm_hazards("kernel_c:\n" + acc + "\ts_nop 15\n\ts_nop 1\n" + read) == []
+    assert build.asm_hazards("kernel_c:\n" + acc + read.replace("a6", "a8")) == []           # another block
+    assert build.asm_hazards("kernel_c:\n" + acc + "\ts_branch .LBB0_9\n" + read) == []     # not the next to run
 
 
 FAKE_HIP = r"""
