@@ -211,23 +211,57 @@ MA_DEV float sum_across_quads(float x) {
     return sum_across_halves(__builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]));
 }
 
-// x of lane (l ^ M), M = 1 or 2: inside groups of four lanes, one instruction
+// Value of another lane of the same row of 16, one vector instruction (through the LDS, as __shfl does it, an exchange is about a
+// hundred clocks of latency): CTRL is a quad permutation, a mirror or a shift.  Lanes that read no lane, and rows outside
+// ROW_MASK, get 0.
+template <int CTRL, int ROW_MASK = 0xf> MA_DEV uint32_t row_exchange(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROW_MASK, 0xf, ROW_MASK == 0xf);
+}
+template <int CTRL> MA_DEV float row_exchange(float x) { return __builtin_bit_cast(float, row_exchange<CTRL>(__builtin_bit_cast(uint32_t, x))); }
+// x of lane (l ^ M), M = 1 or 2: inside groups of four lanes
 template <int M> MA_DEV uint32_t quad_swap(uint32_t x) {
     static_assert(M == 1 || M == 2, "lanes of one group of four");
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, M == 1 ? 0xb1 : 0x4e, 0xf, 0xf, true);   // quad_perm [1,0,3,2] / [2,3,0,1]
+    return row_exchange<M == 1 ? 0xb1 : 0x4e>(x);   // quad_perm [1,0,3,2] / [2,3,0,1]
+}
+// x of lane `lane`, which is the same for all lanes
+MA_DEV int lane_value(int x, int lane) { return __builtin_amdgcn_readlane(x, lane); }
+MA_DEV float lane_value(float x, int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane)); }
+// x summed (its largest value taken) over aligned groups of LANES lanes, in every lane.  The additions are those of
+// `x += __shfl_xor(x, m)` for m = 1, 2, 4 .. LANES / 2: after the quad steps every lane of a quad holds the same sum, so that
+// mirroring half a row or a row reads the same value as the lane m away.
+template <int LANES> MA_DEV float lane_sum(float x) {
+    static_assert(LANES == 8 || LANES == 16 || LANES == 32 || LANES == 64, "whole half rows");
+    x += row_exchange<0xb1>(x);
+    x += row_exchange<0x4e>(x);
+    x += row_exchange<0x141>(x);                        // half row mirrored
+    if (LANES > 8) x += row_exchange<0x140>(x);         // row mirrored
+    if (LANES > 16) {
+        const uint32_t u = __builtin_bit_cast(uint32_t, x);
+        auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        x = __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+    }
+    return LANES > 32 ? sum_across_halves(x) : x;
+}
+MA_DEV float wave_max(float x) {
+    x = max2(x, row_exchange<0xb1>(x));
+    x = max2(x, row_exchange<0x4e>(x));
+    x = max2(x, row_exchange<0x141>(x));
+    x = max2(x, row_exchange<0x140>(x));
+    return max_across_quads(x);
+}
+// Inclusive prefix sum of x over the lanes of a wave: over a row by shifts, then the last lanes of rows 0 and 2 to rows 1 and 3
+// and lane 31 to rows 2 and 3.
+MA_DEV int wave_inclusive_scan(int x) {
+    x += (int)row_exchange<0x111>((uint32_t)x);
+    x += (int)row_exchange<0x112>((uint32_t)x);
+    x += (int)row_exchange<0x114>((uint32_t)x);
+    x += (int)row_exchange<0x118>((uint32_t)x);
+    x += (int)row_exchange<0x142, 0xa>((uint32_t)x);
+    x += (int)row_exchange<0x143, 0xc>((uint32_t)x);
+    return x;
 }
 
 MA_DEV float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
-// Inclusive prefix sum of x over the lanes of a wave.
-MA_DEV int wave_inclusive_scan(int x, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int up = __shfl_up(x, d);
-        if (lane >= d) x += up;
-    }
-    return x;
-}
 
 // Loads and stores of bytes that a kernel touches once (cache rows being streamed, rows of a normalisation):
 // marked non-temporal, so that the caches between the compute units and HBM do not keep the lines.  On this chip

@@ -77,9 +77,9 @@ MA_DEV int work_total(const DecodeParams& p, int lane, bool publish) {
     for (int base = 0; base < p.B; base += 64) {
         const int b = base + lane;
         const int n = b < p.B ? groups_of(p, p.ctx[b]) * pairs : 0;
-        const int incl = wave_inclusive_scan(n, lane);
+        const int incl = wave_inclusive_scan(n);
         if (publish && b < p.B) p.seq_off[b] = offset + incl - n;
-        offset += __builtin_amdgcn_readfirstlane(__shfl(incl, 63));
+        offset += lane_value(incl, 63);
     }
     if (publish && lane == 0) p.seq_off[p.B] = offset;
     return offset;
@@ -98,16 +98,16 @@ MA_DEV void locate_sequence(const DecodeParams& p, int x, int lane, int& b_out, 
         const int b = base + lane;
         const int c = b < p.B ? p.ctx[b] : 0;
         const int n = b < p.B ? groups_of(p, c) * pairs : 0;
-        const int incl = wave_inclusive_scan(n, lane);
-        const int total = __builtin_amdgcn_readfirstlane(__shfl(incl, 63));
+        const int incl = wave_inclusive_scan(n);
+        const int total = lane_value(incl, 63);
         if (x < offset + total) {
             const uint64_t hit = __ballot(x < offset + incl);
-            const int src = __ffsll((unsigned long long)hit) - 1;
+            const int src = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)hit) - 1);
             // every lane holds the same values; saying so keeps the kernel's control flow (and with it
             // the compiler's wait-count bookkeeping in the main loop) scalar
-            b_out = __builtin_amdgcn_readfirstlane(base + src);
-            off_out = __builtin_amdgcn_readfirstlane(offset + __shfl(incl - n, src));
-            ctx_out = __builtin_amdgcn_readfirstlane(__shfl(c, src));
+            b_out = base + src;
+            off_out = offset + lane_value(incl - n, src);
+            ctx_out = lane_value(c, src);
             return;
         }
         offset += total;
@@ -137,8 +137,8 @@ struct SegmentWalk {
         if (p.B <= 64) {   // one scan gives the line's length and the share's first sequence
             c = lane < p.B ? p.ctx[lane] : 0;
             const int n = lane < p.B ? groups_of(p, c) * p.Hkv * p.n_hg : 0;
-            const int incl = wave_inclusive_scan(n, lane);
-            const int total = __builtin_amdgcn_readfirstlane(__shfl(incl, 63));
+            const int incl = wave_inclusive_scan(n);
+            const int total = lane_value(incl, 63);
             if (first) {
                 if (lane < p.B) p.seq_off[lane] = incl - n;
                 if (lane == 0) p.seq_off[p.B] = total;
@@ -146,10 +146,10 @@ struct SegmentWalk {
             quota = work_quota(p, total);
             take_share(total, w);
             if (x >= x_end) return false;
-            const int src = __ffsll((unsigned long long)__ballot(x < incl)) - 1;
-            b = __builtin_amdgcn_readfirstlane(src);
-            off_b = __builtin_amdgcn_readfirstlane(__shfl(incl - n, src));
-            c = __builtin_amdgcn_readfirstlane(__shfl(c, src));
+            const int src = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(x < incl)) - 1);
+            b = src;
+            off_b = lane_value(incl - n, src);
+            c = lane_value(c, src);
         } else {
             const int total = work_total(p, lane, first);
             quota = work_quota(p, total);
@@ -285,11 +285,11 @@ MA_DEV void stream_rows(const DecodeParams& p, int b, int g, int hg, int row_lo,
         }
         // ---- online softmax over this group's 16 keys ------------------------------------------
         float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const bool grow = (mx - m_ref) * c2 > kLazyLog2 || (m_ref == -INFINITY && mx > -INFINITY);
-        if (__any(grow)) {
-            const float m_new = grow ? mx : m_ref;
+        // (one of the head's four lanes holds its largest score: the exchange between them is left to the branch)
+        auto grows = [&](float x) { return (x - m_ref) * c2 > kLazyLog2 || (m_ref == -INFINITY && x > -INFINITY); };
+        if (__any(grows(mx))) {
+            mx = max_across_quads(mx);
+            const float m_new = grows(mx) ? mx : m_ref;
             const float alpha = (m_ref == -INFINITY) ? 0.f : fast_exp2((m_ref - m_new) * c2);
             m_ref = m_new;
             l_sum *= alpha;
@@ -323,10 +323,8 @@ MA_DEV void stream_rows(const DecodeParams& p, int b, int g, int hg, int row_lo,
             load_group(t0 + s + NS, kr[s], vr[s]);
         }
     }
-    l_sum += __shfl_xor(l_sum, 16);
-    l_sum += __shfl_xor(l_sum, 32);
     acc.m = m_ref;
-    acc.l = l_sum;
+    acc.l = sum_across_quads(l_sum);
 }
 
 // The segment's partial result of every head, into the workspace.
@@ -547,11 +545,11 @@ MA_DEV void stream_rows_q8(const DecodeParams& p, int b, int g, int hg, int row_
         }
         // ---- online softmax over this group's 32 keys ----------------------------------------------------
         float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])), fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const bool grow = (mx - m_ref) * c2 > kLazyLog2 || (m_ref == -INFINITY && mx > -INFINITY);
-        if (__any(grow)) {
-            const float m_new = grow ? mx : m_ref;
+        // (one of the head's four lanes holds its largest score: the exchange between them is left to the branch)
+        auto grows = [&](float x) { return (x - m_ref) * c2 > kLazyLog2 || (m_ref == -INFINITY && x > -INFINITY); };
+        if (__any(grows(mx))) {
+            mx = max_across_quads(mx);
+            const float m_new = grows(mx) ? mx : m_ref;
             const float alpha = (m_ref == -INFINITY) ? 0.f : fast_exp2((m_ref - m_new) * c2);
             m_ref = m_new;
             l_sum *= alpha;
@@ -599,10 +597,8 @@ MA_DEV void stream_rows_q8(const DecodeParams& p, int b, int g, int hg, int row_
         for (int s = 0; s < NS; ++s)
             if (t0 + s < n_groups) consume(general_tag, general_tag, t0 + s, ring[s]);
     }
-    l_sum += __shfl_xor(l_sum, 16);
-    l_sum += __shfl_xor(l_sum, 32);
     acc.m = m_ref;
-    acc.l = l_sum;
+    acc.l = sum_across_quads(l_sum);
 }
 
 template <int D>
@@ -655,13 +651,9 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecodeParams 
     const int start = p.seq_off[b] + (hg * p.Hkv + g) * n_b;
     const int ns = n_b > 0 ? (start + n_b - 1) / quota - start / quota + 1 : 0;
     const float m = lane < ns ? m_raw : -INFINITY, l = lane < ns ? l_raw : 0.f;
-    float M = m;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) M = fmaxf(M, __shfl_xor(M, d));
+    const float M = wave_max(m);
     const float wgt = (m > -INFINITY) ? fast_exp2((m - M) * p.scale_log2) : 0.f;
-    float L = l * wgt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) L += __shfl_xor(L, d);
+    const float L = lane_sum<64>(l * wgt);
     float acc[EPL];
 #pragma unroll
     for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
@@ -676,7 +668,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecodeParams 
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const bool on = s0 + u < ns;
-            const float ws = __shfl(wgt, min(s0 + u, 63));
+            const float ws = lane_value(wgt, min(s0 + u, 63));
 #pragma unroll
             for (int e = 0; e < EPL; ++e) acc[e] += on ? x[u][e] * ws : 0.f;
         }

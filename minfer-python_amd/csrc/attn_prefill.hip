@@ -252,14 +252,14 @@ __global__ __launch_bounds__(NW * TEAMS * 64, 2) void prefill_kernel(const Prefi
                 len = min(min(max(p.cu[sq + 1], lo), p.L) - lo, p.max_len);
             }
             const int n = (len + 32 * QBW - 1) / (32 * QBW);
-            const int incl = wave_inclusive_scan(n, lane);
-            const int total = __builtin_amdgcn_readfirstlane(__shfl(incl, 63));
+            const int incl = wave_inclusive_scan(n);
+            const int total = lane_value(incl, 63);
             if (x < total) {
-                const int src = __ffsll((unsigned long long)__ballot(x < incl)) - 1;
-                seq_lo = __builtin_amdgcn_readfirstlane(__shfl(lo, src));
-                seq_len = __builtin_amdgcn_readfirstlane(__shfl(len, src));
-                nt = __builtin_amdgcn_readfirstlane(__shfl(n, src));
-                x -= __builtin_amdgcn_readfirstlane(__shfl(incl - n, src));
+                const int src = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(x < incl)) - 1);
+                seq_lo = lane_value(lo, src);
+                seq_len = lane_value(len, src);
+                nt = lane_value(n, src);
+                x -= lane_value(incl - n, src);
                 found = true;
             } else {
                 x -= total;

@@ -717,10 +717,8 @@ __global__ __launch_bounds__(4 * 64) void gemv_kernel(const GemmParams p, int ro
         if (seg == nseg - 1) {
 #pragma unroll
             for (int m = 0; m < MR; ++m) {
-                float v = acc[m];
+                float v = lane_sum<64>(acc[m]);
                 acc[m] = 0.f;
-#pragma unroll
-                for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
                 if (lane == 0 && m < p.M) {
                     const short* unused; short* out;
                     locate(row, unused, out);
@@ -954,10 +952,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_q8_kernel(const GemmPara
             }
         }
         if (seg == nseg - 1) {                             // the row is complete: add the lanes' sums up and store
-            float v = acc;
+            float v = lane_sum<64>(acc);
             acc = 0.f;
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
             if (lane == 0) {
                 v *= p.alpha;
                 if (p.beta != 0.f) v += p.beta * T::to_float(((const short*)p.C)[row]);

@@ -57,8 +57,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_rows_kernel(const NormPa
         }
 #pragma unroll
         for (int j = 0; j < NCH; ++j) ss += sum_sq8<T>(x[j]);
-#pragma unroll
-        for (int m = 1; m < LANES; m <<= 1) ss += __shfl_xor(ss, m);
+        ss = lane_sum<LANES>(ss);
         const float sc = rsqrtf(ss * p.inv_dim + p.eps);
         short* dst = (short*)p.out + vec * p.dim;
 #pragma unroll
@@ -95,8 +94,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_block_kernel(const NormP
         } else {
             for (int i = tid; i < p.dim; i += kNormThreads) { const float f = T::to_float(src[i]); ss += f * f; }
         }
-#pragma unroll
-        for (int m = 1; m < 64; m <<= 1) ss += __shfl_xor(ss, m);
+        ss = lane_sum<64>(ss);
         __syncthreads();                 // the previous vector's partial sums have been read
         if ((tid & 63) == 0) part[tid >> 6] = ss;
         __syncthreads();

@@ -313,21 +313,6 @@ struct NormRopeParams {
     float eps, inv_dim;
 };
 
-// A lane's value from another lane of its row of 16 (quad permutation, mirror or rotation, chosen by CTRL).
-template <int CTRL> MA_DEV uint32_t row_exchange(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
-}
-// ss summed over the G lanes of a head.  The partners are those of `ss += __shfl_xor(ss, m)`, m = 1, 2, 4, 8 (after
-// the quad steps every lane of a quad holds the same sum, so mirroring the half row or the row reads the same value
-// as the lane m away), the additions therefore the same, at a few cycles each instead of a trip through the LDS.
-template <int G> MA_DEV float sum_over_head(float ss) {
-    ss += __builtin_bit_cast(float, row_exchange<0xB1>(__builtin_bit_cast(uint32_t, ss)));            // lanes 1 0 3 2
-    ss += __builtin_bit_cast(float, row_exchange<0x4E>(__builtin_bit_cast(uint32_t, ss)));            // lanes 2 3 0 1
-    ss += __builtin_bit_cast(float, row_exchange<0x141>(__builtin_bit_cast(uint32_t, ss)));           // half row mirrored
-    if (G == 16) ss += __builtin_bit_cast(float, row_exchange<0x140>(__builtin_bit_cast(uint32_t, ss)));   // row mirrored
-    return ss;
-}
-
 template <class T, int STYLE, bool Q8, int G, bool STREAM>
 __global__ __launch_bounds__(kRopeThreads) void rope_norm_append_kernel(const NormRopeParams np) {
     const RopeParams& p = np.r;
@@ -423,7 +408,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_norm_append_kernel(const No
             const int hd = (int)((unsigned)unit / G);
             const bool is_q = valid && hd < p.H, is_k = valid && hd >= p.H && hd < p.H + p.Hkv;
             // normalise: every lane takes part in the exchanges, the result is used by q and k heads only
-            const float ss = sum_over_head<G>(sum_sq8<T>(x[u]));
+            const float ss = lane_sum<G>(sum_sq8<T>(x[u]));
             const float sc = rsqrtf(ss * np.inv_dim + np.eps);
             s16x8 a = x[u];
             if ((is_q && np.wq) || (is_k && np.wk)) {
