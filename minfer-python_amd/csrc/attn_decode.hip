@@ -52,7 +52,8 @@ struct DecodeParams {
     const int32_t* ctx;
     float* part_o;     // [B][Hq][S][D]
     float* part_ml;    // [B][Hq][S][2]: reference max (raw score units), sum
-    int32_t* seq_off;  // [B + 1]: linear start of every sequence's work, written by workgroup 0 for the combine kernel
+    int32_t* seq_off;  // [B + 2]: linear start of every sequence's work, the line's length and, where pairs are cut into pieces of
+                       // their own, the largest piece (else 0), written by workgroup 0 for the combine kernel
     int64_t q0, q1, kv0, kv1, kv2;
     int B, Hq, Hkv, n_rep, Lmax;
     int n_wg;          // workgroups of the split launch (kDecodeWaves waves each)
@@ -81,7 +82,7 @@ MA_DEV int work_total(const DecodeParams& p, int lane, bool publish) {
         if (publish && b < p.B) p.seq_off[b] = offset + incl - n;
         offset += lane_value(incl, 63);
     }
-    if (publish && lane == 0) p.seq_off[p.B] = offset;
+    if (publish && lane == 0) { p.seq_off[p.B] = offset; p.seq_off[p.B + 1] = 0; }
     return offset;
 }
 MA_DEV int work_quota(const DecodeParams& p, int total) {
@@ -141,7 +142,7 @@ struct SegmentWalk {
             const int total = lane_value(incl, 63);
             if (first) {
                 if (lane < p.B) p.seq_off[lane] = incl - n;
-                if (lane == 0) p.seq_off[p.B] = total;
+                if (lane == 0) { p.seq_off[p.B] = total; p.seq_off[p.B + 1] = 0; }
             }
             quota = work_quota(p, total);
             take_share(total, w);
@@ -178,6 +179,41 @@ struct SegmentWalk {
         g1 = min(n_b, g0 + (x_end - x));
         slot = wave - (off_b + pair * n_b) / quota;
         x += g1 - g0;
+        return true;
+    }
+};
+
+// The other way to share out the work, for up to 64 sequences of few pairs (decode_takes_pieces): every pair is cut into pieces of
+// its own, all of one sequence equal to within a group, and a wave has one piece at most.  A share that crosses from one pair to
+// the next drains the wave's ring, stores, and starts over with the next pair's query rows; here no wave does, and in return the
+// pieces are no longer all of one size: at most `piece` groups, the smallest number that leaves no more pieces than waves.
+struct Piece {
+    int b, ctx, pair, g0, g1, slot;   // groups [g0, g1) of a pair of sequence b; index of the partial result among the pair's
+    MA_DEV bool take(const DecodeParams& p, int lane, int w) {
+        const int pairs = p.Hkv * p.n_hg, n_waves = p.n_wg * kDecodeWaves;
+        const int c = lane < p.B ? min(max(p.ctx[lane], 0), p.Lmax) : 0;
+        const int n = (c + p.group_rows - 1) / p.group_rows;
+        int piece = work_quota(p, lane_value(wave_inclusive_scan(n * pairs), 63));
+        int each, incl, total;
+        // (ends: with a piece of Lmax rows there are no more pieces than pairs, and no more of these than waves)
+        for (;; piece += 1 + piece / 16) {
+            each = (n + piece - 1) / piece;
+            incl = wave_inclusive_scan(each * pairs);
+            total = lane_value(incl, 63);
+            if (total <= n_waves) break;
+        }
+        if (blockIdx.x == 0 && w == 0 && lane == 0) p.seq_off[p.B + 1] = piece;
+        const int x = total <= (int)gridDim.x ? w * (int)gridDim.x + (int)blockIdx.x : (int)blockIdx.x * kDecodeWaves + w;
+        if (x >= total) return false;
+        b = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(x < incl)) - 1);
+        const int k = lane_value(each, b), n_b = lane_value(n, b);
+        const int local = x - (lane_value(incl, b) - k * pairs);
+        ctx = lane_value(c, b);
+        pair = local / k;
+        slot = local - pair * k;
+        const int size = n_b / k, longer = n_b - size * k;   // the first `longer` pieces are a group longer
+        g0 = slot * size + min(slot, longer);
+        g1 = g0 + size + (slot < longer ? 1 : 0);
         return true;
     }
 };
@@ -340,18 +376,24 @@ MA_DEV void store_segment(const DecodeParams& p, int b, int g, int hg, int split
     }
 }
 
-template <class T, int D>
+template <class T, int D, bool PIECES>
 __global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode_split_kernel(const DecodeParams p) {
     __shared__ __attribute__((aligned(1024))) char v_lds[kDecodeWaves][kGroupRows * D * 2];
     __shared__ __attribute__((aligned(1024))) char k_lds[kDecodeWaves][kGroupRows * D * 2];
     const int lane = threadIdx.x & 63, w = wave_id();
-    SegmentWalk walk;
-    if (!walk.start(p, lane, w)) return;   // no share of the work
-    while (walk.next(p)) {
-        const int g = walk.pair % p.Hkv, hg = walk.pair / p.Hkv;
+    auto stream = [&](const auto& seg) __attribute__((always_inline)) {
+        const int g = seg.pair % p.Hkv, hg = seg.pair / p.Hkv;
         DecodeAcc<D> acc;
-        stream_rows<T, D>(p, walk.b, g, hg, walk.g0 * kGroupRows, min(walk.g1 * kGroupRows, walk.ctx), walk.g1 - walk.g0, k_lds[w], v_lds[w], acc);
-        store_segment<D>(p, walk.b, g, hg, walk.slot, acc);
+        stream_rows<T, D>(p, seg.b, g, hg, seg.g0 * kGroupRows, min(seg.g1 * kGroupRows, seg.ctx), seg.g1 - seg.g0, k_lds[w], v_lds[w], acc);
+        store_segment<D>(p, seg.b, g, hg, seg.slot, acc);
+    };
+    if constexpr (PIECES) {
+        Piece piece;
+        if (piece.take(p, lane, w)) stream(piece);
+    } else {
+        SegmentWalk walk;
+        if (!walk.start(p, lane, w)) return;   // no share of the work
+        while (walk.next(p)) stream(walk);
     }
 }
 
@@ -601,17 +643,23 @@ MA_DEV void stream_rows_q8(const DecodeParams& p, int b, int g, int hg, int row_
     acc.l = sum_across_quads(l_sum);
 }
 
-template <int D>
+template <int D, bool PIECES>
 __global__ __launch_bounds__(kDecodeWaves * 64, kDecodeWavesPerSimd) void decode_split_q8_kernel(const DecodeParams p) {
     __shared__ __attribute__((aligned(1024))) char lds[kDecodeWaves][(DecodeGeomQ8<D>::WAVE_LDS + 1023) / 1024 * 1024];
     const int lane = threadIdx.x & 63, w = wave_id();
-    SegmentWalk walk;
-    if (!walk.start(p, lane, w)) return;   // no share of the work
-    while (walk.next(p)) {
-        const int g = walk.pair % p.Hkv, hg = walk.pair / p.Hkv;
+    auto stream = [&](const auto& seg) __attribute__((always_inline)) {
+        const int g = seg.pair % p.Hkv, hg = seg.pair / p.Hkv;
         DecodeAcc<D> acc;
-        stream_rows_q8<D>(p, walk.b, g, hg, walk.g0 * kGroupRowsQ8, min(walk.g1 * kGroupRowsQ8, walk.ctx), walk.g1 - walk.g0, lds[w], acc);
-        store_segment<D>(p, walk.b, g, hg, walk.slot, acc);
+        stream_rows_q8<D>(p, seg.b, g, hg, seg.g0 * kGroupRowsQ8, min(seg.g1 * kGroupRowsQ8, seg.ctx), seg.g1 - seg.g0, lds[w], acc);
+        store_segment<D>(p, seg.b, g, hg, seg.slot, acc);
+    };
+    if constexpr (PIECES) {
+        Piece piece;
+        if (piece.take(p, lane, w)) stream(piece);
+    } else {
+        SegmentWalk walk;
+        if (!walk.start(p, lane, w)) return;   // no share of the work
+        while (walk.next(p)) stream(walk);
     }
 }
 
@@ -646,9 +694,9 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecodeParams 
     for (int u = 0; u < kEarly; ++u) load_o(min(u, p.S - 1), x[u]);
     // the partial results of this row: one per share of the line that overlaps the rows of its (sequence, KV head)
     const int n_b = groups_of(p, p.ctx[b]);
-    const int quota = work_quota(p, p.seq_off[p.B]);
+    const int piece = p.seq_off[p.B + 1], quota = piece > 0 ? piece : work_quota(p, p.seq_off[p.B]);
     const int g = hq / p.n_rep, hg = (hq % p.n_rep) / 16;
-    const int start = p.seq_off[b] + (hg * p.Hkv + g) * n_b;
+    const int start = piece > 0 ? 0 : p.seq_off[b] + (hg * p.Hkv + g) * n_b;
     const int ns = n_b > 0 ? (start + n_b - 1) / quota - start / quota + 1 : 0;
     const float m = lane < ns ? m_raw : -INFINITY, l = lane < ns ? l_raw : 0.f;
     const float M = wave_max(m);
@@ -925,6 +973,16 @@ static int decode_chunk_rows(const DecodeParams& p, int D, bool q8) {
     return chunk <= (full ? 2048 : 1536) ? (int)chunk : 0;
 }
 
+// Whether every pair is cut into pieces of its own (Piece) instead of shares of the line.  Equal pieces of few pairs leave waves
+// idle (784 pairs of 3073 rows, two pieces each, Q8_0 112.5 -> 126.5 us; 960 to 2864 40.2 -> 43.5): up to an eighth as many pairs as
+// waves at any length, and up to a quarter where a share would have 512 rows at most and the crossings weigh more (us, line /
+// pieces: 200 pairs of 2666, Q8_0 35.4 / 33.0; 160 of 2363 36.0 / 35.3; 112 of 20488 181 / 180; 240 of 6511 at D=64 65.4 / 62.3; 320 of
+// 1101 28.0 / 26.3; 408 of 1666, Q8_0 40.3 / 38.3; 512 to 683, Q8_0 20.1 / 18.6; but 512 to 8192 176.7 / 179.0).
+static bool decode_takes_pieces(const DecodeParams& p) {
+    const int64_t pairs = (int64_t)p.B * p.Hkv * p.n_hg, waves = (int64_t)p.n_wg * kDecodeWaves;
+    return p.B <= 64 && (pairs <= waves / 8 || (pairs <= waves / 4 && pairs * p.Lmax <= 512 * waves));
+}
+
 template <class T, int D, bool Q8>
 static int launch_chunks(const DecodeParams& p, int chunk, void* out, int64_t o0, int64_t o1, hipStream_t stream) {
     const unsigned n = (unsigned)((p.Lmax + chunk - 1) / chunk);
@@ -939,7 +997,8 @@ static int launch_chunks(const DecodeParams& p, int chunk, void* out, int64_t o0
 template <class T, int D>
 static int launch_decode(const DecodeParams& p, void* out, int64_t o0, int64_t o1, hipStream_t stream) {
     if (const int chunk = decode_chunk_rows(p, D, false)) return launch_chunks<T, D, false>(p, chunk, out, o0, o1, stream);
-    hipLaunchKernelGGL((decode_split_kernel<T, D>), dim3((unsigned)p.n_wg), dim3(kDecodeWaves * 64), 0, stream, p);
+    if (decode_takes_pieces(p)) hipLaunchKernelGGL((decode_split_kernel<T, D, true>), dim3((unsigned)p.n_wg), dim3(kDecodeWaves * 64), 0, stream, p);
+    else hipLaunchKernelGGL((decode_split_kernel<T, D, false>), dim3((unsigned)p.n_wg), dim3(kDecodeWaves * 64), 0, stream, p);
     if (int rc = check_launch("decode_split_kernel")) return rc;
     hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((p.B * p.Hq + 3) / 4), dim3(256), 0, stream, p, out, o0, o1);
     return check_launch("decode_combine_kernel");
@@ -948,7 +1007,8 @@ static int launch_decode(const DecodeParams& p, void* out, int64_t o0, int64_t o
 template <int D>
 static int launch_decode_q8(const DecodeParams& p, void* out, int64_t o0, int64_t o1, hipStream_t stream) {
     if (const int chunk = decode_chunk_rows(p, D, true)) return launch_chunks<F16, D, true>(p, chunk, out, o0, o1, stream);
-    hipLaunchKernelGGL((decode_split_q8_kernel<D>), dim3((unsigned)p.n_wg), dim3(kDecodeWaves * 64), 0, stream, p);
+    if (decode_takes_pieces(p)) hipLaunchKernelGGL((decode_split_q8_kernel<D, true>), dim3((unsigned)p.n_wg), dim3(kDecodeWaves * 64), 0, stream, p);
+    else hipLaunchKernelGGL((decode_split_q8_kernel<D, false>), dim3((unsigned)p.n_wg), dim3(kDecodeWaves * 64), 0, stream, p);
     if (int rc = check_launch("decode_split_q8_kernel")) return rc;
     hipLaunchKernelGGL((decode_combine_kernel<F16, D>), dim3((p.B * p.Hq + 3) / 4), dim3(256), 0, stream, p, out, o0, o1);
     return check_launch("decode_combine_kernel");

@@ -181,6 +181,32 @@ def test_decode_chunks(Hq, Hkv, Lmax, D):
         assert torch.equal(out, outs[0])
 
 
+@pytest.mark.parametrize("q8", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,Lmax,D", [
+    (2, 4, 2, 40007, 64),      # four pairs of many pieces
+    (12, 20, 1, 9001, 128),    # two head groups
+    (40, 8, 8, 1101, 64),      # 320 pairs
+    (64, 8, 8, 300, 128),      # 512 pairs, one or a few pieces each: as many as are taken
+    (33, 4, 4, 2050, 128),
+])
+def test_decode_pieces(B, Hq, Hkv, Lmax, D, q8):
+    """Pairs cut into pieces of their own: contexts from nothing to the capacity, around a group's and a piece's edges, against the
+    oracle.  Tolerance: that of every fp16 attention result here."""
+    lens = [Lmax, 0, 1, 16, 33, 127, 129, Lmax - 1, Lmax // 2 + 1, 257]
+    q, kc, vc, _ = workloads.decode_cache(seed=B + Lmax, device=DEV, B=B, Hq=Hq, Hkv=Hkv, Lmax=Lmax, D=D, ctx_lo=1, ctx_hi=1)
+    ctx = torch.tensor([lens[i % len(lens)] for i in range(B)], dtype=torch.int32, device=DEV)
+    out = torch.full(q.shape, float("nan"), dtype=q.dtype, device=DEV)
+    if q8:
+        kc, vc = workloads.q8_0_rows(kc), workloads.q8_0_rows(vc)
+        assert capi.flash_attn_decode_q8_0(q, kc, vc, ctx, out) == capi.OK, capi.last_error()
+        want = oracle.flash_attn_decode_q8_0(q.cpu(), kc.cpu(), vc.cpu(), ctx.cpu())
+    else:
+        assert capi.flash_attn_decode(q, kc, vc, ctx, out) == capi.OK, capi.last_error()
+        want = oracle.flash_attn_decode(q, kc, vc, ctx)
+    torch.cuda.synchronize()
+    assert max_err(out, want) <= TOL[torch.float16]
+
+
 def test_merged_parts_on_every_kind_of_stream(monkeypatch):
     """The null stream, the per-thread one (handle 2) and a created one: whether a launch's last workgroups or a second launch
     merge the parts of a decode and add up the K slices of a projection, the bits are the same."""
