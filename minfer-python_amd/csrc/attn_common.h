@@ -5,6 +5,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+#include <utility>
+
 namespace minfer_attn {
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -21,6 +24,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 #define MA_DEV __device__ __forceinline__
+
+template <int A, class F, int... I> MA_DEV void for_range_(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, A + I>{}), ...); }
+// f(A), f(A + 1) .. f(B - 1), the index a compile-time constant
+template <int A, int B, class F> MA_DEV void for_range(F&& f) { for_range_<A>(f, std::make_integer_sequence<int, B - A>{}); }
 
 // 16-bit element types.  Operand fragments travel as raw 16-bit lanes (s16x8 / s16x4) and are
 // bit-cast at the MFMA call, so one kernel body serves both.
@@ -139,11 +146,11 @@ MA_DEV void copy16_global_to_lds(const void* uniform_base, uint32_t lane_byte_of
 }
 
 // Same, for a loop that counts its issue slots: the destination as a wave-uniform LDS address plus a compile-time offset (three
-// instructions; from a generic pointer the address costs two to four more).  The base must be a scalar value long before the call.
-template <int LDS_OFFSET> MA_DEV void copy16_global_to_lds_at(const void* uniform_base, uint32_t lane_byte_offset, uint32_t lds_uniform) {
-    asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
+// instructions; from a generic pointer the address costs two to four more).
+template <int LDS_OFFSET, bool BASE_FRESH = false> MA_DEV void copy16_global_to_lds_at(const void* uniform_base, uint32_t lane_byte_offset, uint32_t lds_uniform) {
+    asm volatile("s_add_u32 m0, %0, %1\n\ts_nop %4\n\tglobal_load_lds_dwordx4 %2, %3"
                  :
-                 : "s"(lds_uniform), "i"(LDS_OFFSET), "v"(lane_byte_offset), "s"((uint64_t)(uintptr_t)uniform_base)
+                 : "s"(lds_uniform), "i"(LDS_OFFSET), "v"(lane_byte_offset), "s"((uint64_t)(uintptr_t)uniform_base), "i"(BASE_FRESH ? 3 : 0)
                  : "memory", "m0", "scc");
 }
 

@@ -184,7 +184,7 @@ template <int D, int NW> struct TileGeom {
 // of its own; the second team's sums go to the first through LDS.  A launch of few workgroups ends with its longest one, whose
 // tiles run one after the other: this halves them.
 template <class T, int D, int MODE, int NW, int TEAMS = 1>
-__global__ __launch_bounds__(NW * TEAMS * 64, 2) void prefill_kernel(const PrefillParams p) {
+__global__ __launch_bounds__(NW * TEAMS * 64, D == 64 && NW == kWavesSmall && TEAMS == 1 && MODE != MODE_DENSE_SELF ? 3 : 2) void prefill_kernel(const PrefillParams p) {
     static_assert(TEAMS == 1 || NW == 4, "the teams' stages and the 32 rows of NW waves fill the LDS");
     using GEO = TileGeom<D, NW>;
     constexpr int RB = GEO::RB, G = GEO::G, RPI = GEO::RPI, NLD = GEO::NLD;
@@ -382,41 +382,47 @@ __global__ __launch_bounds__(NW * TEAMS * 64, 2) void prefill_kernel(const Prefi
     s16x8 qf[2][KC];   // the wave's query rows as B-operand fragments; filled once the first K/V tile has been requested
 
     // ---- global -> LDS tile copy ----------------------------------------------------------
-    // Instruction j of this wave fills rows (j*kWaves + w)*RPI .. +RPI-1 of the tile.  The lane's byte offset from the
-    // first of the instruction's rows is a constant (row and swizzled granule; kWaves*RPI is a multiple of every
-    // swizzle period, so it is the same for every j), and the instruction's first row goes into the scalar base: a
-    // full tile costs no vector ALU work.
+    // Instruction j of this wave fills rows (j*kWaves + w)*RPI .. +RPI-1 of the tile (1 KiB); the lane's byte offset from the tile's
+    // first row is a constant (row and swizzled granule; kWaves*RPI is a multiple of every swizzle period): a full tile costs
+    // no vector ALU work, and three scalar instructions a copy.
     static_assert((kWaves * RPI) % 16 == 0, "the swizzles repeat every 16 rows at most");
-    uint32_t k_off0, v_off0;
+    constexpr int NOFF = D == 128 ? NLD : 1;   // at head_dim 64 the instruction's rows go into the base: two registers less let a third workgroup on a unit
+    uint32_t k_off[NOFF], v_off[NOFF];
     {
         const int row = w * RPI + lane / G, pg = lane % G;
-        k_off0 = (uint32_t)((int64_t)(lane / G) * p.kv2 + 8 * (pg ^ GEO::swz_k(row))) * 2u;
-        v_off0 = (uint32_t)((int64_t)(lane / G) * p.kv2 + 8 * (pg ^ GEO::swz_v(row))) * 2u;
+#pragma unroll
+        for (int j = 0; j < NOFF; ++j) {
+            const int64_t at = (int64_t)(row + j * kWaves * RPI) * p.kv2;
+            k_off[j] = (uint32_t)(at + 8 * (pg ^ GEO::swz_k(row))) * 2u;
+            v_off[j] = (uint32_t)(at + 8 * (pg ^ GEO::swz_v(row))) * 2u;
+        }
     }
-    // In this one instantiation the compiler (out of scalar registers) keeps the row bases in vector registers and moves
+    // In these instantiations the compiler (out of scalar registers) keeps the row bases in vector registers and moves
     // them to scalar ones right in front of every copy, closer than a copy may follow such a move (copy16_global_to_lds);
     // the build's scan of the generated code is what says which instantiations need this.
     constexpr bool kFreshBases = TEAMS > 1 || (MODE == MODE_VARLEN && NW == 4 && D == 128);
-    auto issue_tile = [&](int kt, int stage) {
+    const uint32_t dst0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds_addr(&kv_lds[0][0]) + w * 1024));
+    // copy c (K's, then V's) of the key tile at kbase, vbase into stage STAGE
+    auto copy_one = [&](auto c_tag, auto stage_tag, const short* kbase, const short* vbase) __attribute__((always_inline)) {
+        constexpr int c = decltype(c_tag)::value, is_v = c >= NLD, j = c - is_v * NLD;
+        constexpr int AT = decltype(stage_tag)::value * STAGE_BYTES + is_v * GEO::TILE_BYTES + j * kWaves * 1024;
+        const short* base = (is_v ? vbase : kbase) + (NOFF == 1 ? (int64_t)(j * kWaves * RPI) * p.kv2 : 0);
+        copy16_global_to_lds_at<AT, kFreshBases>(base, (is_v ? v_off : k_off)[NOFF == 1 ? 0 : j], dst0);
+    };
+    auto issue_tile = [&](int kt, auto stage_tag) __attribute__((always_inline)) {
         const int key0 = kt * 64;
         const short* kbase = Kh + (int64_t)key0 * p.kv2;
         const short* vbase = Vh + (int64_t)key0 * p.kv2;
         if (key0 + 64 <= seq_len) {
-#pragma unroll
-            for (int j = 0; j < NLD; ++j) {
-                const int row0 = (j * kWaves + w) * RPI;
-                copy16_global_to_lds<kFreshBases>(kbase + (int64_t)row0 * p.kv2, k_off0, &kv_lds[stage][row0 * RB]);
-                copy16_global_to_lds<kFreshBases>(vbase + (int64_t)row0 * p.kv2, v_off0, &kv_lds[stage][GEO::TILE_BYTES + row0 * RB]);
-            }
+            for_range<0, 2 * NLD>([&](auto c) __attribute__((always_inline)) { copy_one(c, stage_tag, kbase, vbase); });
         } else {   // tile crossing the end of the sequence: rows past it re-read the last row
-#pragma unroll
-            for (int j = 0; j < NLD; ++j) {
-                const int row0 = (j * kWaves + w) * RPI;
-                const int row = row0 + lane / G, pg = lane % G;
+            for_range<0, NLD>([&](auto j) __attribute__((always_inline)) {
+                constexpr int AT = decltype(stage_tag)::value * STAGE_BYTES + j.value * kWaves * 1024;
+                const int row = (j.value * kWaves + w) * RPI + lane / G, pg = lane % G;
                 const int64_t grow = (int64_t)(min(key0 + row, last_row) - key0) * p.kv2;
-                copy16_global_to_lds<kFreshBases>(kbase, (uint32_t)(grow + 8 * (pg ^ GEO::swz_k(row))) * 2u, &kv_lds[stage][row0 * RB]);
-                copy16_global_to_lds<kFreshBases>(vbase, (uint32_t)(grow + 8 * (pg ^ GEO::swz_v(row))) * 2u, &kv_lds[stage][GEO::TILE_BYTES + row0 * RB]);
-            }
+                copy16_global_to_lds_at<AT, kFreshBases>(kbase, (uint32_t)(grow + 8 * (pg ^ GEO::swz_k(row))) * 2u, dst0);
+                copy16_global_to_lds_at<AT + GEO::TILE_BYTES, kFreshBases>(vbase, (uint32_t)(grow + 8 * (pg ^ GEO::swz_v(row))) * 2u, dst0);
+            });
         }
     };
 
@@ -495,9 +501,15 @@ __global__ __launch_bounds__(NW * TEAMS * 64, 2) void prefill_kernel(const Prefi
     };
 
     // ---- one key tile, K/V in LDS stage STAGE (compile-time, so every LDS address is base + immediate) ----
-    auto process_tile = [&](auto stage_tag, int kt, uint32_t cls_w) {
+    constexpr bool kCopiesBetween = NW == kWavesSmall && D == 128;
+    // Three scalar instructions a copy, and with four waves at head_dim 128 the copies between the MFMAs instead of in front of them (32
+    // heads over 8, us: L=512 15.0 -> 14.4, 1000 24.7 -> 23.5, 1777 47.9 -> 46.7, 8 over 2 L=2048 37.1 -> 34.6, packed 32 to 1200, 24
+    // over 8 187 -> 180; with eight waves, where the power budget is the bound, and at head_dim 64 no gain).  With `next` >= 0 the copies of key tile `next`, which lies wholly inside the sequence, are issued into the other stage between
+    // the MFMAs of the first product.
+    auto process_tile = [&](auto stage_tag, int kt, uint32_t cls_w, int next) {
         constexpr int STAGE = decltype(stage_tag)::value;
         constexpr int SOFF = STAGE * STAGE_BYTES;
+        const std::integral_constant<int, STAGE ^ 1> other_tag{};
         const int key0 = kt * 64;
         auto pin = [&]() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
 
@@ -517,31 +529,34 @@ __global__ __launch_bounds__(NW * TEAMS * 64, 2) void prefill_kernel(const Prefi
         // requested.  The accumulators start from -reference (neg_ref, a register block that changes only when the
         // reference does), so the MFMA output is the exponent relative to the reference.
         f32x4 e_acc[4][2];
-        {
+        auto first_product = [&](auto copy_tag) __attribute__((always_inline)) {
+            constexpr bool COPY = decltype(copy_tag)::value;
+            const short* kbase = Kh + (int64_t)next * 64 * p.kv2;
+            const short* vbase = Vh + (int64_t)next * 64 * p.kv2;
             s16x8 kf[2][4];   // [buffer][key block]
 #pragma unroll
             for (int c = 0; c < 2 && c < KC; ++c)
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb) kf[c][kb] = lds_read_b128(k_rd[c], SOFF + 16 * kb * RB);
             pin();
+            for_range<0, KC * 4>([&](auto i_tag) __attribute__((always_inline)) {
+                constexpr int i = decltype(i_tag)::value, c = i / 4, kb = i % 4;
 #pragma unroll
-            for (int c = 0; c < KC; ++c) {
+                for (int qb = 0; qb < 2; ++qb)
+                    e_acc[kb][qb] = T::mfma16(kf[c & 1][kb], qf[qb][c], c == 0 ? neg_ref[qb] : e_acc[kb][qb]);
+                pin();
+                if (c + 2 < KC) {
+                    kf[c & 1][kb] = lds_read_b128(k_rd[c + 2], SOFF + 16 * kb * RB);
+                } else if (c + 1 == KC) {
 #pragma unroll
-                for (int kb = 0; kb < 4; ++kb) {
-#pragma unroll
-                    for (int qb = 0; qb < 2; ++qb)
-                        e_acc[kb][qb] = T::mfma16(kf[c & 1][kb], qf[qb][c], c == 0 ? neg_ref[qb] : e_acc[kb][qb]);
-                    pin();
-                    if (c + 2 < KC) {
-                        kf[c & 1][kb] = lds_read_b128(k_rd[c + 2], SOFF + 16 * kb * RB);
-                    } else if (c + 1 == KC) {
-#pragma unroll
-                        for (int db = kb * (DB / 4); db < (kb + 1) * (DB / 4); ++db) va[db] = read_v(0, db);
-                    }
-                    pin();
+                    for (int db = kb * (DB / 4); db < (kb + 1) * (DB / 4); ++db) va[db] = read_v(0, db);
                 }
-            }
-        }
+                if constexpr (COPY)
+                    for_range<i * 2 * NLD / (KC * 4), (i + 1) * 2 * NLD / (KC * 4)>([&](auto x) __attribute__((always_inline)) { copy_one(x, other_tag, kbase, vbase); });
+                pin();
+            });
+        };
+        if (kCopiesBetween && next >= 0) first_product(std::integral_constant<bool, kCopiesBetween>{}); else first_product(std::false_type{});
 
         // ---- masking ----------------------------------------------------------------------
         // The test by position (keys past the end of the sequence; in a packed batch also keys after the lane's query
@@ -649,7 +664,7 @@ __global__ __launch_bounds__(NW * TEAMS * 64, 2) void prefill_kernel(const Prefi
     int kt_first = 0; uint32_t cls_first = TILE_NONE;
     if (n_own > 0) {
         tile_of(e_cur, 0, kt_first, cls_first);
-        issue_tile(kt_first, 0);
+        issue_tile(kt_first, std::integral_constant<int, 0>{});
     }
     // ---- Q fragments (B operand): lane = query row 16qb + l16, d = 32c + 8 quad + 0..7 --------------------
     // Q is multiplied by scale*log2(e) once, here, so that the MFMA accumulator of Q K^T is directly
@@ -674,14 +689,17 @@ __global__ __launch_bounds__(NW * TEAMS * 64, 2) void prefill_kernel(const Prefi
         const uint32_t e_after = list_entry(it + 2);   // read early, used next iteration
         wait_vmcnt<0>();       // this wave's share of tile `it` (and its mask words) has landed
         __syncthreads();       // everyone's has; stage STAGE^1 is no longer being read
-        if (it + 1 < n_own) issue_tile(ktn, STAGE ^ 1);
+        // the next tile's copies: between this tile's MFMAs, or now where it has none or the next tile crosses the sequence's end
+        const bool on = cls_w != TILE_NONE && (TEAMS == 1 || it < n_own);
+        const bool between = kCopiesBetween && on && it + 1 < n_own && ktn * 64 + 64 <= seq_len;
+        if (it + 1 < n_own && !between) issue_tile(ktn, std::integral_constant<int, STAGE ^ 1>{});
         // The next tile's mask words are requested after this tile's were used; with 4 waves already in front of a tile that
         // uses none (a short problem's few tiles wait for everything they request late: L=256 9.0 -> 8.6 us; with 8 waves the
         // second copy of the requests costs as much as it gives, S=4096 134.4 -> 135.7).
         const bool fetch = kDense && it + 1 < n_own && cn == TILE_MIXED;
         const bool early = NW == kWavesSmall && cls_w != TILE_MIXED;
         if (fetch && early) fetch_mask(ktn);
-        if (cls_w != TILE_NONE && (TEAMS == 1 || it < n_own)) process_tile(stage_tag, kt, cls_w);
+        if (on) process_tile(stage_tag, kt, cls_w, between ? ktn : -1);
         if (fetch && !early) fetch_mask(ktn);
         e_cur = e_next; e_next = e_after;
     };
@@ -773,9 +791,19 @@ static size_t cls_bytes(int64_t B, int64_t L) {
     return (size_t)(B * nt * nt + 255) / 256 * 256;
 }
 
+// At head_dim 64 three four-wave workgroups fit a unit (40 KiB of LDS, 168 registers), which is ahead where they come one after the
+// other (us, two / three to a unit: 16 x 512 rows of 32 heads 43.7 / 38.8, 8 x 300 of 24 heads 17.4 / 15.0, L=8192 292 / 269, 4096 under a
+// window of 256 31.8 / 30.3, packed 32 sequences to 1200 95.2 / 93.4).  Where all of them would be on the chip at once, but not two to a
+// unit, a causal mask's longest share their unit with two others and the launch ends with them: L=3000 56.6 / 59.0, 2 x 1400 31.0 /
+// 32.3, 3 x 800 (600 workgroups) 23.3 / 23.7 (but 2 x 900 of 48 heads, 720 of them, 24.7 / 23.1, and shorter sequences' tiles weigh
+// less than what a workgroup pays once); LDS that nobody uses keeps those to two.
+static unsigned unused_lds(int64_t L, int64_t grid) {
+    return grid > 512 && grid <= 768 && (L > 1024 || (L > 512 && grid < 704)) ? 20 * 1024 : 0;
+}
 template <class T, int D, int MODE, int NW, int TEAMS>
 static int launch_prefill(const PrefillParams& p, int grid, hipStream_t stream) {
-    hipLaunchKernelGGL((prefill_kernel<T, D, MODE, NW, TEAMS>), dim3(grid), dim3(NW * TEAMS * 64), 0, stream, p);
+    const unsigned pad = D == 64 && MODE == MODE_DENSE && NW == kWavesSmall && TEAMS == 1 ? unused_lds(p.L, grid) : 0;
+    hipLaunchKernelGGL((prefill_kernel<T, D, MODE, NW, TEAMS>), dim3(grid), dim3(NW * TEAMS * 64), pad, stream, p);
     return check_launch("prefill_kernel");
 }
 

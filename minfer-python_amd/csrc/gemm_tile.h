@@ -8,9 +8,6 @@
 
 namespace minfer_attn {
 
-template <int A, class F, int... I> MA_DEV void for_range_(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, A + I>{}), ...); }
-// f(A), f(A + 1) .. f(B - 1), the index a compile-time constant
-template <int A, int B, class F> MA_DEV void for_range(F&& f) { for_range_<A>(f, std::make_integer_sequence<int, B - A>{}); }
 typedef s16x8 __attribute__((aligned(8))) s16x8_a8;
 
 // Tile shapes: four waves (2 x 2), a wave owning M16 x N16 blocks of 16 x 16; NS stages of the K ring in LDS (NS - 1 steps in
