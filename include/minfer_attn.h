@@ -238,9 +238,9 @@ int minfer_gemm_ws(int dtype, int b_layout, const void* A, const void* B, const 
  * and an even number of blocks per weight row, a kernel streams the blocks once (34 bytes per 32 weights instead of
  * 64: the projections of a decode step) and no workspace is needed; for 2-64 rows against fewer than 12288 columns
  * minfer_gemm_q8_0_workspace_bytes still names one, for K slices as in minfer_gemm_ws (fp32 partial sums), which the call
- * uses when it is given in full and does without otherwise.  Other shapes dequantise the
- * weight into the workspace and run the fp16 kernels on it: for them a missing or too small workspace is
- * MINFER_ATTN_EWORKSPACE.  This is the case the reference's
+ * uses when it is given in full and does without otherwise.  Other shapes need room for the weight dequantised, which the
+ * fp16 kernels are then run on (65 to 160 rows against a large weight go through the streaming kernels in parts instead): for
+ * them a missing or too small workspace is MINFER_ATTN_EWORKSPACE.  This is the case the reference's
  * gemm_cuda routes to dispatch_quant_abt, whose body is empty (reference: gemm/op.cuh:199-210, 299-312); block format
  * common/types.hpp:141-146, dequantisation cuda/quants/impls.cuh:121-143.
  */

@@ -1581,6 +1581,18 @@ static bool q8_stream_operands(const void* A, const void* C, const void* D, int6
            (beta == 0.0 || (ldc % 4 == 0 && ((uintptr_t)C & 7u) == 0));
 }
 
+// More rows than the kernels that stream the blocks take: in how many calls of theirs a product goes all the same (1: none, the
+// weight is dequantised).  Dequantising writes and reads back twice the blocks' bytes; a second call reads the blocks again,
+// from the last-level cache mostly (us, weights from memory, dequantised / in parts): 65 rows x 14336 x 4096 64.0 / 39.4, 4096 x 14336
+// 61.7 / 42.3, 128256 x 4096 488 / 288, 6144 x 4096 32.8 / 28.6, 4096 x 4096 24.4 / 21.8; 128 rows 72.1 / 46.3, 70.3 / 49.7, 496 / 337,
+// 37.3 / 34.8, 26.3 / 27.0; 160 rows in three 76.2 / 64.9, 73.9 / 69.8, 507 / 483, 40.4 / 48.1; 192 28672 x 4096 124 / 128.
+static int64_t q8_parts(int64_t M, int64_t N, int64_t K, const void* Bq) {
+    if (M <= kQ8SkinnyRows || M > 160 || N * K < (M <= 96 ? INT64_C(16000000) : M <= 128 ? INT64_C(20000000) : INT64_C(50000000))) return 1;
+    const int64_t parts = (M + kQ8SkinnyRows - 1) / kQ8SkinnyRows, rows = M / parts, row_bytes = K / 32 * 34;
+    const bool stripes = q8_stripe_ok(rows, N, K, Bq, row_bytes) || (aligned16(Bq) && row_bytes % 16 == 0 && q8_slices(rows, N, K) > 1);
+    return stripes ? parts : 1;
+}
+
 MINFER_ATTN_EXPORT size_t minfer_gemm_q8_0_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 32 != 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
     if (q8_streams(M, N, K)) {   // optional: K slices of the stripe kernel for a narrow weight
@@ -1617,12 +1629,19 @@ MINFER_ATTN_EXPORT int minfer_gemm_q8_0(const void* A, const void* Bq, const voi
         if (q8_stripe_ok(M, N, K, Bq, row_bytes)) return launch_stripe_q8(p, stream);
         return launch_skinny_q8(p, stream);
     }
-    // otherwise: the weight as fp16 in the workspace, then the fp16 kernels on it
+    // otherwise: the weight as fp16 in the workspace, then the fp16 kernels on it, or the call in parts (q8_parts)
     const size_t deq = q8_dequant_bytes(N, K);
     if (!workspace || !aligned16(workspace) || workspace_bytes < deq)
         return fail(MINFER_ATTN_EWORKSPACE, "gemm_q8_0: this call needs a workspace of N*K*2 bytes (rounded up to 256) for the dequantised weight "
                                             "(more than 64 rows, an odd number of blocks per row, N not a multiple of 4, or A/C/D not aligned for the streaming kernel: "
                                             "A 16 bytes with lda a multiple of 8, C and D 8 bytes with strides multiples of 4)");
+    if (const int64_t parts = q8_parts(M, N, K, Bq); parts > 1 && q8_stream_operands(A, C, D, lda, ldc, ldd, beta)) {
+        const int64_t rows = ((M + parts - 1) / parts + 15) / 16 * 16;
+        for (int64_t m = 0; m < M; m += rows)
+            if (int rc = minfer_gemm_q8_0((const short*)A + m * lda, Bq, C ? (const short*)C + m * ldc : nullptr, (short*)D + m * ldd, std::min(rows, M - m), N, K,
+                                          lda, ldc, ldd, alpha, beta, workspace, workspace_bytes, stream_v)) return rc;
+        return MINFER_ATTN_OK;
+    }
     if (int rc = minfer_dequant_q8_0(MINFER_ATTN_F16, Bq, workspace, N, K, stream_v)) return rc;
     return gemm_impl(MINFER_ATTN_F16, MINFER_GEMM_B_NK, A, workspace, C, D, M, N, K, lda, K, ldc, ldd, alpha, beta,
                      (char*)workspace + deq, workspace_bytes - deq, stream_v);

@@ -528,6 +528,27 @@ def test_gemm_q8_0_weights_against_oracle(M, N, K, alpha, beta):
         assert capi.gemm_q8_0(da, dwq, dc, d, alpha, beta, None) == capi.EWORKSPACE and "workspace" in capi.last_error()
 
 
+@pytest.mark.parametrize("M,N,K,alpha,beta", [
+    (65, 10248, 2048, 2.0, 3.0),     # 48 rows and 17
+    (96, 4104, 4096, 1.0, 0.0),      # 48 and 48 in K slices, in the workspace that a dequantised weight would take
+    (113, 10248, 2048, 1.0, 1.0),    # 64 and 49
+    (128, 6152, 4096, 0.5, 0.0),
+    (130, 12296, 4352, 1.0, 1.0),    # 48, 48 and 34
+])
+def test_gemm_q8_0_in_parts(M, N, K, alpha, beta):
+    """65 to 160 rows against a large weight go through the block-streaming kernels in parts: every element against torch's product
+    with the dequantised weight in 64 bits, within the bound of assert_close; no less workspace is accepted than before."""
+    a, wq, c, w_deq = make_q8(M, N, K, seed=M + N)
+    need = capi.lib().minfer_gemm_q8_0_workspace_bytes(M, N, K)
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=DEV)
+    d = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
+    da, dwq, dc = a.to(DEV), wq.to(DEV), c.to(DEV)
+    assert capi.gemm_q8_0(da, dwq, dc, d, alpha, beta, ws) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    assert_close(d, (alpha * (a.double() @ w_deq.double().T) + beta * c.double()).numpy(), torch.float16)
+    assert capi.gemm_q8_0(da, dwq, dc, d, alpha, beta, ws[:N * K * 2 - 256]) == capi.EWORKSPACE
+
+
 def test_gemm_op_with_q8_0_weight(kerns):
     M, N, K = 8, 2048, 4096
     a, wq, c, w_deq = make_q8(M, N, K, seed=3)
