@@ -149,6 +149,7 @@ struct PrefillParams {
     int n_hg;              // head groups per KV head = n_rep >> hpw_log2
     int NQT, NKT;          // dense: 64-row query / key tile counts of the mask classification
     int NQ;                // workgroup-level query tiles (dense: exact; varlen: upper bound)
+    int fold;              // dense: fold_order's units, or 0
     int n_seqs;
     int max_len;           // varlen: rows of a sequence past this many are not computed (>= every length for a valid call)
     float scale_log2;      // softmax scale * log2(e)
@@ -179,6 +180,15 @@ template <int D, int NW> struct TileGeom {
     static MA_DEV int swz_k(int row) { return (row / RPW) & (G - 1); }
     static MA_DEV int swz_v(int row) { return D == 128 ? ((row & 7) << 1) : (((row >> 1) & 3) << 1); }
 };
+
+// Workgroup id n as the place in the order of work (longest rows first) that it takes.  With `fold` = the chip's units, in a launch
+// whose workgroups are all on the chip at once, the ones after the first round come from the other end: a unit that has one of the
+// longest gets one of the shortest beside it.  by_xcd: within the ids of each XCD, which keep their residue mod 8.
+MA_DEV int fold_order(int n, int count, int fold, bool by_xcd) {
+    if (!fold) return n;
+    const int step = by_xcd ? 8 : 1, at = n / step, first = fold / step, total = count / step;
+    return n + (at < first ? 0 : (at < 2 * first ? total - 1 - (at - first) : at - first) - at) * step;
+}
 
 // TEAMS = 2: two teams of NW waves hold the same query rows and take the even and the odd key tiles of the list, each with stages
 // of its own; the second team's sums go to the first through LDS.  A launch of few workgroups ends with its longest one, whose
@@ -219,7 +229,7 @@ __global__ __launch_bounds__(NW * TEAMS * 64, D == 64 && NW == kWavesSmall && TE
     const int NG = BG * p.n_hg;
     int pidx, rank;
     {
-        const int n = blockIdx.x;
+        const int n = fold_order((int)blockIdx.x, (int)gridDim.x, p.fold, (NG & 7) == 0);
         if ((NG & 7) == 0) {  // keep all workgroups of one (batch, KV head) on one XCD (ids go round-robin)
             const int per = NG >> 3, mm = n >> 3;
             pidx = (mm % per) * 8 + (n & 7);
@@ -927,6 +937,10 @@ MINFER_ATTN_EXPORT int minfer_flash_attn(int dtype, const void* q, const void* k
     p.n_seqs = 0;
     const int64_t grid = (int64_t)p.NQ * B * Hkv * p.n_hg;
     if (grid > 0x7fffffffLL) return fail(MINFER_ATTN_EINVAL, "flash_attn: problem too large for one launch");
+    // Four-wave workgroups that are all on the chip, two to a unit at most: the second ones shortest first (us, in order / folded: 32 heads
+    // over 8 L=1777 47.4 / 45.1, 2048 52.8 / 49.5, 2 x 1000 33.4 / 32.4, 48 heads 1300 37.3 / 35.2, a window of 256 over 1777 23.6 / 22.4, at
+    // head_dim 64 1777 34.5 / 33.3; three to a unit gain nothing by it).
+    p.fold = kWaves == kWavesSmall && grid > 256 && grid <= 512 ? 256 : 0;
 
     // A short problem whose workgroups all fit on the chip at once (2 per CU, 256 CUs) needs no pre-pass: its workgroups
     // classify their own rows, which takes 2-3 us off a call of 9-28 us.  With more workgroups than that the pre-pass is

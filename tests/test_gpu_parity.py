@@ -181,6 +181,27 @@ def test_decode_chunks(Hq, Hkv, Lmax, D):
         assert torch.equal(out, outs[0])
 
 
+@pytest.mark.parametrize("Hq,Hkv,L,D,kind", [
+    (32, 8, 1100, 64, "causal"),     # 280 workgroups of eight (batch, KV head) groups: each XCD's ids folded by themselves
+    (32, 8, 1100, 128, "random"),
+    (6, 2, 5600, 64, "causal"),      # 264 workgroups of six groups: all ids folded together
+    (32, 8, 1100, 64, "blocky"),
+    (36, 9, 930, 64, "causal"),      # 270, classified in the kernel
+])
+def test_dense_workgroups_in_folded_order(Hq, Hkv, L, D, kind):
+    """Launches of more workgroups than units, all on the chip at once, take the second ones in the opposite order: every row is still
+    computed, and as in a batch of copies too many for that, bit for bit."""
+    q, k, v = workloads.dense_prefill(1, Hq, Hkv, L, D, torch.float16, seed=L, device=DEV)
+    mask = make_mask(kind, 1, L, torch.Generator().manual_seed(L))
+    out, outs = torch.full_like(q, float("nan")), torch.full((4, *q.shape[1:]), float("nan"), dtype=q.dtype, device=DEV)
+    assert capi.flash_attn(q, k, v, mask.to(DEV), out) == capi.OK, capi.last_error()
+    copies = [t.expand(4, *t.shape[1:]).contiguous() for t in (q, k, v, mask.to(DEV))]
+    assert capi.flash_attn(*copies, outs) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    assert not torch.isnan(out).any()
+    assert all(torch.equal(out[0], o) for o in outs)
+
+
 @pytest.mark.parametrize("q8", [False, True])
 @pytest.mark.parametrize("B,Hq,Hkv,Lmax,D", [
     (2, 4, 2, 40007, 64),      # four pairs of many pieces
