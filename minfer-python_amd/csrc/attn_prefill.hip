@@ -324,6 +324,9 @@ __global__ __launch_bounds__(NW * TEAMS * 64, D == 64 && NW == kWavesSmall && TE
     // (a workgroup that classifies its own rows does so per 32-row query block: slot = the wave's block)
     const int my_qt64_slot = MODE == MODE_DENSE_SELF ? (w >> p.hpw_log2) : (q_row0 >> 6) - qt64_first;
     int n_active;
+    // A last tile of fewer than 64 keys goes through its mask bytes whatever its class (class 1, all, becomes 2, mixed): fetch_mask
+    // clears those past the end, so that nothing else of a dense problem tests positions.
+    auto cut_tile = [&](uint32_t c, int kt) { return kt * 64 + 64 <= p.L ? c : (c & ~0x55555555u) | ((c & 0x55555555u) << 1); };
     if (MODE == MODE_DENSE_SELF) {
         // Every wave reads 32/HPW rows of its own query block (the HPW waves of a block share its rows), 8 rows in flight:
         // lane l holds the 16 mask bytes of key columns 16l .. 16l+15, so lanes 4t .. 4t+3 cover key tile t.  Rows past the
@@ -355,6 +358,7 @@ __global__ __launch_bounds__(NW * TEAMS * 64, D == 64 && NW == kWavesSmall && TE
                     for (int ww = sb * HPW; ww < (sb + 1) * HPW; ++ww) { a |= any_s[ww][kt]; l &= all_s[ww][kt]; }
                     c |= (a == 0u ? TILE_NONE : (l == 0x01010101u ? TILE_ALL : TILE_MIXED)) << (2 * sb);
                 }
+                c = cut_tile(c, kt);
             }
             const uint64_t bal = __ballot(c != 0);
             if (c) tile_list[__popcll(bal & ((1ull << lane) - 1ull))] = (uint32_t)kt | (c << 16);
@@ -373,6 +377,7 @@ __global__ __launch_bounds__(NW * TEAMS * 64, D == 64 && NW == kWavesSmall && TE
                         const int qs = qt64_first + s;
                         if (qs < p.NQT) c |= (uint32_t)p.cls[((size_t)b * p.NQT + qs) * p.NKT + kt] << (2 * s);
                     }
+                    c = cut_tile(c, kt);
                 }
                 const uint64_t bal = __ballot(c != 0);
                 const int pos = cnt + __popcll(bal & ((1ull << lane) - 1ull));
@@ -496,17 +501,24 @@ __global__ __launch_bounds__(NW * TEAMS * 64, D == 64 && NW == kWavesSmall && TE
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb)
                     mw[qb][kb] = *reinterpret_cast<const u32_any*>(mrow[qb] + key0 + 16 * kb + 4 * quad);
-        } else {  // a tile crossing the end: bytes, clamped (the range test comes later)
+        } else if (p.L >= 4) {  // a tile crossing the end: the row's last word where a word would cross it, shifted; none past the end
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb) {
-                    const int kbase = key0 + 16 * kb + 4 * quad;
-                    uint32_t x = 0;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x |= (uint32_t)mrow[qb][min(kbase + e, last_row)] << (8 * e);
-                    mw[qb][kb] = x;
+                    const int kbase = key0 + 16 * kb + 4 * quad, past = max(kbase - (last_row - 3), 0);
+                    const uint32_t x = *reinterpret_cast<const u32_any*>(mrow[qb] + (kbase - past));
+                    mw[qb][kb] = past < 4 ? x >> (8 * past) : 0u;
                 }
+        } else {                // a row of fewer than four bytes (one tile): byte by byte
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) {
+                uint32_t x = 0;
+                for (int e = 0; e <= last_row; ++e) x |= (uint32_t)mrow[qb][e] << (8 * e);
+                mw[qb][0] = quad == 0 ? x : 0u;
+#pragma unroll
+                for (int kb = 1; kb < 4; ++kb) mw[qb][kb] = 0u;
+            }
         }
     };
 
@@ -569,22 +581,27 @@ __global__ __launch_bounds__(NW * TEAMS * 64, D == 64 && NW == kWavesSmall && TE
         if (kCopiesBetween && next >= 0) first_product(std::integral_constant<bool, kCopiesBetween>{}); else first_product(std::false_type{});
 
         // ---- masking ----------------------------------------------------------------------
-        // The test by position (keys past the end of the sequence; in a packed batch also keys after the lane's query
-        // row) is one compare of a constant with a per-lane limit; dense MIXED tiles test their mask bytes as well.
-        if (cls_w == TILE_MIXED || key0 + 64 > seq_len) {
-            const bool use_bytes = kDense && cls_w == TILE_MIXED;
+        // Dense: the tile's mask bytes, three instructions an element.  Packed: one compare of a constant with a per-lane limit, the
+        // lane's query row or the end of the sequence.  With both tests on the dense elements (324 instructions a tile in place of
+        // 114), and a tile across the end read byte by byte (32 loads in place of 8): L=1003 with a window of 256 37.5 us, now 35.1;
+        // causal L=1000 23.4 / 21.3, L=256 8.3 / 7.9, L=60 9.15 / 7.7, L=4096 132.0 / 131.1.
+        if (kDense) {
+            if (cls_w == TILE_MIXED) {
+#pragma unroll
+                for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+                    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) e_acc[kb][qb][e] = ((mw[qb][kb] >> (8 * e)) & 0xffu) != 0u ? e_acc[kb][qb][e] : -INFINITY;
+            }
+        } else if (cls_w == TILE_MIXED || key0 + 64 > seq_len) {
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb) {
-                int lim = last_row - key0 - 4 * quad;                              // largest kept 16kb + e
-                if (MODE == MODE_VARLEN) lim = min(lim, qrow[qb] - key0 - 4 * quad);
+                const int lim = min(last_row, qrow[qb]) - key0 - 4 * quad;   // largest kept 16kb + e
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        bool keep = 16 * kb + e <= lim;
-                        if (kDense) keep = keep && (!use_bytes || ((mw[qb][kb] >> (8 * e)) & 0xffu) != 0u);
-                        e_acc[kb][qb][e] = keep ? e_acc[kb][qb][e] : -INFINITY;
-                    }
+                    for (int e = 0; e < 4; ++e) e_acc[kb][qb][e] = 16 * kb + e <= lim ? e_acc[kb][qb][e] : -INFINITY;
             }
         }
         // ---- reference update (rare after the first tiles) --------------------------------------

@@ -129,6 +129,17 @@ def test_dense_matches_oracle(dtype, B, Hq, Hkv, L, D, kind, views):
     assert max_err(out, want) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("kind", ["random", "full"])
+@pytest.mark.parametrize("L", [2, 3, 4, 5, 66, 67, 127, 129])
+def test_dense_mask_rows_end_inside_a_word(L, kind):
+    """Mask rows whose last key tile ends one to four bytes into a word, and rows shorter than one word: the tile's words come from
+    the row's end, shifted, and keys past it count for nothing, in mixed tiles and in tiles that every row attends."""
+    q, k, v = workloads.dense_prefill(2, 4, 2, L, 128, torch.float16, seed=L, scale=0.5, device=DEV)
+    mask = make_mask(kind, 2, L, torch.Generator().manual_seed(L))
+    out = run_prefill(q, k, v, mask.to(DEV))
+    assert max_err(out, oracle.flash_attn(q, k, v, mask)) <= TOL[torch.float16]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,Hq,Hkv,L,kind", [
     (3, 32, 8, 1093, "random"),    # n_rep = 4: 64 rows per workgroup, a last key tile of 5 rows
