@@ -399,30 +399,42 @@ static int launch_rows_lds(const GemmParams& p, int groups, hipStream_t stream) 
     return check_launch("gemm_rows_lds_kernel");
 }
 
-// Up to 64 rows against a wide [N, K] weight (a batch of decode steps against an FFN or output-head weight): a workgroup
-// of four waves owns a stripe of 64 columns over the whole of K; K goes by in segments of 256 values, the 64 weight rows
-// and the activation rows copied global -> LDS with instructions whose lanes walk along the rows (512 consecutive bytes
-// of each of two rows, 2 lines per quarter wave); three weight stages (two segments in flight) and two or three
+// Up to 64 rows against an [N, K] weight (a batch of decode steps against a projection, FFN or output-head weight): a workgroup
+// of four waves takes NB blocks of 16 columns at a time over the whole of K; K goes by in segments of 256 values, the 16 NB weight
+// rows and the activation rows copied global -> LDS with instructions whose lanes walk along the rows (512 consecutive bytes
+// of each of two rows, 2 lines per quarter wave); two to five weight stages and two to four
 // activation stages, one workgroup per compute unit (segments of 128 values and two workgroups per unit are 15-25 %
 // slower from 24 rows on).  No K slices across workgroups, so no partial sums in memory: the activations are read once
-// per stripe (N / 64 times in all) and the weight once.  Two rows of a copy share a 1 KiB block of LDS; inside block i
+// per workgroup and the weight once.  Two rows of a copy share a 1 KiB block of LDS; inside block i
 // the 16-byte pieces of a row sit at piece ^ (i & 7), so the 16 rows of a fragment read hit 16 different bank groups
-// without padding (160 KiB exactly at 49-64 rows).  It needs N / 64 stripes to fill the chip.
+// without padding.
+// What bounds it, once the weight does not (5 TB/s), is the copies a unit makes, 50-60 bytes per ns: NB is what the workgroups have,
+// one to four, the four waves share the copies of the rows there are, and the stages that smaller chunks leave room for keep as many
+// bytes in flight.  (With chunks of four whatever the workgroup had, the missing rows copied again, us, before / now: 6144 x 4096 at
+// 16 / 32 / 40 / 64 rows 10.9 / 10.0, 13.7 / 11.0, 14.1 / 12.4, 15.9 / 15.1; 4096 + 1024 + 1024 columns at 24 / 40 rows 13.5 / 11.1, 15.1 /
+// 12.5; 11008 x 4096 at 40 rows 20.4 / 19.5, 22016 x 4096 40.2 / 35.2; where chunks of four are still the choice, 28672 x 4096 at 64
+// rows 48.2 / 46.0, for the even share of the copies.)
 constexpr int kStripeSeg = 256;                                // K values per segment
 constexpr int kStripeBlock = 1024;                             // LDS bytes of two rows' segment
-template <int MB> struct StripeGeom {
-    static constexpr int W_BYTES = 4 * 8 * kStripeBlock;       // 64 weight rows
+template <int MB, int NB = 4> struct StripeGeom {   // 16-row blocks of activations, 16-column blocks of the weight
+    static constexpr int W_BYTES = NB * 8 * kStripeBlock;      // 16 * NB weight rows
     static constexpr int X_BYTES = MB * 8 * kStripeBlock;      // 16 * MB activation rows
-    static constexpr int WST = MB >= 4 ? 2 : 3, XST = MB >= 3 ? 2 : 3;   // 120 / 144 / 144 / 128 KiB
-    static constexpr int CW = 8, CX = 2 * MB;                  // copies per wave and segment
+    static constexpr int WST = NB == 1 ? (MB >= 4 ? 4 : 5) : NB == 2 ? (MB >= 4 ? 3 : 4) : (NB == 4 && MB >= 4 ? 2 : 3);
+    static constexpr int XST = NB == 1 ? (MB >= 4 ? 3 : 4) : NB == 2 ? 3 : (MB + NB >= 7 ? 2 : 3);   // 120 / 144 / 144 / 128 KiB, three blocks 96 / 120 / 144 / 136, two 88 / 112 / 136 / 144, one 72 / 104 / 136 / 128
+    static constexpr int CW = 2 * NB, CX = 2 * MB;             // copies per wave and segment
+    // copies issued after those of segment t, with `after` segments behind it: those of x(t) go out in front of w(t + WST - XST)
+    static constexpr int behind(int after) {
+        const int w = WST > XST ? (after < WST - 1 ? after : WST - 1) - (WST - XST) + 1 : (after < WST - 1 ? after : WST - 1);
+        return (w > 0 ? w : 0) * CW + (after < XST - 1 ? after : XST - 1) * CX;
+    }
 };
 // SLICED: p.splits workgroups per stripe, each over its share of the segments; they leave raw fp32 sums in p.part
 // ([slice][M][N]) for finish_slices.
 // GROUPED: the stripes of up to three weights numbered through (p.grp.end in stripes), alpha = 1 and no C.
-template <class T, int MB, bool SLICED = false, bool GROUPED = false>
+template <class T, int MB, bool SLICED = false, bool GROUPED = false, int NB = 4>
 __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p) {
     static_assert(!(SLICED && GROUPED), "the grouped launch has no workspace");
-    using G = StripeGeom<MB>;
+    using G = StripeGeom<MB, NB>;
     constexpr int WST = G::WST, XST = G::XST;
     __shared__ __attribute__((aligned(16))) char w_lds[WST][G::W_BYTES];
     __shared__ __attribute__((aligned(16))) char x_lds[XST][G::X_BYTES];
@@ -436,12 +448,11 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
     }
     // Which columns.  SLICED: workgroup b / splits owns stripe b / splits.  Plain launches: the 16-column blocks of the weight
     // are shared out evenly: workgroup g of G owns blocks g * blocks / G ..
-    // (g + 1) * blocks / G - 1 and goes through them four at a time, a chunk ending early at the end of the workgroup's
-    // range; the waves without a block of their own in such a chunk copy its last row again (from L2) and
-    // multiply what is never stored.  Every compute unit so streams the same share of the weight to within one block,
+    // (g + 1) * blocks / G - 1 and goes through them NB at a time, a chunk ending early at the end of the workgroup's
+    // range; its missing rows are the last one again (from L2) and
+    // what they multiply is never stored.  Every compute unit so streams the same share of the weight to within one block,
     // whatever the number of columns (448 stripes of 64 columns are one and three quarter rounds of 256 workgroups:
-    // 28672 x 4096 from memory 46.5 -> 41.5-42.3 us), and a narrow weight is spread over the whole chip (6144 x 4096 at
-    // 9-16 rows: 96 stripes 15.2-15.9 us, 256 workgroups of one or two blocks 12.3-12.7).
+    // 28672 x 4096 from memory 46.5 -> 41.5-42.3 us), and a narrow weight is spread over the whole chip.
     // GROUPED: every weight has a run of workgroups of its own (p.grp.end counts them, cumulatively; the host hands them
     // out in proportion to the weights' blocks), and a workgroup's share is worked out inside its weight, once, before the
     // chunk loop: with the lookup of a chunk's weight inside the loop the grouped launch ran 20 us where the plain one ran
@@ -467,16 +478,17 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
     }
     for (int cb = blk_first; cb < blk_last;) {
     const int local = cb;
-    const int nb = min(4, blk_last - cb);
+    const int nb = min(NB, blk_last - cb);
     int N = Nw;
     N = min(N, 16 * (local + nb));                             // rows past the chunk are not this chunk's
-    const int n0 = 16 * local + 16 * w;                        // the columns this wave copies and, at the end, writes
-    // copy instruction for row pair i: lane L lands at byte 16 L of the block and fetches piece (L >> 1) ^ (i & 7) of
-    // row 2i + (L & 1)
-    const short* wsrc[8];
+    // copy instruction for row pair i: lane L lands at byte 16 L of the block and fetches piece (L >> 1) ^ (i & 7) of row
+    // 2i + (L & 1); the wave's pairs are w, w + 4, .., eight in a row in K slices, whose chunks are full (40 rows of 6144 x 4096
+    // 14.1 against 14.3 us)
+    auto pair = [&](int j) { return SLICED ? 8 * w + j : w + 4 * j; };
+    const short* wsrc[2 * NB];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-        wsrc[i] = Bg + (int64_t)min(n0 + 2 * i + (lane & 1), N - 1) * ldb + 8 * ((lane >> 1) ^ i);
+    for (int j = 0; j < 2 * NB; ++j)
+        wsrc[j] = Bg + (int64_t)min(16 * local + 2 * pair(j) + (lane & 1), N - 1) * ldb + 8 * ((lane >> 1) ^ (pair(j) & 7));
     const short* xsrc[2 * MB];                                 // this wave's share of the activation rows: row pairs w, w + 4, ...
 #pragma unroll
     for (int j = 0; j < 2 * MB; ++j)
@@ -489,7 +501,7 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
         char* st = w_lds[t % WST];
         const int k0 = seg_k0(t);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) copy16_global_to_lds(wsrc[i] + k0, st + (w * 8 + i) * kStripeBlock);
+        for (int j = 0; j < 2 * NB; ++j) copy16_global_to_lds(wsrc[j] + k0, st + pair(j) * kStripeBlock);
     };
     auto issue_x = [&](int t) {
         char* st = x_lds[t % XST];
@@ -505,9 +517,9 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
     int frag[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) frag[s] = row_off + 32 * ((4 * (2 * w + s) + quad) ^ (l16 >> 1));
-    f32x4 acc[4][MB];
+    f32x4 acc[NB][MB];
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < NB; ++c)
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) acc[c][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -519,28 +531,27 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
         __syncthreads();                                       // every wave has read segment t - 1: its stages may be refilled
         if (t + XST - 1 < nseg) issue_x(t + XST - 1);
         if (t + WST - 1 < nseg) issue_w(t + WST - 1);
-        // segment t has landed once at most the copies issued after it are outstanding: the weight of the next two
-        // segments and the activations of the next XST - 1
+        // segment t has landed once at most the copies issued after it are outstanding
         const int after = nseg - 1 - t;
-        if (after >= 2) wait_vmcnt<(WST - 1) * G::CW + (XST - 1) * G::CX>(); else if (after == 1) wait_vmcnt<G::CW + G::CX>(); else wait_vmcnt<0>();
+        if (WST >= 5 && after >= 4) wait_vmcnt<G::behind(4)>(); else if (after >= 3) wait_vmcnt<G::behind(3)>(); else if (after == 2) wait_vmcnt<G::behind(2)>(); else if (after == 1) wait_vmcnt<G::behind(1)>(); else wait_vmcnt<0>();
         __syncthreads();                                       // ... for every wave's copies
         const char* wb = w_lds[t % WST];
         const char* xb = x_lds[t % XST];
         // all fragments of the wave's two k steps first, then the MFMAs: left to itself the compiler pipelines these reads
         // in one instantiation and waits for each before its MFMA in another (the grouped one ran twice as long for it)
-        s16x8 a[2][4], b[2][MB];
+        s16x8 a[2][NB], b[2][MB];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) b[s][mb] = *reinterpret_cast<const s16x8*>(xb + mb * 8 * kStripeBlock + frag[s]);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) a[s][c] = *reinterpret_cast<const s16x8*>(wb + c * 8 * kStripeBlock + frag[s]);
+            for (int c = 0; c < NB; ++c) a[s][c] = *reinterpret_cast<const s16x8*>(wb + c * 8 * kStripeBlock + frag[s]);
         }
         __builtin_amdgcn_sched_barrier(0);                     // (the scheduler moves nothing across this)
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
+            for (int c = 0; c < NB; ++c)
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb) acc[c][mb] = T::mfma16(a[s][c], b[s][mb], acc[c][mb]);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // fragments in registers before the barrier that frees the stage
@@ -550,18 +561,18 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
     __syncthreads();
     f32x4* red = reinterpret_cast<f32x4*>(&w_lds[0][0]);   // 16 MB KiB of the 96
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < NB; ++c)
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) red[((w * 4 + c) * MB + mb) * 64 + lane] = acc[c][mb];
+        for (int mb = 0; mb < MB; ++mb) red[((w * NB + c) * MB + mb) * 64 + lane] = acc[c][mb];
     __syncthreads();
-    const int n = n0 + 4 * quad;                               // register r of a lane: weight row n + r, activation row 16mb + l16
+    const int n = 16 * local + 16 * w + 4 * quad;                              // register r of a lane: weight row n + r, activation row 16mb + l16
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
         const int m = 16 * mb + l16;
         if (m >= p.M || n >= N) continue;
-        f32x4 sum = red[((0 * 4 + w) * MB + mb) * 64 + lane];
+        f32x4 sum = red[(w * MB + mb) * 64 + lane];
 #pragma unroll
-        for (int u = 1; u < 4; ++u) sum += red[((u * 4 + w) * MB + mb) * 64 + lane];
+        for (int u = 1; u < 4; ++u) sum += red[((u * NB + w) * MB + mb) * 64 + lane];
         if (SLICED) {
             store_slice4(p, slice, m, n, sum);
             continue;
@@ -588,25 +599,54 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
     }
 }
 // Which widths it takes (in stripes of 64 columns; weights coming from memory): from 96 on every row count that reaches
-// it (14336 x 4096 at 2-32 rows 22.8-23.7 us, the 16-column kernel 24.3-32.4; 6144 x 4096 at 9-32 rows 12.3-15.5 against
-// 14.4-21.5); 80 from 8 rows on and 64 from 32 rows on, where no workspace allows K slices (5120 x 5120 at 16 rows 15.8
-// against 20.5; 4096 x 4096 at 32 rows 13.6 against 16.3); an output head from 5 rows on (128256 x 4096 at 8 rows 179 against
-// 183, 57344 x 8192 166 against 185; up to 4 rows the kernels that keep more workgroups on a compute unit are ahead).
+// it (14336 x 4096 at 2-32 rows 22.8-23.7 us, the 16-column kernel 24.3-32.4); an output head from 5 rows on (128256 x 4096 at 8
+// rows 179 against 183, 57344 x 8192 166 against 185; up to 4 rows the kernels that keep more workgroups on a compute unit are
+// ahead); narrower ones down to 32 stripes from 5 rows on, up to 8 when their rows are long enough to matter, against the 16-column
+// and few-row kernels (us: 2048 x 4096 at 16 / 17 / 64 rows 9.1 / 7.2, 13.9 / 8.0, 21.3 / 12.2; 5120 x 5120 at 5 / 16 rows 14.1 / 10.9,
+// 13.4 / 11.0; 3072 x 8192 at 8 / 32 rows 14.9 / 10.8, 29.6 / 14.2; 4096 x 14336 at 8 / 64 rows 24.0 / 21.5, 54.9 / 44.9).
 static bool stripe_takes(int64_t M, int64_t stripes, int64_t K) {
     if (M < 1 || M > 64 || K % kStripeSeg != 0) return false;
     if (stripes > 640) return M >= 5;
-    return stripes >= 96 || (stripes >= 80 && M >= 8) || (stripes >= 64 && M >= 32);
+    return stripes >= 96 || (stripes >= 80 && M >= 8) || (stripes >= 32 && M >= 5 && (M > 8 || K >= 2560));
+}
+// Where it is also ahead of its K slices, whose workgroups copy less each but leave partial sums that a second launch adds up: by the rows
+// a unit copies, (NB + MB) x 16 of K values, the narrower the weight the fewer (us, slices / whole rows: 6144 x 4096 at 64 rows 15.9 /
+// 15.1, 5632 x 4096 15.5 / 15.1, 4608 x 4096 13.8 / 14.9 and at 33 rows 12.7 / 11.7; 4096 x 6144 at 33 / 64 rows 13.9 / 13.4, 15.2 /
+// 16.5; 3584 x 8192 at 32 / 48 rows 14.5 / 14.3, 16.1 / 18.2; 2560 x 5120 at 32 / 33 rows 10.7 / 10.1, 11.4 / 11.7; 2048 x 4096 at 32 /
+// 64 rows 9.3 / 8.4, 11.2 / 12.2; 2048 x 8192 at 5 rows 9.5 / 10.4; 4096 x 14336 at 16 / 24 rows 24.0 / 24.1, 24.8 / 27.8).
+static bool stripe_blocks_pay(int64_t M, int64_t stripes, int64_t K) {
+    const int64_t most = stripes < 48 ? 16000 : stripes <= 64 || stripes >= 80 ? 25000 : 22000;
+    return stripe_takes(M, stripes, K) && (stripes >= 96 || ((stripes > 64 ? 2 : 1) + (M + 15) / 16) * K <= most);
+}
+// The smallest NB that goes through the `most` blocks of a workgroup in as few chunks as four would (five blocks as three and two: 18944 x 3584
+// at 32 rows 33.4 -> 30.5 us).
+template <class T, int MB, bool SLICED, bool GROUPED>
+static void launch_stripe_rows(const GemmParams& p, int most, dim3 grid, hipStream_t stream) {
+    const dim3 block(4 * 64);
+    if constexpr (!SLICED) {
+        if (most == 1) { hipLaunchKernelGGL((gemm_stripe_kernel<T, MB, false, GROUPED, 1>), grid, block, 0, stream, p); return; }
+        if (most == 2) { hipLaunchKernelGGL((gemm_stripe_kernel<T, MB, false, GROUPED, 2>), grid, block, 0, stream, p); return; }
+        if ((most + 2) / 3 == (most + 3) / 4) { hipLaunchKernelGGL((gemm_stripe_kernel<T, MB, false, GROUPED, 3>), grid, block, 0, stream, p); return; }
+    }
+    hipLaunchKernelGGL((gemm_stripe_kernel<T, MB, SLICED, GROUPED>), grid, block, 0, stream, p);
 }
 // `blocks`: 16-column blocks in all (GROUPED: workgroups in all, p.grp.end counting them per weight).
 template <class T, bool SLICED = false, bool GROUPED = false>
 static int launch_stripe(const GemmParams& p0, int blocks, hipStream_t stream) {
     GemmParams p = p0;
     p.tiles_n = blocks;
-    const dim3 grid(SLICED ? (blocks + 3) / 4 * p.splits : GROUPED ? blocks : std::min(blocks, 256)), block(4 * 64);   // (GROUPED: `blocks` is the number of workgroups)
-    if (p.M <= 16) hipLaunchKernelGGL((gemm_stripe_kernel<T, 1, SLICED, GROUPED>), grid, block, 0, stream, p);
-    else if (p.M <= 32) hipLaunchKernelGGL((gemm_stripe_kernel<T, 2, SLICED, GROUPED>), grid, block, 0, stream, p);
-    else if (p.M <= 48) hipLaunchKernelGGL((gemm_stripe_kernel<T, 3, SLICED, GROUPED>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((gemm_stripe_kernel<T, 4, SLICED, GROUPED>), grid, block, 0, stream, p);
+    const dim3 grid(SLICED ? (blocks + 3) / 4 * p.splits : GROUPED ? blocks : std::min(blocks, 256));   // (GROUPED: `blocks` is the number of workgroups)
+    int most = 0;   // the 16-column blocks of a workgroup
+    if (GROUPED) {
+        for (int s = 0, at = 0; s < kMaxGroup; at = p.grp.end[s++])
+            if (p.grp.end[s] > at) most = std::max(most, ((p.grp.N[s] + 15) / 16 + p.grp.end[s] - at - 1) / (p.grp.end[s] - at));
+    } else {
+        most = (blocks + (int)grid.x - 1) / (int)grid.x;
+    }
+    if (p.M <= 16) launch_stripe_rows<T, 1, SLICED, GROUPED>(p, most, grid, stream);
+    else if (p.M <= 32) launch_stripe_rows<T, 2, SLICED, GROUPED>(p, most, grid, stream);
+    else if (p.M <= 48) launch_stripe_rows<T, 3, SLICED, GROUPED>(p, most, grid, stream);
+    else launch_stripe_rows<T, 4, SLICED, GROUPED>(p, most, grid, stream);
     return check_launch("gemm_stripe_kernel");
 }
 // A weight of fewer than 192 stripes: with a workspace, K slices bring the workgroups up to the chip's 256 compute units
@@ -1372,9 +1412,9 @@ static int launch_grouped(GemmParams& p, int n_w, hipStream_t stream) {
         for (int s = 0; s < kMaxGroup; ++s) { if (s < n_w) acc += p.grp.N[s]; p.grp.end[s] = acc; }
         return launch_gemv<T, true>(p, (int)n_sum, stream);
     }
-    // a batch of decode steps: the stripe kernel over the three weights from 5 rows on (4096 + 1024 + 1024 columns of 4096
-    // values, weights coming from memory: 8 rows 12.3 us against 14.2 for the 16-column kernel, 16 rows 12.7 against 17.4,
-    // 32 rows 15.6 against 21.5; up to 4 rows both take 12.1-12.6)
+    // a batch of decode steps: the stripe kernel over the three weights from 5 rows on (us, the 16-column and few-row kernels / it: 4096 +
+    // 1024 + 1024 columns of 4096 values at 5 / 16 rows 12.6 / 10.3, 17.4 / 10.5, up to 4 rows level; 2560 + 640 + 640 of 2560 at 16 / 24 / 64
+    // rows 6.7 / 6.4, 11.1 / 6.8, 15.4 / 9.3)
     {
         int64_t stripes = 0;
         for (int s = 0; s < n_w; ++s) stripes += (p.grp.N[s] + 63) / 64;
@@ -1490,10 +1530,10 @@ static int gemm_impl(int dtype, int b_layout, const void* A, const void* B, cons
     // 8192 at 2-3 rows 33.2-34.6 against 36.3; 8192 x 8192 30.5-33.9 against 29.2-29.6, and rows of 4096 values gain nothing)
     if (fast && nt && M >= 2 && gemv_takes(M, K) && K >= 8192 && N >= 10240 && (M <= 3 || N >= 16384))
         return dtype == MINFER_ATTN_F16 ? launch_gemv<F16>(p, p.N, stream) : launch_gemv<BF16>(p, p.N, stream);
-    // up to 8 rows against fewer than 96 stripes, and up to 4 against an output head: the 16-column kernel (4096 x 14336 at
-    // 2-8 rows: 23.5-24.4 us against 32.5 for the stripes' blocks shared out; 128256 x 4096 at 2-4 rows 166-170 against
-    // 176-178; 28672 x 4096 at 2-8 rows 42.2-44.5 against 41.5-41.7 and 14336 x 4096 24.3-25.8 against 22.8-23.0: those go on)
-    const bool rows_first = rows_takes && ((M <= 8 && stripes < 96) || (M <= 4 && stripes > 640));
+    // up to 4 rows (8 where stripe_takes says no) against fewer than 96 stripes, and up to 4 against an output head: the 16-column
+    // kernel (128256 x 4096 at 2-4 rows 166-170 against 176-178; 28672 x 4096 at 2-8 rows 42.2-44.5 against 41.5-41.7 and 14336 x
+    // 4096 24.3-25.8 against 22.8-23.0: those go on)
+    const bool rows_first = rows_takes && ((M <= 8 && stripes < 96 && !stripe_takes(M, stripes, K)) || (M <= 4 && stripes > 640));
     const int slices = fast && nt && workspace && aligned16(workspace) ? stripe_slices(M, N, K) : 1;
     const bool sliceable = slices > 1 && workspace_bytes >= (size_t)slices * (size_t)M * (size_t)N * sizeof(float);
     // ... except long rows of a narrow weight when a workspace allows K slices: one wave per 16 columns walks a whole row
@@ -1502,17 +1542,11 @@ static int gemm_impl(int dtype, int b_layout, const void* A, const void* B, cons
     const bool long_rows_few_stripes = K >= 8192 && ((M >= 5 && stripes <= 32) || (M >= 2 && stripes <= 24));
     if (fast && nt && rows_first && !(sliceable && long_rows_few_stripes))
         return dtype == MINFER_ATTN_F16 ? launch_rows_lds<F16>(p, (int)((N + 15) / 16), stream) : launch_rows_lds<BF16>(p, (int)((N + 15) / 16), stream);
-    // with a workspace, K slices of the stripes: fewer than 96 stripes from 9 rows on (4096 x 14336 at 16 rows 24.5 us against
-    // 29.1 for the 16-column kernel and 33 for the blocks shared out; 5120 x 5120 14.6 / 20.5 / 15.8), 96-191 stripes from 33
-    // rows on (6144 x 4096 at 64 rows 18.6 against 20.2, 8192 x 8192 33.9 against 37.8; up to 32 rows the blocks shared out
-    // are ahead: 6144 x 4096 at 16 rows 12.7 against 14.3).  Two launches, 10.5 us at least, where one launch over rows of
-    // 4096 values takes 8-10 at 9-16 rows: up to 16 rows only for 25 M weight values or rows of 6144 values and more (2048 x
-    // 8192 at 9-16 rows 12.7-13.0 against 13.9-16.5, 1024 x 14336 13.7-14.6 against 21.5-26.7; 4096 x 4096 12.0 against
-    // 9.3-10.2), from 17 rows on for 8 M values where the other choice is gemm_skinny_kernel (2048 x 4096 at 24-64 rows
-    // 10.9-13.0 against 13.9-16.7, 4096 x 2048 at 24 rows 10.8 against 12.3) and 16 M where it is the blocks shared out
-    // (4096 x 2048 at 32 / 64 rows: 10.8 / 12.6 against 8.9 / 11.5).
-    const bool slices_pay = stripes >= 96 ? M > 32 && N * K >= (INT64_C(1) << 24)
-        : long_rows_few_stripes || (M >= 9 && (N * K >= INT64_C(25000000) || K >= 6144 || (M >= 17 && N * K >= (INT64_C(1) << (stripe_takes(M, stripes, K) ? 24 : 23)))));
+    // with a workspace, K slices of the stripes, from 9 rows on, where whole rows are not ahead (stripe_blocks_pay): two launches, 10.5
+    // us at least, where one launch over rows of 4096 values takes 8-10 at 9-16 rows: up to 16 rows only for 25 M weight values or
+    // rows of 6144 values and more (2048 x 8192 at 9-16 rows 12.7-13.0 against 13.9-16.5, 1024 x 14336 13.7-14.6 against 21.5-26.7),
+    // from 17 rows on for 8 M values (1536 x 5632 and the like: gemm_skinny_kernel is the other choice)
+    const bool slices_pay = !stripe_blocks_pay(M, stripes, K) && (long_rows_few_stripes || (M >= 9 && (N * K >= INT64_C(25000000) || K >= 6144 || (M >= 17 && N * K >= (INT64_C(1) << 23)))));
     if (sliceable && slices_pay) {
         p.splits = slices; p.part = (float*)workspace;
         return dtype == MINFER_ATTN_F16 ? launch_stripe_slices<F16>(p, stream) : launch_stripe_slices<BF16>(p, stream);

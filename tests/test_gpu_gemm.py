@@ -70,12 +70,12 @@ def make(M, N, K, layout, dtype, seed):
     (16, 4104, 1024, 1.0, 1.0),
     (3, 8, 512, 1.0, 0.0),           # a single half-empty group
     (9, 2048, 14336, 0.5, 0.0),      # 28 segments per wave
-    # 1-64 rows against a weight of 12288 columns or more, K a multiple of 256: 64-column stripes over the whole of K
+    # 1-64 rows, K a multiple of 256: 16-column blocks over the whole of K
     (2, 12288, 256, 1.0, 0.0),       # one segment
     (1, 12296, 1024, 2.0, 3.0),      # one row
     (1, 6144, 4096, 1.0, 0.0),       # 96 stripes: the narrowest weight it takes at any row count
-    (8, 5120, 768, 2.0, 3.0),        # 80 stripes from 8 rows on
-    (40, 4104, 1024, 1.0, 1.0),      # 65 stripes from 32 rows on, the last one of 8 columns
+    (8, 5120, 768, 2.0, 3.0),        # 80 stripes
+    (40, 4104, 1024, 1.0, 1.0),      # 65 stripes, the last one of 8 columns
     (9, 12296, 512, 2.0, 3.0),       # a last stripe of 8 columns; two segments (fewer than the three stages)
     (16, 14336, 1024, 1.0, 1.0),
     (17, 12288, 768, 1.0, 0.0),      # two blocks of activation rows, the second with one row
@@ -173,6 +173,29 @@ def test_gemm_every_tile_shape(layout, M, N, K):
     assert capi.gemm(a.to(DEV), b.to(DEV), c.to(DEV), d, alpha, beta, layout) == capi.OK, capi.last_error()
     torch.cuda.synchronize()
     assert_close(d, (alpha * (a.double() @ (b if layout == KN else b.T).double()) + beta * c.double()).numpy(), dtype)
+
+
+@pytest.mark.parametrize("M", [9, 24, 40, 64])
+@pytest.mark.parametrize("N,K", [
+    (2056, 256),      # one 16-column block a workgroup, the last of 8 columns; one segment
+    (4096, 512),
+    (2048, 2560),     # more segments than the five stages
+    (4104, 1280),     # two blocks
+    (8184, 768),
+    (8200, 1024),     # three
+    (18440, 512),     # five: three and two
+    (28680, 1024),    # eight at most: four by four
+])
+def test_gemm_stripe_blocks(M, N, K):
+    """Every number of 16-column blocks that the stripe kernel takes at a time, from fewer segments of K than stages to more, every number
+    of activation row blocks: all elements against torch's product in 64 bits, within the bound of assert_close."""
+    dtype = torch.float16 if (M + K // 256) % 2 else torch.bfloat16
+    a, b, c = make(M, N, K, NK, dtype, M + N + K)
+    alpha, beta = (2.0, 3.0) if M % 16 else (1.0, 0.0)
+    d = torch.full((M, N), float("nan"), dtype=dtype, device=DEV)
+    assert capi.gemm(a.to(DEV), b.to(DEV), c.to(DEV), d, alpha, beta, NK) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    assert_close(d, (alpha * (a.double() @ b.T.double()) + beta * c.double()).numpy(), dtype)
 
 
 def test_gemm_golden_strided_and_in_place():
@@ -313,7 +336,7 @@ def test_qkv_op_and_reference_checks(kerns):
 @pytest.mark.parametrize("layout", [KN, NK])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K,alpha,beta", [
-    (64, 4096, 4096, 1.0, 0.0),      # [K, N]: 32 tiles of 128 columns, 8 slices of 8 steps; [N, K]: four slices of 64 stripes
+    (64, 4096, 4096, 1.0, 0.0),      # [K, N]: 32 tiles of 128 columns, 8 slices of 8 steps; [N, K]: 256 blocks of 16 columns, no slices
     (100, 1032, 2048, 2.0, 3.0),     # ragged rows and columns, C read by the second kernel
     (256, 2048, 1024, 0.5, 1.0),     # two tile rows
     (40, 512, 1984, 1.0, 0.0),       # K steps (31) not a multiple of the slice count
@@ -321,7 +344,7 @@ def test_qkv_op_and_reference_checks(kerns):
     (24, 1024, 2048, 1.0, 1.0),      # 17-32 rows: with a workspace [K, N] slices of 128 columns, [N, K] the sliced tiles
     (256, 8192, 1024, 1.0, 1.0),     # 128 tiles: two slices, so that two workgroups share a compute unit
     # [N, K] weights of fewer than 192 stripes of 64 columns: K slices of the stripe kernel
-    (8, 5120, 5120, 2.0, 3.0),       # 80 stripes, three slices of 6, 7 and 7 segments
+    (8, 5120, 5120, 2.0, 3.0),       # 80 stripes, 320 blocks of 16 columns shared out: the workspace is not needed
     (16, 4104, 8192, 1.0, 1.0),      # a last stripe of 8 columns
     (33, 8192, 2048, 0.5, 0.0),      # three blocks of activation rows, two slices of four segments
     (1, 8192, 4096, 1.0, 0.0),       # one row
