@@ -402,15 +402,14 @@ static int launch_rows_lds(const GemmParams& p, int groups, hipStream_t stream) 
 // Up to 64 rows against an [N, K] weight (a batch of decode steps against a projection, FFN or output-head weight): a workgroup
 // of four waves takes NB blocks of 16 columns at a time over the whole of K; K goes by in segments of 256 values, the 16 NB weight
 // rows and the activation rows copied global -> LDS with instructions whose lanes walk along the rows (512 consecutive bytes
-// of each of two rows, 2 lines per quarter wave); two to five weight stages and two to four
+// of each of two rows, 2 lines per quarter wave); two or three weight stages and two or three
 // activation stages, one workgroup per compute unit (segments of 128 values and two workgroups per unit are 15-25 %
 // slower from 24 rows on).  No K slices across workgroups, so no partial sums in memory: the activations are read once
 // per workgroup and the weight once.  Two rows of a copy share a 1 KiB block of LDS; inside block i
 // the 16-byte pieces of a row sit at piece ^ (i & 7), so the 16 rows of a fragment read hit 16 different bank groups
 // without padding.
 // What bounds it, once the weight does not (5 TB/s), is the copies a unit makes, 50-60 bytes per ns: NB is what the workgroups have,
-// one to four, the four waves share the copies of the rows there are, and the stages that smaller chunks leave room for keep as many
-// bytes in flight.  (With chunks of four whatever the workgroup had, the missing rows copied again, us, before / now: 6144 x 4096 at
+// one to four, and the four waves share the copies of the rows there are.  (With chunks of four whatever the workgroup had, the missing rows copied again, us, before / now: 6144 x 4096 at
 // 16 / 32 / 40 / 64 rows 10.9 / 10.0, 13.7 / 11.0, 14.1 / 12.4, 15.9 / 15.1; 4096 + 1024 + 1024 columns at 24 / 40 rows 13.5 / 11.1, 15.1 /
 // 12.5; 11008 x 4096 at 40 rows 20.4 / 19.5, 22016 x 4096 40.2 / 35.2; where chunks of four are still the choice, 28672 x 4096 at 64
 // rows 48.2 / 46.0, for the even share of the copies.)
@@ -419,15 +418,23 @@ constexpr int kStripeBlock = 1024;                             // LDS bytes of t
 template <int MB, int NB = 4> struct StripeGeom {   // 16-row blocks of activations, 16-column blocks of the weight
     static constexpr int W_BYTES = NB * 8 * kStripeBlock;      // 16 * NB weight rows
     static constexpr int X_BYTES = MB * 8 * kStripeBlock;      // 16 * MB activation rows
-    static constexpr int WST = NB == 1 ? (MB >= 4 ? 4 : 5) : NB == 2 ? (MB >= 4 ? 3 : 4) : (NB == 4 && MB >= 4 ? 2 : 3);
-    static constexpr int XST = NB == 1 ? (MB >= 4 ? 3 : 4) : NB == 2 ? 3 : (MB + NB >= 7 ? 2 : 3);   // 120 / 144 / 144 / 128 KiB, three blocks 96 / 120 / 144 / 136, two 88 / 112 / 136 / 144, one 72 / 104 / 136 / 128
+    // 120 / 144 / 144 / 128 KiB with four blocks, 48 / 72 / 96 / 120 with one; a fourth and fifth stage of the smaller chunks cost 2-7 % (3072 x
+    // 8192 at 16 rows 10.3 -> 11.1 us, 6144 x 4096 at 32 10.6 -> 11.0, Q8_0 14336 x 4096 at 16 16.7 -> 18.2)
+    static constexpr int WST = NB == 4 && MB >= 4 ? 2 : 3, XST = MB + NB >= 7 ? 2 : 3;
     static constexpr int CW = 2 * NB, CX = 2 * MB;             // copies per wave and segment
-    // copies issued after those of segment t, with `after` segments behind it: those of x(t) go out in front of w(t + WST - XST)
-    static constexpr int behind(int after) {
-        const int w = WST > XST ? (after < WST - 1 ? after : WST - 1) - (WST - XST) + 1 : (after < WST - 1 ? after : WST - 1);
-        return (w > 0 ? w : 0) * CW + (after < XST - 1 ? after : XST - 1) * CX;
-    }
 };
+// Copies issued after those of segment t, with `after` segments behind it: those of x(t) go out in front of w(t + WST - XST).
+template <class G> constexpr int copies_behind(int after) {
+    const int w = std::min(after, G::WST - 1) - (G::WST > G::XST ? G::WST - G::XST - 1 : 0);
+    return std::max(w, 0) * G::CW + std::min(after, G::XST - 1) * G::CX;
+}
+// ... which is how many may be outstanding once segment t has landed
+template <class G> MA_DEV void wait_behind(int after) {
+    static_assert(G::WST <= 3 && G::XST <= G::WST, "three cases");
+    if (after >= 2) wait_vmcnt<copies_behind<G>(2)>();
+    else if (after >= 1) wait_vmcnt<copies_behind<G>(1)>();
+    else wait_vmcnt<0>();
+}
 // SLICED: p.splits workgroups per stripe, each over its share of the segments; they leave raw fp32 sums in p.part
 // ([slice][M][N]) for finish_slices.
 // GROUPED: the stripes of up to three weights numbered through (p.grp.end in stripes), alpha = 1 and no C.
@@ -533,7 +540,7 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
         if (t + WST - 1 < nseg) issue_w(t + WST - 1);
         // segment t has landed once at most the copies issued after it are outstanding
         const int after = nseg - 1 - t;
-        if (WST >= 5 && after >= 4) wait_vmcnt<G::behind(4)>(); else if (after >= 3) wait_vmcnt<G::behind(3)>(); else if (after == 2) wait_vmcnt<G::behind(2)>(); else if (after == 1) wait_vmcnt<G::behind(1)>(); else wait_vmcnt<0>();
+        wait_behind<G>(after);
         __syncthreads();                                       // ... for every wave's copies
         const char* wb = w_lds[t % WST];
         const char* xb = x_lds[t % XST];
@@ -1048,16 +1055,21 @@ static int launch_skinny_q8(const GemmParams& p, hipStream_t stream) {
 // and dequantises them exactly as minfer_dequant_q8_0 does (dequant8_shifted; block 2 w starts on a word boundary,
 // block 2 w + 1 two bytes past one), so the result is that of the fp16 kernels on the dequantised weight.
 constexpr int kQ8SegBytes = 272;
-constexpr int kQ8Stage = 22 * 1024;                            // 17 KiB of row segments, 3 KiB the extra copies land in; three stages hold the 64 KiB of partial sums
+template <int MB, int NB> struct Q8StripeGeom {
+    static constexpr int X_BYTES = MB * 8 * kStripeBlock, CW = (17 * NB + 15) / 16, CX = 2 * MB;   // copies per wave and segment
+    static constexpr int WST = 3, XST = MB + NB >= 7 ? 2 : 3;
+    static constexpr int SUM_BYTES = 4 * NB * MB * 1024;   // the partial sums reuse the weight stages
+    static constexpr int W_BYTES = 4 * CW * 1024 * WST >= SUM_BYTES ? 4 * CW * 1024 : (SUM_BYTES / 1024 + WST - 1) / WST * 1024;   // the row segments and what the extra copies land in
+    static_assert(WST * W_BYTES + XST * X_BYTES < 160 * 1024, "with a word to spare for finish_slices");
+};
 // SLICED: p.splits workgroups per chunk of four blocks, each over its share of the segments; raw fp32 sums into p.part
 // ([slice][M][N]) for finish_slices (a narrow weight with a workspace, as gemm_stripe_kernel has it).
-template <int MB, bool SLICED = false>
+template <int MB, bool SLICED = false, int NB = 4>
 __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams p) {
     using T = F16;
-    using G = StripeGeom<MB>;
-    constexpr int WST = 3, XST = MB >= 3 ? 2 : 3, CW = 5, CX = 2 * MB;   // 90 / 114 / 114 / 130 KiB
-    static_assert(WST * kQ8Stage >= 4 * 4 * MB * 64 * 16, "the partial sums reuse the weight stages");
-    __shared__ __attribute__((aligned(16))) char w_lds[WST][kQ8Stage];
+    using G = Q8StripeGeom<MB, NB>;
+    constexpr int WST = G::WST, XST = G::XST, CW = G::CW, CX = G::CX;
+    __shared__ __attribute__((aligned(16))) char w_lds[WST][G::W_BYTES];
     __shared__ __attribute__((aligned(16))) char x_lds[XST][G::X_BYTES];
     const int lane = threadIdx.x & 63, w = wave_id();
     const int l16 = lane & 15, quad = lane >> 4;
@@ -1077,12 +1089,12 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams
     for (int s = 0; s < 2; ++s) frag[s] = row_off + 32 * ((4 * (2 * w + s) + quad) ^ (l16 >> 1));
     const int wfrag = kQ8SegBytes * l16 + 68 * w + 8 * quad;
     for (int cb = blk_first; cb < blk_last;) {
-    const int nb = min(4, blk_last - cb);
+    const int nb = min(NB, blk_last - cb);
     const int N = min(p.N, 16 * (cb + nb));                    // rows past the chunk are not this chunk's
     const char* wsrc[CW];
 #pragma unroll
     for (int i = 0; i < CW; ++i) {
-        const int pc = min(64 * (w + 4 * i) + lane, 64 * 17 - 1), row = pc / 17;
+        const int pc = min(64 * (w + 4 * i) + lane, 16 * NB * 17 - 1), row = pc / 17;
         wsrc[i] = (const char*)p.B + (int64_t)min(16 * cb + row, N - 1) * p.ldb + 16 * (pc - 17 * row);
     }
     const short* xsrc[CX];
@@ -1103,9 +1115,9 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams
 #pragma unroll
         for (int j = 0; j < CX; ++j) copy16_global_to_lds(xsrc[j] + k0, st + (w + 4 * j) * kStripeBlock);
     };
-    f32x4 acc[4][MB];
+    f32x4 acc[NB][MB];
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < NB; ++c)
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) acc[c][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -1118,18 +1130,18 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams
         if (t + XST - 1 < nseg) issue_x(t + XST - 1);
         if (t + WST - 1 < nseg) issue_w(t + WST - 1);
         const int after = nseg - 1 - t;
-        if (after >= 2) wait_vmcnt<(WST - 1) * CW + (XST - 1) * CX>(); else if (after == 1) wait_vmcnt<CW + CX>(); else wait_vmcnt<0>();
+        wait_behind<G>(after);
         __syncthreads();                                       // ... for every wave's copies
         const char* wb = w_lds[t % WST] + wfrag;
         const char* xb = x_lds[t % XST];
-        uint32_t wq[2][4][3], dbits[2][4];
+        uint32_t wq[2][NB][3], dbits[2][NB];
         s16x8 b[2][MB];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) b[s][mb] = *reinterpret_cast<const s16x8*>(xb + mb * 8 * kStripeBlock + frag[s]);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
+            for (int c = 0; c < NB; ++c) {
                 const uint32_t* wp = reinterpret_cast<const uint32_t*>(wb + 16 * kQ8SegBytes * c + 32 * s);
                 wq[s][c][0] = wp[0]; wq[s][c][1] = wp[1]; wq[s][c][2] = wp[2];
                 dbits[s][c] = *reinterpret_cast<const uint16_t*>(wb + 16 * kQ8SegBytes * c + 34 * s - 8 * quad);
@@ -1139,7 +1151,7 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
+            for (int c = 0; c < NB; ++c) {
                 const _Float16 dh = __builtin_bit_cast(_Float16, (uint16_t)dbits[s][c]);
                 const s16x8 a = dequant8_shifted(wq[s][c][0], wq[s][c][1], wq[s][c][2], s == 0 ? kQ8SelEven : kQ8SelOdd, h16x2{dh, dh});
 #pragma unroll
@@ -1148,20 +1160,20 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // fragments in registers before the barrier that frees the stage
     }
     __syncthreads();
-    f32x4* red = reinterpret_cast<f32x4*>(&w_lds[0][0]);   // 16 MB KiB of the 66
+    f32x4* red = reinterpret_cast<f32x4*>(&w_lds[0][0]);
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < NB; ++c)
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) red[((w * 4 + c) * MB + mb) * 64 + lane] = acc[c][mb];
+        for (int mb = 0; mb < MB; ++mb) red[((w * NB + c) * MB + mb) * 64 + lane] = acc[c][mb];
     __syncthreads();
     const int n = 16 * cb + 16 * w + 4 * quad;               // register r of a lane: weight row n + r, activation row 16mb + l16
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
         const int m = 16 * mb + l16;
         if (m >= p.M || n >= N) continue;
-        f32x4 sum = red[((0 * 4 + w) * MB + mb) * 64 + lane];
+        f32x4 sum = red[(w * MB + mb) * 64 + lane];
 #pragma unroll
-        for (int u = 1; u < 4; ++u) sum += red[((u * 4 + w) * MB + mb) * 64 + lane];
+        for (int u = 1; u < 4; ++u) sum += red[((u * NB + w) * MB + mb) * 64 + lane];
         if (SLICED) {
             store_slice4(p, slice, m, n, sum);
             continue;
@@ -1190,15 +1202,27 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams
 // Which calls it takes: 2-64 rows, whole segments of 8 blocks, rows that start on 16-byte boundaries, and a weight wide
 // enough for two and a half blocks per workgroup, or two from 16 rows, or one and a half above 32 (weights coming from memory:
 // 14336 x 4096 at 2-16 rows 16.7-16.9 us against 20.8-26.8 for gemm_skinny_q8_kernel, 64 rows 23.4 against 50.9; 28672 x
-// 4096 29.7-43.4 against 36.8-97.7; 8192 x 8192 at 2 rows 27.0 against 23.5, at 16 rows 27.4 against 28.4; 6144 x 4096 at
-// 16 rows 15.7 against 15.2, at 64 rows 22.9 against 25.9).  A chunk of fewer than four blocks dequantises and multiplies
-// all four all the same: skipping the missing ones by a branch cost the full chunks a third (16.7 -> 22.8 us).
+// 4096 29.7-43.4 against 36.8-97.7), or q8_blocks_pay.  Chunks of as many blocks as a workgroup has, as for the 16-bit weights (11008 x 4096
+// at 2 / 24 / 64 rows 15.4 -> 13.3, 18.4 -> 15.6, 23.3 -> 20.6; 18944 x 3584 at 2 / 40 rows 25.6 -> 21.6, 34.1 -> 31.3): all of a
+// chunk's blocks are dequantised and multiplied, there or not (skipping the missing ones of four by a branch cost the full chunks a
+// third).
+// Where it is ahead of its K slices and of gemm_skinny_q8_kernel on a weight of fewer than 192 stripes: rows of up to 4096 values, by the rows a
+// unit copies, (NB + MB) x 16 of K values (us, the other / it: 8192 x 4096 at 2 / 16 / 32 rows 11.8 / 11.0, 12.7 / 11.1, 14.9 / 12.8;
+// 6144 x 4096 at 16 / 24 / 40 rows 12.3 / 11.0, 14.1 / 12.1, 15.2 / 15.4; 6144 x 2048 at 16 rows 9.1 / 6.7; 5120 x 4096 at 24 / 40 12.6 /
+// 12.0, 14.0 / 15.1; 4096 x 4096 at 16 / 64 9.7 / 8.2, 13.9 / 13.2; 4096 x 2048 at 8 / 16 / 64 5.4 / 5.9, 8.7 / 5.5, 11.7 / 8.6; 2048 x 4096
+// at 16 / 24 / 40 8.8 / 8.0, 9.9 / 9.6, 10.7 / 11.2; 5120 x 5120 at 16 rows 12.1 / 12.7).
 // K slices of it for a weight of fewer than 192 stripes when a workspace is given (1 = none): 256 / stripes workgroups
 // per chunk of four blocks, full chunks whatever the width (weights coming from memory: 4096 x 14336 at 16 / 32 / 64 rows
 // 19.0 / 21.8 / 26.4 us against 29.6 / 43.0 / 68.4 for gemm_skinny_q8_kernel, 8192 x 8192 at 2-64 rows 19.6-28.5 against
 // 23.7-40.3, 6144 x 4096 12.4-17.7 against 12.7-22.2; 4096 x 4096 up to 8 rows 10.2 against 7.7-8.3: two launches, so a
 // weight of 16 M values or fewer only from 16 rows on, or from 8 when its rows are 6144 values and longer, or from 2
 // when they are 8192 values and longer and the stripes 24 at most, as for the 16-bit weights).
+static bool q8_blocks_pay(int64_t M, int64_t N, int64_t K) {
+    const int64_t stripes = (N + 63) / 64, rows = (stripes > 64 ? 2 : 1) + (M + 15) / 16;
+    if (K > 4096 || M < 2 || M > 64 || stripes < 32 || stripes >= 192) return false;
+    if (stripes >= 96) return rows * K <= 17000 && (M >= 8 || N * K >= INT64_C(20000000));
+    return M >= 16 && rows * K <= (stripes < 64 ? 12500 : stripes == 64 ? 20500 : 17000);
+}
 static int q8_slices(int64_t M, int64_t N, int64_t K) {
     if (M < 2 || M > 64 || K % kStripeSeg != 0 || N % 8 != 0) return 1;
     const bool long_rows = (K >= 6144 && M >= 8) || (K >= 8192 && N <= 24 * 64);
@@ -1207,17 +1231,28 @@ static int q8_slices(int64_t M, int64_t N, int64_t K) {
 }
 static bool q8_stripe_ok(int64_t M, int64_t N, int64_t K, const void* Bq, int64_t row_bytes) {
     return M >= 2 && M <= 64 && K % kStripeSeg == 0 && aligned16(Bq) && row_bytes % 16 == 0 &&
-           (N >= 10240 || (N >= 8192 && M >= 16) || (N >= 6144 && M > 32));
+           (N >= 10240 || (N >= 8192 && M >= 16) || (N >= 6144 && M > 32) || q8_blocks_pay(M, N, K));
+}
+template <int MB, bool SLICED>
+static void launch_stripe_q8_rows(const GemmParams& p, int most, dim3 grid, hipStream_t stream) {   // (NB as in launch_stripe_rows)
+    const dim3 block(4 * 64);
+    if constexpr (!SLICED) {
+        if (most == 1) { hipLaunchKernelGGL((gemm_stripe_q8_kernel<MB, false, 1>), grid, block, 0, stream, p); return; }
+        if (most == 2) { hipLaunchKernelGGL((gemm_stripe_q8_kernel<MB, false, 2>), grid, block, 0, stream, p); return; }
+        if ((most + 2) / 3 == (most + 3) / 4) { hipLaunchKernelGGL((gemm_stripe_q8_kernel<MB, false, 3>), grid, block, 0, stream, p); return; }
+    }
+    hipLaunchKernelGGL((gemm_stripe_q8_kernel<MB, SLICED>), grid, block, 0, stream, p);
 }
 template <bool SLICED = false>
 static int launch_stripe_q8(const GemmParams& p0, hipStream_t stream) {
     GemmParams p = p0;
     p.tiles_n = (p.N + 15) / 16;
-    const dim3 grid(SLICED ? (p.tiles_n + 3) / 4 * p.splits : std::min(p.tiles_n, 256)), block(4 * 64);
-    if (p.M <= 16) hipLaunchKernelGGL((gemm_stripe_q8_kernel<1, SLICED>), grid, block, 0, stream, p);
-    else if (p.M <= 32) hipLaunchKernelGGL((gemm_stripe_q8_kernel<2, SLICED>), grid, block, 0, stream, p);
-    else if (p.M <= 48) hipLaunchKernelGGL((gemm_stripe_q8_kernel<3, SLICED>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((gemm_stripe_q8_kernel<4, SLICED>), grid, block, 0, stream, p);
+    const dim3 grid(SLICED ? (p.tiles_n + 3) / 4 * p.splits : std::min(p.tiles_n, 256));
+    const int most = (p.tiles_n + (int)grid.x - 1) / (int)grid.x;
+    if (p.M <= 16) launch_stripe_q8_rows<1, SLICED>(p, most, grid, stream);
+    else if (p.M <= 32) launch_stripe_q8_rows<2, SLICED>(p, most, grid, stream);
+    else if (p.M <= 48) launch_stripe_q8_rows<3, SLICED>(p, most, grid, stream);
+    else launch_stripe_q8_rows<4, SLICED>(p, most, grid, stream);
     return check_launch("gemm_stripe_q8_kernel");
 }
 
@@ -1655,7 +1690,7 @@ MINFER_ATTN_EXPORT int minfer_gemm_q8_0(const void* A, const void* Bq, const voi
         p.A = A; p.B = Bq; p.C = beta != 0.0 ? C : nullptr; p.D = D; p.M = (int)M; p.N = (int)N; p.K = (int)K;
         p.lda = lda; p.ldb = row_bytes; p.ldc = ldc; p.ldd = ldd; p.alpha = (float)alpha; p.beta = (float)beta;
         if (q8_gemv_ok(M, K, Bq, row_bytes)) return launch_gemv_q8(p, stream);
-        const int slices = aligned16(Bq) && row_bytes % 16 == 0 ? q8_slices(M, N, K) : 1;
+        const int slices = aligned16(Bq) && row_bytes % 16 == 0 && !q8_blocks_pay(M, N, K) ? q8_slices(M, N, K) : 1;
         if (slices > 1 && workspace && aligned16(workspace) && workspace_bytes >= (size_t)slices * (size_t)M * (size_t)N * sizeof(float)) {
             p.splits = slices; p.part = (float*)workspace;
             return launch_stripe_q8_slices(p, stream);

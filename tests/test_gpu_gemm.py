@@ -198,6 +198,30 @@ def test_gemm_stripe_blocks(M, N, K):
     assert_close(d, (alpha * (a.double() @ b.T.double()) + beta * c.double()).numpy(), dtype)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (16, 2056, 256),      # one block a workgroup, the last of 8 columns; one segment
+    (33, 4096, 2048),
+    (64, 2048, 2560),
+    (17, 4104, 1280),     # two
+    (9, 8184, 768),
+    (32, 6144, 4096),
+    (2, 10248, 512),      # three
+    (40, 18440, 768),     # five: three and two
+    (64, 12280, 1024),
+])
+def test_gemm_q8_0_stripe_blocks(M, N, K):
+    """The same over Q8_0 blocks, with and without a workspace, of each number of column blocks at a time: every element against torch's product
+    with the dequantised weight in 64 bits, within the bound of assert_close."""
+    a, wq, c, w = make_q8(M, N, K, seed=M + N + K)
+    want = (2.0 * (a.double() @ w.double().T) + c.double()).numpy()
+    ws = torch.empty(capi.lib().minfer_gemm_q8_0_workspace_bytes(M, N, K), dtype=torch.uint8, device=DEV)
+    for space in (None, ws if ws.numel() else None):
+        d = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
+        assert capi.gemm_q8_0(a.to(DEV), wq.to(DEV), c.to(DEV), d, 2.0, 1.0, space) == capi.OK, capi.last_error()
+        torch.cuda.synchronize()
+        assert_close(d, want, torch.float16)
+
+
 def test_gemm_golden_strided_and_in_place():
     z = np.load(os.path.join(os.path.dirname(__file__), "golden", "gemm_small.npz"))
     a, b, c = (torch.from_numpy(z[k]).to(DEV) for k in "abc")
