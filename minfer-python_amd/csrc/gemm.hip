@@ -1355,7 +1355,9 @@ static int compute_units() {
 // partly filled one at 0.76 + 0.24 of its share (its units run faster), a round its K steps at 20 ns per pair of 16-row blocks (two
 // workgroups on a unit 1.84 of one; with two stages a step that is shorter than the largest tile's does not cover its copies) and
 // 3.8 us of first and last copies and results; the copies of all tiles at 31 TB/s and the weight at 7 TB/s, which are hidden behind
-// that in part: the three add up as their squares; 3.6 us around it, 0.9 more for the launch that adds the slices up, and 0.29 us
+// that in part: the three add up as their squares; past one round, where the clock has come down to what the power budget leaves, the
+// more the more a tile copies per flop (3072 x 8192 x 4096: 128 x 256 tiles 177.7 us, 192 x 256 167.1, without this estimated 171.7 and
+// 172.9; 4096 x 5120 x 4096 150.9 and 137.0); 3.6 us around it, 0.9 more for the launch that adds the slices up, and 0.29 us
 // per MB of sums.  Fitted to 4700 timed calls (150 shapes of 65 to 7000 rows, both layouts, up to 40 choices each): the choice it
 // makes is 1.0 % behind the best one on average, fixed rules for 128 x 128 and 128 x 256 slices and a table of rounds 6 %.
 static double plan_cost(const GemmTile& t, int64_t tiles, int slices, int64_t M, int64_t N, int64_t K, int cus) {
@@ -1363,7 +1365,8 @@ static double plan_cost(const GemmTile& t, int64_t tiles, int slices, int64_t M,
     const double step = (0.0201 * area + 0.0738) * (t.occ == 2 ? 1.84 : 1.0) + (t.ns == 2 && t.occ == 1 ? 0.0147 + 0.0076 * (64 - area) : 0.0);
     const int64_t wgs = tiles * slices, per = (int64_t)cus * t.occ, full = wgs / per, rest = wgs % per;
     const double rounds = (double)full + (rest ? 0.76 + 0.24 * (double)rest / (double)per : 0.0);
-    const double compute = rounds * (step * steps + 3.8), weight = (double)N * (double)K * 2 / 7.0e6;
+    const double power = wgs > per ? 1.0 + ((t.m16 + t.n16) / area - 0.25) : 1.0;
+    const double compute = rounds * (step * steps + 3.8) * power, weight = (double)N * (double)K * 2 / 7.0e6;
     const double copies = (double)tiles * (double)(K / kBK) * (t.m16 + t.n16) * 4096 / 31.3e6;
     const double launch = 3.6 + sqrt(compute * compute + copies * copies + weight * weight);
     return slices > 1 ? launch + 0.9 + 0.286e-6 * slices * (double)M * (double)N * 4 : launch;

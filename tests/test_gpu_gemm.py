@@ -158,6 +158,7 @@ def test_gemm_tiles_between_the_small_and_the_large_one(layout, dtype, M, N, K, 
     (NK, 1773, 4904, 448),        # 224 x 192
     (KN, 1561, 6440, 640),        # 224 x 256
     (NK, 2119, 4824, 64),         # 224 x 256
+    (NK, 1949, 5656, 320),        # 256 x 192
     (NK, 2025, 4888, 128),        # 256 x 224
     (KN, 2027, 5976, 192),        # 256 x 256
     (NK, 1807, 7192, 256),        # 256 x 256
