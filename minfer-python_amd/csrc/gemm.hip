@@ -1319,7 +1319,8 @@ static int launch_stripe_slices(GemmParams& p, hipStream_t stream) {
 }
 
 // [K, N] weights of up to 64 rows: slices of K bring the column tiles up to the chip's 256 compute units, every slice two
-// steps of 64 at least; from 17 rows on four and at most 32 slices, since the sums grow with the rows.
+// steps of 64 at least; from 17 rows on four and at most 32 slices, since the sums grow with the rows.  The workspace is for these; a call that
+// has it takes 8 or 16 of them at most.
 constexpr int64_t kKnRows = 64;
 static int kn_slices(int64_t M, int64_t N, int64_t K) {
     if (M < 1 || M > kKnRows || K % kBK != 0 || K < 8 * kBK || N % 8 != 0) return 1;
@@ -1600,8 +1601,11 @@ static int gemm_impl(int dtype, int b_layout, const void* A, const void* B, cons
     if (fast && nt && (M <= 16 || (!can_split && (M <= 32 || (M <= 64 && N * K <= (INT64_C(1) << 25))))))
         return dtype == MINFER_ATTN_F16 ? launch_skinny<F16>(p, stream) : launch_skinny<BF16>(p, stream);
     if (fast && !nt && M <= kKnRows) {
-        const int kn = kn_slices(M, N, K);   // a smaller workspace: as many slices as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
-        p.splits = fit < (size_t)kn ? std::max((int)fit, 1) : kn;
+        // eight slices at most, 16 for rows of 80 K steps and more: further ones save less streaming than their sums cost (us, as many as fill
+        // the chip / these: 1000 x 4096 at 1 / 9 / 16 rows 10.5 / 7.6, 13.5 / 8.7, 15.5 / 9.4; 2560 x 2560 at 12 10.0 / 8.1; 2048 x 4096 at 40 13.7 /
+        // 11.9; 1024 x 14336 at 9 / 40 15.4 / 12.8, 19.4 / 17.2; 512 x 8192 at 9 17.0 / 9.6; the size reported stays that of filling it)
+        const int kn = kn_slices(M, N, K), most = K >= 80 * kBK ? 16 : 8;   // a smaller workspace: as many slices as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
+        p.splits = fit < (size_t)kn ? std::max((int)fit, 1) : std::min(kn, most);
         p.part = (float*)workspace;
         return dtype == MINFER_ATTN_F16 ? launch_kn_rows<F16>(p, stream) : launch_kn_rows<BF16>(p, stream);
     }
