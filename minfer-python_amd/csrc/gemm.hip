@@ -7,8 +7,8 @@
 //
 // Design.  From 65 rows on a workgroup of four waves owns a tile of D of 128 to 256 rows and columns (gemm_tile.h) and walks K in
 // steps of 64; the A and B panels of a step are copied global->LDS without passing through registers into a ring of two or three
-// stages, one barrier per step.  Which tile, and whether K is cut into slices that meet in a workspace, is what plan_tiles estimates
-// to be quickest.  Up to 64 rows the work is reading the weight once: the kernels of this file.
+// stages, one barrier per step.  Which tile, and whether K is cut into slices that meet in a workspace, is what plan_tiles (gemm_plan.h,
+// which has the rules of the dispatch) estimates to be quickest.  Up to 64 rows the work is reading the weight once: the kernels of this file.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -306,7 +306,6 @@ static void launch_skinny_nr(const GemmParams& p, hipStream_t stream) {
 // fourth 128-wide K segment, each wave with its own two-stage LDS area (no barrier until the final sum): per segment
 // 4 copies for the 16 weight rows, 4 for up to 16 activation rows, 4 MFMAs.  Four rows of a copy share a 1 KiB block
 // of LDS, blocks 64 bytes apart in the banks, so that the 16 rows of a fragment read hit 16 different bank groups.
-constexpr int kRowsSeg = 128;                                  // K values per segment
 constexpr int kRowsBlock = 1024 + 64;                          // LDS bytes of four rows' segment, padded
 constexpr int kRowsStage = 4 * kRowsBlock;                     // 16 rows
 // XI: copy instructions that hold activation rows (four rows each, M <= 4 * XI); fragment columns past them multiply
@@ -388,7 +387,6 @@ __global__ __launch_bounds__(4 * 64) void gemm_rows_lds_kernel(const GemmParams 
     *reinterpret_cast<uint2*>(Dg + (int64_t)m * ldd + n) = pk;
 }
 // (16 rows at most, K a multiple of 512)
-static bool rows_lds_takes(int64_t M, int64_t K) { return M <= 16 && K % (4 * kRowsSeg) == 0; }
 template <class T, bool GROUPED = false>
 static int launch_rows_lds(const GemmParams& p, int groups, hipStream_t stream) {
     const dim3 grid(groups), block(4 * 64);
@@ -413,7 +411,6 @@ static int launch_rows_lds(const GemmParams& p, int groups, hipStream_t stream) 
 // 16 / 32 / 40 / 64 rows 10.9 / 10.0, 13.7 / 11.0, 14.1 / 12.4, 15.9 / 15.1; 4096 + 1024 + 1024 columns at 24 / 40 rows 13.5 / 11.1, 15.1 /
 // 12.5; 11008 x 4096 at 40 rows 20.4 / 19.5, 22016 x 4096 40.2 / 35.2; where chunks of four are still the choice, 28672 x 4096 at 64
 // rows 48.2 / 46.0, for the even share of the copies.)
-constexpr int kStripeSeg = 256;                                // K values per segment
 constexpr int kStripeBlock = 1024;                             // LDS bytes of two rows' segment
 template <int MB, int NB = 4> struct StripeGeom {   // 16-row blocks of activations, 16-column blocks of the weight
     static constexpr int W_BYTES = NB * 8 * kStripeBlock;      // 16 * NB weight rows
@@ -605,26 +602,6 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
         finish_slices<T, 4 * 64>(p, (int)blockIdx.x / p.splits, 0, p.M, 16 * blk_first, min(16 * blk_last, p.N), &last_s);
     }
 }
-// Which widths it takes (in stripes of 64 columns; weights coming from memory): from 96 on every row count that reaches
-// it (14336 x 4096 at 2-32 rows 22.8-23.7 us, the 16-column kernel 24.3-32.4); an output head from 5 rows on (128256 x 4096 at 8
-// rows 179 against 183, 57344 x 8192 166 against 185; up to 4 rows the kernels that keep more workgroups on a compute unit are
-// ahead); narrower ones down to 32 stripes from 5 rows on, up to 8 when their rows are long enough to matter, against the 16-column
-// and few-row kernels (us: 2048 x 4096 at 16 / 17 / 64 rows 9.1 / 7.2, 13.9 / 8.0, 21.3 / 12.2; 5120 x 5120 at 5 / 16 rows 14.1 / 10.9,
-// 13.4 / 11.0; 3072 x 8192 at 8 / 32 rows 14.9 / 10.8, 29.6 / 14.2; 4096 x 14336 at 8 / 64 rows 24.0 / 21.5, 54.9 / 44.9).
-static bool stripe_takes(int64_t M, int64_t stripes, int64_t K) {
-    if (M < 1 || M > 64 || K % kStripeSeg != 0) return false;
-    if (stripes > 640) return M >= 5;
-    return stripes >= 96 || (stripes >= 80 && M >= 8) || (stripes >= 32 && M >= 5 && (M > 8 || K >= 2560));
-}
-// Where it is also ahead of its K slices, whose workgroups copy less each but leave partial sums that a second launch adds up: by the rows
-// a unit copies, (NB + MB) x 16 of K values, the narrower the weight the fewer (us, slices / whole rows: 6144 x 4096 at 64 rows 15.9 /
-// 15.1, 5632 x 4096 15.5 / 15.1, 4608 x 4096 13.8 / 14.9 and at 33 rows 12.7 / 11.7; 4096 x 6144 at 33 / 64 rows 13.9 / 13.4, 15.2 /
-// 16.5; 3584 x 8192 at 32 / 48 rows 14.5 / 14.3, 16.1 / 18.2; 2560 x 5120 at 32 / 33 rows 10.7 / 10.1, 11.4 / 11.7; 2048 x 4096 at 32 /
-// 64 rows 9.3 / 8.4, 11.2 / 12.2; 2048 x 8192 at 5 rows 9.5 / 10.4; 4096 x 14336 at 16 / 24 rows 24.0 / 24.1, 24.8 / 27.8).
-static bool stripe_blocks_pay(int64_t M, int64_t stripes, int64_t K) {
-    const int64_t most = stripes < 48 ? 16000 : stripes <= 64 || stripes >= 80 ? 25000 : 22000;
-    return stripe_takes(M, stripes, K) && (stripes >= 96 || ((stripes > 64 ? 2 : 1) + (M + 15) / 16) * K <= most);
-}
 // The smallest NB that goes through the `most` blocks of a workgroup in as few chunks as four would (five blocks as three and two: 18944 x 3584
 // at 32 rows 33.4 -> 30.5 us).
 template <class T, int MB, bool SLICED, bool GROUPED>
@@ -656,14 +633,6 @@ static int launch_stripe(const GemmParams& p0, int blocks, hipStream_t stream) {
     else launch_stripe_rows<T, 4, SLICED, GROUPED>(p, most, grid, stream);
     return check_launch("gemm_stripe_kernel");
 }
-// A weight of fewer than 192 stripes: with a workspace, K slices bring the workgroups up to the chip's 256 compute units
-// (every slice four segments at least); the slices' sums are added up by finish_slices or gemm_reduce_kernel (slice_counters).
-// 1 = no slices.
-static int stripe_slices(int64_t M, int64_t N, int64_t K) {
-    const int64_t stripes = (N + 63) / 64;
-    if (M < 1 || M > 64 || K % kStripeSeg != 0 || N % 8 != 0 || stripes >= 192) return 1;
-    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / stripes, K / kStripeSeg / 4), 16));
-}
 
 // One row against an [N, K] weight (a decode step's projection): a wave streams whole weight rows as consecutive 16-byte
 // pieces (1 KiB per instruction, where the MFMA kernel above takes 128 bytes of each of 16 rows) and multiplies in the
@@ -671,7 +640,6 @@ static int stripe_slices(int64_t M, int64_t N, int64_t K) {
 // a row.  A row is cut into segments of 4096 values (8 pieces per lane); when it is a single segment the lane keeps the
 // activations it needs in registers (XREG), otherwise the workgroup keeps the activation row in LDS.  A wave owns a run
 // of consecutive rows and has the next two segments in flight.
-constexpr int kGemvSegHalfs = 4096;
 constexpr int kGemvSegPieces = kGemvSegHalfs / 8 / 64;     // 16-byte pieces per lane and segment
 template <class T> MA_DEV float dot8(uint4 a, uint4 b, float acc);
 template <> MA_DEV float dot8<F16>(uint4 a, uint4 b, float acc) {
@@ -689,7 +657,6 @@ template <> MA_DEV float dot8<BF16>(uint4 a, uint4 b, float acc) {   // a bf16 i
     }
     return acc;
 }
-constexpr int kGemvMaxKHalfs = 16384;                      // activation row kept in LDS: 32 KiB
 // GROUPED: the rows of up to three weights numbered through (p.grp.end[s] = rows of weights 0 .. s), every weight with
 // its own output; alpha = 1, no C.
 // MR: activation rows (1-4; more than one only ungrouped): every weight piece is multiplied with the same piece of each.
@@ -800,7 +767,6 @@ static int launch_gemv(const GemmParams& p, int n_rows, hipStream_t stream) {
     return check_launch("gemv_kernel");
 }
 // which calls it takes: one row, or up to four rows longer than a segment whose activations fit its LDS area
-static bool gemv_takes(int64_t M, int64_t K) { return M >= 1 && M <= 4 && K <= kGemvMaxKHalfs && (M == 1 || (K > kGemvSegHalfs && M * K <= 2 * kGemvMaxKHalfs)); }
 
 template <class T>
 static int launch_skinny(const GemmParams& p, hipStream_t stream) {
@@ -1318,15 +1284,6 @@ static int launch_stripe_slices(GemmParams& p, hipStream_t stream) {
     return launch_reduce<T>(p, stream);
 }
 
-// [K, N] weights of up to 64 rows: slices of K bring the column tiles up to the chip's 256 compute units, every slice two
-// steps of 64 at least; from 17 rows on four and at most 32 slices, since the sums grow with the rows.  The workspace is for these; a call that
-// has it takes 8 or 16 of them at most.
-constexpr int64_t kKnRows = 64;
-static int kn_slices(int64_t M, int64_t N, int64_t K) {
-    if (M < 1 || M > kKnRows || K % kBK != 0 || K < 8 * kBK || N % 8 != 0) return 1;
-    const int64_t tiles = (N + 127) / 128;
-    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, K / kBK / (M <= 16 ? 2 : 4)), M <= 16 ? 64 : 32));
-}
 template <class T>
 static int launch_kn_rows(GemmParams& p, hipStream_t stream) {
     const dim3 grid((unsigned)((p.N + 127) / 128 * p.splits)), block(4 * 64);
@@ -1339,8 +1296,7 @@ static int launch_kn_rows(GemmParams& p, hipStream_t stream) {
     return p.splits > 1 ? launch_reduce<T>(p, stream) : MINFER_ATTN_OK;
 }
 
-// ---- which tiles, how many K slices --------------------------------------------------------------------------
-static int64_t tile_count(int64_t M, int64_t N, int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
+
 static int compute_units() {
     static std::atomic<int> cached[64];
     int dev = 0;
@@ -1352,79 +1308,13 @@ static int compute_units() {
     }
     return cus;
 }
-// Microseconds of a launch of `tiles` tiles in `slices` K slices each, weights from memory: whole rounds of the chip, the last,
-// partly filled one at 0.76 + 0.24 of its share (its units run faster), a round its K steps at 20 ns per pair of 16-row blocks (two
-// workgroups on a unit 1.84 of one; with two stages a step that is shorter than the largest tile's does not cover its copies) and
-// 3.8 us of first and last copies and results; the copies of all tiles at 31 TB/s and the weight at 7 TB/s, which are hidden behind
-// that in part: the three add up as their squares; past one round, where the clock has come down to what the power budget leaves, the
-// more the more a tile copies per flop (3072 x 8192 x 4096: 128 x 256 tiles 177.7 us, 192 x 256 167.1, without this estimated 171.7 and
-// 172.9; 4096 x 5120 x 4096 150.9 and 137.0); 3.6 us around it, 0.9 more for the launch that adds the slices up, and 0.29 us
-// per MB of sums.  Fitted to 4700 timed calls (150 shapes of 65 to 7000 rows, both layouts, up to 40 choices each): the choice it
-// makes is 1.0 % behind the best one on average, fixed rules for 128 x 128 and 128 x 256 slices and a table of rounds 6 %.
-static double plan_cost(const GemmTile& t, int64_t tiles, int slices, int64_t M, int64_t N, int64_t K, int cus) {
-    const double steps = (double)((K / kBK + slices - 1) / slices), area = t.m16 * t.n16;
-    const double step = (0.0201 * area + 0.0738) * (t.occ == 2 ? 1.84 : 1.0) + (t.ns == 2 && t.occ == 1 ? 0.0147 + 0.0076 * (64 - area) : 0.0);
-    const int64_t wgs = tiles * slices, per = (int64_t)cus * t.occ, full = wgs / per, rest = wgs % per;
-    const double rounds = (double)full + (rest ? 0.76 + 0.24 * (double)rest / (double)per : 0.0);
-    const double power = wgs > per ? 1.0 + ((t.m16 + t.n16) / area - 0.25) : 1.0;
-    const double compute = rounds * (step * steps + 3.8) * power, weight = (double)N * (double)K * 2 / 7.0e6;
-    const double copies = (double)tiles * (double)(K / kBK) * (t.m16 + t.n16) * 4096 / 31.3e6;
-    const double launch = 3.6 + sqrt(compute * compute + copies * copies + weight * weight);
-    return slices > 1 ? launch + 0.9 + 0.286e-6 * slices * (double)M * (double)N * 4 : launch;
-}
-// The cheapest tile shape and number of slices, up to max_slices of them (what a workspace holds): slices that bring the
-// workgroups to one or two rounds of the chip or just below, 3 steps long at least, with 64 MiB of sums at most.
-struct TilePlan { int tile, slices; };
-static TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, bool nt, int64_t max_slices) {
-    const int cus = compute_units();
-    const int64_t room = std::min<int64_t>(std::min<int64_t>(32, max_slices), std::min<int64_t>(K / kBK / 3, (INT64_C(16) << 20) / (M * N)));
-    TilePlan best{0, 1};
-    double cost = 0;
-    for (int i = 0; i < kGemmTileCount; ++i) {
-        const GemmTile& t = kGemmTiles[i];
-        if (!nt && t.n16 % 4 != 0) continue;
-        const int64_t tiles = tile_count(M, N, 32 * t.m16, 32 * t.n16), fill = (int64_t)cus * t.occ / tiles;
-        if (t.occ == 2 && tiles * std::max<int64_t>(room, 1) <= cus) continue;   // one workgroup to a unit: the other entry's three stages
-        const int64_t options[5] = {1, fill, fill - 1, fill * 3 / 4, 2 * fill};
-        for (int o = 0; o < 5; ++o) {
-            if (options[o] > room && options[o] != 1) continue;
-            if (options[o] < 1 || (o > 0 && options[o] == 1)) continue;
-            const double c = plan_cost(t, tiles, (int)options[o], M, N, K, cus);
-            if (cost == 0 || c < cost) { cost = c; best = {i, (int)options[o]}; }
-        }
-    }
-    return best;
-}
-// The plan a shape gets with all the workspace it wants.  A call asks twice (for the workspace and to launch), so the last few
-// are kept; they depend on nothing but the sizes (and the chip's units, which do not differ between the devices of a process).
-static TilePlan full_plan(int64_t M, int64_t N, int64_t K, bool nt) {
-    struct Entry { int64_t M, N, K; bool nt; TilePlan plan; };
-    static thread_local Entry kept[16];
-    Entry& e = kept[(uint64_t)(M * 31 + N * 7 + K + nt) % 16];
-    if (e.M != M || e.N != N || e.K != K || e.nt != nt) e = Entry{M, N, K, nt, plan_tiles(M, N, K, nt, 1 << 20)};
-    return e.plan;
-}
-// Slices that a workspace is sized for: the plan's, and no fewer than bring 128 x 128 tiles to one round of the chip (to two while
-// a slice stays 16 steps long), four steps long at least: the size has been that, and callers may keep a workspace by it.
-static int gemm_slices(int64_t M, int64_t N, int64_t K, bool nt) {
-    if (K <= 0 || K % kBK != 0 || N % 8 != 0) return 1;
-    int64_t s = 1;
-    const int64_t tiles = tile_count(M, N, 128, 128), kt = K / kBK;
-    if (tiles <= 256 && kt >= 8) {
-        s = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, kt / 4), 32));
-        if (tiles >= 64 && tiles * s <= 256 && kt / (2 * s) >= 16 && (s >= 2 || kt >= 192)) s *= 2;
-    }
-    return std::max((int)s, full_plan(M, N, K, nt).slices);
-}
-
 template <class T> static int launch_tile(const GemmParams& p, bool nt, int tile, hipStream_t stream) {
     return std::is_same<T, F16>::value ? launch_gemm_tile_f16(p, nt, tile, stream) : launch_gemm_tile_bf16(p, nt, tile, stream);
 }
 template <class T>
-static int launch_gemm(GemmParams& p, bool nt, const TilePlan& plan, hipStream_t stream) {
-    p.splits = plan.slices;
-    if (int rc = launch_tile<T>(p, nt, plan.tile, stream)) return rc;
-    return plan.slices > 1 ? launch_reduce<T>(p, stream) : MINFER_ATTN_OK;
+static int launch_gemm(GemmParams& p, bool nt, int tile, hipStream_t stream) {   // (p.splits K slices)
+    if (int rc = launch_tile<T>(p, nt, tile, stream)) return rc;
+    return p.splits > 1 ? launch_reduce<T>(p, stream) : MINFER_ATTN_OK;
 }
 
 template <class T, bool NT>
@@ -1432,6 +1322,22 @@ static int launch_plain(const GemmParams& p, hipStream_t stream) {
     const int grid = (int)std::min<int64_t>(((int64_t)p.M * p.N + 255) / 256, 256 * 16);
     hipLaunchKernelGGL((gemm_plain_kernel<T, NT>), dim3(grid), dim3(256), 0, stream, p);
     return check_launch("gemm_plain_kernel");
+}
+
+template <class T>
+static int launch_route(GemmParams& p, bool nt, const GemmRoute& route, hipStream_t stream) {
+    p.splits = route.slices;
+    switch (route.kernel) {
+        case GemmKernel::gemv: return launch_gemv<T>(p, p.N, stream);
+        case GemmKernel::rows_lds: return launch_rows_lds<T>(p, (p.N + 15) / 16, stream);
+        case GemmKernel::skinny: return launch_skinny<T>(p, stream);
+        case GemmKernel::stripe: return launch_stripe<T>(p, (p.N + 15) / 16, stream);
+        case GemmKernel::stripe_slices: return launch_stripe_slices<T>(p, stream);
+        case GemmKernel::kn_rows: return launch_kn_rows<T>(p, stream);
+        case GemmKernel::tiles: return launch_gemm<T>(p, nt, route.tile, stream);
+        case GemmKernel::plain: break;
+    }
+    return nt ? launch_plain<T, true>(p, stream) : launch_plain<T, false>(p, stream);
 }
 
 // Up to three weights [N_s, K] against one A in one launch (alpha = 1, no C): the tiled kernel over the concatenated
@@ -1489,7 +1395,8 @@ static int launch_grouped(GemmParams& p, int n_w, hipStream_t stream) {
     }
     fill_ends(1);   // the tiled kernel takes the weights' columns numbered through
     p.N = (int)n_sum;
-    return launch_gemm<T>(p, true, plan_tiles(p.M, n_sum, p.K, true, 1), stream);
+    p.splits = 1;
+    return launch_gemm<T>(p, true, tile_plan(p.M, n_sum, p.K, true, 1, compute_units()).tile, stream);
 }
 
 }  // namespace minfer_attn
@@ -1554,69 +1461,10 @@ static int gemm_impl(int dtype, int b_layout, const void* A, const void* B, cons
                       aligned16(A) && aligned16(B) && ((uintptr_t)D & 7u) == 0 && ((uintptr_t)C & 7u) == 0 &&
                       (int64_t)256 * lda < (1LL << 30) && (int64_t)256 * ldb < (1LL << 30);
     hipStream_t stream = (hipStream_t)stream_v;
-    // A decode step's few tokens against an [N, K] weight: stream the weight once.  Which kernel does that best was
-    // measured with the calls cycling over copies of the weight, 640 MiB in all: a weight of up to 256 MiB called again
-    // and again is served by the chip's last-level cache, where the order of the kernels is a different one (14336 x
-    // 4096 at one row: stripes 18.0 us against 19.5 for whole rows per wave from the cache, 24.2 against 21.9 from memory).
     const size_t fit = workspace && aligned16(workspace) ? workspace_bytes / ((size_t)M * (size_t)N * sizeof(float)) : 0;   // slices the workspace holds
-    const bool can_split = fast && fit > 1 && full_plan(M, N, K, nt).slices > 1;
-    const int64_t stripes = (N + 63) / 64;
-    const bool rows_takes = rows_lds_takes(M, K);
-    // one row: whole weight rows per wave (14336 x 4096: 21.9 us, the 16-column kernel 23.6, stripes 24.2; 28672 x 8192:
-    // 75.8 / 91 / 97); a weight under 32 M values goes to the 16-column kernel when it takes it (4096 x 4096: 8.5 against 10.5)
-    if (fast && nt && M == 1 && K <= kGemvMaxKHalfs && (N * K >= (INT64_C(1) << 25) || !rows_takes))
-        return dtype == MINFER_ATTN_F16 ? launch_gemv<F16>(p, p.N, stream) : launch_gemv<BF16>(p, p.N, stream);
-    // two to four rows against long rows of a wide weight go the same way, every weight piece multiplied with the same
-    // piece of each activation row (28672 x 8192 at 2-4 rows: 78.6-82.6 us against 93-95 for the 16-column kernel, 10240 x
-    // 8192 at 2-3 rows 33.2-34.6 against 36.3; 8192 x 8192 30.5-33.9 against 29.2-29.6, and rows of 4096 values gain nothing)
-    if (fast && nt && M >= 2 && gemv_takes(M, K) && K >= 8192 && N >= 10240 && (M <= 3 || N >= 16384))
-        return dtype == MINFER_ATTN_F16 ? launch_gemv<F16>(p, p.N, stream) : launch_gemv<BF16>(p, p.N, stream);
-    // up to 4 rows (8 where stripe_takes says no) against fewer than 96 stripes, and up to 4 against an output head: the 16-column
-    // kernel (128256 x 4096 at 2-4 rows 166-170 against 176-178; 28672 x 4096 at 2-8 rows 42.2-44.5 against 41.5-41.7 and 14336 x
-    // 4096 24.3-25.8 against 22.8-23.0: those go on)
-    const bool rows_first = rows_takes && ((M <= 8 && stripes < 96 && !stripe_takes(M, stripes, K)) || (M <= 4 && stripes > 640));
-    const int slices = fast && nt && workspace && aligned16(workspace) ? stripe_slices(M, N, K) : 1;
-    const bool sliceable = slices > 1 && workspace_bytes >= (size_t)slices * (size_t)M * (size_t)N * sizeof(float);
-    // ... except long rows of a narrow weight when a workspace allows K slices: one wave per 16 columns walks a whole row
-    // by itself (1024 x 14336 at 2-8 rows 16.5-20.8 us, in slices 13.1-14.1; 1536 x 8960 15.2-17.4 and 11.8-12.5; 2048 x
-    // 8192 at 5-8 rows 12.5-13.4 and 12.5-12.6, at 2-4 rows and for rows of 6144 values no gain)
-    const bool long_rows_few_stripes = K >= 8192 && ((M >= 5 && stripes <= 32) || (M >= 2 && stripes <= 24));
-    if (fast && nt && rows_first && !(sliceable && long_rows_few_stripes))
-        return dtype == MINFER_ATTN_F16 ? launch_rows_lds<F16>(p, (int)((N + 15) / 16), stream) : launch_rows_lds<BF16>(p, (int)((N + 15) / 16), stream);
-    // with a workspace, K slices of the stripes, from 9 rows on, where whole rows are not ahead (stripe_blocks_pay): two launches, 10.5
-    // us at least, where one launch over rows of 4096 values takes 8-10 at 9-16 rows: up to 16 rows only for 25 M weight values or
-    // rows of 6144 values and more (2048 x 8192 at 9-16 rows 12.7-13.0 against 13.9-16.5, 1024 x 14336 13.7-14.6 against 21.5-26.7),
-    // from 17 rows on for 8 M values (1536 x 5632 and the like: gemm_skinny_kernel is the other choice)
-    const bool slices_pay = !stripe_blocks_pay(M, stripes, K) && (long_rows_few_stripes || (M >= 9 && (N * K >= INT64_C(25000000) || K >= 6144 || (M >= 17 && N * K >= (INT64_C(1) << 23)))));
-    if (sliceable && slices_pay) {
-        p.splits = slices; p.part = (float*)workspace;
-        return dtype == MINFER_ATTN_F16 ? launch_stripe_slices<F16>(p, stream) : launch_stripe_slices<BF16>(p, stream);
-    }
-    if (fast && nt && stripe_takes(M, stripes, K))
-        return dtype == MINFER_ATTN_F16 ? launch_stripe<F16>(p, (int)((N + 15) / 16), stream) : launch_stripe<BF16>(p, (int)((N + 15) / 16), stream);
-    if (fast && nt && rows_takes)
-        return dtype == MINFER_ATTN_F16 ? launch_rows_lds<F16>(p, (int)((N + 15) / 16), stream) : launch_rows_lds<BF16>(p, (int)((N + 15) / 16), stream);
-    if (fast && nt && M == 1 && K <= kGemvMaxKHalfs)
-        return dtype == MINFER_ATTN_F16 ? launch_gemv<F16>(p, p.N, stream) : launch_gemv<BF16>(p, p.N, stream);
-    if (fast && nt && (M <= 16 || (!can_split && (M <= 32 || (M <= 64 && N * K <= (INT64_C(1) << 25))))))
-        return dtype == MINFER_ATTN_F16 ? launch_skinny<F16>(p, stream) : launch_skinny<BF16>(p, stream);
-    if (fast && !nt && M <= kKnRows) {
-        // eight slices at most, 16 for rows of 80 K steps and more: further ones save less streaming than their sums cost (us, as many as fill
-        // the chip / these: 1000 x 4096 at 1 / 9 / 16 rows 10.5 / 7.6, 13.5 / 8.7, 15.5 / 9.4; 2560 x 2560 at 12 10.0 / 8.1; 2048 x 4096 at 40 13.7 /
-        // 11.9; 1024 x 14336 at 9 / 40 15.4 / 12.8, 19.4 / 17.2; 512 x 8192 at 9 17.0 / 9.6; the size reported stays that of filling it)
-        const int kn = kn_slices(M, N, K), most = K >= 80 * kBK ? 16 : 8;   // a smaller workspace: as many slices as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
-        p.splits = fit < (size_t)kn ? std::max((int)fit, 1) : std::min(kn, most);
-        p.part = (float*)workspace;
-        return dtype == MINFER_ATTN_F16 ? launch_kn_rows<F16>(p, stream) : launch_kn_rows<BF16>(p, stream);
-    }
-    if (fast) {
-        TilePlan plan = full_plan(M, N, K, nt);
-        if ((size_t)plan.slices > std::max<size_t>(fit, 1)) plan = plan_tiles(M, N, K, nt, std::max<int64_t>((int64_t)fit, 1));
-        p.part = (float*)workspace;
-        return dtype == MINFER_ATTN_F16 ? launch_gemm<F16>(p, nt, plan, stream) : launch_gemm<BF16>(p, nt, plan, stream);
-    }
-    if (dtype == MINFER_ATTN_F16) return nt ? launch_plain<F16, true>(p, stream) : launch_plain<F16, false>(p, stream);
-    return nt ? launch_plain<BF16, true>(p, stream) : launch_plain<BF16, false>(p, stream);
+    p.part = (float*)workspace;
+    const GemmRoute route = gemm_route(M, N, K, nt, fast, (int64_t)std::min<size_t>(fit, 2 * kMostSlices), compute_units);
+    return dtype == MINFER_ATTN_F16 ? launch_route<F16>(p, nt, route, stream) : launch_route<BF16>(p, nt, route, stream);
 }
 
 MINFER_ATTN_EXPORT int minfer_gemm(int dtype, int b_layout, const void* A, const void* B, const void* C, void* D,
@@ -1628,14 +1476,15 @@ MINFER_ATTN_EXPORT int minfer_gemm(int dtype, int b_layout, const void* A, const
 MINFER_ATTN_EXPORT size_t minfer_gemm_layout_workspace_bytes(int b_layout, int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
     int splits;   // the most slices that a route of gemm_impl cuts K into for this layout
-    if (b_layout == MINFER_GEMM_B_KN) splits = M <= kKnRows ? kn_slices(M, N, K) : gemm_slices(M, N, K, false);
-    else splits = std::max(stripe_slices(M, N, K), M > 16 ? gemm_slices(M, N, K, true) : 1);
+    if (b_layout == MINFER_GEMM_B_KN) splits = M <= kKnRows ? kn_slices(M, N, K) : gemm_slices(M, N, K, false, compute_units());
+    else splits = std::max(stripe_slices(M, N, K), M > 16 ? gemm_slices(M, N, K, true, compute_units()) : 1);
     return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
 MINFER_ATTN_EXPORT size_t minfer_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
-    const int splits = std::max(std::max(gemm_slices(M, N, K, true), gemm_slices(M, N, K, false)), std::max(stripe_slices(M, N, K), kn_slices(M, N, K)));
+    const int cus = compute_units();
+    const int splits = std::max(std::max(gemm_slices(M, N, K, true, cus), gemm_slices(M, N, K, false, cus)), std::max(stripe_slices(M, N, K), kn_slices(M, N, K)));
     return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 

@@ -7,10 +7,10 @@
 
 #include "attn_common.h"
 #include "attn_host.h"
+#include "gemm_plan.h"
 
 namespace minfer_attn {
 
-constexpr int kBK = 64;                     // K values of a step of the tiled kernels
 constexpr int kRowTile = 8192;              // sub-tile [64 rows][64 k], 128-byte rows (A, and B as [N, K])
 constexpr int kColTile = 16384;             // sub-tile [64 k][128 n], 256-byte rows (B as [K, N])
 
@@ -60,14 +60,6 @@ template <class T> MA_DEV void store_result(const GemmParams& p, int m, int n, f
 MA_DEV int swz_row_tile(int row) { return (row >> 1) & 7; }        // 128-byte rows, read 32 rows x 16 bytes
 MA_DEV int swz_col_tile(int row) { return ((row & 3) << 2) | ((row >> 2) & 2); }   // 256-byte rows, transposing reads of 4 rows x 32 bytes by each of two 16-lane groups 8 rows apart
 
-// The tiled kernel's shapes: 32 m16 x 32 n16, ns stages, occ workgroups to a unit (GemmShape).  The more there are the closer a
-// problem's tiles come to whole rounds of the chip (plan_tiles); of the 26 from 128 to 256 in steps of 32 these lose 0.3 % to all
-// over random shapes (256 x 192 takes 4096 x 6144 x 4096 in two rounds: 163.8 us, the others 167.8 at best).  A [K, N] weight is staged in sub-tiles of 128 columns and takes those whose n16 is a multiple of 4.
-struct GemmTile { int m16, n16, ns, occ; };
-constexpr GemmTile kGemmTiles[] = {
-    {8, 8, 2, 1}, {8, 7, 2, 1}, {7, 8, 2, 1}, {6, 8, 2, 1}, {5, 8, 3, 1}, {4, 8, 3, 1}, {7, 6, 3, 1}, {6, 6, 3, 1},
-    {4, 6, 3, 1}, {5, 7, 3, 1}, {7, 4, 3, 1}, {6, 4, 3, 1}, {5, 4, 3, 1}, {4, 4, 3, 1}, {4, 4, 2, 2}, {8, 6, 2, 1}};
-constexpr int kGemmTileCount = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 int launch_gemm_tile_f16(const GemmParams& p, bool nt, int tile, hipStream_t stream);
 int launch_gemm_tile_bf16(const GemmParams& p, bool nt, int tile, hipStream_t stream);
 

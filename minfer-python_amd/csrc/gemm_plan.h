@@ -1,0 +1,210 @@
+// Which kernel of the GEMM family takes a call, in which tiles and in how many K slices: the rules on sizes, types and alignment, with
+// what was measured on both sides of each line.  Host code only, without a GPU header, so that the rules can be run on their own.
+#pragma once
+
+#include <math.h>
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace minfer_attn {
+
+constexpr int kBK = 64;                     // K values of a step of the tiled kernels
+constexpr int kRowsSeg = 128;               // ... of a segment of gemm_rows_lds_kernel
+constexpr int kStripeSeg = 256;             // ... of the stripe kernels
+constexpr int kGemvSegHalfs = 4096;         // ... of gemv_kernel
+constexpr int kGemvMaxKHalfs = 16384;       // the longest activation row that gemv_kernel keeps in LDS: 32 KiB
+
+// The tiled kernel's shapes: 32 m16 x 32 n16, ns stages, occ workgroups to a unit (GemmShape).  The more there are the closer a
+// problem's tiles come to whole rounds of the chip (plan_tiles); of the 26 from 128 to 256 in steps of 32 these lose 0.3 % to all
+// over random shapes (256 x 192 takes 4096 x 6144 x 4096 in two rounds: 163.8 us, the others 167.8 at best).  A [K, N] weight is
+// staged in sub-tiles of 128 columns and takes those whose n16 is a multiple of 4.
+struct GemmTile { int m16, n16, ns, occ; };
+constexpr GemmTile kGemmTiles[] = {
+    {8, 8, 2, 1}, {8, 7, 2, 1}, {7, 8, 2, 1}, {6, 8, 2, 1}, {5, 8, 3, 1}, {4, 8, 3, 1}, {7, 6, 3, 1}, {6, 6, 3, 1},
+    {4, 6, 3, 1}, {5, 7, 3, 1}, {7, 4, 3, 1}, {6, 4, 3, 1}, {5, 4, 3, 1}, {4, 4, 3, 1}, {4, 4, 2, 2}, {8, 6, 2, 1}};
+constexpr int kGemmTileCount = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
+
+// ---- few rows against an [N, K] weight -----------------------------------------------------------------------
+
+// gemm_rows_lds_kernel: four waves that take a segment each.
+inline bool rows_lds_takes(int64_t M, int64_t K) { return M <= 16 && K % (4 * kRowsSeg) == 0; }
+// gemv_kernel: one to four rows that its LDS area holds.
+inline bool gemv_takes(int64_t M, int64_t K) { return M >= 1 && M <= 4 && K <= kGemvMaxKHalfs && (M == 1 || (K > kGemvSegHalfs && M * K <= 2 * kGemvMaxKHalfs)); }
+// gemm_stripe_kernel.  Which widths it takes (in stripes of 64 columns; weights coming from memory): from 96 on every row count that reaches
+// it (14336 x 4096 at 2-32 rows 22.8-23.7 us, the 16-column kernel 24.3-32.4); an output head from 5 rows on (128256 x 4096 at 8
+// rows 179 against 183, 57344 x 8192 166 against 185; up to 4 rows the kernels that keep more workgroups on a compute unit are
+// ahead); narrower ones down to 32 stripes from 5 rows on, up to 8 when their rows are long enough to matter, against the 16-column
+// and few-row kernels (us: 2048 x 4096 at 16 / 17 / 64 rows 9.1 / 7.2, 13.9 / 8.0, 21.3 / 12.2; 5120 x 5120 at 5 / 16 rows 14.1 / 10.9,
+// 13.4 / 11.0; 3072 x 8192 at 8 / 32 rows 14.9 / 10.8, 29.6 / 14.2; 4096 x 14336 at 8 / 64 rows 24.0 / 21.5, 54.9 / 44.9).
+inline bool stripe_takes(int64_t M, int64_t stripes, int64_t K) {
+    if (M < 1 || M > 64 || K % kStripeSeg != 0) return false;
+    if (stripes > 640) return M >= 5;
+    return stripes >= 96 || (stripes >= 80 && M >= 8) || (stripes >= 32 && M >= 5 && (M > 8 || K >= 2560));
+}
+// Where it is also ahead of its K slices, whose workgroups copy less each but leave partial sums that a second launch adds up: by the rows
+// a unit copies, (NB + MB) x 16 of K values, the narrower the weight the fewer (us, slices / whole rows: 6144 x 4096 at 64 rows 15.9 /
+// 15.1, 5632 x 4096 15.5 / 15.1, 4608 x 4096 13.8 / 14.9 and at 33 rows 12.7 / 11.7; 4096 x 6144 at 33 / 64 rows 13.9 / 13.4, 15.2 /
+// 16.5; 3584 x 8192 at 32 / 48 rows 14.5 / 14.3, 16.1 / 18.2; 2560 x 5120 at 32 / 33 rows 10.7 / 10.1, 11.4 / 11.7; 2048 x 4096 at 32 /
+// 64 rows 9.3 / 8.4, 11.2 / 12.2; 2048 x 8192 at 5 rows 9.5 / 10.4; 4096 x 14336 at 16 / 24 rows 24.0 / 24.1, 24.8 / 27.8).
+inline bool stripe_blocks_pay(int64_t M, int64_t stripes, int64_t K) {
+    const int64_t most = stripes < 48 ? 16000 : stripes <= 64 || stripes >= 80 ? 25000 : 22000;
+    return stripe_takes(M, stripes, K) && (stripes >= 96 || ((stripes > 64 ? 2 : 1) + (M + 15) / 16) * K <= most);
+}
+// A weight of fewer than 192 stripes: with a workspace, K slices bring the workgroups up to the chip's 256 compute units
+// (every slice four segments at least); the slices' sums are added up by finish_slices or gemm_reduce_kernel (slice_counters).
+// 1 = no slices.
+inline int stripe_slices(int64_t M, int64_t N, int64_t K) {
+    const int64_t stripes = (N + 63) / 64;
+    if (M < 1 || M > 64 || K % kStripeSeg != 0 || N % 8 != 0 || stripes >= 192) return 1;
+    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / stripes, K / kStripeSeg / 4), 16));
+}
+
+// ---- few rows against a [K, N] weight ------------------------------------------------------------------------
+
+// [K, N] weights of up to 64 rows: slices of K bring the column tiles up to the chip's 256 compute units, every slice two
+// steps of 64 at least; from 17 rows on four and at most 32 slices, since the sums grow with the rows.  The workspace is for these; a call that
+// has it takes 8 or 16 of them at most.
+constexpr int64_t kKnRows = 64;
+inline int kn_slices(int64_t M, int64_t N, int64_t K) {
+    if (M < 1 || M > kKnRows || K % kBK != 0 || K < 8 * kBK || N % 8 != 0) return 1;
+    const int64_t tiles = (N + 127) / 128;
+    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, K / kBK / (M <= 16 ? 2 : 4)), M <= 16 ? 64 : 32));
+}
+
+// ---- which tiles, how many K slices --------------------------------------------------------------------------
+inline int64_t tile_count(int64_t M, int64_t N, int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
+// Microseconds of a launch of `tiles` tiles in `slices` K slices each, weights from memory: whole rounds of the chip, the last,
+// partly filled one at 0.76 + 0.24 of its share (its units run faster), a round its K steps at 20 ns per pair of 16-row blocks (two
+// workgroups on a unit 1.84 of one; with two stages a step that is shorter than the largest tile's does not cover its copies) and
+// 3.8 us of first and last copies and results; the copies of all tiles at 31 TB/s and the weight at 7 TB/s, which are hidden behind
+// that in part: the three add up as their squares; past one round, where the clock has come down to what the power budget leaves, the
+// more the more a tile copies per flop (3072 x 8192 x 4096: 128 x 256 tiles 177.7 us, 192 x 256 167.1, without this estimated 171.7 and
+// 172.9; 4096 x 5120 x 4096 150.9 and 137.0); 3.6 us around it, 0.9 more for the launch that adds the slices up, and 0.29 us
+// per MB of sums.  Fitted to 4700 timed calls (150 shapes of 65 to 7000 rows, both layouts, up to 40 choices each): the choice it
+// makes is 1.0 % behind the best one on average, fixed rules for 128 x 128 and 128 x 256 slices and a table of rounds 6 %.
+inline double plan_cost(const GemmTile& t, int64_t tiles, int slices, int64_t M, int64_t N, int64_t K, int cus) {
+    const double steps = (double)((K / kBK + slices - 1) / slices), area = t.m16 * t.n16;
+    const double step = (0.0201 * area + 0.0738) * (t.occ == 2 ? 1.84 : 1.0) + (t.ns == 2 && t.occ == 1 ? 0.0147 + 0.0076 * (64 - area) : 0.0);
+    const int64_t wgs = tiles * slices, per = (int64_t)cus * t.occ, full = wgs / per, rest = wgs % per;
+    const double rounds = (double)full + (rest ? 0.76 + 0.24 * (double)rest / (double)per : 0.0);
+    const double power = wgs > per ? 1.0 + ((t.m16 + t.n16) / area - 0.25) : 1.0;
+    const double compute = rounds * (step * steps + 3.8) * power, weight = (double)N * (double)K * 2 / 7.0e6;
+    const double copies = (double)tiles * (double)(K / kBK) * (t.m16 + t.n16) * 4096 / 31.3e6;
+    const double launch = 3.6 + sqrt(compute * compute + copies * copies + weight * weight);
+    return slices > 1 ? launch + 0.9 + 0.286e-6 * slices * (double)M * (double)N * 4 : launch;
+}
+// The cheapest tile shape and number of slices, up to max_slices of them (what a workspace holds): slices that bring the
+// workgroups to one or two rounds of the chip or just below, 3 steps long at least, with 64 MiB of sums at most.
+constexpr int64_t kMostSlices = 32;
+struct TilePlan { int tile, slices; };
+inline TilePlan plan_tiles(int64_t M, int64_t N, int64_t K, bool nt, int64_t max_slices, int cus) {
+    const int64_t room = std::min<int64_t>(std::min<int64_t>(kMostSlices, max_slices), std::min<int64_t>(K / kBK / 3, (INT64_C(16) << 20) / (M * N)));
+    TilePlan best{0, 1};
+    double cost = 0;
+    for (int i = 0; i < kGemmTileCount; ++i) {
+        const GemmTile& t = kGemmTiles[i];
+        if (!nt && t.n16 % 4 != 0) continue;
+        const int64_t tiles = tile_count(M, N, 32 * t.m16, 32 * t.n16), fill = (int64_t)cus * t.occ / tiles;
+        if (t.occ == 2 && tiles * std::max<int64_t>(room, 1) <= cus) continue;   // one workgroup to a unit: the other entry's three stages
+        const int64_t options[5] = {1, fill, fill - 1, fill * 3 / 4, 2 * fill};
+        for (int o = 0; o < 5; ++o) {
+            if (options[o] > room && options[o] != 1) continue;
+            if (options[o] < 1 || (o > 0 && options[o] == 1)) continue;
+            const double c = plan_cost(t, tiles, (int)options[o], M, N, K, cus);
+            if (cost == 0 || c < cost) { cost = c; best = {i, (int)options[o]}; }
+        }
+    }
+    return best;
+}
+// plan_tiles, remembered: estimating takes a microsecond and more, and a call asks twice (for the workspace and to launch), as does every
+// next token or chunk for all the projections of a layer.  The last 16 plans of a thread, looked through from one end to the other
+// (4 to 10 ns): a place by some hash of the sizes is shared sooner or later by the projections of one model, which then push each other out.  A
+// plan depends on nothing but what it is looked up by.
+constexpr int kPlansKept = 16;
+inline TilePlan tile_plan(int64_t M, int64_t N, int64_t K, bool nt, int64_t max_slices, int cus) {
+    struct Entry { int64_t M, N, K, max_slices; int nt, cus; TilePlan plan; };
+    static thread_local Entry kept[kPlansKept];
+    static thread_local unsigned oldest = 0;
+    max_slices = std::min<int64_t>(max_slices, kMostSlices);
+    for (const Entry& e : kept)
+        if (e.M == M && e.N == N && e.K == K && e.max_slices == max_slices && e.nt == (int)nt && e.cus == cus) return e.plan;
+    Entry& e = kept[oldest];
+    oldest = (oldest + 1) % kPlansKept;
+    e = Entry{M, N, K, max_slices, (int)nt, cus, plan_tiles(M, N, K, nt, max_slices, cus)};
+    return e.plan;
+}
+// Slices that a workspace is sized for: the plan's, and no fewer than bring 128 x 128 tiles to one round of the chip (to two while
+// a slice stays 16 steps long), four steps long at least: the size has been that, and callers may keep a workspace by it.
+inline int gemm_slices(int64_t M, int64_t N, int64_t K, bool nt, int cus) {
+    if (K <= 0 || K % kBK != 0 || N % 8 != 0) return 1;
+    int64_t s = 1;
+    const int64_t tiles = tile_count(M, N, 128, 128), kt = K / kBK;
+    if (tiles <= 256 && kt >= 8) {
+        s = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, kt / 4), 32));
+        if (tiles >= 64 && tiles * s <= 256 && kt / (2 * s) >= 16 && (s >= 2 || kt >= 192)) s *= 2;
+    }
+    return std::max((int)s, tile_plan(M, N, K, nt, kMostSlices, cus).slices);
+}
+
+// ---- the dispatch ----------------------------------------------------------------------------------------------
+// Which kernel, and for the sliced ones (stripe_slices, kn_rows, tiles) in how many K slices; `tile` is an index of kGemmTiles.
+enum class GemmKernel { plain, gemv, rows_lds, skinny, stripe, stripe_slices, kn_rows, tiles };
+struct GemmRoute { GemmKernel kernel; int slices, tile; };
+
+// `fast`: sizes, strides and alignment are those of the kernels that move 16-byte pieces and whole K steps.  `fit`: slices of M x N fp32
+// sums that the workspace holds.  `units`: says how many compute units the chip has.
+//
+// A decode step's few tokens against an [N, K] weight: stream the weight once.  Which kernel does that best was
+// measured with the calls cycling over copies of the weight, 640 MiB in all: a weight of up to 256 MiB called again
+// and again is served by the chip's last-level cache, where the order of the kernels is a different one (14336 x
+// 4096 at one row: stripes 18.0 us against 19.5 for whole rows per wave from the cache, 24.2 against 21.9 from memory).
+// These calls are bound by the host: no rule for up to 16 rows asks for a plan of tiles.
+inline GemmRoute gemm_route(int64_t M, int64_t N, int64_t K, bool nt, bool fast, int64_t fit, int (*units)()) {
+    if (!fast) return {GemmKernel::plain, 1, 0};
+    if (nt && M <= 64) {
+        const int64_t stripes = (N + 63) / 64;
+        const bool rows_takes = rows_lds_takes(M, K);
+        // one row: whole weight rows per wave (14336 x 4096: 21.9 us, the 16-column kernel 23.6, stripes 24.2; 28672 x 8192:
+        // 75.8 / 91 / 97); a weight under 32 M values goes to the 16-column kernel when it takes it (4096 x 4096: 8.5 against 10.5)
+        if (M == 1 && K <= kGemvMaxKHalfs && (N * K >= (INT64_C(1) << 25) || !rows_takes)) return {GemmKernel::gemv, 1, 0};
+        // two to four rows against long rows of a wide weight go the same way, every weight piece multiplied with the same
+        // piece of each activation row (28672 x 8192 at 2-4 rows: 78.6-82.6 us against 93-95 for the 16-column kernel, 10240 x
+        // 8192 at 2-3 rows 33.2-34.6 against 36.3; 8192 x 8192 30.5-33.9 against 29.2-29.6, and rows of 4096 values gain nothing)
+        if (M >= 2 && gemv_takes(M, K) && K >= 8192 && N >= 10240 && (M <= 3 || N >= 16384)) return {GemmKernel::gemv, 1, 0};
+        // up to 4 rows (8 where stripe_takes says no) against fewer than 96 stripes, and up to 4 against an output head: the 16-column
+        // kernel (128256 x 4096 at 2-4 rows 166-170 against 176-178; 28672 x 4096 at 2-8 rows 42.2-44.5 against 41.5-41.7 and 14336 x
+        // 4096 24.3-25.8 against 22.8-23.0: those go on)
+        const bool rows_first = rows_takes && ((M <= 8 && stripes < 96 && !stripe_takes(M, stripes, K)) || (M <= 4 && stripes > 640));
+        const int slices = stripe_slices(M, N, K);
+        const bool sliceable = slices > 1 && fit >= slices;
+        // ... except long rows of a narrow weight when a workspace allows K slices: one wave per 16 columns walks a whole row
+        // by itself (1024 x 14336 at 2-8 rows 16.5-20.8 us, in slices 13.1-14.1; 1536 x 8960 15.2-17.4 and 11.8-12.5; 2048 x
+        // 8192 at 5-8 rows 12.5-13.4 and 12.5-12.6, at 2-4 rows and for rows of 6144 values no gain)
+        const bool long_rows_few_stripes = K >= 8192 && ((M >= 5 && stripes <= 32) || (M >= 2 && stripes <= 24));
+        if (rows_first && !(sliceable && long_rows_few_stripes)) return {GemmKernel::rows_lds, 1, 0};
+        // with a workspace, K slices of the stripes, from 9 rows on, where whole rows are not ahead (stripe_blocks_pay): two launches, 10.5
+        // us at least, where one launch over rows of 4096 values takes 8-10 at 9-16 rows: up to 16 rows only for 25 M weight values or
+        // rows of 6144 values and more (2048 x 8192 at 9-16 rows 12.7-13.0 against 13.9-16.5, 1024 x 14336 13.7-14.6 against 21.5-26.7),
+        // from 17 rows on for 8 M values (1536 x 5632 and the like: gemm_skinny_kernel is the other choice)
+        const bool slices_pay = !stripe_blocks_pay(M, stripes, K) && (long_rows_few_stripes || (M >= 9 && (N * K >= INT64_C(25000000) || K >= 6144 || (M >= 17 && N * K >= (INT64_C(1) << 23)))));
+        if (sliceable && slices_pay) return {GemmKernel::stripe_slices, slices, 0};
+        if (stripe_takes(M, stripes, K)) return {GemmKernel::stripe, 1, 0};
+        if (rows_takes) return {GemmKernel::rows_lds, 1, 0};
+        if (M == 1 && K <= kGemvMaxKHalfs) return {GemmKernel::gemv, 1, 0};
+        if (M <= 16) return {GemmKernel::skinny, 1, 0};
+        if ((M <= 32 || N * K <= (INT64_C(1) << 25)) && !(fit > 1 && tile_plan(M, N, K, nt, kMostSlices, units()).slices > 1)) return {GemmKernel::skinny, 1, 0};
+    }
+    if (!nt && M <= kKnRows) {
+        // eight slices at most, 16 for rows of 80 K steps and more: further ones save less streaming than their sums cost (us, as many as fill
+        // the chip / these: 1000 x 4096 at 1 / 9 / 16 rows 10.5 / 7.6, 13.5 / 8.7, 15.5 / 9.4; 2560 x 2560 at 12 10.0 / 8.1; 2048 x 4096 at 40 13.7 /
+        // 11.9; 1024 x 14336 at 9 / 40 15.4 / 12.8, 19.4 / 17.2; 512 x 8192 at 9 17.0 / 9.6; the size reported stays that of filling it)
+        const int kn = kn_slices(M, N, K), most = K >= 80 * kBK ? 16 : 8;   // a smaller workspace: as many slices as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
+        return {GemmKernel::kn_rows, fit < kn ? std::max((int)fit, 1) : std::min(kn, most), 0};
+    }
+    TilePlan plan = tile_plan(M, N, K, nt, kMostSlices, units());
+    if (plan.slices > std::max<int64_t>(fit, 1)) plan = tile_plan(M, N, K, nt, std::max<int64_t>(fit, 1), units());
+    return {GemmKernel::tiles, plan.slices, plan.tile};
+}
+
+}  // namespace minfer_attn

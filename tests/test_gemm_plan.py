@@ -1,0 +1,95 @@
+"""The rules of the GEMM dispatch (csrc/gemm_plan.h), compiled for the host: which kernel takes a call, when a plan of tiles is
+estimated and how often."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+import capi
+
+PLAIN, GEMV, ROWS_LDS, SKINNY, STRIPE, STRIPE_SLICES, KN_ROWS, TILES = range(8)   # enum GemmKernel
+KN, NK = False, True
+
+PROBE = """
+#include <math.h>
+#include <algorithm>
+static long estimates = 0;
+static double counting_sqrt(double x) { ++estimates; return sqrt(x); }
+#define sqrt counting_sqrt                      // plan_cost takes one square root
+#include "gemm_plan.h"
+using namespace minfer_attn;
+extern "C" void route(int64_t M, int64_t N, int64_t K, int nt, int fast, int64_t fit, int* out) {
+    const GemmRoute r = gemm_route(M, N, K, nt, fast, fit, []() { return 256; });
+    const GemmTile& t = kGemmTiles[r.tile];
+    const int v[] = {(int)r.kernel, r.slices, 32 * t.m16, 32 * t.n16, t.occ};
+    std::copy(v, v + 5, out);
+}
+extern "C" int grouped_tile(int64_t M, int64_t N, int64_t K) { return tile_plan(M, N, K, true, 1, 256).tile; }
+extern "C" long estimates_made() { return estimates; }
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    tmp = tmp_path_factory.mktemp("plan")
+    (tmp / "probe.cpp").write_text(PROBE)
+    so = tmp / "probe.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", os.path.join(capi.ROOT, "minfer-python_amd", "csrc"),
+                    str(tmp / "probe.cpp"), "-o", str(so)], check=True)
+    L = ctypes.CDLL(str(so))
+    i64 = ctypes.c_int64
+    L.route.argtypes = [i64, i64, i64, ctypes.c_int, ctypes.c_int, i64, ctypes.POINTER(ctypes.c_int)]
+    L.grouped_tile.argtypes = [i64, i64, i64]
+    L.estimates_made.restype = ctypes.c_long
+
+    def route(M, N, K, nt, fit=0, fast=True):
+        """(kernel, slices, rows of a tile, its columns, workgroups of it to a unit)"""
+        out = (ctypes.c_int * 5)()
+        L.route(M, N, K, nt, fast, fit, out)
+        return tuple(out)
+    route.grouped_tile, route.estimates = L.grouped_tile, L.estimates_made
+    return route
+
+
+# (out, in) of the projections of a layer: q, k and v fused, output, gate and up, down; and the sizes of a narrower model
+LAYERS = [[(6144, 4096), (4096, 4096), (28672, 4096), (14336, 4096), (4096, 14336)], [(10240, 8192), (8192, 8192), (57344, 8192), (8192, 28672)],
+          [(2048, 1536), (1536, 1536), (17920, 1536), (8960, 1536), (1536, 8960)]]
+
+
+@pytest.mark.parametrize("M", [65, 100, 200, 600, 1777, 4096])
+@pytest.mark.parametrize("layer", LAYERS)
+def test_the_projections_of_a_layer_keep_their_plans(plan, layer, M):
+    """The second walk through a layer estimates nothing, with weights of either layout, a workspace or none, and the grouped projection."""
+    def walk():
+        for N, K in layer:
+            for nt in (KN, NK):
+                plan(M, N, K, nt, 64)
+        plan.grouped_tile(M, layer[0][0], layer[0][1])
+    walk()
+    before = plan.estimates()
+    walk()
+    assert plan.estimates() == before
+
+
+def test_a_call_with_a_smaller_workspace_keeps_its_plan(plan):
+    assert plan(100, 4096, 14336, NK, 64)[1] > 2
+    plan(100, 4096, 14336, NK, 2)
+    before = plan.estimates()
+    assert plan(100, 4096, 14336, NK, 2)[1] <= 2 and plan(100, 4096, 14336, NK, 64)[1] > 2
+    assert plan.estimates() == before
+
+
+def test_few_rows_need_no_plan_of_tiles(plan):
+    """Up to 16 rows of an [N, K] weight, up to 64 of a [K, N] weight, and up to 64 where K is whole segments of the stripe kernel."""
+    before = plan.estimates()
+    for fit in (0, 1, 2, 64):
+        for N, K in [s for layer in LAYERS for s in layer] + [(1000, 4160), (264, 16448), (128256, 4096), (512, 64)]:
+            for M in (1, 2, 5, 16):
+                assert plan(M, N, K, NK, fit)[0] not in (TILES, PLAIN)
+            for M in (1, 16, 17, 64):
+                assert plan(M, N, K, KN, fit)[0] == KN_ROWS
+            if K % 256 == 0 and N >= 6144:
+                for M in (17, 40, 64):
+                    assert plan(M, N, K, NK, fit)[0] in (STRIPE, STRIPE_SLICES)
+    assert plan.estimates() == before
