@@ -1475,9 +1475,9 @@ MINFER_ATTN_EXPORT int minfer_gemm(int dtype, int b_layout, const void* A, const
 
 MINFER_ATTN_EXPORT size_t minfer_gemm_layout_workspace_bytes(int b_layout, int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || N > 0x7fffffffLL || K > 0x7fffffffLL) return 0;
-    int splits;   // the most slices that a route of gemm_impl cuts K into for this layout
-    if (b_layout == MINFER_GEMM_B_KN) splits = M <= kKnRows ? kn_slices(M, N, K) : gemm_slices(M, N, K, false, compute_units());
-    else splits = std::max(stripe_slices(M, N, K), M > 16 ? gemm_slices(M, N, K, true, compute_units()) : 1);
+    // what gemm_route cuts K into for this layout when it has all the room it wants (sizes the tiled kernels take; others use none)
+    const bool fast = K % kBK == 0 && N % 8 == 0;
+    const int splits = gemm_route(M, N, K, b_layout != MINFER_GEMM_B_KN, fast, 2 * kMostSlices, compute_units).slices;
     return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
@@ -1526,7 +1526,8 @@ MINFER_ATTN_EXPORT size_t minfer_gemm_q8_0_workspace_bytes(int64_t M, int64_t N,
         const int slices = q8_slices(M, N, K);
         return slices > 1 ? (size_t)slices * (size_t)M * (size_t)N * sizeof(float) : 0;
     }
-    return q8_dequant_bytes(N, K) + minfer_gemm_layout_workspace_bytes(MINFER_GEMM_B_NK, M, N, K);
+    const int slices = std::max(stripe_slices(M, N, K), M > 16 ? gemm_slices(M, N, K, true, compute_units()) : 1);   // (the size has been that)
+    return q8_dequant_bytes(N, K) + (slices > 1 ? (size_t)slices * (size_t)M * (size_t)N * sizeof(float) : 0);
 }
 
 MINFER_ATTN_EXPORT int minfer_gemm_q8_0(const void* A, const void* Bq, const void* C, void* D, int64_t M, int64_t N, int64_t K,

@@ -93,3 +93,26 @@ def test_few_rows_need_no_plan_of_tiles(plan):
                 for M in (17, 40, 64):
                     assert plan(M, N, K, NK, fit)[0] in (STRIPE, STRIPE_SLICES)
     assert plan.estimates() == before
+
+
+def layout_slices(layout, M, N, K):
+    need = capi.lib().minfer_gemm_layout_workspace_bytes(layout, M, N, K)
+    assert need % (4 * M * N) == 0
+    return need // (4 * M * N)
+
+
+def test_workspace_of_a_layout_is_what_its_route_uses(plan):
+    """minfer_gemm_layout_workspace_bytes: no less than a call can use, and no more."""
+    # whole rows of an [N, K] weight: from 96 stripes of 64 columns on always, and where stripe_blocks_pay says so
+    for M, N, K in ((40, 8192, 2048), (64, 6144, 4096), (9, 12280, 8192), (64, 4096, 4096), (24, 2048, 4096)):
+        assert layout_slices(capi.GEMM_B_NK, M, N, K) == 0
+    # a [K, N] weight: eight slices, or sixteen of long rows, however many would fill the chip
+    assert layout_slices(capi.GEMM_B_KN, 9, 1000, 4096) == 8 and layout_slices(capi.GEMM_B_KN, 9, 1000, 8192) == 16
+    for M in (1, 3, 9, 16, 17, 40, 64, 65, 100, 300, 600, 1777):
+        for N in (8, 520, 1000, 1536, 4096, 4104, 6144, 8192, 14336):
+            for K in (64, 256, 512, 1984, 4096, 4160, 8192, 8960, 14336):
+                for layout, nt in ((capi.GEMM_B_KN, KN), (capi.GEMM_B_NK, NK)):
+                    slices = layout_slices(layout, M, N, K)
+                    assert slices * 4 * M * N <= capi.lib().minfer_gemm_workspace_bytes(M, N, K)
+                    best = plan(M, N, K, nt, 64)
+                    assert plan(M, N, K, nt, slices) == best and best[1] == max(slices, 1), (M, N, K, layout)
