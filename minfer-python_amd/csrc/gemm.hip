@@ -891,7 +891,6 @@ constexpr int kGemvWaves = 4;
 constexpr int kGemvSegBlocks = 128;                       // blocks per segment: two per lane
 constexpr int kGemvSegBytes = kGemvSegBlocks * 34;        // 4352
 constexpr int kGemvPieces = (kGemvSegBytes + 1023) / 1024;   // 16-byte pieces per lane and segment (5, the last one partly)
-constexpr int kGemvMaxK = 16384;                          // activation row kept in LDS: 32 KiB
 template <bool XREG>
 __global__ __launch_bounds__(kGemvWaves * 64) void gemv_q8_kernel(const GemmParams p, int rows_per_wave) {
     using T = F16;
@@ -980,10 +979,6 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_q8_kernel(const GemmPara
     }
 }
 
-// which calls the row-streaming kernel takes: one row, whole segments of 16-byte pieces, an activation row that fits its LDS area
-static bool q8_gemv_ok(int64_t M, int64_t K, const void* Bq, int64_t row_bytes) {
-    return M == 1 && K % 256 == 0 && K <= kGemvMaxK && aligned16(Bq) && row_bytes % 16 == 0;
-}
 static int launch_gemv_q8(const GemmParams& p, hipStream_t stream) {
     // as many waves as the chip holds at a time when there are rows enough for them: two workgroups per compute unit
     const int max_waves = 256 * 2 * kGemvWaves;
@@ -1166,40 +1161,6 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams
         __shared__ int last_s;
         finish_slices<T, 4 * 64>(p, (int)blockIdx.x / p.splits, 0, p.M, 16 * blk_first, min(16 * blk_last, p.N), &last_s);
     }
-}
-// Which calls it takes: 2-64 rows, whole segments of 8 blocks, rows that start on 16-byte boundaries, and a weight wide
-// enough for two and a half blocks per workgroup, or two from 16 rows, or one and a half above 32 (weights coming from memory:
-// 14336 x 4096 at 2-16 rows 16.7-16.9 us against 20.8-26.8 for gemm_skinny_q8_kernel, 64 rows 23.4 against 50.9; 28672 x
-// 4096 29.7-43.4 against 36.8-97.7), or q8_blocks_pay.  Chunks of as many blocks as a workgroup has, as for the 16-bit weights (11008 x 4096
-// at 2 / 24 / 64 rows 15.4 -> 13.3, 18.4 -> 15.6, 23.3 -> 20.6; 18944 x 3584 at 2 / 40 rows 25.6 -> 21.6, 34.1 -> 31.3): all of a
-// chunk's blocks are dequantised and multiplied, there or not (skipping the missing ones of four by a branch cost the full chunks a
-// third).
-// Where it is ahead of its K slices and of gemm_skinny_q8_kernel on a weight of fewer than 192 stripes: rows of up to 4096 values, by the rows a
-// unit copies, (NB + MB) x 16 of K values (us, the other / it: 8192 x 4096 at 2 / 16 / 32 rows 11.8 / 11.0, 12.7 / 11.1, 14.9 / 12.8;
-// 6144 x 4096 at 16 / 24 / 40 rows 12.3 / 11.0, 14.1 / 12.1, 15.2 / 15.4; 6144 x 2048 at 16 rows 9.1 / 6.7; 5120 x 4096 at 24 / 40 12.6 /
-// 12.0, 14.0 / 15.1; 4096 x 4096 at 16 / 64 9.7 / 8.2, 13.9 / 13.2; 4096 x 2048 at 8 / 16 / 64 5.4 / 5.9, 8.7 / 5.5, 11.7 / 8.6; 2048 x 4096
-// at 16 / 24 / 40 8.8 / 8.0, 9.9 / 9.6, 10.7 / 11.2; 5120 x 5120 at 16 rows 12.1 / 12.7).
-// K slices of it for a weight of fewer than 192 stripes when a workspace is given (1 = none): 256 / stripes workgroups
-// per chunk of four blocks, full chunks whatever the width (weights coming from memory: 4096 x 14336 at 16 / 32 / 64 rows
-// 19.0 / 21.8 / 26.4 us against 29.6 / 43.0 / 68.4 for gemm_skinny_q8_kernel, 8192 x 8192 at 2-64 rows 19.6-28.5 against
-// 23.7-40.3, 6144 x 4096 12.4-17.7 against 12.7-22.2; 4096 x 4096 up to 8 rows 10.2 against 7.7-8.3: two launches, so a
-// weight of 16 M values or fewer only from 16 rows on, or from 8 when its rows are 6144 values and longer, or from 2
-// when they are 8192 values and longer and the stripes 24 at most, as for the 16-bit weights).
-static bool q8_blocks_pay(int64_t M, int64_t N, int64_t K) {
-    const int64_t stripes = (N + 63) / 64, rows = (stripes > 64 ? 2 : 1) + (M + 15) / 16;
-    if (K > 4096 || M < 2 || M > 64 || stripes < 32 || stripes >= 192) return false;
-    if (stripes >= 96) return rows * K <= 17000 && (M >= 8 || N * K >= INT64_C(20000000));
-    return M >= 16 && rows * K <= (stripes < 64 ? 12500 : stripes == 64 ? 20500 : 17000);
-}
-static int q8_slices(int64_t M, int64_t N, int64_t K) {
-    if (M < 2 || M > 64 || K % kStripeSeg != 0 || N % 8 != 0) return 1;
-    const bool long_rows = (K >= 6144 && M >= 8) || (K >= 8192 && N <= 24 * 64);
-    if (N * K <= (INT64_C(1) << 24) && M < 16 && !long_rows) return 1;
-    return stripe_slices(M, N, K);
-}
-static bool q8_stripe_ok(int64_t M, int64_t N, int64_t K, const void* Bq, int64_t row_bytes) {
-    return M >= 2 && M <= 64 && K % kStripeSeg == 0 && aligned16(Bq) && row_bytes % 16 == 0 &&
-           (N >= 10240 || (N >= 8192 && M >= 16) || (N >= 6144 && M > 32) || q8_blocks_pay(M, N, K));
 }
 template <int MB, bool SLICED>
 static void launch_stripe_q8_rows(const GemmParams& p, int most, dim3 grid, hipStream_t stream) {   // (NB as in launch_stripe_rows)
@@ -1495,29 +1456,13 @@ MINFER_ATTN_EXPORT int minfer_gemm_ws(int dtype, int b_layout, const void* A, co
 }
 
 // ---- weights stored as Q8_0 blocks ------------------------------------------------------------------------------
-constexpr int64_t kQ8SkinnyRows = 64;    // up to here the kernel that streams the blocks; above, dequantise once and run the tiles
-
 static size_t q8_dequant_bytes(int64_t N, int64_t K) { return ((size_t)N * (size_t)K * 2 + 255) & ~(size_t)255; }
 
-// the streaming kernel takes up to 64 rows, needs weight rows that are multiples of 4 bytes (an even number of blocks)
-// and stores 8-byte pieces of D (N a multiple of 4); every other shape goes through the dequantised weight
-static bool q8_streams(int64_t M, int64_t N, int64_t K) { return M <= kQ8SkinnyRows && (K / 32) % 2 == 0 && N % 4 == 0; }
-// ... and it reads 16-byte pieces of A and aligned 8-byte pieces of C (only when beta != 0) and D
+// What the kernels that stream the blocks (q8_streams) need besides: 16-byte pieces of A, aligned 8-byte pieces of C (only when beta != 0)
+// and D.
 static bool q8_stream_operands(const void* A, const void* C, const void* D, int64_t lda, int64_t ldc, int64_t ldd, double beta) {
     return aligned16(A) && lda % 8 == 0 && ldd % 4 == 0 && ((uintptr_t)D & 7u) == 0 &&
            (beta == 0.0 || (ldc % 4 == 0 && ((uintptr_t)C & 7u) == 0));
-}
-
-// More rows than the kernels that stream the blocks take: in how many calls of theirs a product goes all the same (1: none, the
-// weight is dequantised).  Dequantising writes and reads back twice the blocks' bytes; a second call reads the blocks again,
-// from the last-level cache mostly (us, weights from memory, dequantised / in parts): 65 rows x 14336 x 4096 64.0 / 39.4, 4096 x 14336
-// 61.7 / 42.3, 128256 x 4096 488 / 288, 6144 x 4096 32.8 / 28.6, 4096 x 4096 24.4 / 21.8; 128 rows 72.1 / 46.3, 70.3 / 49.7, 496 / 337,
-// 37.3 / 34.8, 26.3 / 27.0; 160 rows in three 76.2 / 64.9, 73.9 / 69.8, 507 / 483, 40.4 / 48.1; 192 28672 x 4096 124 / 128.
-static int64_t q8_parts(int64_t M, int64_t N, int64_t K, const void* Bq) {
-    if (M <= kQ8SkinnyRows || M > 160 || N * K < (M <= 96 ? INT64_C(16000000) : M <= 128 ? INT64_C(20000000) : INT64_C(50000000))) return 1;
-    const int64_t parts = (M + kQ8SkinnyRows - 1) / kQ8SkinnyRows, rows = M / parts, row_bytes = K / 32 * 34;
-    const bool stripes = q8_stripe_ok(rows, N, K, Bq, row_bytes) || (aligned16(Bq) && row_bytes % 16 == 0 && q8_slices(rows, N, K) > 1);
-    return stripes ? parts : 1;
 }
 
 MINFER_ATTN_EXPORT size_t minfer_gemm_q8_0_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -1548,23 +1493,23 @@ MINFER_ATTN_EXPORT int minfer_gemm_q8_0(const void* A, const void* Bq, const voi
         GemmParams p{};
         p.A = A; p.B = Bq; p.C = beta != 0.0 ? C : nullptr; p.D = D; p.M = (int)M; p.N = (int)N; p.K = (int)K;
         p.lda = lda; p.ldb = row_bytes; p.ldc = ldc; p.ldd = ldd; p.alpha = (float)alpha; p.beta = (float)beta;
-        if (q8_gemv_ok(M, K, Bq, row_bytes)) return launch_gemv_q8(p, stream);
-        const int slices = aligned16(Bq) && row_bytes % 16 == 0 && !q8_blocks_pay(M, N, K) ? q8_slices(M, N, K) : 1;
-        if (slices > 1 && workspace && aligned16(workspace) && workspace_bytes >= (size_t)slices * (size_t)M * (size_t)N * sizeof(float)) {
-            p.splits = slices; p.part = (float*)workspace;
-            return launch_stripe_q8_slices(p, stream);
+        const size_t fit = workspace && aligned16(workspace) ? workspace_bytes / ((size_t)M * (size_t)N * sizeof(float)) : 0;
+        const Q8Route route = q8_route(M, N, K, aligned16(Bq), (int64_t)std::min<size_t>(fit, kMostSlices));
+        p.splits = route.slices; p.part = (float*)workspace;
+        switch (route.kernel) {
+            case Q8Kernel::gemv: return launch_gemv_q8(p, stream);
+            case Q8Kernel::stripe_slices: return launch_stripe_q8_slices(p, stream);
+            case Q8Kernel::stripe: return launch_stripe_q8(p, stream);
+            case Q8Kernel::skinny: return launch_skinny_q8(p, stream);
         }
-        if (q8_stripe_ok(M, N, K, Bq, row_bytes)) return launch_stripe_q8(p, stream);
-        return launch_skinny_q8(p, stream);
     }
-    // otherwise: the weight as fp16 in the workspace, then the fp16 kernels on it, or the call in parts (q8_parts)
+    // otherwise: the weight as fp16 in the workspace, then the fp16 kernels on it, or the call in parts (q8_part_rows)
     const size_t deq = q8_dequant_bytes(N, K);
     if (!workspace || !aligned16(workspace) || workspace_bytes < deq)
         return fail(MINFER_ATTN_EWORKSPACE, "gemm_q8_0: this call needs a workspace of N*K*2 bytes (rounded up to 256) for the dequantised weight "
                                             "(more than 64 rows, an odd number of blocks per row, N not a multiple of 4, or A/C/D not aligned for the streaming kernel: "
                                             "A 16 bytes with lda a multiple of 8, C and D 8 bytes with strides multiples of 4)");
-    if (const int64_t parts = q8_parts(M, N, K, Bq); parts > 1 && q8_stream_operands(A, C, D, lda, ldc, ldd, beta)) {
-        const int64_t rows = ((M + parts - 1) / parts + 15) / 16 * 16;
+    if (const int64_t rows = q8_part_rows(M, N, K, aligned16(Bq)); rows < M && q8_stream_operands(A, C, D, lda, ldc, ldd, beta)) {
         for (int64_t m = 0; m < M; m += rows)
             if (int rc = minfer_gemm_q8_0((const short*)A + m * lda, Bq, C ? (const short*)C + m * ldc : nullptr, (short*)D + m * ldd, std::min(rows, M - m), N, K,
                                           lda, ldc, ldd, alpha, beta, workspace, workspace_bytes, stream_v)) return rc;

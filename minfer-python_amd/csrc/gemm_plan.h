@@ -207,4 +207,76 @@ inline GemmRoute gemm_route(int64_t M, int64_t N, int64_t K, bool nt, bool fast,
     return {GemmKernel::tiles, plan.slices, plan.tile};
 }
 
+// ---- weights stored as Q8_0 blocks -----------------------------------------------------------------------------
+constexpr int64_t kQ8SkinnyRows = 64;       // up to here the kernels that stream the blocks; above, dequantise once and run the tiles
+constexpr int kGemvMaxK = 16384;            // the longest activation row that gemv_q8_kernel keeps in LDS: 32 KiB
+
+// the streaming kernel takes up to 64 rows, needs weight rows that are multiples of 4 bytes (an even number of blocks)
+// and stores 8-byte pieces of D (N a multiple of 4); every other shape goes through the dequantised weight
+inline bool q8_streams(int64_t M, int64_t N, int64_t K) { return M <= kQ8SkinnyRows && (K / 32) % 2 == 0 && N % 4 == 0; }
+// gemm_stripe_q8_kernel.  Which calls it takes: 2-64 rows, whole segments of 8 blocks, rows that start on 16-byte boundaries, and a weight wide
+// enough for two and a half blocks per workgroup, or two from 16 rows, or one and a half above 32 (weights coming from memory:
+// 14336 x 4096 at 2-16 rows 16.7-16.9 us against 20.8-26.8 for gemm_skinny_q8_kernel, 64 rows 23.4 against 50.9; 28672 x
+// 4096 29.7-43.4 against 36.8-97.7), or q8_blocks_pay.  Chunks of as many blocks as a workgroup has, as for the 16-bit weights (11008 x 4096
+// at 2 / 24 / 64 rows 15.4 -> 13.3, 18.4 -> 15.6, 23.3 -> 20.6; 18944 x 3584 at 2 / 40 rows 25.6 -> 21.6, 34.1 -> 31.3): all of a
+// chunk's blocks are dequantised and multiplied, there or not (skipping the missing ones of four by a branch cost the full chunks a
+// third).
+// Where it is ahead of its K slices and of gemm_skinny_q8_kernel on a weight of fewer than 192 stripes: rows of up to 4096 values, by the rows a
+// unit copies, (NB + MB) x 16 of K values (us, the other / it: 8192 x 4096 at 2 / 16 / 32 rows 11.8 / 11.0, 12.7 / 11.1, 14.9 / 12.8;
+// 6144 x 4096 at 16 / 24 / 40 rows 12.3 / 11.0, 14.1 / 12.1, 15.2 / 15.4; 6144 x 2048 at 16 rows 9.1 / 6.7; 5120 x 4096 at 24 / 40 12.6 /
+// 12.0, 14.0 / 15.1; 4096 x 4096 at 16 / 64 9.7 / 8.2, 13.9 / 13.2; 4096 x 2048 at 8 / 16 / 64 5.4 / 5.9, 8.7 / 5.5, 11.7 / 8.6; 2048 x 4096
+// at 16 / 24 / 40 8.8 / 8.0, 9.9 / 9.6, 10.7 / 11.2; 5120 x 5120 at 16 rows 12.1 / 12.7).
+// K slices of it for a weight of fewer than 192 stripes when a workspace is given (1 = none): 256 / stripes workgroups
+// per chunk of four blocks, full chunks whatever the width (weights coming from memory: 4096 x 14336 at 16 / 32 / 64 rows
+// 19.0 / 21.8 / 26.4 us against 29.6 / 43.0 / 68.4 for gemm_skinny_q8_kernel, 8192 x 8192 at 2-64 rows 19.6-28.5 against
+// 23.7-40.3, 6144 x 4096 12.4-17.7 against 12.7-22.2; 4096 x 4096 up to 8 rows 10.2 against 7.7-8.3: two launches, so a
+// weight of 16 M values or fewer only from 16 rows on, or from 8 when its rows are 6144 values and longer, or from 2
+// when they are 8192 values and longer and the stripes 24 at most, as for the 16-bit weights).
+inline bool q8_blocks_pay(int64_t M, int64_t N, int64_t K) {
+    const int64_t stripes = (N + 63) / 64, rows = (stripes > 64 ? 2 : 1) + (M + 15) / 16;
+    if (K > 4096 || M < 2 || M > 64 || stripes < 32 || stripes >= 192) return false;
+    if (stripes >= 96) return rows * K <= 17000 && (M >= 8 || N * K >= INT64_C(20000000));
+    return M >= 16 && rows * K <= (stripes < 64 ? 12500 : stripes == 64 ? 20500 : 17000);
+}
+inline int q8_slices(int64_t M, int64_t N, int64_t K) {
+    if (M < 2 || M > 64 || K % kStripeSeg != 0 || N % 8 != 0) return 1;
+    const bool long_rows = (K >= 6144 && M >= 8) || (K >= 8192 && N <= 24 * 64);
+    if (N * K <= (INT64_C(1) << 24) && M < 16 && !long_rows) return 1;
+    return stripe_slices(M, N, K);
+}
+inline bool q8_stripe_ok(int64_t M, int64_t N, int64_t K, bool aligned) {
+    return M >= 2 && M <= 64 && K % kStripeSeg == 0 && aligned &&
+           (N >= 10240 || (N >= 8192 && M >= 16) || (N >= 6144 && M > 32) || q8_blocks_pay(M, N, K));
+}
+
+// Which of the kernels that stream the blocks takes a call that q8_streams.  `aligned`: the weight starts on a 16-byte boundary (its rows
+// of whole segments, 272 bytes each, then do too); `fit` as in gemm_route.
+enum class Q8Kernel { gemv, stripe, stripe_slices, skinny };
+struct Q8Route { Q8Kernel kernel; int slices; };
+inline Q8Route q8_route(int64_t M, int64_t N, int64_t K, bool aligned, int64_t fit) {
+    // one row of whole segments: whole weight rows per wave
+    if (M == 1 && K % 256 == 0 && K <= kGemvMaxK && aligned) return {Q8Kernel::gemv, 1};
+    const int slices = aligned && !q8_blocks_pay(M, N, K) ? q8_slices(M, N, K) : 1;
+    if (slices > 1 && fit >= slices) return {Q8Kernel::stripe_slices, slices};
+    return {q8_stripe_ok(M, N, K, aligned) ? Q8Kernel::stripe : Q8Kernel::skinny, 1};
+}
+
+// More rows than the kernels that stream the blocks take: the rows of each of the calls of theirs in which a product goes all
+// the same (the last one takes what remains; M: none, the weight is dequantised).  Dequantising writes and reads back twice the blocks' bytes; a second call reads the blocks again,
+// from the last-level cache mostly (us, weights from memory, dequantised / in parts): 65 rows x 14336 x 4096 64.0 / 39.4, 4096 x 14336
+// 61.7 / 42.3, 128256 x 4096 488 / 288, 6144 x 4096 32.8 / 28.6, 4096 x 4096 24.4 / 21.8; 128 rows 72.1 / 46.3, 70.3 / 49.7, 496 / 337,
+// 37.3 / 34.8, 26.3 / 27.0; 160 rows in three 76.2 / 64.9, 73.9 / 69.8, 507 / 483, 40.4 / 48.1; 192 28672 x 4096 124 / 128.
+// Judged by the parts as they run, the shorter last one too: every one has to be a product that a kernel streams (a part that is not
+// dequantises the weight by itself), and the stripe kernels have to take it, or else the dequantised weight is one that
+// the tiled kernel does not take (N no multiple of 8: 65 x 4100 x 4096 3645 us, in parts through gemm_skinny_q8_kernel 40).
+inline int64_t q8_part_rows(int64_t M, int64_t N, int64_t K, bool aligned) {
+    if (M <= kQ8SkinnyRows || M > 160 || N * K < (M <= 96 ? INT64_C(16000000) : M <= 128 ? INT64_C(20000000) : INT64_C(50000000))) return M;
+    const int64_t parts = (M + kQ8SkinnyRows - 1) / kQ8SkinnyRows, rows = ((M + parts - 1) / parts + 15) / 16 * 16;
+    for (const int64_t r : {rows, M - (parts - 1) * rows}) {
+        // (the room of the dequantised weight holds the slices of a part)
+        if (!q8_streams(r, N, K) || (N % 8 == 0 && q8_route(r, N, K, aligned, kMostSlices).kernel == Q8Kernel::skinny)) return M;
+    }
+    return rows;
+}
+
 }  // namespace minfer_attn

@@ -25,6 +25,8 @@ extern "C" void route(int64_t M, int64_t N, int64_t K, int nt, int fast, int64_t
     const int v[] = {(int)r.kernel, r.slices, 32 * t.m16, 32 * t.n16, t.occ};
     std::copy(v, v + 5, out);
 }
+extern "C" int q8_kernel(int64_t M, int64_t N, int64_t K, int aligned, int64_t fit) { return (int)q8_route(M, N, K, aligned, fit).kernel; }
+extern "C" int64_t q8_rows_of_a_part(int64_t M, int64_t N, int64_t K, int aligned) { return q8_part_rows(M, N, K, aligned); }
 extern "C" int grouped_tile(int64_t M, int64_t N, int64_t K) { return tile_plan(M, N, K, true, 1, 256).tile; }
 extern "C" long estimates_made() { return estimates; }
 """
@@ -42,6 +44,8 @@ def plan(tmp_path_factory):
     L.route.argtypes = [i64, i64, i64, ctypes.c_int, ctypes.c_int, i64, ctypes.POINTER(ctypes.c_int)]
     L.grouped_tile.argtypes = [i64, i64, i64]
     L.estimates_made.restype = ctypes.c_long
+    L.q8_kernel.argtypes = [i64, i64, i64, ctypes.c_int, i64]
+    L.q8_rows_of_a_part.restype, L.q8_rows_of_a_part.argtypes = i64, [i64, i64, i64, ctypes.c_int]
 
     def route(M, N, K, nt, fit=0, fast=True):
         """(kernel, slices, rows of a tile, its columns, workgroups of it to a unit)"""
@@ -49,6 +53,7 @@ def plan(tmp_path_factory):
         L.route(M, N, K, nt, fast, fit, out)
         return tuple(out)
     route.grouped_tile, route.estimates = L.grouped_tile, L.estimates_made
+    route.q8_kernel, route.q8_part_rows = L.q8_kernel, L.q8_rows_of_a_part
     return route
 
 
@@ -116,3 +121,28 @@ def test_workspace_of_a_layout_is_what_its_route_uses(plan):
                     assert slices * 4 * M * N <= capi.lib().minfer_gemm_workspace_bytes(M, N, K)
                     best = plan(M, N, K, nt, 64)
                     assert plan(M, N, K, nt, slices) == best and best[1] == max(slices, 1), (M, N, K, layout)
+
+
+Q8_GEMV, Q8_STRIPE, Q8_STRIPE_SLICES, Q8_SKINNY = range(4)   # enum Q8Kernel
+
+
+def test_parts_of_a_q8_0_product_are_streamed(plan):
+    """65 to 160 rows against a large Q8_0 weight: whatever goes in parts, every part as it runs is a product that a kernel streams, one of
+    the stripe kernels wherever the tiled kernel could take the dequantised weight."""
+    assert plan.q8_part_rows(65, 14336, 4096, 1) == 48 and plan.q8_part_rows(160, 14336, 4096, 1) == 64
+    assert plan.q8_part_rows(64, 14336, 4096, 1) == 64 and plan.q8_part_rows(161, 14336, 4096, 1) == 161   # whole
+    assert plan.q8_part_rows(65, 10246, 4096, 1) == 65      # a width that no kernel streams: dequantised once, not once a part
+    assert plan.q8_part_rows(65, 14336, 4096, 0) == 65      # a weight off the 16-byte boundaries
+    assert plan.q8_part_rows(96, 4100, 4096, 1) == 48       # streamed, and no width for the tiled kernel
+    in_parts = 0
+    for M in range(65, 161):
+        for N in (1024, 1536, 2048, 3000, 4096, 4100, 4104, 5120, 6144, 6146, 8192, 8196, 10240, 10244, 14336, 28672, 128256):
+            for K in (1024, 2048, 4096, 4160, 8192, 8960, 14336):
+                rows = plan.q8_part_rows(M, N, K, 1)
+                room = N * K * 2
+                for m in range(0, M, rows) if rows < M else ():
+                    r = min(rows, M - m)
+                    assert N % 4 == 0 and (K // 32) % 2 == 0, (M, N, K, r)
+                    assert N % 8 != 0 or plan.q8_kernel(r, N, K, 1, room // (r * N * 4)) in (Q8_STRIPE, Q8_STRIPE_SLICES), (M, N, K, r)
+                    in_parts += 1
+    assert in_parts > 5000

@@ -582,6 +582,8 @@ def test_gemm_q8_0_weights_against_oracle(M, N, K, alpha, beta):
     (113, 10248, 2048, 1.0, 1.0),    # 64 and 49
     (128, 6152, 4096, 0.5, 0.0),
     (130, 12296, 4352, 1.0, 1.0),    # 48, 48 and 34
+    (96, 4100, 4096, 2.0, 1.0),      # 48 and 48 where the dequantised weight is no width for the tiled kernel
+    (65, 4100, 4160, 1.0, 0.0),      # ... and K is no whole segments
 ])
 def test_gemm_q8_0_in_parts(M, N, K, alpha, beta):
     """65 to 160 rows against a large weight go through the block-streaming kernels in parts: every element against torch's product
