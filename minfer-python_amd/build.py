@@ -38,18 +38,35 @@ def asm_hazards(asm_text):
     """Distances the compiler cannot keep because one end is inside an asm statement, looked for in the device code:
     (1) a global->LDS copy (always emitted from asm here) whose scalar address pair was written by a vector instruction
         (readfirstlane / readlane) fewer than five instructions earlier;
-    (2) a matrix instruction that reads a register written inside an asm statement fewer than two instructions earlier;
+    (2) a matrix instruction that reads a register (an operand's or its accumulator's) written inside an asm statement fewer than
+        two issue slots earlier, or, when the matrix instruction is itself inside one, written by any vector instruction
+        that close in front of it;
     (3) an instruction outside asm statements that touches an accumulation register fewer than 18 issue slots after a matrix
         instruction inside one wrote it (16x16x32: 11 are needed).
     Returns a list of (function, offending instruction, the write it follows too closely)."""
     import re
     found, func, window, in_asm = [], "?", [], False
 
+    def regs(text, bank):
+        out = set()
+        for m in re.finditer(r"\b%s(?:\[(\d+):(\d+)\]|(\d+)\b)" % bank, text):
+            out.update((bank, r) for r in (range(int(m.group(1)), int(m.group(2)) + 1) if m.group(1) else (int(m.group(3)),)))
+        return out
+
     def acc_regs(text):
-        regs = set()
-        for m in re.finditer(r"\ba(?:\[(\d+):(\d+)\]|(\d+)\b)", text):
-            regs.update(range(int(m.group(1)), int(m.group(2)) + 1) if m.group(1) else (int(m.group(3)),))
-        return regs
+        return regs(text, "a")
+
+    def vector_regs(text):
+        return regs(text, "v") | regs(text, "a")
+
+    def written(text):
+        operands = text.split(None, 1)[1] if len(text.split()) > 1 else ""
+        return vector_regs(operands if "swap" in text.split()[0] else operands.split(",", 1)[0])
+
+    def issue_slots(text):   # s_nop N fills N + 1
+        n = re.match(r"s_nop (\d+)", text)
+        return int(n.group(1)) + 1 if n else 1
+
     for raw in asm_text.split("\n"):
         line = raw.strip()
         if line.startswith(";;#ASMSTART"):
@@ -72,27 +89,23 @@ def asm_hazards(asm_text):
             m = re.search(r"s\[(\d+):(\d+)\]", line)
             if m:
                 pair = {int(m.group(1)), int(m.group(2))}
-                states = 0   # issue slots between the write and this instruction: s_nop N fills N + 1
+                states = 0   # issue slots between the write and this instruction
                 for prev, _ in reversed(window):
                     if states >= 5:
                         break
                     w = re.match(r"v_read(?:first)?lane_b32 s(\d+)", prev)
                     if w and int(w.group(1)) in pair:
                         found.append((func, line, prev))
-                    n = re.match(r"s_nop (\d+)", prev)
-                    states += int(n.group(1)) + 1 if n else 1
+                    states += issue_slots(prev)
         elif op.startswith("v_mfma"):
-            srcs = set()
-            for m in re.finditer(r"v\[(\d+):(\d+)\]", line.split(",", 1)[1] if "," in line else ""):
-                srcs.update(range(int(m.group(1)), int(m.group(2)) + 1))
-            for prev, prev_in_asm in window[-2:]:
-                if prev_in_asm and prev.startswith("v_"):
-                    d = re.match(r"\S+\s+v(\d+)", prev) or re.match(r"\S+\s+v\[(\d+):(\d+)\]", prev)
-                    if d:
-                        lo = int(d.group(1))
-                        hi = int(d.group(2)) if d.lastindex and d.lastindex >= 2 else lo
-                        if srcs.intersection(range(lo, hi + 1)):
-                            found.append((func, line, prev))
+            srcs, states = vector_regs(line.split(",", 1)[1] if "," in line else ""), 0
+            for prev, prev_in_asm in reversed(window):
+                if states >= 2:
+                    break
+                if prev.startswith("v_") and not prev.startswith("v_mfma") and (prev_in_asm or in_asm):
+                    if srcs & written(prev):
+                        found.append((func, line, prev))
+                states += issue_slots(prev)
         if not in_asm and window:
             touched = acc_regs(line)
             states = 0
@@ -101,8 +114,7 @@ def asm_hazards(asm_text):
                     break
                 if prev_in_asm and prev.startswith("v_mfma") and touched.intersection(acc_regs(prev.split(",", 1)[0])):
                     found.append((func, line, prev))
-                n = re.match(r"s_nop (\d+)", prev)
-                states += int(n.group(1)) + 1 if n else 1
+                states += issue_slots(prev)
         window.append((line, in_asm))
         if len(window) > 20:
             window.pop(0)

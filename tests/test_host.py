@@ -384,7 +384,7 @@ def test_workload_generators_are_seeded():
 
 
 def test_build_scan_finds_dependences_too_close_to_an_asm_statement():
-    """build.py scans the generated device code for the two distances the compiler cannot keep when one end lies inside
+    """build.py scans the generated device code for the distances the compiler cannot keep when one end lies inside
     an asm statement; the scan itself is checked here on small pieces of assembly text."""
     import importlib.util
     spec = importlib.util.spec_from_file_location("minfer_build", f"{capi.ROOT}/minfer-python_amd/build.py")
@@ -408,6 +408,25 @@ def test_build_scan_finds_dependences_too_close_to_an_asm_statement():
     assert build.asm_hazards("kernel_c:\n" + acc + "\ts_nop 15\n\ts_nop 1\n" + read) == []
     assert build.asm_hazards("kernel_c:\n" + acc + read.replace("a6", "a8")) == []           # another block
     assert build.asm_hazards("kernel_c:\n" + acc + "\ts_branch .LBB0_9\n" + read) == []     # not the next to run
+
+
+def test_build_scan_finds_writes_in_front_of_a_matrix_instruction_inside_an_asm_statement():
+    """The other end of the same distance: the matrix instruction is the asm statement, the write the compiler's."""
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("minfer_build", f"{capi.ROOT}/minfer-python_amd/build.py")
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    mfma = "\t;;#ASMSTART\n\tv_mfma_f32_16x16x32_f16 a[4:7], v[50:53], v[58:61], a[4:7]\n\t;;#ASMEND\n"
+    for write in ("v_mov_b32_e32 v51, v9", "v_accvgpr_write_b32 a6, 0", "v_pk_mul_f16 v58, v63, v136", "v_lshlrev_b64 v[60:61], 1, v[2:3]",
+                  "v_accvgpr_mov_b32 a4, a9", "v_permlane32_swap_b32_e32 v9, v61"):
+        assert len(build.asm_hazards(f"kernel_d:\n\t{write}\n" + mfma)) == 1, write
+        assert len(build.asm_hazards(f"kernel_d:\n\t{write}\n\ts_add_u32 s2, s2, s3\n" + mfma)) == 1, write
+        assert build.asm_hazards(f"kernel_d:\n\t{write}\n\ts_add_u32 s2, s2, s3\n\tv_add_u32_e32 v1, v2, v3\n" + mfma) == [], write
+        assert build.asm_hazards(f"kernel_d:\n\t{write}\n\ts_nop 1\n" + mfma) == [], write
+    for other in ("v_mov_b32_e32 v54, v51", "v_accvgpr_write_b32 a8, 0", "v_accvgpr_read_b32 v3, a9", "v_cmp_gt_i32_e32 vcc, 0, v51", "s_nop 0"):
+        assert build.asm_hazards(f"kernel_d:\n\t{other}\n" + mfma) == [], other
+    assert build.asm_hazards("kernel_d:\n" + mfma + mfma) == []    # one after the other into one accumulator: the pipe's own order
+    assert build.asm_hazards("kernel_d:\n\tv_mov_b32_e32 v51, v9\n" + mfma.replace("\t;;#ASMSTART\n", "").replace("\t;;#ASMEND\n", "")) == []   # the compiler's own
 
 
 FAKE_HIP = r"""
