@@ -789,6 +789,7 @@ __global__ __launch_bounds__(NW * TEAMS * 64, D == 64 && NW == kWavesSmall && TE
                 *(lds_u32x2*)(uintptr_t)(so + row * RB + 16 * (gi ^ (row & (G - 1))) + 8 * (quad & 1)) = pk;
             }
         }
+        wave_lds_order();
         if (q_row0 + 32 <= seq_len) {   // every row exists: a wave-uniform base per store plus one 32-bit lane offset
             const int row_in = lane / G, gi = lane % G;
             const uint32_t lane_off = (uint32_t)((int64_t)row_in * p.o2 + 8 * gi) * 2u;

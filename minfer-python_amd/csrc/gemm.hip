@@ -939,6 +939,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_q8_kernel(const GemmPara
 #pragma unroll
         for (int j = 0; j < kGemvPieces; ++j)
             *reinterpret_cast<u32x4*>(my_raw + 16 * min(64 * j + lane, pieces - 1)) = un.piece[j];
+        wave_lds_order();
         request(u + 2, un);                                // the registers are free again: two units ahead
 #pragma unroll
         for (int i = 0; i < 2; ++i) {

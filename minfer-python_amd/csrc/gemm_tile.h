@@ -302,6 +302,7 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
         if (mw >= p.M) break;
 #pragma unroll
         for (int nb = 0; nb < N16; ++nb) *(lds_f32x4*)(uintptr_t)(area + l16 * ROW + 16 * (4 * nb + quad)) = acc[nb][mb];
+        wave_lds_order();
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
             const int m = mw + i_row[it];
@@ -326,6 +327,7 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
             pk.x = T::pack2(v[0], v[1]); pk.y = T::pack2(v[2], v[3]); pk.z = T::pack2(v[4], v[5]); pk.w = T::pack2(v[6], v[7]);
             *reinterpret_cast<s16x8_a8*>(d_col[it] + (int64_t)m * i_ldd[it]) = __builtin_bit_cast(s16x8, pk);
         }
+        wave_lds_order();
     }
 }
 
