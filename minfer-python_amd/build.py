@@ -123,6 +123,13 @@ def asm_hazards(asm_text):
     return found
 
 
+def scratch_users(asm_text):
+    """Kernels whose registers did not suffice: (name, bytes of scratch memory per lane) of those that have any."""
+    import re
+    sizes = re.findall(r"^    \.name:\s*(\S+)\n    \.private_segment_fixed_size:\s*(\d+)$", asm_text, flags=re.M)
+    return [(name, int(size)) for name, size in sizes if int(size)]
+
+
 def build_core(verbose=False):
     os.makedirs(LIB_DIR, exist_ok=True)
     obj_dir = os.path.join(HERE, "build")
@@ -138,10 +145,13 @@ def build_core(verbose=False):
         print("".join(outs))
     for a in asms:
         with open(a) as f:
-            bad = asm_hazards(f.read())
+            text = f.read()
+        bad = asm_hazards(text)
         if bad:
             raise RuntimeError("asm statement too close to an instruction that depends on it in %s:\n%s" % (
                 os.path.basename(a), "\n".join("  %s: %s  <-  %s" % b for b in bad[:20])))
+        if scratch_users(text):   # (every kernel here is meant to fit its registers: set-up alone is felt by the short calls)
+            raise RuntimeError("scratch memory in %s:\n%s" % (os.path.basename(a), "\n".join("  %s: %d bytes" % u for u in scratch_users(text))))
     _run(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", CORE_SO, *objs])
     return CORE_SO
 

@@ -290,6 +290,14 @@ __global__ __launch_bounds__(NW * TEAMS * 64, D == 64 && NW == kWavesSmall && TE
     const short* Kh = (const short*)p.k + (kDense ? (int64_t)b * p.kv0 : 0) + (int64_t)g * p.kv1 + (int64_t)seq_lo * p.kv2;
     const short* Vh = (const short*)p.v + (kDense ? (int64_t)b * p.kv0 : 0) + (int64_t)g * p.kv1 + (int64_t)seq_lo * p.kv2;
     short* Oh = (short*)p.out + (kDense ? (int64_t)b * p.o0 : 0) + (int64_t)head * p.o1 + (int64_t)seq_lo * p.o2;
+    // Mask rows of the lane's two query rows: a pointer each, or, with four waves, whose instantiations are at the end of their registers,
+    // a wave-uniform row and 32-bit offsets from it (31 rows of at most 2^17 bytes; the loads then take a scalar base), which is what
+    // keeps those out of scratch memory (4 x 1003 under a window of 256 35.2 -> 35.1 us, 8 heads over 2 L=256 7.96 -> 7.93).  Eight
+    // waves have registers to spare and gain nothing (L=4096 139.6 / 140.2).
+    constexpr bool kMaskOffsets = NW == kWavesSmall;
+    const int mrow0 = min(q_row0, last_row);
+    const uint8_t* const mbase = kDense ? p.mask + ((size_t)b * p.L + mrow0) * p.L : nullptr;
+    const uint32_t moff[2] = {(uint32_t)(min(qrow[0], last_row) - mrow0) * (uint32_t)p.L, (uint32_t)(min(qrow[1], last_row) - mrow0) * (uint32_t)p.L};
     const uint8_t* mrow[2] = {kDense ? p.mask + ((size_t)b * p.L + min(qrow[0], last_row)) * p.L : nullptr,
                               kDense ? p.mask + ((size_t)b * p.L + min(qrow[1], last_row)) * p.L : nullptr};
 
@@ -500,21 +508,21 @@ __global__ __launch_bounds__(NW * TEAMS * 64, D == 64 && NW == kWavesSmall && TE
             for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb)
-                    mw[qb][kb] = *reinterpret_cast<const u32_any*>(mrow[qb] + key0 + 16 * kb + 4 * quad);
+                    mw[qb][kb] = *reinterpret_cast<const u32_any*>(kMaskOffsets ? mbase + key0 + 16 * kb + (moff[qb] + 4 * quad) : mrow[qb] + key0 + 16 * kb + 4 * quad);
         } else if (p.L >= 4) {  // a tile crossing the end: the row's last word where a word would cross it, shifted; none past the end
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb) {
                     const int kbase = key0 + 16 * kb + 4 * quad, past = max(kbase - (last_row - 3), 0);
-                    const uint32_t x = *reinterpret_cast<const u32_any*>(mrow[qb] + (kbase - past));
+                    const uint32_t x = *reinterpret_cast<const u32_any*>(kMaskOffsets ? mbase + (moff[qb] + (uint32_t)(kbase - past)) : mrow[qb] + (kbase - past));
                     mw[qb][kb] = past < 4 ? x >> (8 * past) : 0u;
                 }
         } else {                // a row of fewer than four bytes (one tile): byte by byte
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb) {
                 uint32_t x = 0;
-                for (int e = 0; e <= last_row; ++e) x |= (uint32_t)mrow[qb][e] << (8 * e);
+                for (int e = 0; e <= last_row; ++e) x |= (uint32_t)(kMaskOffsets ? mbase[moff[qb] + e] : mrow[qb][e]) << (8 * e);
                 mw[qb][0] = quad == 0 ? x : 0u;
 #pragma unroll
                 for (int kb = 1; kb < 4; ++kb) mw[qb][kb] = 0u;
@@ -819,7 +827,7 @@ static size_t cls_bytes(int64_t B, int64_t L) {
     return (size_t)(B * nt * nt + 255) / 256 * 256;
 }
 
-// At head_dim 64 three four-wave workgroups fit a unit (40 KiB of LDS, 168 registers), which is ahead where they come one after the
+// At head_dim 64 three four-wave workgroups fit a unit (40 KiB of LDS, 166 registers of the 168 that leaves), which is ahead where they come one after the
 // other (us, two / three to a unit: 16 x 512 rows of 32 heads 43.7 / 38.8, 8 x 300 of 24 heads 17.4 / 15.0, L=8192 292 / 269, 4096 under a
 // window of 256 31.8 / 30.3, packed 32 sequences to 1200 95.2 / 93.4).  Where all of them would be on the chip at once, but not two to a
 // unit, a causal mask's longest share their unit with two others and the launch ends with them: L=3000 56.6 / 59.0, 2 x 1400 31.0 /

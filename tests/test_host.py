@@ -429,6 +429,19 @@ def test_build_scan_finds_writes_in_front_of_a_matrix_instruction_inside_an_asm_
     assert build.asm_hazards("kernel_d:\n\tv_mov_b32_e32 v51, v9\n" + mfma.replace("\t;;#ASMSTART\n", "").replace("\t;;#ASMEND\n", "")) == []   # the compiler's own
 
 
+def test_build_refuses_kernels_that_use_scratch_memory():
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("minfer_build", f"{capi.ROOT}/minfer-python_amd/build.py")
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    meta = "amdhsa.kernels:\n" + "".join(
+        f"  - .agpr_count:     0\n    .args:\n      - .offset:         0\n        .size:           8\n    .max_flat_workgroup_size: 256\n    .name:           {name}\n"
+        f"    .private_segment_fixed_size: {size}\n    .sgpr_count:     72\n" for name, size in (("kernel_a", 0), ("kernel_b", 12), ("kernel_c", 0))) + "amdhsa.version:\n"
+    assert build.scratch_users(meta) == [("kernel_b", 12)]
+    assert build.scratch_users(meta.replace("size: 12", "size: 0")) == []
+    assert "scratch_users(" in inspect.getsource(build.build_core)
+
+
 FAKE_HIP = r"""
 #pragma once
 #include <stddef.h>
