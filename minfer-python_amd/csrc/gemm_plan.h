@@ -199,8 +199,8 @@ inline GemmRoute gemm_route(int64_t M, int64_t N, int64_t K, bool nt, bool fast,
         // eight slices at most, 16 for rows of 80 K steps and more: further ones save less streaming than their sums cost (us, as many as fill
         // the chip / these: 1000 x 4096 at 1 / 9 / 16 rows 10.5 / 7.6, 13.5 / 8.7, 15.5 / 9.4; 2560 x 2560 at 12 10.0 / 8.1; 2048 x 4096 at 40 13.7 /
         // 11.9; 1024 x 14336 at 9 / 40 15.4 / 12.8, 19.4 / 17.2; 512 x 8192 at 9 17.0 / 9.6; minfer_gemm_workspace_bytes stays that of filling it)
-        const int kn = kn_slices(M, N, K), most = K >= 80 * kBK ? 16 : 8;   // a smaller workspace: as many slices as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
-        return {GemmKernel::kn_rows, fit < kn ? std::max((int)fit, 1) : std::min(kn, most), 0};
+        const int most = std::min(kn_slices(M, N, K), K >= 80 * kBK ? 16 : 8);   // a smaller workspace: as many of these as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
+        return {GemmKernel::kn_rows, std::max((int)std::min<int64_t>(most, fit), 1), 0};
     }
     TilePlan plan = tile_plan(M, N, K, nt, kMostSlices, units());
     if (plan.slices > std::max<int64_t>(fit, 1)) plan = tile_plan(M, N, K, nt, std::max<int64_t>(fit, 1), units());

@@ -100,6 +100,13 @@ def test_few_rows_need_no_plan_of_tiles(plan):
     assert plan.estimates() == before
 
 
+@pytest.mark.parametrize("M,N,K,most", [(9, 1000, 4096, 8), (1, 512, 8192, 16), (40, 4096, 4096, 8), (17, 264, 14336, 16), (64, 14336, 4096, 2), (64, 33000, 4096, 1)])
+def test_a_kn_weight_gets_no_more_slices_from_a_smaller_workspace(plan, M, N, K, most):
+    """As many as it holds, up to what a call with all the room takes."""
+    for fit in range(65):
+        assert plan(M, N, K, KN, fit)[:2] == (KN_ROWS, max(1, min(fit, most))), fit
+
+
 def layout_slices(layout, M, N, K):
     need = capi.lib().minfer_gemm_layout_workspace_bytes(layout, M, N, K)
     assert need % (4 * M * N) == 0

@@ -440,7 +440,7 @@ def test_few_rows_against_a_kn_weight(dtype, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(9, 1000, 4096), (40, 4096, 4096), (64, 2056, 2048)])
 def test_few_rows_against_a_kn_weight_in_a_smaller_workspace(M, N, K):
     """A workspace one byte short of minfer_gemm_workspace_bytes, one of two slices and one of less than two: as many slices as it
-    holds, none past its end; the bound is this file's."""
+    holds, eight at most, none past its end; the bound is this file's."""
     a, b, c = make(M, N, K, KN, torch.float16, seed=M + N)
     exact = oracle.gemm(a.float().numpy(), b.float().numpy(), c.float().numpy(), 2.0, 3.0, KN)
     da, db, dc = a.to(DEV), b.to(DEV), c.to(DEV)
@@ -453,7 +453,7 @@ def test_few_rows_against_a_kn_weight_in_a_smaller_workspace(M, N, K):
         assert_close(d, exact, torch.float16, f"{size} bytes")
         slices = ws[:need // (4 * M * N) * 4 * M * N].view(-1, 4 * M * N)
         written = [bool((s != 0xFF).any()) for s in slices]
-        fit = size // (4 * M * N)
+        fit = min(size // (4 * M * N), 8)
         assert written == [i < fit and fit > 1 for i in range(len(written))], (size, written)
 
 
