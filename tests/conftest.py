@@ -24,3 +24,9 @@ def kerns():
     import minfer.kernels.torch_ext  # noqa: F401
     from minfer.kernels import KernelBackend
     return KernelBackend("torch_ext")
+
+
+@pytest.fixture(scope="session")
+def gemm_plan(tmp_path_factory):
+    from gemm_plan_probe import GemmPlan
+    return GemmPlan(str(tmp_path_factory.mktemp("plan")))

@@ -1,60 +1,14 @@
 """The rules of the GEMM dispatch (csrc/gemm_plan.h), compiled for the host: which kernel takes a call, when a plan of tiles is
 estimated and how often."""
-import ctypes
-import os
-import subprocess
-
 import pytest
 
 import capi
-
-PLAIN, GEMV, ROWS_LDS, SKINNY, STRIPE, STRIPE_SLICES, KN_ROWS, TILES = range(8)   # enum GemmKernel
-KN, NK = False, True
-
-PROBE = """
-#include <math.h>
-#include <algorithm>
-static long estimates = 0;
-static double counting_sqrt(double x) { ++estimates; return sqrt(x); }
-#define sqrt counting_sqrt                      // plan_cost takes one square root
-#include "gemm_plan.h"
-using namespace minfer_attn;
-extern "C" void route(int64_t M, int64_t N, int64_t K, int nt, int fast, int64_t fit, int* out) {
-    const GemmRoute r = gemm_route(M, N, K, nt, fast, fit, []() { return 256; });
-    const GemmTile& t = kGemmTiles[r.tile];
-    const int v[] = {(int)r.kernel, r.slices, 32 * t.m16, 32 * t.n16, t.occ};
-    std::copy(v, v + 5, out);
-}
-extern "C" int q8_kernel(int64_t M, int64_t N, int64_t K, int aligned, int64_t fit) { return (int)q8_route(M, N, K, aligned, fit).kernel; }
-extern "C" int64_t q8_rows_of_a_part(int64_t M, int64_t N, int64_t K, int aligned) { return q8_part_rows(M, N, K, aligned); }
-extern "C" int grouped_tile(int64_t M, int64_t N, int64_t K) { return tile_plan(M, N, K, true, 1, 256).tile; }
-extern "C" long estimates_made() { return estimates; }
-"""
+from gemm_plan_probe import KN, KN_ROWS, NK, PLAIN, Q8_STRIPE, Q8_STRIPE_SLICES, STRIPE, STRIPE_SLICES, TILES
 
 
-@pytest.fixture(scope="module")
-def plan(tmp_path_factory):
-    tmp = tmp_path_factory.mktemp("plan")
-    (tmp / "probe.cpp").write_text(PROBE)
-    so = tmp / "probe.so"
-    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", os.path.join(capi.ROOT, "minfer-python_amd", "csrc"),
-                    str(tmp / "probe.cpp"), "-o", str(so)], check=True)
-    L = ctypes.CDLL(str(so))
-    i64 = ctypes.c_int64
-    L.route.argtypes = [i64, i64, i64, ctypes.c_int, ctypes.c_int, i64, ctypes.POINTER(ctypes.c_int)]
-    L.grouped_tile.argtypes = [i64, i64, i64]
-    L.estimates_made.restype = ctypes.c_long
-    L.q8_kernel.argtypes = [i64, i64, i64, ctypes.c_int, i64]
-    L.q8_rows_of_a_part.restype, L.q8_rows_of_a_part.argtypes = i64, [i64, i64, i64, ctypes.c_int]
-
-    def route(M, N, K, nt, fit=0, fast=True):
-        """(kernel, slices, rows of a tile, its columns, workgroups of it to a unit)"""
-        out = (ctypes.c_int * 5)()
-        L.route(M, N, K, nt, fast, fit, out)
-        return tuple(out)
-    route.grouped_tile, route.estimates = L.grouped_tile, L.estimates_made
-    route.q8_kernel, route.q8_part_rows = L.q8_kernel, L.q8_rows_of_a_part
-    return route
+@pytest.fixture
+def plan(gemm_plan):
+    return gemm_plan
 
 
 # (out, in) of the projections of a layer: q, k and v fused, output, gate and up, down; and the sizes of a narrower model
@@ -130,9 +84,6 @@ def test_workspace_of_a_layout_is_what_its_route_uses(plan):
                     assert plan(M, N, K, nt, slices) == best and best[1] == max(slices, 1), (M, N, K, layout)
 
 
-Q8_GEMV, Q8_STRIPE, Q8_STRIPE_SLICES, Q8_SKINNY = range(4)   # enum Q8Kernel
-
-
 def test_parts_of_a_q8_0_product_are_streamed(plan):
     """65 to 160 rows against a large Q8_0 weight: whatever goes in parts, every part as it runs is a product that a kernel streams, one of
     the stripe kernels wherever the tiled kernel could take the dequantised weight."""
@@ -150,6 +101,6 @@ def test_parts_of_a_q8_0_product_are_streamed(plan):
                 for m in range(0, M, rows) if rows < M else ():
                     r = min(rows, M - m)
                     assert N % 4 == 0 and (K // 32) % 2 == 0, (M, N, K, r)
-                    assert N % 8 != 0 or plan.q8_kernel(r, N, K, 1, room // (r * N * 4)) in (Q8_STRIPE, Q8_STRIPE_SLICES), (M, N, K, r)
+                    assert N % 8 != 0 or plan.q8(r, N, K, 1, min(room // (r * N * 4), 32))[0] in (Q8_STRIPE, Q8_STRIPE_SLICES), (M, N, K, r)
                     in_parts += 1
     assert in_parts > 5000

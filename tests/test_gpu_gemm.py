@@ -12,6 +12,7 @@ import pytest
 import torch
 
 import capi
+import gemm_plan_probe as rules
 import oracle
 import workloads
 
@@ -56,13 +57,15 @@ def make(M, N, K, layout, dtype, seed):
     (8, 4096, 4096, 1.0, 0.0),       # a decode step's tokens: kernels that stream the weight once
     (64, 1024, 1792, 2.0, 3.0),      # their largest row count; K steps not a multiple of the eight waves
     (48, 8192, 8192, 1.0, 0.0),      # more than 32 rows against a large weight
-    (2048, 6144, 128, 1.0, 1.0),     # [N, K]: 256 x 192 tiles (one full round instead of three quarters of one)
-    (1800, 6144, 64, 2.0, 3.0),      # the same with a ragged last tile row
+    (2048, 6144, 128, 1.0, 1.0),     # 256 x 256, three quarters of a round
+    (1800, 6144, 64, 2.0, 3.0),      # the same with a ragged last tile row, one K step
     (30, 5200, 128, 2.0, 1.0),       # wide enough for two column groups per workgroup, the last one ragged
     (37, 24, 192, 0.5, 1.0),         # ragged rows, a last group of 16 columns that is half empty
     (17, 4104, 64, 1.0, 1.0),        # one K step: seven of the eight waves have nothing to add
-    (64, 6144, 4096, 2.0, 3.0),      # 64 rows, two column groups per workgroup: the few-row kernel's largest instantiation
-    (40, 5128, 1024, 1.0, 1.0),      # 40 rows (three row blocks), two column groups, the last one ragged
+    (64, 6144, 4096, 2.0, 3.0),      # 64 rows, 96 stripes
+    (40, 5128, 1024, 1.0, 1.0),      # 40 rows (three row blocks), 81 stripes, the last one of 8 columns
+    (64, 5152, 192, 2.0, 3.0),       # K no multiple of 256, two column groups per workgroup: the few-row kernel's largest instantiation
+    (40, 5128, 448, 1.0, 1.0),       # ... with three row blocks, the last group ragged
     # up to 16 rows against an [N, K] weight with K a multiple of 512: weight and activation rows copied to LDS along the rows
     (2, 4096, 4096, 1.0, 0.0),
     (5, 264, 512, 1.0, 1.0),         # one segment per wave; rows 5..7 of the second activation copy do not exist
@@ -83,9 +86,10 @@ def make(M, N, K, layout, dtype, seed):
     (33, 12288, 512, 1.0, 1.0),      # four blocks of activation rows, two stages
     (64, 14336, 1792, 2.0, 0.0),
     # one row against an [N, K] weight: whole weight rows per wave (segments of 4096 values)
-    (1, 4096, 4096, 1.0, 0.0),       # one segment, the activations in registers; two rows per wave
+    (1, 4096, 4096, 1.0, 0.0),       # a small weight and K a multiple of 512: the LDS-staged few-row kernel
+    (1, 8200, 4096, 2.0, 3.0),       # one segment, the activations in registers; three rows per wave, a last wave with fewer
     (1, 1000, 4160, 2.0, 3.0),       # a second segment of 64 values, the activations in LDS
-    (1, 1000, 8192, 2.0, 3.0),       # longer than a segment and a multiple of 512: the LDS-staged few-row kernel instead
+    (1, 1000, 8192, 2.0, 3.0),       # longer than a segment and a multiple of 512: the LDS-staged few-row kernel as well
     (1, 20000, 64, 2.0, 3.0),        # ten short rows per wave
     (1, 264, 16384, 1.0, 1.0),       # the longest activation row its LDS area holds
     (1, 264, 16448, 1.0, 0.0),       # longer: the 16-rows-per-instruction kernel
@@ -115,17 +119,17 @@ def test_gemm_matches_oracle(layout, dtype, M, N, K, alpha, beta):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("layout,M,N,K,alpha,beta", [
     (NK, 593, 14344, 64, 1.0, 0.0),      # 160 x 256: one K step of the three stages, a ragged last tile row and column
-    (NK, 470, 16392, 256, 2.0, 3.0),     # four steps
+    (NK, 470, 16392, 256, 2.0, 3.0),     # 160 x 224: four steps
     (NK, 900, 8200, 320, 1.0, 1.0),      # five steps
-    (NK, 1003, 8200, 192, 2.0, 3.0),     # 256 x 192 over a width that is no multiple of 192
-    (NK, 385, 8200, 128, 1.0, 1.0),      # 128 x 256: two steps; a last tile row of one row
-    (NK, 130, 16392, 448, 2.0, 3.0),
+    (NK, 1003, 8200, 192, 2.0, 3.0),     # 160 x 256: a last tile of 8 columns
+    (NK, 385, 8200, 128, 1.0, 1.0),      # 224 x 128: two steps
+    (NK, 130, 16392, 448, 2.0, 3.0),     # 160 x 128
     (KN, 385, 8200, 192, 1.0, 0.0),
     (KN, 257, 12296, 64, 2.0, 3.0),
-    (KN, 520, 14344, 64, 1.0, 1.0),      # 192 x 256
-    (KN, 385, 16392, 320, 2.0, 3.0),     # a last tile row of one row, an odd number of steps
-    (NK, 1545, 4904, 192, 2.0, 3.0),     # 128 x 128, two workgroups per unit: a width that larger tiles would round up
-    (KN, 1545, 4904, 192, 2.0, 3.0),
+    (KN, 520, 14344, 64, 1.0, 1.0),      # 160 x 256
+    (KN, 385, 16392, 320, 2.0, 3.0),     # an odd number of steps
+    (NK, 1545, 4904, 192, 2.0, 3.0),     # 160 x 224
+    (KN, 1545, 4904, 192, 2.0, 3.0),     # 128 x 128, two workgroups to a unit
 ])
 def test_gemm_tiles_between_the_small_and_the_large_one(layout, dtype, M, N, K, alpha, beta):
     """Every element against torch's product in 64 bits, within the bound of assert_close."""
@@ -136,37 +140,39 @@ def test_gemm_tiles_between_the_small_and_the_large_one(layout, dtype, M, N, K, 
     assert_close(d, (alpha * (a.double() @ (b if layout == KN else b.T).double()) + beta * c.double()).numpy(), dtype)
 
 
-@pytest.mark.parametrize("layout,M,N,K", [
-    (KN, 977, 4152, 64),          # 128 x 128, two to a unit
-    (KN, 71, 424, 192),           # 128 x 128
-    (NK, 67, 360, 256),           # 128 x 128
-    (NK, 1147, 3640, 320),        # 128 x 192
-    (KN, 899, 6536, 448),         # 128 x 256
-    (NK, 905, 6568, 640),         # 128 x 256
-    (KN, 137, 1944, 64),          # 160 x 128
-    (NK, 137, 3816, 128),         # 160 x 128
-    (NK, 897, 6632, 192),         # 160 x 224
-    (KN, 1059, 7192, 256),        # 160 x 256
-    (NK, 1349, 6296, 320),        # 160 x 256
-    (KN, 651, 6584, 448),         # 192 x 128
-    (NK, 647, 6568, 640),         # 192 x 128
-    (NK, 903, 3592, 64),          # 192 x 192
-    (KN, 1287, 7176, 128),        # 192 x 256
-    (NK, 1811, 5416, 192),        # 192 x 256
-    (KN, 645, 6200, 256),         # 224 x 128
-    (NK, 657, 6632, 320),         # 224 x 128
-    (NK, 1773, 4904, 448),        # 224 x 192
-    (KN, 1561, 6440, 640),        # 224 x 256
-    (NK, 2119, 4824, 64),         # 224 x 256
-    (NK, 1949, 5656, 320),        # 256 x 192
-    (NK, 2025, 4888, 128),        # 256 x 224
-    (KN, 2027, 5976, 192),        # 256 x 256
-    (NK, 1807, 7192, 256),        # 256 x 256
+@pytest.mark.parametrize("layout,M,N,K,tile", [   # tile: rows, columns, workgroups to a unit
+    (KN, 977, 4152, 64, (128, 128, 2)),
+    (NK, 1173, 3384, 64, (128, 128, 2)),
+    (KN, 71, 424, 192, (128, 128, 1)),
+    (NK, 67, 360, 256, (128, 128, 1)),
+    (NK, 1147, 3640, 320, (128, 192, 1)),
+    (KN, 899, 6536, 448, (128, 256, 1)),
+    (NK, 905, 6568, 640, (128, 256, 1)),
+    (KN, 137, 1944, 64, (160, 128, 1)),
+    (NK, 137, 3816, 128, (160, 128, 1)),
+    (NK, 897, 6632, 192, (160, 224, 1)),
+    (KN, 1059, 7192, 256, (160, 256, 1)),
+    (NK, 1349, 6296, 320, (160, 256, 1)),
+    (KN, 651, 6584, 448, (192, 128, 1)),
+    (NK, 647, 6568, 640, (192, 128, 1)),
+    (NK, 903, 3592, 64, (192, 192, 1)),
+    (KN, 1287, 7176, 128, (192, 256, 1)),
+    (NK, 1811, 5416, 192, (192, 256, 1)),
+    (KN, 645, 6200, 256, (224, 128, 1)),
+    (NK, 657, 6632, 320, (224, 128, 1)),
+    (NK, 1773, 4904, 448, (224, 192, 1)),
+    (KN, 1561, 6440, 640, (224, 256, 1)),
+    (NK, 2119, 4824, 64, (224, 256, 1)),
+    (NK, 1949, 5656, 320, (256, 192, 1)),
+    (NK, 2025, 4888, 128, (256, 224, 1)),
+    (KN, 2027, 5976, 192, (256, 256, 1)),
+    (NK, 1807, 7192, 256, (256, 256, 1)),
 ])
-def test_gemm_every_tile_shape(layout, M, N, K):
-    """A shape for which plan_tiles takes each tile (as the comments say; without a workspace, on 256 compute units), the last tile
-    row and column ragged, from one K step (fewer than the ring has stages) to ten: every element against torch's product in 64
-    bits, within the bound of assert_close."""
+def test_gemm_every_tile_shape(gemm_plan, layout, M, N, K, tile):
+    """A shape for which plan_tiles takes each tile (without a workspace, on 256 compute units), the last tile row and column
+    ragged, from one K step (fewer than the ring has stages) to ten: every element against torch's product in 64 bits, within the
+    bound of assert_close."""
+    assert gemm_plan(M, N, K, layout == NK, 0) == (rules.TILES, 1, *tile)
     dtype = torch.float16 if (M + K // 64) % 2 else torch.bfloat16
     alpha, beta = (2.0, 3.0) if K % 128 else (1.0, 0.0)
     a, b, c = make(M, N, K, layout, dtype, M + N + K)
@@ -180,7 +186,7 @@ def test_gemm_every_tile_shape(layout, M, N, K):
 @pytest.mark.parametrize("N,K", [
     (2056, 256),      # one 16-column block a workgroup, the last of 8 columns; one segment
     (4096, 512),
-    (2048, 2560),     # more segments than the five stages
+    (2048, 2560),     # more segments than the ring has stages
     (4104, 1280),     # two blocks
     (8184, 768),
     (8200, 1024),     # three
@@ -269,25 +275,30 @@ def test_gemm_op_reference_test_recipe(kerns, S, alpha, beta):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,K,Nq,Nk,Nv", [
     (4096, 4096, 4096, 1024, 1024),    # Llama-3-8B prefill: 256 x 192 tiles over the weights' columns numbered through (two full rounds)
-    (2000, 128, 4096, 1024, 1024),     # the same tiling with a ragged last tile row; tiles that hold columns of q and k, of k and v
-    (4096, 128, 4096, 2048, 2048),     # 8192 columns: no multiple of 192, 256 x 256 tiles per weight
+    (2000, 128, 4096, 1024, 1024),     # 224 x 256: a ragged last tile row and column
+    (4096, 128, 4096, 2048, 2048),     # 256 x 256
     (512, 6144, 6144, 1024, 1024),     # the reference test's head shape at a smaller batch: 128 x 128 tiles
     (300, 256, 200, 72, 136),          # ragged rows, widths that end inside a tile
     (593, 128, 12288, 1024, 1088),     # 160 x 256 tiles over the columns numbered through, the last one past the third weight's end
-    (300, 320, 12288, 1024, 1088),     # 128 x 256 ones
-    (1003, 64, 8192, 1024, 1088),      # 256 x 192 ones
-    (1, 4096, 4096, 1024, 1024),       # a decode step: whole weight rows per wave, the three weights' rows numbered through
-    (1, 8192, 1032, 8, 520),           # the same with the activations in LDS and runs of rows that cross from one weight to the next
+    (300, 320, 12288, 1024, 1088),     # 160 x 128 ones
+    (1003, 64, 8192, 1024, 1088),      # 256 x 256 ones
+    (1, 4096, 4096, 1024, 1024),       # a decode step, 25 M weight values: the LDS-staged few-row kernel over the three weights' column groups
+    (1, 8192, 1032, 8, 520),           # the same with ragged last groups
+    (1, 4096, 7176, 1032, 8),          # 33 M: whole weight rows per wave, the three weights' rows numbered through, runs that cross from one to the next
+    (1, 8256, 1032, 8, 520),           # the same with the activations in LDS
     (2, 4096, 4096, 1024, 1024),       # up to 16 rows, K a multiple of 512: the LDS-staged few-row kernel over the three weights' column groups
     (13, 1024, 520, 264, 8),           # the same with ragged last groups
     (16, 576, 4096, 1024, 1024),       # K not a multiple of 512: the few-row kernel that loads fragments directly
-    (24, 1024, 5120, 1280, 1288),      # few rows, two column groups per workgroup, a ragged last group
-    (64, 512, 768, 256, 256),          # few-row kernel at its largest row count
+    (24, 1024, 5120, 1280, 1288),      # stripes of 64 columns, see below
+    (24, 192, 4104, 1024, 1032),       # the few-row kernel, two column groups per workgroup, ragged last groups; two blocks of rows
+    (40, 448, 5120, 520, 8),           # ... three
+    (64, 192, 4096, 1024, 1032),       # ... four
+    (64, 512, 768, 256, 256),          # the few-row kernel at its largest row count, one column group per workgroup
     (33, 50, 17, 17, 9),               # nothing tileable: three plain launches
-    # 5-64 rows, K a multiple of 256, 96 stripes of 64 columns or more over the three weights: the stripe kernel, every weight
-    # with workgroups of its own in proportion to its width
     (300, 320, 1000, 72, 136),         # tiles and 16-column blocks that hold columns of two or three weights
     (1100, 192, 1032, 1000, 8),
+    # 5-64 rows, K a multiple of 256, 96 stripes of 64 columns or more over the three weights: the stripe kernel, every weight
+    # with workgroups of its own in proportion to its width
     (5, 4096, 4096, 1024, 1024),
     (16, 512, 4096, 1024, 1032),       # a last stripe of 8 columns in the third weight
     (40, 1024, 4104, 1024, 1024),      # ... in the first; three blocks of activation rows
@@ -362,21 +373,21 @@ def test_qkv_op_and_reference_checks(kerns):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K,alpha,beta", [
     (64, 4096, 4096, 1.0, 0.0),      # [K, N]: 32 tiles of 128 columns, 8 slices of 8 steps; [N, K]: 256 blocks of 16 columns, no slices
-    (100, 1032, 2048, 2.0, 3.0),     # ragged rows and columns, C read by the second kernel
-    (256, 2048, 1024, 0.5, 1.0),     # two tile rows
-    (40, 512, 1984, 1.0, 0.0),       # K steps (31) not a multiple of the slice count
+    (100, 1032, 2048, 2.0, 3.0),     # tiles of whole rows: the workspace is not needed
+    (256, 2048, 1024, 0.5, 1.0),
+    (40, 512, 1984, 1.0, 0.0),       # [K, N]: 31 K steps in 7 slices; [N, K]: whole rows
     (1, 4096, 4096, 1.0, 1.0),       # one row: with [K, N] slices of 128 columns, with [N, K] still the few-row kernel
-    (24, 1024, 2048, 1.0, 1.0),      # 17-32 rows: with a workspace [K, N] slices of 128 columns, [N, K] the sliced tiles
-    (256, 8192, 1024, 1.0, 1.0),     # 128 tiles: two slices, so that two workgroups share a compute unit
-    # [N, K] weights of fewer than 192 stripes of 64 columns: K slices of the stripe kernel
+    (24, 1024, 2048, 1.0, 1.0),      # [K, N]: 8 slices of four steps; [N, K]: whole rows
+    (256, 8192, 1024, 1.0, 1.0),     # 128 tiles of whole rows
+    # [N, K] weights of fewer than 192 stripes of 64 columns: K slices of the stripe kernel, or whole rows where those are ahead
     (8, 5120, 5120, 2.0, 3.0),       # 80 stripes, 320 blocks of 16 columns shared out: the workspace is not needed
-    (16, 4104, 8192, 1.0, 1.0),      # a last stripe of 8 columns
-    (33, 8192, 2048, 0.5, 0.0),      # three blocks of activation rows, two slices of four segments
-    (1, 8192, 4096, 1.0, 0.0),       # one row
-    (64, 6144, 4096, 1.0, 1.0),
+    (16, 4104, 8192, 1.0, 1.0),      # three slices, a last stripe of 8 columns
+    (33, 8192, 2048, 0.5, 0.0),      # whole rows
+    (1, 8192, 4096, 1.0, 0.0),       # one row: whole rows
+    (64, 6144, 4096, 1.0, 1.0),      # whole rows
     (12, 1024, 14336, 1.0, 0.0),     # long rows of a small weight: 16 stripes, 14 slices of 4 segments
-    (24, 2048, 4096, 2.0, 1.0),      # 8 M weight values from 17 rows on: 8 slices of 2 segments, two blocks of rows
-    (3, 1536, 8960, 1.0, 1.0),       # long rows, 24 stripes: slices from 2 rows on (10 slices of 3 or 4 segments)
+    (24, 2048, 4096, 2.0, 1.0),      # whole rows
+    (3, 1536, 8960, 1.0, 1.0),       # long rows, 24 stripes: slices from 2 rows on (8 slices of 4 or 5 segments)
 ])
 def test_gemm_k_slices_against_oracle(layout, dtype, M, N, K, alpha, beta):
     a, b, c = make(M, N, K, layout, dtype, seed=M + N + K)
@@ -457,21 +468,82 @@ def test_few_rows_against_a_kn_weight_in_a_smaller_workspace(M, N, K):
         assert written == [i < fit and fit > 1 for i in range(len(written))], (size, written)
 
 
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("layout,M,N,K", [
-    (NK, 70, 8136, 8256),      # eight slices of 16 and 17 steps; a last tile of 200 columns
-    (KN, 70, 8136, 8256),
-    (NK, 250, 8072, 4160),     # four; a last tile row of 122
-    (KN, 129, 8072, 4160),     # ... of one
-])
-def test_gemm_k_slices_of_wide_tiles(layout, dtype, M, N, K):
-    """Slices of 128 x 256 tiles, every element against torch's product in 64 bits within the bound of assert_close."""
-    a, b, c = make(M, N, K, layout, dtype, M + N + K)
+def sliced_call(a, b, c, layout, M, N, K):
+    """2 A B + 3 C with a workspace of minfer_gemm_workspace_bytes that holds a NaN pattern: every slot read must have been written."""
     ws = torch.full((capi.lib().minfer_gemm_workspace_bytes(M, N, K),), 0xFF, dtype=torch.uint8, device=DEV)
-    d = torch.full((M, N), float("nan"), dtype=dtype, device=DEV)
-    assert capi.gemm_ws(a.to(DEV), b.to(DEV), c.to(DEV), d, 2.0, 3.0, ws, layout) == capi.OK, capi.last_error()
+    d = torch.full((M, N), float("nan"), dtype=a.dtype, device=DEV)
+    assert capi.gemm_ws(a, b, c, d, 2.0, 3.0, ws, layout) == capi.OK, capi.last_error()
     torch.cuda.synchronize()
-    assert_close(d, (2.0 * (a.double() @ (b if layout == KN else b.T).double()) + 3.0 * c.double()).numpy(), dtype)
+    return ws, d
+
+
+def written_slices(ws, M, N):
+    """How many slices of M x N sums the call wrote, from the workspace's start on and without a gap."""
+    written = [bool((x != 0xFF).any()) for x in ws[:ws.numel() // (4 * M * N) * 4 * M * N].view(-1, 4 * M * N)]
+    assert written == sorted(written, reverse=True)
+    return sum(written)
+
+
+@pytest.mark.parametrize("layout,M,N,K,slices,tile", [   # tile: rows, columns, workgroups to a unit
+    (NK, 70, 8136, 8256, 4, (128, 128, 1)),
+    (KN, 70, 8136, 8256, 4, (128, 128, 1)),
+    (NK, 250, 8072, 4160, 2, (128, 128, 1)),
+    (KN, 129, 8072, 4160, 3, (160, 128, 1)),
+    (KN, 130, 272, 5952, 31, (128, 128, 1)),
+    (KN, 987, 2616, 8000, 3, (128, 128, 2)),
+    (KN, 65, 8312, 7936, 7, (128, 256, 1)),
+    (KN, 964, 136, 2496, 13, (160, 128, 1)),
+    (KN, 261, 5560, 6848, 5, (160, 256, 1)),
+    (KN, 162, 5488, 2112, 3, (192, 128, 1)),
+    (KN, 517, 6864, 8384, 3, (192, 256, 1)),
+    (KN, 199, 5384, 4160, 5, (224, 128, 1)),
+    (KN, 391, 5384, 8896, 5, (224, 256, 1)),
+    (KN, 487, 8584, 8064, 3, (256, 256, 1)),
+    (NK, 129, 264, 6080, 31, (128, 128, 1)),
+    (NK, 487, 3112, 11200, 5, (128, 128, 2)),
+    (NK, 67, 8208, 5056, 5, (128, 192, 1)),
+    (NK, 322, 5488, 4032, 3, (128, 256, 1)),
+    (NK, 980, 136, 2496, 13, (160, 128, 1)),
+    (NK, 258, 5424, 5376, 5, (160, 224, 1)),
+    (NK, 261, 5744, 6720, 5, (160, 256, 1)),
+    (NK, 163, 2064, 6336, 11, (192, 128, 1)),
+    (NK, 327, 5400, 4544, 4, (192, 192, 1)),
+    (NK, 527, 4104, 16960, 5, (192, 256, 1)),
+    (NK, 193, 5464, 4160, 5, (224, 128, 1)),
+    (NK, 387, 5448, 5312, 4, (224, 192, 1)),
+    (NK, 386, 6296, 9920, 5, (224, 256, 1)),
+    (NK, 485, 3096, 19264, 9, (256, 224, 1)),
+    (NK, 227, 8240, 14784, 7, (256, 256, 1)),
+])
+def test_gemm_k_slices_of_tiles(gemm_plan, layout, M, N, K, slices, tile):
+    """Every tile that the plan cuts K for, in each layout, a last tile row and column that are not full, slices of different lengths: so
+    many slices written and no more, every element against torch's product in 64 bits within the bound of assert_close."""
+    assert gemm_plan(M, N, K, layout == NK, rules.MOST_SLICES) == (rules.TILES, slices, *tile)
+    dtype = torch.float16 if (M + K // 64) % 2 else torch.bfloat16
+    a, b, c = (x.to(DEV) for x in make(M, N, K, layout, dtype, M + N + K))
+    ws, d = sliced_call(a, b, c, layout, M, N, K)
+    assert written_slices(ws, M, N) == slices
+    exact = 2.0 * torch.mm(a.double(), (b if layout == KN else b.T.contiguous()).double()) + 3.0 * c.double()
+    assert_close(d, exact.cpu().numpy(), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,slices", [
+    (9, 520, 6144, 6),       # one block of activation rows; a last stripe of 8 columns
+    (17, 520, 8448, 8),      # two, the second of one row; 33 segments
+    (32, 3080, 8448, 5),
+    (33, 2056, 4352, 4),     # three; 17 segments
+    (48, 1544, 9216, 9),
+    (49, 1032, 8448, 8),     # four
+    (64, 3080, 6144, 5),
+])
+def test_gemm_k_slices_of_stripes(gemm_plan, dtype, M, N, K, slices):
+    """K slices of the stripe kernel with every number of activation row blocks, their edges: as above."""
+    assert gemm_plan(M, N, K, rules.NK, rules.MOST_SLICES)[:2] == (rules.STRIPE_SLICES, slices)
+    a, b, c = (x.to(DEV) for x in make(M, N, K, NK, dtype, M + N + K))
+    ws, d = sliced_call(a, b, c, NK, M, N, K)
+    assert written_slices(ws, M, N) == slices
+    assert_close(d, (2.0 * torch.mm(a.double(), b.T.contiguous().double()) + 3.0 * c.double()).cpu().numpy(), dtype)
 
 
 def test_gemm_workspace_bytes_is_zero_where_tiles_fill_the_chip():
