@@ -585,9 +585,12 @@ def make_q8(M, N, K, seed):
     (1, 4096, 4096, 1.0, 0.0),       # a decode step against a Llama-3-8B projection: the kernel that streams the blocks
     (8, 1024, 4096, 1.0, 1.0),
     (16, 256, 14336, 2.0, 3.0),      # a long contraction split over the eight waves
-    (17, 5152, 256, 1.0, 0.0),       # two column groups per workgroup, a ragged last one
-    (4, 5200, 512, 1.0, 1.0),        # the same with one block of rows
-    (40, 5152, 512, 2.0, 1.0),       # three and four blocks of rows with two column groups
+    (17, 5152, 192, 1.0, 0.0),       # two column groups per workgroup, a ragged last one
+    (4, 5200, 512, 1.0, 1.0),        # one block of rows
+    (40, 5160, 448, 2.0, 1.0),       # three and four blocks of rows with two column groups
+    (64, 5120, 192, 1.0, 0.0),
+    (17, 5152, 256, 1.0, 0.0),       # K a multiple of 256: the stripe kernel, see below
+    (40, 5152, 512, 2.0, 1.0),
     (64, 5120, 256, 1.0, 0.0),
     (64, 264, 192, 0.5, 1.0),        # its largest row count; K a multiple of 64 but not of 128: a short last step
     (37, 24, 64, 1.0, 1.0),          # one step, half-empty column group
@@ -616,9 +619,9 @@ def make_q8(M, N, K, seed):
     (16, 4096, 14336, 1.0, 1.0),     # 4 slices of 14 segments
     (33, 5120, 5120, 2.0, 0.0),      # 3 slices of 7, 7 and 6 segments; three blocks of rows
     (8, 8192, 8192, 1.0, 0.0),       # 2 slices
-    (64, 4104, 2048, 0.5, 1.0),      # 65 stripes, the last of 8 columns: 2 slices of 4 segments; a small weight, from 16 rows
-    (2, 6144, 4096, 1.0, 0.0),
-    (3, 1536, 8960, 1.0, 1.0),       # long rows, 24 stripes: 10 slices of 3 or 4 segments
+    (64, 4104, 2048, 0.5, 1.0),      # 65 stripes, the last of 8 columns: whole rows, the workspace is not needed
+    (2, 6144, 4096, 1.0, 0.0),       # ... as here
+    (3, 1536, 8960, 1.0, 1.0),       # long rows, 24 stripes: 8 slices of 4 or 5 segments
 ])
 def test_gemm_q8_0_weights_against_oracle(M, N, K, alpha, beta):
     a, wq, c, w_deq = make_q8(M, N, K, seed=M * 7 + N + K)
@@ -646,6 +649,26 @@ def test_gemm_q8_0_weights_against_oracle(M, N, K, alpha, beta):
     assert_close(d_ref, exact, torch.float16, "fp16 kernel on the dequantised weight")
     if not streams:
         assert capi.gemm_q8_0(da, dwq, dc, d, alpha, beta, None) == capi.EWORKSPACE and "workspace" in capi.last_error()
+
+
+@pytest.mark.parametrize("M,N,K,slices", [
+    (9, 1544, 8448, 8),      # one block of activation rows; a last stripe of 8 columns; 33 segments
+    (17, 2056, 6144, 6),     # two, the second of one row
+    (32, 4104, 4352, 3),     # 17 segments
+    (48, 3080, 6144, 5),     # three
+    (64, 2056, 4608, 4),     # four
+])
+def test_gemm_q8_0_k_slices_of_stripes(gemm_plan, M, N, K, slices):
+    """K slices of the stripe kernel over Q8_0 blocks with every number of activation row blocks: so many slices written, every element
+    against torch's product with the dequantised weight in 64 bits, within the bound of assert_close."""
+    assert gemm_plan.q8(M, N, K, True, slices) == (rules.Q8_STRIPE_SLICES, slices)
+    a, wq, c, w = make_q8(M, N, K, seed=M + N + K)
+    ws = torch.full((capi.lib().minfer_gemm_q8_0_workspace_bytes(M, N, K),), 0xFF, dtype=torch.uint8, device=DEV)
+    d = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
+    assert capi.gemm_q8_0(a.to(DEV), wq.to(DEV), c.to(DEV), d, 2.0, 3.0, ws) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    assert written_slices(ws, M, N) == slices
+    assert_close(d, (2.0 * (a.double() @ w.double().T) + 3.0 * c.double()).numpy(), torch.float16)
 
 
 @pytest.mark.parametrize("M,N,K,alpha,beta", [
