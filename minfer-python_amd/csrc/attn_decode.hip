@@ -917,7 +917,8 @@ static int decode_slots(int64_t Lmax, int floor_rows) { return (int)(Lmax / deco
 
 static size_t decode_ws_bytes(int64_t B, int64_t Hq, int64_t Lmax, int64_t D, int floor_rows) {
     const int64_t S = decode_slots(Lmax, floor_rows);
-    return (size_t)(B * Hq * S * (D + 2) * 4 + 255) / 256 * 256 + (size_t)((B + 1) * 4 + 255) / 256 * 256 + 256;
+    // seq_off's B + 2 entries and 252 bytes that nothing uses: the size has been that, and callers may keep a workspace by it
+    return (size_t)(B * Hq * S * (D + 2) * 4 + 255) / 256 * 256 + (size_t)((B + 2) * 4 + 252 + 255) / 256 * 256;
 }
 
 // Workgroups of the split launch: as many as the chip holds at once (kDecodeWgPerCu per compute unit: LDS and

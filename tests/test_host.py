@@ -37,9 +37,13 @@ def test_workspace_sizes():
     assert L.minfer_flash_attn_workspace_bytes(2, 100) >= 2 * 2 * 2
     assert L.minfer_flash_attn_workspace_bytes(1, 32768) >= 512 * 512
     # fp32 partials (D values + max + sum), one per share of at least 256 rows that can overlap a (sequence, head)'s rows
-    # (8192/256 + 2 of them), plus one line offset per sequence
+    # (8192/256 + 2 of them), plus the line offsets: one per sequence, the line's length and the largest piece
     need = L.minfer_flash_attn_decode_workspace_bytes(64, 32, 8192, 128)
     assert 64 * 32 * 34 * 130 * 4 + 65 * 4 <= need <= 2 * 64 * 32 * 34 * 130 * 4
+    # the offsets that fill whole 256 bytes with and without their last entry; the sizes are those that callers keep workspaces by
+    for B, offsets in ((1, 512), (62, 512), (63, 512), (64, 768), (126, 768), (127, 768), (128, 1024)):
+        partials = (B * 7 * 66 * 4 + 255) // 256 * 256   # one head of 64 values over 512 rows: four shares of 128 and three more
+        assert L.minfer_flash_attn_decode_workspace_bytes(B, 1, 512, 64) - partials == offsets >= (B + 2) * 4
     # never more than 64 partials per row, however long the cache
     assert L.minfer_flash_attn_decode_workspace_bytes(1, 8, 1 << 20, 128) <= 8 * 64 * 130 * 4 + 4096
 
