@@ -214,9 +214,9 @@ int minfer_gemm(int dtype, int b_layout, const void* A, const void* B, const voi
  * that run as separate workgroups and meet in the workspace as fp32 partial sums, which the last workgroup of a
  * tile (small sums on a device's null stream, stream 0) or a second kernel adds up, with the same result to the bit
  * (alpha, beta and C applied there, one rounding): slices of tiles, or, up to 64 rows, of
- * 128-column tiles of a [K, N] weight, or of an [N, K] weight of fewer than 12288 columns, of 64-column stripes
- * (where two launches pay: from 9 rows on below 6144 columns, from 2 on rows of 8192 values and more of at most
- * 1536 columns, from 33 between 6144 and 12288 columns).  With a null workspace the call is minfer_gemm; a
+ * 128-column tiles of a [K, N] weight, or, for an [N, K] weight of at most 6080 columns, of 64-column stripes
+ * (where that pays: from 9 rows on, or from 2 on rows of 8192 values and more of at most 1536 columns, and only
+ * where streaming whole rows in one launch is not ahead).  With a null workspace the call is minfer_gemm; a
  * workspace smaller than minfer_gemm_workspace_bytes is used only by a path whose slices fit in it, and from 65 rows
  * on, or against a [K, N] weight, for as many slices as it holds.  minfer_gemm_workspace_bytes is enough for either
  * layout; minfer_gemm_layout_workspace_bytes is what one of them (MINFER_GEMM_B_KN, MINFER_GEMM_B_NK) can use,

@@ -832,7 +832,8 @@ static size_t cls_bytes(int64_t B, int64_t L) {
 // window of 256 31.8 / 30.3, packed 32 sequences to 1200 95.2 / 93.4).  Where all of them would be on the chip at once, but not two to a
 // unit, a causal mask's longest share their unit with two others and the launch ends with them: L=3000 56.6 / 59.0, 2 x 1400 31.0 /
 // 32.3, 3 x 800 (600 workgroups) 23.3 / 23.7 (but 2 x 900 of 48 heads, 720 of them, 24.7 / 23.1, and shorter sequences' tiles weigh
-// less than what a workgroup pays once); LDS that nobody uses keeps those to two.
+// less than what a workgroup pays once); LDS that nobody uses keeps those to two.  The host does not see the mask: a window's rows, which are
+// alike, would not need it; timed under causal masks only.
 static unsigned unused_lds(int64_t L, int64_t grid) {
     return grid > 512 && grid <= 768 && (L > 1024 || (L > 512 && grid < 704)) ? 20 * 1024 : 0;
 }

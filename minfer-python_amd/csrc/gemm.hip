@@ -1316,7 +1316,7 @@ static int launch_grouped(GemmParams& p, int n_w, hipStream_t stream) {
         }
         return acc;
     };
-    if (p.M == 1 && p.K <= kGemvMaxKHalfs && (n_sum * p.K >= (INT64_C(1) << 25) || !rows_lds_takes(p.M, p.K))) {   // one row: whole weight rows per wave, numbered through (the rule of gemm_impl)
+    if (p.M == 1 && p.K <= kGemvMaxKHalfs && (n_sum * p.K >= (INT64_C(1) << 25) || !rows_lds_takes(p.M, p.K))) {   // one row: whole weight rows per wave, numbered through (the rule of gemm_route)
         int acc = 0;
         for (int s = 0; s < kMaxGroup; ++s) { if (s < n_w) acc += p.grp.N[s]; p.grp.end[s] = acc; }
         return launch_gemv<T, true>(p, (int)n_sum, stream);

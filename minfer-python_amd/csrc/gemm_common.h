@@ -14,8 +14,9 @@ namespace minfer_attn {
 constexpr int kRowTile = 8192;              // sub-tile [64 rows][64 k], 128-byte rows (A, and B as [N, K])
 constexpr int kColTile = 16384;             // sub-tile [64 k][128 n], 256-byte rows (B as [K, N])
 
-// Several weights that share A in one launch (the QKV projection): the column tiles (tiled kernel) or column groups
-// (few-row kernel) of weight s follow those of weight s - 1; `end` holds the cumulative counts.  No C operand.
+// [N, K] weights that share A in one launch (the QKV projection): the column units of weight s follow those of weight s - 1, and `end`
+// holds the cumulative counts: columns for the tiled kernel, whose tiles may hold columns of two weights, and gemv_kernel, column groups or
+// workgroups for the other few-row kernels.  More than one weight: no C operand.
 constexpr int kMaxGroup = 3;
 struct GemmGroup {
     const void* B[kMaxGroup]; void* D[kMaxGroup];
@@ -31,7 +32,7 @@ struct GemmParams {
     int splits;                   // SPLIT instantiations: K is cut into this many slices, one workgroup per (tile, slice)
     float* part;                  // their fp32 partial products, [splits][M][N]
     uint32_t* done;               // zeroed arrival counters, one per tile (stripe), left zero; null: gemm_reduce_kernel adds the slices up
-    GemmGroup grp;                // used by the GROUPED instantiations only
+    GemmGroup grp;                // used by the GROUPED instantiations, and by every [N, K] launch of the tiled kernel (one weight: a group of one)
 };
 // Which weight column unit `c` (a tile column or a column group) belongs to, and its index inside that weight.
 MA_DEV int group_of_unit(const GemmGroup& g, int c, int& local) {

@@ -47,6 +47,8 @@ inline bool stripe_takes(int64_t M, int64_t stripes, int64_t K) {
 // 15.1, 5632 x 4096 15.5 / 15.1, 4608 x 4096 13.8 / 14.9 and at 33 rows 12.7 / 11.7; 4096 x 6144 at 33 / 64 rows 13.9 / 13.4, 15.2 /
 // 16.5; 3584 x 8192 at 32 / 48 rows 14.5 / 14.3, 16.1 / 18.2; 2560 x 5120 at 32 / 33 rows 10.7 / 10.1, 11.4 / 11.7; 2048 x 4096 at 32 /
 // 64 rows 9.3 / 8.4, 11.2 / 12.2; 2048 x 8192 at 5 rows 9.5 / 10.4; 4096 x 14336 at 16 / 24 rows 24.0 / 24.1, 24.8 / 27.8).
+// The lines lie between these: below 48 stripes a quarter of the units and more have no column block and whole rows pay less; from 65 to
+// 79 a few units have two blocks where the others have one.
 inline bool stripe_blocks_pay(int64_t M, int64_t stripes, int64_t K) {
     const int64_t most = stripes < 48 ? 16000 : stripes <= 64 || stripes >= 80 ? 25000 : 22000;
     return stripe_takes(M, stripes, K) && (stripes >= 96 || ((stripes > 64 ? 2 : 1) + (M + 15) / 16) * K <= most);
@@ -214,6 +216,30 @@ constexpr int kGemvMaxK = 16384;            // the longest activation row that g
 // the streaming kernel takes up to 64 rows, needs weight rows that are multiples of 4 bytes (an even number of blocks)
 // and stores 8-byte pieces of D (N a multiple of 4); every other shape goes through the dequantised weight
 inline bool q8_streams(int64_t M, int64_t N, int64_t K) { return M <= kQ8SkinnyRows && (K / 32) % 2 == 0 && N % 4 == 0; }
+// Where gemm_stripe_q8_kernel over whole rows is ahead of its K slices and of gemm_skinny_q8_kernel on a weight of fewer than 192 stripes: rows of up to 4096 values, by the rows a
+// unit copies, (NB + MB) x 16 of K values (us, the other / it: 8192 x 4096 at 2 / 16 / 32 rows 11.8 / 11.0, 12.7 / 11.1, 14.9 / 12.8;
+// 6144 x 4096 at 16 / 24 / 40 rows 12.3 / 11.0, 14.1 / 12.1, 15.2 / 15.4; 6144 x 2048 at 16 rows 9.1 / 6.7; 5120 x 4096 at 24 / 40 12.6 /
+// 12.0, 14.0 / 15.1; 4096 x 4096 at 16 / 64 9.7 / 8.2, 13.9 / 13.2; 4096 x 2048 at 8 / 16 / 64 5.4 / 5.9, 8.7 / 5.5, 11.7 / 8.6; 2048 x 4096
+// at 16 / 24 / 40 8.8 / 8.0, 9.9 / 9.6, 10.7 / 11.2; 5120 x 5120 at 16 rows 12.1 / 12.7).  64 stripes are 253 to 256 column blocks, one to a unit
+// with no unit idle, and have a line of their own: 4096 x 4096 still gains at 64 rows, 20480 by this count.
+inline bool q8_blocks_pay(int64_t M, int64_t N, int64_t K) {
+    const int64_t stripes = (N + 63) / 64, rows = (stripes > 64 ? 2 : 1) + (M + 15) / 16;
+    if (K > 4096 || M < 2 || M > 64 || stripes < 32 || stripes >= 192) return false;
+    if (stripes >= 96) return rows * K <= 17000 && (M >= 8 || N * K >= INT64_C(20000000));
+    return M >= 16 && rows * K <= (stripes < 64 ? 12500 : stripes == 64 ? 20500 : 17000);
+}
+// K slices of gemm_stripe_q8_kernel for a weight of fewer than 192 stripes when a workspace is given (1 = none): 256 / stripes workgroups
+// per chunk of four blocks, full chunks whatever the width (weights coming from memory: 4096 x 14336 at 16 / 32 / 64 rows
+// 19.0 / 21.8 / 26.4 us against 29.6 / 43.0 / 68.4 for gemm_skinny_q8_kernel, 8192 x 8192 at 2-64 rows 19.6-28.5 against
+// 23.7-40.3, 6144 x 4096 12.4-17.7 against 12.7-22.2; 4096 x 4096 up to 8 rows 10.2 against 7.7-8.3: two launches, so a
+// weight of 16 M values or fewer only from 16 rows on, or from 8 when its rows are 6144 values and longer, or from 2
+// when they are 8192 values and longer and the stripes 24 at most, as for the 16-bit weights).
+inline int q8_slices(int64_t M, int64_t N, int64_t K) {
+    if (M < 2 || M > 64 || K % kStripeSeg != 0 || N % 8 != 0) return 1;
+    const bool long_rows = (K >= 6144 && M >= 8) || (K >= 8192 && N <= 24 * 64);
+    if (N * K <= (INT64_C(1) << 24) && M < 16 && !long_rows) return 1;
+    return stripe_slices(M, N, K);
+}
 // gemm_stripe_q8_kernel.  Which calls it takes: 2-64 rows, whole segments of 8 blocks, rows that start on 16-byte boundaries, and a weight wide
 // enough for two and a half blocks per workgroup, or two from 16 rows, or one and a half above 32 (weights coming from memory:
 // 14336 x 4096 at 2-16 rows 16.7-16.9 us against 20.8-26.8 for gemm_skinny_q8_kernel, 64 rows 23.4 against 50.9; 28672 x
@@ -221,29 +247,6 @@ inline bool q8_streams(int64_t M, int64_t N, int64_t K) { return M <= kQ8SkinnyR
 // at 2 / 24 / 64 rows 15.4 -> 13.3, 18.4 -> 15.6, 23.3 -> 20.6; 18944 x 3584 at 2 / 40 rows 25.6 -> 21.6, 34.1 -> 31.3): all of a
 // chunk's blocks are dequantised and multiplied, there or not (skipping the missing ones of four by a branch cost the full chunks a
 // third).
-// Where it is ahead of its K slices and of gemm_skinny_q8_kernel on a weight of fewer than 192 stripes: rows of up to 4096 values, by the rows a
-// unit copies, (NB + MB) x 16 of K values (us, the other / it: 8192 x 4096 at 2 / 16 / 32 rows 11.8 / 11.0, 12.7 / 11.1, 14.9 / 12.8;
-// 6144 x 4096 at 16 / 24 / 40 rows 12.3 / 11.0, 14.1 / 12.1, 15.2 / 15.4; 6144 x 2048 at 16 rows 9.1 / 6.7; 5120 x 4096 at 24 / 40 12.6 /
-// 12.0, 14.0 / 15.1; 4096 x 4096 at 16 / 64 9.7 / 8.2, 13.9 / 13.2; 4096 x 2048 at 8 / 16 / 64 5.4 / 5.9, 8.7 / 5.5, 11.7 / 8.6; 2048 x 4096
-// at 16 / 24 / 40 8.8 / 8.0, 9.9 / 9.6, 10.7 / 11.2; 5120 x 5120 at 16 rows 12.1 / 12.7).
-// K slices of it for a weight of fewer than 192 stripes when a workspace is given (1 = none): 256 / stripes workgroups
-// per chunk of four blocks, full chunks whatever the width (weights coming from memory: 4096 x 14336 at 16 / 32 / 64 rows
-// 19.0 / 21.8 / 26.4 us against 29.6 / 43.0 / 68.4 for gemm_skinny_q8_kernel, 8192 x 8192 at 2-64 rows 19.6-28.5 against
-// 23.7-40.3, 6144 x 4096 12.4-17.7 against 12.7-22.2; 4096 x 4096 up to 8 rows 10.2 against 7.7-8.3: two launches, so a
-// weight of 16 M values or fewer only from 16 rows on, or from 8 when its rows are 6144 values and longer, or from 2
-// when they are 8192 values and longer and the stripes 24 at most, as for the 16-bit weights).
-inline bool q8_blocks_pay(int64_t M, int64_t N, int64_t K) {
-    const int64_t stripes = (N + 63) / 64, rows = (stripes > 64 ? 2 : 1) + (M + 15) / 16;
-    if (K > 4096 || M < 2 || M > 64 || stripes < 32 || stripes >= 192) return false;
-    if (stripes >= 96) return rows * K <= 17000 && (M >= 8 || N * K >= INT64_C(20000000));
-    return M >= 16 && rows * K <= (stripes < 64 ? 12500 : stripes == 64 ? 20500 : 17000);
-}
-inline int q8_slices(int64_t M, int64_t N, int64_t K) {
-    if (M < 2 || M > 64 || K % kStripeSeg != 0 || N % 8 != 0) return 1;
-    const bool long_rows = (K >= 6144 && M >= 8) || (K >= 8192 && N <= 24 * 64);
-    if (N * K <= (INT64_C(1) << 24) && M < 16 && !long_rows) return 1;
-    return stripe_slices(M, N, K);
-}
 inline bool q8_stripe_ok(int64_t M, int64_t N, int64_t K, bool aligned) {
     return M >= 2 && M <= 64 && K % kStripeSeg == 0 && aligned &&
            (N >= 10240 || (N >= 8192 && M >= 16) || (N >= 6144 && M > 32) || q8_blocks_pay(M, N, K));
