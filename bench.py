@@ -54,13 +54,14 @@ TRAFFIC_MEASURED_AGAINST = {
     "rmsnorm.hip": "f6c4e575f461",
     "gemm.hip": "e8a1ab9b2e5c",
 }
+_PREFILL_SOURCES, _DECODE_SOURCES = ("attn_common.h", "attn_prefill.hip"), ("attn_common.h", "attn_decode.hip", "quant_q8.h")
+_ROPE_SOURCES, _NORM_SOURCES = ("attn_common.h", "rope.hip", "quant_q8.h"), ("attn_common.h", "rmsnorm.hip")
+_GEMM_SOURCES = ("attn_common.h", "gemm.hip", "gemm_common.h", "gemm_plan.h", "quant_q8.h")
+_TILE_SOURCES = _GEMM_SOURCES + ("gemm_tile.h", "gemm_tile_f16.hip", "gemm_tile_bf16.hip")
 TRAFFIC_ROW_SOURCES = {
-    "": ("attn_common.h", "attn_prefill.hip"), "long_context": ("attn_common.h", "attn_prefill.hip"), "ragged": ("attn_common.h", "attn_prefill.hip"),
-    "decode": ("attn_common.h", "attn_decode.hip"), "decode_q8_0": ("attn_common.h", "attn_decode.hip", "quant_q8.h"),
-    "rope": ("attn_common.h", "rope.hip"), "rope_kv_append": ("attn_common.h", "rope.hip"),
-    "rope_kv_append_q8_0": ("attn_common.h", "rope.hip", "quant_q8.h"), "rope_kv_append_norm": ("attn_common.h", "rope.hip"),
-    "rmsnorm": ("attn_common.h", "rmsnorm.hip"), "gemm": ("attn_common.h", "gemm.hip"), "qkv": ("attn_common.h", "gemm.hip"),
-    "gemm_q8_0": ("attn_common.h", "gemm.hip", "quant_q8.h"), "gemm_decode": ("attn_common.h", "gemm.hip"),
+    "": _PREFILL_SOURCES, "long_context": _PREFILL_SOURCES, "ragged": _PREFILL_SOURCES, "decode": _DECODE_SOURCES, "decode_q8_0": _DECODE_SOURCES,
+    "rope": _ROPE_SOURCES, "rope_kv_append": _ROPE_SOURCES, "rope_kv_append_q8_0": _ROPE_SOURCES, "rope_kv_append_norm": _ROPE_SOURCES,
+    "rmsnorm": _NORM_SOURCES, "gemm": _TILE_SOURCES, "qkv": _TILE_SOURCES, "gemm_q8_0": _GEMM_SOURCES, "gemm_decode": _GEMM_SOURCES,
 }
 
 
@@ -72,7 +73,7 @@ def source_digest(name):
 
 def mark_stale_traffic(rec):
     """Adds "traffic_stale" to every roofline that quotes a traffic constant."""
-    changed = {n for n, d in TRAFFIC_MEASURED_AGAINST.items() if source_digest(n) != d}
+    changed = {n for n in set().union(*TRAFFIC_ROW_SOURCES.values()) if source_digest(n) != TRAFFIC_MEASURED_AGAINST.get(n)}
     for row, sources in TRAFFIC_ROW_SOURCES.items():
         roof = (rec if row == "" else rec[row]).get("roofline", {})
         if roof.get("traffic") is not None:

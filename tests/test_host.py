@@ -491,3 +491,25 @@ extern "C" uintptr_t probe(uintptr_t stream, int current, int owner) {
     assert probe(0x7000, 0, 1) == 0                 # another device's stream
     assert probe(0x7000, 1, 1) == 0                 # a created stream, and the next one at its address
     assert probe(0, 64, 0) == 0                     # a device past the table
+
+
+def test_bench_traffic_is_stale_when_any_source_of_its_kernel_changes():
+    """Every row's sources are its kernel files and the headers that these include, but for those of the host's checks; the digests name
+    files that exist."""
+    import os
+    import re
+
+    import bench
+    csrc = os.path.join(capi.ROOT, "minfer-python_amd", "csrc")
+
+    def included(name):
+        with open(os.path.join(csrc, name)) as f:
+            found = {h for h in re.findall(r'#include "([^"]+)"', f.read()) if h not in ("attn_host.h", "minfer_attn.h")}
+        return found.union(*(included(h) for h in found))
+    for row, sources in bench.TRAFFIC_ROW_SOURCES.items():
+        kernels = [n for n in sources if n.endswith(".hip")]
+        assert kernels, row
+        assert set(sources) == set(kernels).union(*(included(n) for n in kernels)), row
+    assert {"gemm_tile_f16.hip", "gemm_tile_bf16.hip"} <= set(bench.TRAFFIC_ROW_SOURCES["gemm"]) & set(bench.TRAFFIC_ROW_SOURCES["qkv"])
+    for name in bench.TRAFFIC_MEASURED_AGAINST:
+        bench.source_digest(name)
