@@ -20,8 +20,8 @@ template <int M16_, int N16_, int NS_, int OCC_ = 1> struct GemmShape {
 };
 
 // The tiled kernel: a workgroup of four waves (2 x 2) owns a BM x BN tile of D, wave (wm, wn) 16 M16 rows x 16 N16 columns of it.
-// What bounds it: from a round of the largest tiles on the power budget (4096 x 4096 x 14336 runs at 1.6-1.7 GHz of 2.4 with the
-// matrix pipes busy 71-74 % of the cycles, whatever the order of the instructions), below that what a wave issues between its
+// What bounds it: from a round of the largest tiles on the power budget (4096 x 14336 x 4096 and 4096^3 run at 1.6-1.7 GHz of
+// 2.4 with the matrix pipes busy 74 and 76 % of the cycles, whatever the order of the instructions), below that what a wave issues between its
 // MFMAs and the copies.  Four waves rather than eight read a third fewer LDS bytes per flop (a fragment feeds M16 or N16 MFMAs), and
 // with one wave per SIMD everything has to fit in the 12 clocks that an MFMA leaves the issue port: a K step is one basic block, a
 // copy three instructions, and reads and copies share no slot.  Eight waves (2 x 4 or 4 x 2, a copy of seven instructions, results
@@ -270,7 +270,8 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
 
     // ---- epilogue: D = alpha * acc + beta * C.  Register e of a block is n = 4 quad + e, m = l16: stored from the registers an
     // instruction would write 32 bytes to each of 16 rows.  A block row of 16 rows goes through the wave's own part of the LDS
-    // (rows padded by 16 bytes: no conflicts) and leaves in 16-byte pieces of whole rows, C coming in the same way.
+    // (rows padded by 16 bytes: no bank conflicts with N16 = 8, 4 N16 clocks a block row,
+    // 0.5 % of the kernel, with 6 and 7) and leaves in 16-byte pieces of whole rows, C coming in the same way.
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");        // the last MFMAs' results
     __syncthreads();
     constexpr int ROW = N16 * 64 + 16, ITEMS = 32 * N16, IT = (ITEMS + 63) / 64;   // bytes of a padded row; pieces of 8 columns
