@@ -29,30 +29,35 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 # same counter reads for a 1 GiB copy: x2.0 and x1.0), classify+main and split+combine respectively
 # These are figures from those earlier counter runs, not measured in the run that prints them.
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels_pmc.md (rocprofv3 --pmc runs of the same workloads; not re-measured by this run)"
-PREFILL_TRAFFIC_BYTES = 107416 * 1024
-DECODE_TRAFFIC_BYTES = 1092984 * 1024
+PREFILL_TRAFFIC_BYTES = 107316 * 1024
+DECODE_TRAFFIC_BYTES = 1092924 * 1024
 ROPE_TRAFFIC_BYTES = 393314 * 1024          # il_rope on [8,4096,48,128], rotary 64
-APPEND_TRAFFIC_BYTES = 786534 * 1024        # rope_kv_append, B=8 L=4096 Llama-3-8B heads
-NORM_TRAFFIC_BYTES = 786696 * 1024          # rmsnorm on [8,4096,6144]
-GEMM_TRAFFIC_BYTES = 229746 * 1024          # gemm 4096^3 (A and B panels are re-read by several XCDs)
-DECODE_Q8_TRAFFIC_BYTES = 598481 * 1024     # decode over Q8_0 caches (split + combine)
-APPEND_Q8_TRAFFIC_BYTES = 737591 * 1024     # rope_kv_append into Q8_0 caches
-APPEND_NORM_TRAFFIC_BYTES = 786615 * 1024   # rope_kv_append_norm, the same shape
-QKV_TRAFFIC_BYTES = 377777 * 1024           # qkv in one launch, M=K=4096, N=4096+1024+1024
-LONG_TRAFFIC_BYTES = 2721865 * 1024         # long-context prefill (classify + main), S=32768 bf16: the 1 GiB mask once, K/V re-fetched past the 4 MiB L2s
-RAGGED_TRAFFIC_BYTES = 748150 * 1024        # packed ragged prefill (T=20514, Hq=64)
-GEMM_Q8_TRAFFIC_BYTES = 61121 * 1024        # one token against a 14336 x 4096 weight of Q8_0 blocks
-GEMM_DECODE_TRAFFIC_BYTES = 120713 * 1024   # 64 tokens against the same weight in fp16, [N, K]
+APPEND_TRAFFIC_BYTES = 786533 * 1024        # rope_kv_append, B=8 L=4096 Llama-3-8B heads
+NORM_TRAFFIC_BYTES = 786682 * 1024          # rmsnorm on [8,4096,6144]
+GEMM_TRAFFIC_BYTES = 229795 * 1024          # gemm 4096^3 (A and B panels are re-read by several XCDs)
+DECODE_Q8_TRAFFIC_BYTES = 598309 * 1024     # decode over Q8_0 caches (split + combine)
+APPEND_Q8_TRAFFIC_BYTES = 737593 * 1024     # rope_kv_append into Q8_0 caches
+APPEND_NORM_TRAFFIC_BYTES = 786638 * 1024   # rope_kv_append_norm, the same shape
+QKV_TRAFFIC_BYTES = 377984 * 1024           # qkv in one launch, M=K=4096, N=4096+1024+1024
+LONG_TRAFFIC_BYTES = 2721616 * 1024         # long-context prefill (classify + main), S=32768 bf16: the 1 GiB mask once, K/V re-fetched past the 4 MiB L2s
+RAGGED_TRAFFIC_BYTES = 748032 * 1024        # packed ragged prefill (T=20514, Hq=64)
+GEMM_Q8_TRAFFIC_BYTES = 61123 * 1024        # one token against a 14336 x 4096 weight of Q8_0 blocks
+GEMM_DECODE_TRAFFIC_BYTES = 120711 * 1024   # 64 tokens against the same weight in fp16, [N, K]
 # The kernel sources the counter runs were made against (first 12 hex digits of each file's sha1).  A row one of whose
 # sources has changed since carries "traffic_stale": true, so a constant that describes an earlier kernel says so.
 TRAFFIC_MEASURED_AGAINST = {
-    "attn_common.h": "efe4f3bf88e9",
-    "attn_prefill.hip": "c946efbc805b",
-    "attn_decode.hip": "72ec9ae9463e",
+    "attn_common.h": "f00da2487c24",
+    "attn_prefill.hip": "4aa50ccd63dd",
+    "attn_decode.hip": "322fe3fdb487",
     "quant_q8.h": "4fea6a94e300",
-    "rope.hip": "b4fd0618b44e",
-    "rmsnorm.hip": "f6c4e575f461",
-    "gemm.hip": "e8a1ab9b2e5c",
+    "rope.hip": "f03d700b34e7",
+    "rmsnorm.hip": "90740d99856e",
+    "gemm.hip": "106d5e4e5211",
+    "gemm_common.h": "608850fcbd9f",
+    "gemm_plan.h": "a390cbf53d12",
+    "gemm_tile.h": "f07b752e72ff",
+    "gemm_tile_f16.hip": "969b3f4315b6",
+    "gemm_tile_bf16.hip": "d2866de7d66d",
 }
 _PREFILL_SOURCES, _DECODE_SOURCES = ("attn_common.h", "attn_prefill.hip"), ("attn_common.h", "attn_decode.hip", "quant_q8.h")
 _ROPE_SOURCES, _NORM_SOURCES = ("attn_common.h", "rope.hip", "quant_q8.h"), ("attn_common.h", "rmsnorm.hip")
@@ -150,7 +155,7 @@ def cpu_baseline(torch, workloads, refs, L):
 
 
 def cpu_baseline_plumbing(torch, workloads, refs):
-    """BASELINE configs[0] (B=1, Hq=8, Hkv=2, S=256, D=64, fp32): the reference's CPU path on it."""
+    """The CPU-plumbing shape (B=1, Hq=8, Hkv=2, S=256, D=64, fp32): the reference's CPU path on it."""
     q, k, v, mask = workloads.cpu_plumbing(seed=0)
     k, v = k.repeat_interleave(4, 1), v.repeat_interleave(4, 1)
     refs.flash_attn(q, k, v, mask)
@@ -486,7 +491,7 @@ def main():
     q8_gbs = q8bytes / (q8_avg_ms * 1e-3) / 1e9
     del wq8, wq8s, xa, xo
 
-    # ... and for the decode batch of BASELINE configs[2]: 64 tokens against the fp16 weight as [N, K]
+    # ... and for the decode batch: its 64 tokens against the fp16 weight as [N, K]
     gwn = workloads.gemm_input(16, 14336, 4096, seed=3, device=dev)[1].t().contiguous()      # [14336, 4096]
     gwns = [gwn] + [gwn.clone() for _ in range(5)]                                             # 6 x 112 MiB
     gxa = workloads.gemm_input(64, 16, 4096, seed=5, device=dev)[0]                            # [1, 64, 4096]
@@ -503,7 +508,7 @@ def main():
     gd_gbs = gdbytes / (gd_avg_ms * 1e-3) / 1e9
     del gwn, gwns, gxa, gxo
 
-    # ---- BASELINE configs[0] (the CPU-plumbing shape: B=1, Hq=8, Hkv=2, S=256, D=64) through the GPU op; its fp32
+    # ---- the CPU-plumbing shape (B=1, Hq=8, Hkv=2, S=256, D=64) through the GPU op; its fp32
     # inputs are rounded to fp16, the op having no fp32 form.  Two launches of a few microseconds: launch-bound.
     cq, ck, cv, cmask = workloads.cpu_plumbing(seed=0)
     cq, ck, cv, cmask = cq.half().to(dev), ck.half().to(dev), cv.half().to(dev), cmask.to(dev)
@@ -543,13 +548,13 @@ def main():
         "dtype": "f16", "data": "synthetic", "launch": "hipgraph replay of one op call" if args.graph else "eager",
         "ms_is": "every row's ms: back-to-back calls between ONE pair of HIP events on the op's stream, divided by the calls (a pair around "
                  "every call adds 2-3 us, a tenth of the shortest kernels here); median_ms: a pair around every call",
-        "config": {"workload": "prefill B=1 Hq=32 Hkv=8 S=4096 D=128 fp16 causal dense-mask (BASELINE configs[1])",
+        "config": {"workload": "prefill B=1 Hq=32 Hkv=8 S=4096 D=128 fp16 causal dense-mask",
                    "global_batch": 1, "seq_len": L, "parallelism": "single-gpu"},
         "roofline": mfma_roofline(achieved, sus_f16, mix_f16, traffic=PREFILL_TRAFFIC_BYTES, traffic_source=TRAFFIC_SOURCE,
                                   kernel="classify_mask_kernel + prefill_kernel<F16,128,dense>",
                                   algorithmic_flops=flops, avg_ms=avg_ms, median_ms=med_ms),
         "decode": {"value": d_gbs, "unit": "GB/s", "ms": d_avg_ms, "median_ms": d_med_ms,
-                   "workload": "decode B=64 Hq=32 Hkv=8 D=128 fp16 ctx~U[512,8192] cache [64,8,8192,128] (BASELINE configs[2])",
+                   "workload": "decode B=64 Hq=32 Hkv=8 D=128 fp16 ctx~U[512,8192] cache [64,8,8192,128]",
                    "roofline": {"bound": "hbm", "achieved": d_gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                                 "frac": d_gbs / PEAK_HBM_GBS, "traffic": DECODE_TRAFFIC_BYTES, "traffic_source": TRAFFIC_SOURCE,
                                 "kernel": "decode_split_kernel<F16,128> + decode_combine_kernel",
@@ -563,11 +568,11 @@ def main():
                                        "kernel": "decode_split_q8_kernel<128> + decode_combine_kernel",
                                        "algorithmic_bytes": d8bytes}}
     rec["long_context"] = {"value": l_tf, "unit": "TFLOP/s", "ms": l_avg_ms, "median_ms": l_med_ms,
-                           "workload": "prefill B=1 Hq=32 Hkv=8 S=32768 D=128 bf16 causal dense-mask, mask 1 GiB (BASELINE configs[3])",
+                           "workload": "prefill B=1 Hq=32 Hkv=8 S=32768 D=128 bf16 causal dense-mask, mask 1 GiB",
                            "roofline": mfma_roofline(l_tf, sus_bf16, mix_bf16, traffic=LONG_TRAFFIC_BYTES, traffic_source=TRAFFIC_SOURCE,
                                                      kernel="classify_mask_kernel + prefill_kernel<BF16,128,dense>", algorithmic_flops=lflops)}
     rec["ragged"] = {"value": v_tf, "unit": "TFLOP/s", "ms": v_avg_ms, "median_ms": v_med_ms,
-                     "workload": f"packed prefill of 16 sequences, lengths U[128,2048] (T={sum(vlens)}), Hq=64 Hkv=8 D=128 fp16, causal within a sequence (BASELINE configs[4])",
+                     "workload": f"packed prefill of 16 sequences, lengths U[128,2048] (T={sum(vlens)}), Hq=64 Hkv=8 D=128 fp16, causal within a sequence",
                      "roofline": mfma_roofline(v_tf, sus_f16, mix_f16, traffic=RAGGED_TRAFFIC_BYTES, traffic_source=TRAFFIC_SOURCE,
                                                kernel="prefill_kernel<F16,128,varlen>", algorithmic_flops=vflops)}
     rec["rope_kv_append_q8_0"] = {"value": a8_gbs, "unit": "GB/s", "ms": a8_avg_ms, "median_ms": a8_med_ms,
@@ -601,7 +606,7 @@ def main():
                           "roofline": {"bound": "hbm", "achieved": gd_gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": gd_gbs / PEAK_HBM_GBS,
                                        "traffic": GEMM_DECODE_TRAFFIC_BYTES, "traffic_source": TRAFFIC_SOURCE, "kernel": "gemm_stripe_kernel<F16,4>", "algorithmic_bytes": gdbytes}}
     rec["cpu_plumbing"] = {"value": cflops / (c_avg_ms * 1e-3) / 1e12, "unit": "TFLOP/s", "ms": c_avg_ms, "median_ms": c_med_ms,
-                           "workload": "prefill B=1 Hq=8 Hkv=2 S=256 D=64 causal dense-mask, fp32 inputs rounded to fp16 for the GPU op (BASELINE configs[0]); launch-bound"}
+                           "workload": "prefill B=1 Hq=8 Hkv=2 S=256 D=64 causal dense-mask, fp32 inputs rounded to fp16 for the GPU op; launch-bound"}
     rec["calibration"] = {"mfma_only_f16_random": sus_f16, "mfma_only_bf16_random": sus_bf16,
                           "attention_mix_f16_random": mix_f16, "attention_mix_bf16_random": mix_bf16,
                           "note": "mfma_only: v_mfma_f32_16x16x32 alone (the instruction the prefill and GEMM kernels use), two waves per SIMD on every compute unit, operands 0.5*N(0,1); "
