@@ -246,7 +246,7 @@ def main():
     args = ap.parse_args()
     if args.gpus != 1:
         sys.exit("bench.py measures one GPU: the attention path shards by batch / KV head without any "
-                 "exchange, and this build has no multi-GPU launcher. Run with --gpus 1.")
+                 "exchange, and this package has no multi-GPU launcher. Run with --gpus 1.")
 
     import torch
     import workloads
