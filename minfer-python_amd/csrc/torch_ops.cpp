@@ -12,10 +12,11 @@
 // fails in the dispatcher instead of falling back to anything.
 #include <Python.h>
 
+#include <optional>
+
 #include <torch/csrc/inductor/aoti_torch/c/shim.h>
 #include <torch/csrc/stable/accelerator.h>
 #include <torch/csrc/stable/library.h>
-#include <torch/csrc/stable/ops.h>
 #include <torch/csrc/stable/tensor.h>
 #include <torch/headeronly/core/ScalarType.h>
 #include <torch/headeronly/util/Exception.h>
@@ -31,7 +32,6 @@ PyObject* PyInit__C(void) {
 
 namespace minfer {
 
-using torch::headeronly::DeviceType;
 using torch::headeronly::ScalarType;
 using torch::stable::Tensor;
 
@@ -44,20 +44,51 @@ void* current_stream() {
     return stream;
 }
 
-bool on_gpu(const Tensor& t) { return t.device().type() == DeviceType::CUDA; }
+// An operator looks at the type and device of up to nine tensors.  Asked for through the ABI's own numbers they take 3 ns each;
+// as ScalarType and Device they go through the translation of an argument (25 and 16 ns).
+const int32_t kHalf = aoti_torch_dtype_float16(), kBFloat16 = aoti_torch_dtype_bfloat16(), kFloat = aoti_torch_dtype_float32(),
+              kByte = aoti_torch_dtype_uint8(), kInt = aoti_torch_dtype_int32(), kBool = aoti_torch_dtype_bool();
+
+// The types that these operators take; Undefined for any other.
+ScalarType type_of(const Tensor& t) {
+    int32_t d = 0;
+    TORCH_ERROR_CODE_CHECK(aoti_torch_get_dtype(t.get(), &d));
+    if (d == kHalf) return ScalarType::Half;
+    if (d == kBFloat16) return ScalarType::BFloat16;
+    if (d == kByte) return ScalarType::Byte;
+    if (d == kInt) return ScalarType::Int;
+    if (d == kBool) return ScalarType::Bool;
+    return d == kFloat ? ScalarType::Float : ScalarType::Undefined;
+}
+
+bool on_gpu(const Tensor& t) { return t.is_cuda(); }
 
 int dtype_code(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const char* op) {
-    const ScalarType t = q.scalar_type();
+    const ScalarType t = type_of(q);
     STD_TORCH_CHECK(t == ScalarType::Half || t == ScalarType::BFloat16, op, ": q must be float16 or bfloat16");
-    STD_TORCH_CHECK(k.scalar_type() == t && v.scalar_type() == t && out.scalar_type() == t, op,
+    STD_TORCH_CHECK(type_of(k) == t && type_of(v) == t && type_of(out) == t, op,
                     ": q, k, v and out must share one dtype");
     return t == ScalarType::Half ? MINFER_ATTN_F16 : MINFER_ATTN_BF16;
 }
 
-Tensor byte_workspace(const Tensor& like, size_t nbytes) {
-    const int64_t n = (int64_t)nbytes;
-    return torch::stable::new_empty(like, {n}, ScalarType::Byte);
-}
+// Scratch memory on a tensor's device, from torch's allocator and so for the current stream; none at all for a call that needs
+// none.  (new_empty by the name of its operator, for every call, was 0.9 us of the 6 that issuing one took.)
+class Workspace {
+public:
+    Workspace(const Tensor& like, size_t nbytes) {
+        if (nbytes == 0) return;
+        const int64_t n = (int64_t)nbytes, one = 1;
+        AtenTensorHandle h = nullptr;
+        TORCH_ERROR_CODE_CHECK(aoti_torch_empty_strided(1, &n, &one, kByte, aoti_torch_device_type_cuda(), like.get_device_index(), &h));
+        memory_.emplace(h);
+        ptr_ = memory_->mutable_data_ptr();
+    }
+    void* ptr() const { return ptr_; }
+
+private:
+    std::optional<Tensor> memory_;
+    void* ptr_ = nullptr;
+};
 
 void check_rc(int rc, const char* op) {
     STD_TORCH_CHECK(rc == MINFER_ATTN_OK, op, ": ", minfer_attn_last_error());
@@ -78,14 +109,14 @@ static void flash_attn_q8_0(int64_t qblock_size, int64_t qtype_size, const Tenso
                     "flash_attn: Q8_0 has qblock_size 32 and qtype_size 34");
     STD_TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4 && out.dim() == 4 && mask.dim() == 4,
                     "flash_attn: q, k, v, mask and out must be 4-D");
-    STD_TORCH_CHECK(q.scalar_type() == ScalarType::Half && out.scalar_type() == ScalarType::Half,
+    STD_TORCH_CHECK(type_of(q) == ScalarType::Half && type_of(out) == ScalarType::Half,
                     "flash_attn: q and out must be float16 over Q8_0 k/v");
-    STD_TORCH_CHECK(k.scalar_type() == ScalarType::Byte && v.scalar_type() == ScalarType::Byte, "flash_attn: Q8_0 k and v must be uint8");
+    STD_TORCH_CHECK(type_of(k) == ScalarType::Byte && type_of(v) == ScalarType::Byte, "flash_attn: Q8_0 k and v must be uint8");
     STD_TORCH_CHECK(q.stride(-1) == 1 && k.stride(-1) == 1 && v.stride(-1) == 1 && out.stride(-1) == 1,
                     "flash_attn: q, k, v and out must be contiguous in their last dimension");
     STD_TORCH_CHECK(k.stride(0) == v.stride(0) && k.stride(1) == v.stride(1) && k.stride(2) == v.stride(2),
                     "flash_attn: k and v must share strides");
-    STD_TORCH_CHECK(mask.is_contiguous() && mask.scalar_type() == ScalarType::Bool, "flash_attn: mask must be contiguous bool");
+    STD_TORCH_CHECK(mask.is_contiguous() && type_of(mask) == ScalarType::Bool, "flash_attn: mask must be contiguous bool");
     STD_TORCH_CHECK(q.sizes().equals(out.sizes()) && k.sizes().equals(v.sizes()), "flash_attn: q/out or k/v shapes differ");
     const int64_t B = q.size(0), Hq = q.size(1), Hkv = k.size(1), L = q.size(2), D = q.size(3);
     STD_TORCH_CHECK(D == 128 || D == 64, "flash_attn: head_dim must be 128 or 64");
@@ -95,10 +126,10 @@ static void flash_attn_q8_0(int64_t qblock_size, int64_t qtype_size, const Tenso
     if (B == 0 || L == 0) return;
     const minfer_attn_strides st = strides_of(q, k, out);   // a byte tensor's strides are byte strides
     const size_t ws_bytes = minfer_flash_attn_q8_0_workspace_bytes(B, Hkv, L, D);
-    Tensor ws = byte_workspace(q, ws_bytes);
+    const Workspace ws(q, ws_bytes);
     check_rc(minfer_flash_attn_q8_0(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(),
                                     static_cast<const uint8_t*>(mask.const_data_ptr()), out.mutable_data_ptr(), B, Hq, Hkv, L, D,
-                                    &st, ws.mutable_data_ptr(), ws_bytes, current_stream()),
+                                    &st, ws.ptr(), ws_bytes, current_stream()),
              "flash_attn");
 }
 
@@ -119,7 +150,7 @@ void flash_attn_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype_size,
         flash_attn_q8_0(qblock_size, qtype_size, q, k, v, mask, out);
         return;
     }
-    STD_TORCH_CHECK(k.scalar_type() != ScalarType::Byte, "flash_attn: byte k/v need qtype_int = 8 (Q8_0)");
+    STD_TORCH_CHECK(type_of(k) != ScalarType::Byte, "flash_attn: byte k/v need qtype_int = 8 (Q8_0)");
     STD_TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4 && out.dim() == 4 && mask.dim() == 4,
                     "flash_attn: q, k, v, mask and out must be 4-D");
     STD_TORCH_CHECK(q.stride(-1) == 1 && k.stride(-1) == 1 && v.stride(-1) == 1 && out.stride(-1) == 1,
@@ -128,7 +159,7 @@ void flash_attn_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype_size,
                     "flash_attn: k and v must share strides");
     STD_TORCH_CHECK(mask.is_contiguous(), "flash_attn: mask must be contiguous");
     const int dtype = dtype_code(q, k, v, out, "flash_attn");
-    STD_TORCH_CHECK(mask.scalar_type() == ScalarType::Bool, "flash_attn: mask must be bool");
+    STD_TORCH_CHECK(type_of(mask) == ScalarType::Bool, "flash_attn: mask must be bool");
     STD_TORCH_CHECK(q.sizes().equals(out.sizes()), "flash_attn: q and out shapes differ");
     STD_TORCH_CHECK(k.sizes().equals(v.sizes()), "flash_attn: k and v shapes differ");
     STD_TORCH_CHECK(q.size(0) == k.size(0) && q.size(0) == mask.size(0) && mask.size(1) == 1 &&
@@ -141,10 +172,10 @@ void flash_attn_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype_size,
 
     const minfer_attn_strides st = strides_of(q, k, out);
     const size_t ws_bytes = minfer_flash_attn_workspace_bytes(B, L);
-    Tensor ws = byte_workspace(q, ws_bytes);
+    const Workspace ws(q, ws_bytes);
     check_rc(minfer_flash_attn(dtype, q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(),
                                static_cast<const uint8_t*>(mask.const_data_ptr()), out.mutable_data_ptr(),
-                               B, Hq, Hkv, L, D, &st, ws.mutable_data_ptr(), ws_bytes, current_stream()),
+                               B, Hq, Hkv, L, D, &st, ws.ptr(), ws_bytes, current_stream()),
              "flash_attn");
 }
 
@@ -157,15 +188,15 @@ static void flash_attn_decode_q8_0(int64_t qblock_size, int64_t qtype_size, cons
                     "flash_attn_decode: Q8_0 has qblock_size 32 and qtype_size 34");
     STD_TORCH_CHECK(q.dim() == 4 && k_cache.dim() == 4 && v_cache.dim() == 4 && out.dim() == 4 && ctx_lens.dim() == 1,
                     "flash_attn_decode: q, k_cache, v_cache, out must be 4-D and ctx_lens 1-D");
-    STD_TORCH_CHECK(q.scalar_type() == ScalarType::Half && out.scalar_type() == ScalarType::Half,
+    STD_TORCH_CHECK(type_of(q) == ScalarType::Half && type_of(out) == ScalarType::Half,
                     "flash_attn_decode: q and out must be float16 over Q8_0 caches");
-    STD_TORCH_CHECK(k_cache.scalar_type() == ScalarType::Byte && v_cache.scalar_type() == ScalarType::Byte,
+    STD_TORCH_CHECK(type_of(k_cache) == ScalarType::Byte && type_of(v_cache) == ScalarType::Byte,
                     "flash_attn_decode: Q8_0 caches must be uint8");
     STD_TORCH_CHECK(q.stride(-1) == 1 && k_cache.stride(-1) == 1 && v_cache.stride(-1) == 1 && out.stride(-1) == 1,
                     "flash_attn_decode: tensors must be contiguous in their last dimension");
     STD_TORCH_CHECK(k_cache.stride(0) == v_cache.stride(0) && k_cache.stride(1) == v_cache.stride(1) &&
                     k_cache.stride(2) == v_cache.stride(2), "flash_attn_decode: k_cache and v_cache must share strides");
-    STD_TORCH_CHECK(ctx_lens.scalar_type() == ScalarType::Int && ctx_lens.is_contiguous(),
+    STD_TORCH_CHECK(type_of(ctx_lens) == ScalarType::Int && ctx_lens.is_contiguous(),
                     "flash_attn_decode: ctx_lens must be contiguous int32");
     STD_TORCH_CHECK(q.sizes().equals(out.sizes()), "flash_attn_decode: q and out shapes differ");
     STD_TORCH_CHECK(k_cache.sizes().equals(v_cache.sizes()), "flash_attn_decode: cache shapes differ");
@@ -177,10 +208,10 @@ static void flash_attn_decode_q8_0(int64_t qblock_size, int64_t qtype_size, cons
     if (B == 0) return;
     const minfer_attn_strides st = strides_of(q, k_cache, out);   // a byte tensor's strides are byte strides
     const size_t ws_bytes = minfer_flash_attn_decode_workspace_bytes(B, Hq, Lmax, D);
-    Tensor ws = byte_workspace(q, ws_bytes);
+    const Workspace ws(q, ws_bytes);
     check_rc(minfer_flash_attn_decode_q8_0(q.const_data_ptr(), k_cache.const_data_ptr(), v_cache.const_data_ptr(),
                                            static_cast<const int32_t*>(ctx_lens.const_data_ptr()), out.mutable_data_ptr(),
-                                           B, Hq, Hkv, Lmax, D, &st, ws.mutable_data_ptr(), ws_bytes, current_stream()),
+                                           B, Hq, Hkv, Lmax, D, &st, ws.ptr(), ws_bytes, current_stream()),
              "flash_attn_decode");
 }
 
@@ -198,7 +229,7 @@ void flash_attn_decode_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype
         return;
     }
     // any other value describes caches of q's own type, as the reference's callers pass it (F16 = 1)
-    STD_TORCH_CHECK(k_cache.scalar_type() != ScalarType::Byte, "flash_attn_decode: byte caches need qtype_int = 8 (Q8_0)");
+    STD_TORCH_CHECK(type_of(k_cache) != ScalarType::Byte, "flash_attn_decode: byte caches need qtype_int = 8 (Q8_0)");
     STD_TORCH_CHECK(q.dim() == 4 && k_cache.dim() == 4 && v_cache.dim() == 4 && out.dim() == 4 && ctx_lens.dim() == 1,
                     "flash_attn_decode: q, k_cache, v_cache, out must be 4-D and ctx_lens 1-D");
     STD_TORCH_CHECK(q.stride(-1) == 1 && k_cache.stride(-1) == 1 && v_cache.stride(-1) == 1 && out.stride(-1) == 1,
@@ -206,7 +237,7 @@ void flash_attn_decode_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype
     STD_TORCH_CHECK(k_cache.stride(0) == v_cache.stride(0) && k_cache.stride(1) == v_cache.stride(1) &&
                     k_cache.stride(2) == v_cache.stride(2), "flash_attn_decode: k_cache and v_cache must share strides");
     const int dtype = dtype_code(q, k_cache, v_cache, out, "flash_attn_decode");
-    STD_TORCH_CHECK(ctx_lens.scalar_type() == ScalarType::Int && ctx_lens.is_contiguous(),
+    STD_TORCH_CHECK(type_of(ctx_lens) == ScalarType::Int && ctx_lens.is_contiguous(),
                     "flash_attn_decode: ctx_lens must be contiguous int32");
     STD_TORCH_CHECK(q.sizes().equals(out.sizes()), "flash_attn_decode: q and out shapes differ");
     STD_TORCH_CHECK(k_cache.sizes().equals(v_cache.sizes()), "flash_attn_decode: cache shapes differ");
@@ -219,10 +250,10 @@ void flash_attn_decode_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype
 
     const minfer_attn_strides st = strides_of(q, k_cache, out);
     const size_t ws_bytes = minfer_flash_attn_decode_workspace_bytes(B, Hq, Lmax, D);
-    Tensor ws = byte_workspace(q, ws_bytes);
+    const Workspace ws(q, ws_bytes);
     check_rc(minfer_flash_attn_decode(dtype, q.const_data_ptr(), k_cache.const_data_ptr(), v_cache.const_data_ptr(),
                                       static_cast<const int32_t*>(ctx_lens.const_data_ptr()), out.mutable_data_ptr(),
-                                      B, Hq, Hkv, Lmax, D, &st, ws.mutable_data_ptr(), ws_bytes, current_stream()),
+                                      B, Hq, Hkv, Lmax, D, &st, ws.ptr(), ws_bytes, current_stream()),
              "flash_attn_decode");
 }
 
@@ -241,13 +272,13 @@ void flash_attn_varlen_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype
     if (qtype_int == MINFER_Q8_0) {   // k and v as Q8_0 blocks: uint8 [1, n_kv_heads, T, HEAD_DIM/32 * 34], q and out float16
         STD_TORCH_CHECK(qblock_size == MINFER_Q8_0_BLOCK && qtype_size == MINFER_Q8_0_BLOCK_BYTES,
                         "flash_attn_varlen: Q8_0 has qblock_size 32 and qtype_size 34");
-        STD_TORCH_CHECK(q.scalar_type() == ScalarType::Half && out.scalar_type() == ScalarType::Half &&
-                        k.scalar_type() == ScalarType::Byte && v.scalar_type() == ScalarType::Byte,
+        STD_TORCH_CHECK(type_of(q) == ScalarType::Half && type_of(out) == ScalarType::Half &&
+                        type_of(k) == ScalarType::Byte && type_of(v) == ScalarType::Byte,
                         "flash_attn_varlen: over Q8_0 k/v, q and out must be float16 and k, v uint8");
         STD_TORCH_CHECK(q.stride(-1) == 1 && k.stride(-1) == 1 && v.stride(-1) == 1 && out.stride(-1) == 1 &&
                         k.stride(1) == v.stride(1) && k.stride(2) == v.stride(2),
                         "flash_attn_varlen: tensors must be contiguous in their last dimension, k and v share strides");
-        STD_TORCH_CHECK(cu_seqlens.scalar_type() == ScalarType::Int && cu_seqlens.is_contiguous() && cu_seqlens.size(0) >= 1,
+        STD_TORCH_CHECK(type_of(cu_seqlens) == ScalarType::Int && cu_seqlens.is_contiguous() && cu_seqlens.size(0) >= 1,
                         "flash_attn_varlen: cu_seqlens must be contiguous int32 with at least one entry");
         STD_TORCH_CHECK(q.sizes().equals(out.sizes()) && k.sizes().equals(v.sizes()), "flash_attn_varlen: q/out or k/v shapes differ");
         const int64_t Hq8 = q.size(1), Hkv8 = k.size(1), T8 = q.size(2), D8 = q.size(3);
@@ -258,20 +289,20 @@ void flash_attn_varlen_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype
         if (n8 == 0 || T8 == 0) return;
         const minfer_attn_strides st8 = strides_of(q, k, out);
         const size_t ws_bytes = minfer_flash_attn_varlen_q8_0_workspace_bytes(Hkv8, T8, D8);
-        Tensor ws = byte_workspace(q, ws_bytes);
+        const Workspace ws(q, ws_bytes);
         check_rc(minfer_flash_attn_varlen_q8_0(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(),
                                                static_cast<const int32_t*>(cu_seqlens.const_data_ptr()), n8, max_seqlen,
-                                               out.mutable_data_ptr(), Hq8, Hkv8, T8, D8, &st8, ws.mutable_data_ptr(), ws_bytes,
+                                               out.mutable_data_ptr(), Hq8, Hkv8, T8, D8, &st8, ws.ptr(), ws_bytes,
                                                current_stream()),
                  "flash_attn_varlen");
         return;
     }
-    STD_TORCH_CHECK(k.scalar_type() != ScalarType::Byte, "flash_attn_varlen: byte k/v need qtype_int = 8 (Q8_0)");
+    STD_TORCH_CHECK(type_of(k) != ScalarType::Byte, "flash_attn_varlen: byte k/v need qtype_int = 8 (Q8_0)");
     STD_TORCH_CHECK(q.stride(-1) == 1 && k.stride(-1) == 1 && v.stride(-1) == 1 && out.stride(-1) == 1,
                     "flash_attn_varlen: tensors must be contiguous in head_dim");
     STD_TORCH_CHECK(k.stride(1) == v.stride(1) && k.stride(2) == v.stride(2), "flash_attn_varlen: k and v must share strides");
     const int dtype = dtype_code(q, k, v, out, "flash_attn_varlen");
-    STD_TORCH_CHECK(cu_seqlens.scalar_type() == ScalarType::Int && cu_seqlens.is_contiguous() && cu_seqlens.size(0) >= 1,
+    STD_TORCH_CHECK(type_of(cu_seqlens) == ScalarType::Int && cu_seqlens.is_contiguous() && cu_seqlens.size(0) >= 1,
                     "flash_attn_varlen: cu_seqlens must be contiguous int32 with at least one entry");
     STD_TORCH_CHECK(q.sizes().equals(out.sizes()), "flash_attn_varlen: q and out shapes differ");
     STD_TORCH_CHECK(k.sizes().equals(v.sizes()), "flash_attn_varlen: k and v shapes differ");
@@ -298,7 +329,7 @@ void rope_hip(int style, const char* op, int64_t rotary_dim, int64_t start_pos, 
     STD_TORCH_CHECK(on_gpu(x), op, ": x must be on the GPU");
     STD_TORCH_CHECK(x.is_contiguous(), op, ": x must be contiguous");
     STD_TORCH_CHECK(x.dim() == 4, op, ": x must be 4-D");
-    const ScalarType t = x.scalar_type();
+    const ScalarType t = type_of(x);
     STD_TORCH_CHECK(t == ScalarType::Half || t == ScalarType::BFloat16, op, ": x must be float16 or bfloat16");
     STD_TORCH_CHECK(rotary_dim <= x.size(3), op, ": rotary_dim exceeds head_dim");
     check_rc(minfer_rope(t == ScalarType::Half ? MINFER_ATTN_F16 : MINFER_ATTN_BF16, style, x.mutable_data_ptr(),
@@ -331,10 +362,10 @@ void rope_kv_append_hip(int64_t style, int64_t rotary_dim, double freq_base,
                     "rope_kv_append: q, k, v and the caches must be 4-D and positions 1-D");
     STD_TORCH_CHECK(q.is_contiguous() && k.is_contiguous() && v.is_contiguous(), "rope_kv_append: q, k and v must be contiguous");
     STD_TORCH_CHECK(style == MINFER_ROPE_INTERLEAVED || style == MINFER_ROPE_NEOX, "rope_kv_append: style must be 0 (interleaved) or 1 (NeoX)");
-    const bool q8 = k_cache.scalar_type() == ScalarType::Byte;   // Q8_0 caches: [B, n_kv_heads, Lmax, head_dim/32 * 34] bytes
+    const bool q8 = type_of(k_cache) == ScalarType::Byte;   // Q8_0 caches: [B, n_kv_heads, Lmax, head_dim/32 * 34] bytes
     const int dtype = dtype_code(q, k, v, q8 ? q : k_cache, "rope_kv_append");
-    STD_TORCH_CHECK(v_cache.scalar_type() == k_cache.scalar_type(), "rope_kv_append: caches must share q's dtype, or both be uint8 (Q8_0)");
-    STD_TORCH_CHECK(positions.scalar_type() == ScalarType::Int && positions.is_contiguous(), "rope_kv_append: positions must be contiguous int32");
+    STD_TORCH_CHECK(type_of(v_cache) == type_of(k_cache), "rope_kv_append: caches must share q's dtype, or both be uint8 (Q8_0)");
+    STD_TORCH_CHECK(type_of(positions) == ScalarType::Int && positions.is_contiguous(), "rope_kv_append: positions must be contiguous int32");
     STD_TORCH_CHECK(k.sizes().equals(v.sizes()) && k_cache.sizes().equals(v_cache.sizes()), "rope_kv_append: k/v or cache shapes differ");
     STD_TORCH_CHECK(k_cache.stride(-1) == 1 && v_cache.stride(-1) == 1 && k_cache.stride(0) == v_cache.stride(0) &&
                     k_cache.stride(1) == v_cache.stride(1) && k_cache.stride(2) == v_cache.stride(2),
@@ -381,12 +412,12 @@ void rope_kv_append_norm_hip(int64_t style, int64_t rotary_dim, double freq_base
     STD_TORCH_CHECK(q.is_contiguous() && k.is_contiguous() && v.is_contiguous() && wq_norm.is_contiguous() && wk_norm.is_contiguous(),
                     "rope_kv_append_norm: q, k, v and the norm weights must be contiguous");
     STD_TORCH_CHECK(style == MINFER_ROPE_INTERLEAVED || style == MINFER_ROPE_NEOX, "rope_kv_append_norm: style must be 0 (interleaved) or 1 (NeoX)");
-    const bool q8 = k_cache.scalar_type() == ScalarType::Byte;
+    const bool q8 = type_of(k_cache) == ScalarType::Byte;
     const int dtype = dtype_code(q, k, v, q8 ? q : k_cache, "rope_kv_append_norm");
-    STD_TORCH_CHECK(wq_norm.scalar_type() == q.scalar_type() && wk_norm.scalar_type() == q.scalar_type(),
+    STD_TORCH_CHECK(type_of(wq_norm) == type_of(q) && type_of(wk_norm) == type_of(q),
                     "rope_kv_append_norm: norm weights must have q's dtype");
-    STD_TORCH_CHECK(v_cache.scalar_type() == k_cache.scalar_type(), "rope_kv_append_norm: caches must share q's dtype, or both be uint8 (Q8_0)");
-    STD_TORCH_CHECK(positions.scalar_type() == ScalarType::Int && positions.is_contiguous(), "rope_kv_append_norm: positions must be contiguous int32");
+    STD_TORCH_CHECK(type_of(v_cache) == type_of(k_cache), "rope_kv_append_norm: caches must share q's dtype, or both be uint8 (Q8_0)");
+    STD_TORCH_CHECK(type_of(positions) == ScalarType::Int && positions.is_contiguous(), "rope_kv_append_norm: positions must be contiguous int32");
     STD_TORCH_CHECK(k.sizes().equals(v.sizes()) && k_cache.sizes().equals(v_cache.sizes()), "rope_kv_append_norm: k/v or cache shapes differ");
     STD_TORCH_CHECK(k_cache.stride(-1) == 1 && v_cache.stride(-1) == 1 && k_cache.stride(0) == v_cache.stride(0) &&
                     k_cache.stride(1) == v_cache.stride(1) && k_cache.stride(2) == v_cache.stride(2),
@@ -413,9 +444,9 @@ void rmsnorm_hip(double eps,
                  Tensor& out) {      // same shape as in
     STD_TORCH_CHECK(on_gpu(in) && on_gpu(w) && on_gpu(out), "rmsnorm: all tensors must be on the GPU");
     STD_TORCH_CHECK(in.is_contiguous() && out.is_contiguous() && w.is_contiguous(), "rmsnorm: tensors must be contiguous");
-    const ScalarType t = in.scalar_type();
+    const ScalarType t = type_of(in);
     STD_TORCH_CHECK(t == ScalarType::Half || t == ScalarType::BFloat16, "rmsnorm: input must be float16 or bfloat16");
-    STD_TORCH_CHECK(out.scalar_type() == t && w.scalar_type() == t, "rmsnorm: input, w and out must share one dtype");
+    STD_TORCH_CHECK(type_of(out) == t && type_of(w) == t, "rmsnorm: input, w and out must share one dtype");
     STD_TORCH_CHECK(in.dim() == 3 || in.dim() == 4, "rmsnorm: input must be 3-D or 4-D");
     STD_TORCH_CHECK(in.sizes().equals(out.sizes()), "rmsnorm: input and out shapes differ");
     STD_TORCH_CHECK(w.dim() == 1 && w.size(0) > 0 && (in.size(-1) == w.size(0) || in.size(-1) % w.size(0) == 0),
@@ -442,9 +473,9 @@ void gemm_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype_size, double
         // B [out_dim, in_dim / 32 * 34] bytes: alpha * A B^T + beta * C over the dequantised weight (reference:
         // gemm/op.cuh:299-312 routes this case to dispatch_quant_abt, which is empty there)
         STD_TORCH_CHECK(qblock_size == 32 && qtype_size == 34, "gemm: Q8_0 is (qblock_size, qtype_size) = (32, 34)");
-        STD_TORCH_CHECK(A.scalar_type() == ScalarType::Half && C.scalar_type() == ScalarType::Half && D.scalar_type() == ScalarType::Half,
+        STD_TORCH_CHECK(type_of(A) == ScalarType::Half && type_of(C) == ScalarType::Half && type_of(D) == ScalarType::Half,
                         "gemm: A, C and D must be float16 with a Q8_0 weight");
-        STD_TORCH_CHECK(B.scalar_type() == ScalarType::Byte, "gemm: a Q8_0 weight is a uint8 tensor");
+        STD_TORCH_CHECK(type_of(B) == ScalarType::Byte, "gemm: a Q8_0 weight is a uint8 tensor");
         STD_TORCH_CHECK(A.dim() == 3 && B.dim() == 2 && C.dim() == 3 && D.dim() == 3, "gemm: A, C, D must be 3-D and B 2-D");
         STD_TORCH_CHECK(A.is_contiguous() && B.is_contiguous() && C.is_contiguous() && D.is_contiguous(), "gemm: tensors must be contiguous");
         const int64_t K = A.size(-1), M = A.numel() / (K > 0 ? K : 1), N = B.size(0);
@@ -459,16 +490,16 @@ void gemm_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype_size, double
         const auto misaligned = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) != 0; };
         if (ws_bytes == 0 && (misaligned(A.const_data_ptr()) || misaligned(D.const_data_ptr()) || (beta != 0.0 && misaligned(C.const_data_ptr()))))
             ws_bytes = ((static_cast<size_t>(N) * static_cast<size_t>(K) * 2 + 255) & ~static_cast<size_t>(255)) + minfer_gemm_layout_workspace_bytes(MINFER_GEMM_B_NK, M, N, K);
-        Tensor ws = byte_workspace(A, ws_bytes);
+        const Workspace ws(A, ws_bytes);
         check_rc(minfer_gemm_q8_0(A.const_data_ptr(), B.const_data_ptr(), C.const_data_ptr(), D.mutable_data_ptr(), M, N, K, K, N, N,
-                                  alpha, beta, ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, current_stream()),
+                                  alpha, beta, ws.ptr(), ws_bytes, current_stream()),
                  "gemm");
         return;
     }
     (void)qblock_size; (void)qtype_size;
-    const ScalarType t = A.scalar_type();
+    const ScalarType t = type_of(A);
     STD_TORCH_CHECK(t == ScalarType::Half || t == ScalarType::BFloat16, "gemm: A must be float16 or bfloat16");
-    STD_TORCH_CHECK(B.scalar_type() == t && C.scalar_type() == t && D.scalar_type() == t, "gemm: A, B, C and D must share one dtype");
+    STD_TORCH_CHECK(type_of(B) == t && type_of(C) == t && type_of(D) == t, "gemm: A, B, C and D must share one dtype");
     STD_TORCH_CHECK(A.dim() == 3 && B.dim() == 2 && C.dim() == 3 && D.dim() == 3, "gemm: A, C, D must be 3-D and B 2-D");
     STD_TORCH_CHECK(A.is_contiguous() && B.is_contiguous() && C.is_contiguous() && D.is_contiguous(), "gemm: tensors must be contiguous");
     const int64_t K = A.size(-1), M = A.numel() / (K > 0 ? K : 1);
@@ -480,10 +511,10 @@ void gemm_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype_size, double
     STD_TORCH_CHECK(alpha != 0.0, "gemm: alpha must not be 0");
     // a few dozen rows against a wide weight run as K slices that meet in a workspace
     const size_t ws_bytes = minfer_gemm_layout_workspace_bytes(kn ? MINFER_GEMM_B_KN : MINFER_GEMM_B_NK, M, N, K);
-    Tensor ws = byte_workspace(A, ws_bytes);
+    const Workspace ws(A, ws_bytes);
     check_rc(minfer_gemm_ws(t == ScalarType::Half ? MINFER_ATTN_F16 : MINFER_ATTN_BF16, kn ? MINFER_GEMM_B_KN : MINFER_GEMM_B_NK,
                             A.const_data_ptr(), B.const_data_ptr(), C.const_data_ptr(), D.mutable_data_ptr(), M, N, K, K,
-                            kn ? N : K, N, N, alpha, beta, ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, current_stream()),
+                            kn ? N : K, N, N, alpha, beta, ws.ptr(), ws_bytes, current_stream()),
              "gemm");
 }
 
@@ -502,7 +533,7 @@ void qkv_hip(int64_t q_qtype_int, int64_t k_qtype_int, int64_t v_qtype_int, int6
              Tensor& v_out) {    // [B, L, kv_dim]
     const int64_t qtypes[3] = {q_qtype_int, k_qtype_int, v_qtype_int};
     const int64_t qblocks[3] = {q_qblock_size, k_qblock_size, v_qblock_size}, qsizes[3] = {q_qtype_size, k_qtype_size, v_qtype_size};
-    const ScalarType t = x.scalar_type();
+    const ScalarType t = type_of(x);
     STD_TORCH_CHECK(t == ScalarType::Half || t == ScalarType::BFloat16, "qkv: x must be float16 or bfloat16");
     STD_TORCH_CHECK(x.dim() == 3 && x.is_contiguous() && on_gpu(x), "qkv: x must be a contiguous 3-D GPU tensor");
     const int64_t K = x.size(-1), M = x.numel() / (K > 0 ? K : 1);
@@ -523,27 +554,26 @@ void qkv_hip(int64_t q_qtype_int, int64_t k_qtype_int, int64_t v_qtype_int, int6
             const size_t need = qtypes[i] == MINFER_Q8_0 ? minfer_gemm_q8_0_workspace_bytes(M, N, K) : minfer_gemm_layout_workspace_bytes(MINFER_GEMM_B_NK, M, N, K);
             ws_max = need > ws_max ? need : ws_max;
         }
-        Tensor wsp = byte_workspace(x, ws_max);
-        void* wsp_ptr = ws_max ? wsp.mutable_data_ptr() : nullptr;
-        for (int i = 0; i < 3; ++i) {
+        const Workspace wsp(x, ws_max);
+            for (int i = 0; i < 3; ++i) {
             const Tensor& w = *ws[i];
             Tensor& o = *outs[i];
-            STD_TORCH_CHECK(on_gpu(w) && on_gpu(o) && o.scalar_type() == t, names[i], ": dtype or device mismatch");
+            STD_TORCH_CHECK(on_gpu(w) && on_gpu(o) && type_of(o) == t, names[i], ": dtype or device mismatch");
             STD_TORCH_CHECK(w.dim() == 2 && o.dim() == 3 && w.is_contiguous() && o.is_contiguous(), names[i], ": weight must be contiguous 2-D, output contiguous 3-D");
             STD_TORCH_CHECK(o.size(0) == x.size(0) && o.size(1) == x.size(1), names[i], ": output must be [B, L, out_dim]");
             const int64_t N = o.size(-1);
             if (qtypes[i] == MINFER_Q8_0) {
                 STD_TORCH_CHECK(qblocks[i] == MINFER_Q8_0_BLOCK && qsizes[i] == MINFER_Q8_0_BLOCK_BYTES, names[i], ": Q8_0 is (qblock_size, qtype_size) = (32, 34)");
-                STD_TORCH_CHECK(w.scalar_type() == ScalarType::Byte && w.size(0) == N && w.size(1) == K / 32 * 34, names[i],
+                STD_TORCH_CHECK(type_of(w) == ScalarType::Byte && w.size(0) == N && w.size(1) == K / 32 * 34, names[i],
                                 ": a Q8_0 weight is uint8 [out_dim, hidden_dim / 32 * 34]");
                 check_rc(minfer_gemm_q8_0(x.const_data_ptr(), w.const_data_ptr(), nullptr, o.mutable_data_ptr(), M, N, K, K, N, N, 1.0, 0.0,
-                                          wsp_ptr, ws_max, stream),
+                                          wsp.ptr(), ws_max, stream),
                          names[i]);
             } else {
-                STD_TORCH_CHECK(qtypes[i] == 1 && w.scalar_type() == t && w.size(0) == N && w.size(1) == K, names[i],
+                STD_TORCH_CHECK(qtypes[i] == 1 && type_of(w) == t && w.size(0) == N && w.size(1) == K, names[i],
                                 ": next to a Q8_0 weight, a 16-bit weight must be float16 [out_dim, hidden_dim]");
                 check_rc(minfer_gemm_ws(dtype, MINFER_GEMM_B_NK, x.const_data_ptr(), w.const_data_ptr(), nullptr, o.mutable_data_ptr(), M, N, K, K, K, N, N,
-                                        1.0, 0.0, wsp_ptr, ws_max, stream),
+                                        1.0, 0.0, wsp.ptr(), ws_max, stream),
                          names[i]);
             }
         }
@@ -555,7 +585,7 @@ void qkv_hip(int64_t q_qtype_int, int64_t k_qtype_int, int64_t v_qtype_int, int6
     for (int i = 0; i < 3; ++i) {
         const Tensor& w = *ws[i];
         Tensor& o = *outs[i];
-        STD_TORCH_CHECK(on_gpu(w) && on_gpu(o) && w.scalar_type() == t && o.scalar_type() == t, names[i], ": dtype or device mismatch");
+        STD_TORCH_CHECK(on_gpu(w) && on_gpu(o) && type_of(w) == t && type_of(o) == t, names[i], ": dtype or device mismatch");
         STD_TORCH_CHECK(w.dim() == 2 && o.dim() == 3 && w.is_contiguous() && o.is_contiguous(), names[i], ": weight must be contiguous 2-D, output contiguous 3-D");
         const int64_t N = o.size(-1);
         STD_TORCH_CHECK(o.size(0) == x.size(0) && o.size(1) == x.size(1), names[i], ": output must be [B, L, out_dim]");
@@ -591,12 +621,12 @@ void dequant_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype_size, con
     STD_TORCH_CHECK(on_gpu(x) && on_gpu(y), "dequant: x and y must be on the GPU");
     STD_TORCH_CHECK(x.dim() == 2 && y.dim() == 2);
     STD_TORCH_CHECK(x.size(0) == y.size(0), "x and y must have the same number of rows");
-    STD_TORCH_CHECK(x.scalar_type() == ScalarType::Byte, "x must be uint8 (byte)");
-    STD_TORCH_CHECK(y.scalar_type() == ScalarType::Float || y.scalar_type() == ScalarType::Half, "y must be float32 or float16");
+    STD_TORCH_CHECK(type_of(x) == ScalarType::Byte, "x must be uint8 (byte)");
+    STD_TORCH_CHECK(type_of(y) == ScalarType::Float || type_of(y) == ScalarType::Half, "y must be float32 or float16");
     STD_TORCH_CHECK(x.is_contiguous(), "x must be contiguous");
     STD_TORCH_CHECK(y.is_contiguous(), "y must be contiguous");
     STD_TORCH_CHECK(y.size(1) % 32 == 0 && x.size(1) == y.size(1) / 32 * 34, "dequant: x rows must hold y.size(1)/32 blocks of 34 bytes");
-    check_rc(minfer_dequant_q8_0(y.scalar_type() == ScalarType::Float ? MINFER_ATTN_F32 : MINFER_ATTN_F16, x.const_data_ptr(),
+    check_rc(minfer_dequant_q8_0(type_of(y) == ScalarType::Float ? MINFER_ATTN_F32 : MINFER_ATTN_F16, x.const_data_ptr(),
                                  y.mutable_data_ptr(), y.size(0), y.size(1), current_stream()),
              "dequant");
 }
@@ -607,9 +637,9 @@ void quant_hip(int64_t qtype_int, int64_t qblock_size, int64_t qtype_size, const
     STD_TORCH_CHECK(on_gpu(x) && on_gpu(y), "quant: x and y must be on the GPU");
     STD_TORCH_CHECK(x.dim() == 2 && y.dim() == 2);
     STD_TORCH_CHECK(x.size(0) == y.size(0), "x and y must have same number of rows");
-    const ScalarType t = x.scalar_type();
+    const ScalarType t = type_of(x);
     STD_TORCH_CHECK(t == ScalarType::Float || t == ScalarType::Half || t == ScalarType::BFloat16, "x must be float32 (or float16 / bfloat16)");
-    STD_TORCH_CHECK(y.scalar_type() == ScalarType::Byte, "y must be uint8 (byte)");
+    STD_TORCH_CHECK(type_of(y) == ScalarType::Byte, "y must be uint8 (byte)");
     STD_TORCH_CHECK(x.is_contiguous(), "x must be contiguous");
     STD_TORCH_CHECK(y.is_contiguous(), "y must be contiguous");
     STD_TORCH_CHECK(x.size(1) % 32 == 0 && y.size(1) == x.size(1) / 32 * 34, "quant: y rows must hold x.size(1)/32 blocks of 34 bytes");
