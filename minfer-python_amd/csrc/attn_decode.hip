@@ -503,6 +503,7 @@ MA_DEV void stream_rows_q8(const DecodeParams& p, int b, int g, int hg, int row_
     };
     const std::false_type general_tag{};
     const std::true_type inner_group_tag{};
+    const struct NoGroup {} no_group{};
 #pragma unroll
     for (int s = 0; s < NS; ++s) { load_k(general_tag, s, ring[s]); load_v(general_tag, s, ring[s]); }
 
@@ -526,7 +527,7 @@ MA_DEV void stream_rows_q8(const DecodeParams& p, int b, int g, int hg, int row_
         return h16x2{dh, dh};
     };
 
-    // (next_tag: whether group t + NS, requested during this turn, is an inner one)
+    // (next_tag: whether group t + NS, requested during this turn, is an inner one, or that there is none)
     auto consume = [&](auto inner_tag, auto next_tag, int t, Stage& st) __attribute__((always_inline)) {
         constexpr bool INNER = decltype(inner_tag)::value;
         const int r0 = row_lo + t * GR;
@@ -537,7 +538,7 @@ MA_DEV void stream_rows_q8(const DecodeParams& p, int b, int g, int hg, int row_
             const int off = INNER ? inner_off[j] : piece_offset(t, j, last_k, goff);
             *reinterpret_cast<u32x4*>(raw_k + off) = st.k[j];
         }
-        load_k(next_tag, t + NS, st);
+        if constexpr (!std::is_same_v<decltype(next_tag), NoGroup>) load_k(next_tag, t + NS, st);
         // ---- S^T = K Q^T for the two 16-key halves: lane gets head l16, keys 16h + 4*quad + r ---------------
         f32x4 s[2];
 #pragma unroll
@@ -568,7 +569,7 @@ MA_DEV void stream_rows_q8(const DecodeParams& p, int b, int g, int hg, int row_
             const int off = INNER ? inner_off[j] : piece_offset(t, j, last_v, goff);
             *reinterpret_cast<u32x4*>(raw_v + off) = st.v[j];
         }
-        load_v(next_tag, t + NS, st);
+        if constexpr (!std::is_same_v<decltype(next_tag), NoGroup>) load_v(next_tag, t + NS, st);
 #pragma unroll
         for (int i = 0; i < GR * BPR / 64; ++i) {
             const int idx = 64 * i + lane, row = idx / BPR, c = idx % BPR;
@@ -629,16 +630,25 @@ MA_DEV void stream_rows_q8(const DecodeParams& p, int b, int g, int hg, int row_
     };
 
     int t0 = 0;
-    // rounds in which every group consumed and every group requested is an inner one
+    // Three kinds of rounds, so that no path joins another inside one: with a loop over the last groups that may skip a round's second
+    // one, every wait of its first group covered what the second had just requested, half the ring, and a wave's share is six
+    // groups where 40 sequences of 1101 rows meet.  (us, before / after: these, 8 KV heads, 26.4 / 25.9; 3 of 200 to 3000 11.7 / 11.4; one of 32000
+    // 23.9 / 23.4; 64 to 8192 119.1 / 118.1; head_dim 64, 30 to 2000 13.7 / 13.5.)
+    // (1) every group consumed and every group requested is an inner one
     for (; t0 + 2 * NS < n_groups; t0 += NS) {
 #pragma unroll
         for (int s = 0; s < NS; ++s) consume(inner_group_tag, inner_group_tag, t0 + s, ring[s]);
     }
-    for (; t0 < n_groups; t0 += NS) {
+    // (2) at most once: inner groups are consumed, the last ones requested
+    if (t0 + NS < n_groups) {
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
-            if (t0 + s < n_groups) consume(general_tag, general_tag, t0 + s, ring[s]);
+        for (int s = 0; s < NS; ++s) consume(inner_group_tag, general_tag, t0 + s, ring[s]);
+        t0 += NS;
     }
+    // (3) the last one or two, with nothing left to request
+    static_assert(NS == 2, "one or two groups are left");
+    consume(general_tag, no_group, t0, ring[0]);
+    if (t0 + 1 < n_groups) consume(general_tag, no_group, t0 + 1, ring[1]);
     acc.m = m_ref;
     acc.l = sum_across_quads(l_sum);
 }

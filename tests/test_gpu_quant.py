@@ -126,6 +126,19 @@ def test_decode_q8_matches_oracle_and_fp16_path(B, Hq, Hkv, Lmax, D, lo, hi):
     assert float((out.float() - out16.float()).abs().max()) <= TOL
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_decode_q8_every_number_of_groups(D):
+    """256 pairs of up to 2048 rows, a context per workgroup: its eight waves stream 1 to 8 groups of 32 rows each, the last wave
+    with rows less, groups less or none (the rounds of inner, requested and last groups)."""
+    B, H, Lmax = 32, 8, 2048
+    ctx = torch.tensor([256 * g - less for g in range(1, 9) for less in (0, 1, 45, 31 * g)], dtype=torch.int32)
+    q = torch.randn(B, H, 1, D, generator=torch.Generator().manual_seed(D)).half()
+    kq, vq = q8_cache(D, B, H, Lmax, D), q8_cache(D + 1, B, H, Lmax, D)
+    out = run_decode_q8(q.to(DEV), kq.to(DEV), vq.to(DEV), ctx.to(DEV))
+    want = oracle.flash_attn_decode_q8_0(q, kq, vq, ctx)
+    assert float(np.abs(out.float().cpu().numpy() - want).max()) <= TOL
+
+
 def test_decode_q8_ignores_rows_past_ctx_and_takes_strided_caches():
     B, Hq, Hkv, Lmax, D = 4, 16, 4, 600, 128
     g = torch.Generator().manual_seed(1)
