@@ -182,6 +182,27 @@ def test_gemm_every_tile_shape(gemm_plan, layout, M, N, K, tile):
     assert_close(d, (alpha * (a.double() @ (b if layout == KN else b.T).double()) + beta * c.double()).numpy(), dtype)
 
 
+@pytest.mark.parametrize("layout,M,N,K", [   # tiles of 4 to 8 block rows a wave, 4 to 8 blocks across, the last ones not full
+    (NK, 65, 136, 64), (KN, 129, 264, 128), (NK, 300, 1000, 192), (NK, 258, 5424, 384), (KN, 487, 8584, 128),
+    (NK, 1949, 5656, 320), (NK, 2025, 4888, 128), (KN, 2027, 5976, 192),
+])
+def test_gemm_adds_c_in_place(layout, M, N, K):
+    """The residual added in place, in rows of a wider buffer: C's pieces are requested block rows before the same places are
+    stored, bit-equal to the call with C apart, nothing else written."""
+    a, b, c = (x.to(DEV) for x in make(M, N, K, layout, torch.float16, M + N + K))
+    d = torch.full_like(c, float("nan"))
+    assert capi.gemm(a, b, c, d, 2.0, 3.0, layout) == capi.OK, capi.last_error()
+    wide = torch.full((M + 3, N + 24), float("nan"), dtype=c.dtype, device=DEV)
+    view = wide[1:M + 1, 8:N + 8]
+    view.copy_(c)
+    assert capi.gemm(a, b, view, view, 2.0, 3.0, layout) == capi.OK, capi.last_error()
+    torch.cuda.synchronize()
+    assert_close(d, (2.0 * torch.mm(a.double(), (b if layout == KN else b.T.contiguous()).double()) + 3.0 * c.double()).cpu().numpy(), torch.float16)
+    assert torch.equal(view, d)
+    view.fill_(float("nan"))
+    assert torch.isnan(wide).all()
+
+
 @pytest.mark.parametrize("M", [9, 24, 40, 64])
 @pytest.mark.parametrize("N,K", [
     (2056, 256),      # one 16-column block a workgroup, the last of 8 columns; one segment
