@@ -1202,22 +1202,34 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const GemmParams p) {
     }
 }
 
-// D = alpha * (sum of the K slices' partial products) + beta * C, four columns per thread.
-template <class T>
+// D = alpha * (sum of the K slices' partial products) + beta * C, four columns per thread, the slices added in their order.
+// Bound by latency: the sums of AT slices (eight at most) and C are requested together (one after the other, each with the memory's
+// latency, 4 us beside a product of 7: 40 x 4096 x 4096 `[K, N]` with C 12.8 -> 11.7 us, 64 x 2048 x 8192 15.7 -> 13.8, 24 x 2048 x 8192
+// `[N, K]` 11.9 -> 10.4, 24 x 4096 x 14336 Q8_0 20.0 -> 19.2), and a thread's place is a 32-bit division.  Many rows of few slices are bound by
+// their bytes: AT divides the slices as evenly as it can, since the loads past the last one repeat it (500 x 4096 x 4096, two slices, 26.3 before; two
+// loads 26.3, up to eight behind a branch each 27.2; 400 x 2048 x 8192, five slices, 25.8; five read as eight 26.1).
+template <class T, int AT>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmParams p) {
-    const int n4 = p.N >> 2;
-    const int64_t total = (int64_t)p.M * n4;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+    const uint32_t n4 = (uint32_t)p.N >> 2, total = (uint32_t)p.M * n4;   // (64 rows of under 16 K columns, or 8 M sums of a slice, at most)
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
         const int m = (int)(i / n4), n = 4 * (int)(i % n4);
-        f32x4 sum = *reinterpret_cast<const f32x4*>(p.part + (int64_t)m * p.N + n);
-        for (int sl = 1; sl < p.splits; ++sl) sum += *reinterpret_cast<const f32x4*>(p.part + ((int64_t)sl * p.M + m) * p.N + n);
-        store_result<T>(p, m, n, sum);
+        const s16x4 c = load_c4(p, m, n);
+        const float* src = p.part + (int64_t)m * p.N + n;
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f}, x[AT];
+        for (int s0 = 0; s0 < p.splits; s0 += AT) {
+#pragma unroll
+            for (int u = 0; u < AT; ++u) x[u] = *reinterpret_cast<const f32x4*>(src + (int64_t)min(s0 + u, p.splits - 1) * p.M * p.N);
+#pragma unroll
+            for (int u = 0; u < AT; ++u)
+                if (s0 + u < p.splits) sum = s0 + u == 0 ? x[u] : sum + x[u];
+        }
+        store_result<T>(p, m, n, sum, c);
     }
 }
 
 // The counters of a sliced launch, when its workgroups are to add the slices up themselves: up to 16 rows and 2 MiB of sums.
 // Written through to where every XCD sees them they pass at about a microsecond per MiB, so larger ones are left to a second
-// launch (fused / two launches: 1 MiB 12.2 / 13.4 us, 1.9 MiB 23.7 / 25.3, 2.4 MiB 18.0 / 15.0, 5 MiB 16.7 / 13.7), and so are
+// launch (fused / two launches, the latter 1 us less since it reads its slices together: 1 MiB 12.2 / 13.4 us, 1.9 MiB 23.7 / 25.3, 2.4 MiB 18.0 / 15.0, 5 MiB 16.7 / 13.7), and so are
 // more rows, and so the slices of gemm_kernel, whose tiles' last workgroups add up what a second launch spreads over the chip (17 x 528 x 1152 9.5 / 8.7, 40 x
 // 808 x 1600 13.3 / 9.8, 24 x 3424 x 1408 11.3 / 9.7).  At most 256 tiles.
 static uint32_t* slice_counters(const GemmParams& p, hipStream_t stream) {
@@ -1229,7 +1241,16 @@ template <class T>
 static int launch_reduce(const GemmParams& p, hipStream_t stream) {
     if (p.done) return MINFER_ATTN_OK;
     const int grid = (int)std::min<int64_t>(((int64_t)p.M * (p.N / 4) + 255) / 256, 256 * 8);
-    hipLaunchKernelGGL((gemm_reduce_kernel<T>), dim3(grid), dim3(256), 0, stream, p);
+    const int rounds = (p.splits + 7) / 8;
+    switch ((p.splits + rounds - 1) / rounds) {
+        case 2: hipLaunchKernelGGL((gemm_reduce_kernel<T, 2>), dim3(grid), dim3(256), 0, stream, p); break;
+        case 3: hipLaunchKernelGGL((gemm_reduce_kernel<T, 3>), dim3(grid), dim3(256), 0, stream, p); break;
+        case 4: hipLaunchKernelGGL((gemm_reduce_kernel<T, 4>), dim3(grid), dim3(256), 0, stream, p); break;
+        case 5: hipLaunchKernelGGL((gemm_reduce_kernel<T, 5>), dim3(grid), dim3(256), 0, stream, p); break;
+        case 6: hipLaunchKernelGGL((gemm_reduce_kernel<T, 6>), dim3(grid), dim3(256), 0, stream, p); break;
+        case 7: hipLaunchKernelGGL((gemm_reduce_kernel<T, 7>), dim3(grid), dim3(256), 0, stream, p); break;
+        default: hipLaunchKernelGGL((gemm_reduce_kernel<T, 8>), dim3(grid), dim3(256), 0, stream, p);
+    }
     return check_launch("gemm_reduce_kernel");
 }
 

@@ -41,13 +41,18 @@ MA_DEV int group_of_unit(const GemmGroup& g, int c, int& local) {
     return s;
 }
 
-// Four consecutive columns of D from the sums in fp32: alpha, beta and C, one rounding.
-template <class T> MA_DEV void store_result(const GemmParams& p, int m, int n, f32x4 sum) {
+// Four consecutive columns of C, which are requested together with the sums that they are added to; not read where beta is 0.
+MA_DEV s16x4 load_c4(const GemmParams& p, int m, int n) {
+    s16x4 c = {0, 0, 0, 0};
+    if (p.beta != 0.f) c = *reinterpret_cast<const s16x4*>((const short*)p.C + (int64_t)m * p.ldc + n);
+    return c;
+}
+// Four consecutive columns of D from the sums in fp32 and those of C: alpha, beta and C, one rounding.
+template <class T> MA_DEV void store_result(const GemmParams& p, int m, int n, f32x4 sum, s16x4 c) {
     float v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = p.alpha * sum[e];
     if (p.beta != 0.f) {
-        const s16x4 c = *reinterpret_cast<const s16x4*>((const short*)p.C + (int64_t)m * p.ldc + n);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] += p.beta * T::to_float(c[e]);
     }
@@ -56,6 +61,7 @@ template <class T> MA_DEV void store_result(const GemmParams& p, int m, int n, f
     pk.y = T::pack2(v[2], v[3]);
     *reinterpret_cast<uint2*>((short*)p.D + (int64_t)m * p.ldd + n) = pk;
 }
+template <class T> MA_DEV void store_result(const GemmParams& p, int m, int n, f32x4 sum) { store_result<T>(p, m, n, sum, load_c4(p, m, n)); }
 
 // swizzles: granule index of a row XORed with a function of the row (see the attention kernel's TileGeom)
 MA_DEV int swz_row_tile(int row) { return (row >> 1) & 7; }        // 128-byte rows, read 32 rows x 16 bytes
