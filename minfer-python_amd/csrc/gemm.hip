@@ -49,6 +49,18 @@ MA_DEV f32x4 load_slice4(const GemmParams& p, int slice, int m, int n) {
 template <class T, int THREADS>
 MA_DEV void finish_slices(const GemmParams& p, int tile, int m0, int m1, int n0, int n1, int* flag) {
     if (!p.done) return;
+    // C is requested before it is known who adds up, while the sums are on their way (slice_counters: up to 16 rows of 128 columns, so a
+    // thread has two pieces of four columns at most), and a thread without a piece reads nothing (us, before / after: 16 x 2560 x 2560 `[K, N]` 9.0 /
+    // 8.3, 4096 x 4096 at one row 9.7 / 9.4, 16 x 2048 x 8192 `[N, K]` 10.8 / 10.3, Q8_0 10.5 / 10.1; requested with the slices 8 x 1000 x 4096 was slower, 7.6 / 7.8, now 7.5)
+    const int n4 = (n1 - n0) >> 2, total = (m1 - m0) * n4;
+    int m[2], n[2];
+    s16x4 c[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int i = min((int)threadIdx.x + e * THREADS, total - 1), r = i / n4;
+        m[e] = m0 + r; n[e] = n0 + 4 * (i - r * n4);
+        c[e] = load_c4(p, m[e], n[e]);
+    }
     wait_vmcnt<0>();   // the thread's sums have arrived
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -57,32 +69,24 @@ MA_DEV void finish_slices(const GemmParams& p, int tile, int m0, int m1, int n0,
         if (*flag) __hip_atomic_store(p.done + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
-    if (!*flag) return;
-    const int n4 = (n1 - n0) >> 2, total = (m1 - m0) * n4;
-    // two pieces of four columns and eight slices at a time, so that sixteen loads of a thread are in flight
-    for (int i0 = threadIdx.x; i0 < total; i0 += 2 * THREADS) {
-        int m[2], n[2];
-        f32x4 sum[2], x[2][8];
+    if (!*flag || (int)threadIdx.x >= total) return;
+    // two pieces and eight slices at a time, so that sixteen loads of a thread are in flight
+    f32x4 sum[2], x[2][8];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int i = min(i0 + e * THREADS, total - 1), r = i / n4;
-            m[e] = m0 + r; n[e] = n0 + 4 * (i - r * n4);
-            sum[e] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        for (int s0 = 0; s0 < p.splits; s0 += 8) {
+    for (int e = 0; e < 2; ++e) sum[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < p.splits; s0 += 8) {
 #pragma unroll
-            for (int e = 0; e < 2; ++e)
+        for (int e = 0; e < 2; ++e)
 #pragma unroll
-                for (int u = 0; u < 8; ++u) x[e][u] = load_slice4(p, min(s0 + u, p.splits - 1), m[e], n[e]);
+            for (int u = 0; u < 8; ++u) x[e][u] = load_slice4(p, min(s0 + u, p.splits - 1), m[e], n[e]);
 #pragma unroll
-            for (int e = 0; e < 2; ++e)
+        for (int e = 0; e < 2; ++e)
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (s0 + u < p.splits) sum[e] = s0 + u == 0 ? x[e][u] : sum[e] + x[e][u];
-        }
-        store_result<T>(p, m[0], n[0], sum[0]);
-        if (i0 + THREADS < total) store_result<T>(p, m[1], n[1], sum[1]);
+            for (int u = 0; u < 8; ++u)
+                if (s0 + u < p.splits) sum[e] = s0 + u == 0 ? x[e][u] : sum[e] + x[e][u];
     }
+    store_result<T>(p, m[0], n[0], sum[0], c[0]);
+    if ((int)threadIdx.x + THREADS < total) store_result<T>(p, m[1], n[1], sum[1], c[1]);
 }
 
 // Up to 64 rows against a weight stored [K, N] (what a square weight is taken for): the work is reading the weight once.  A
