@@ -51,6 +51,10 @@ inline bool stripe_takes(int64_t M, int64_t stripes, int64_t K) {
 // 79 a few units have two blocks where the others have one.
 inline bool stripe_blocks_pay(int64_t M, int64_t stripes, int64_t K) {
     const int64_t most = stripes < 48 ? 16000 : stripes <= 64 || stripes >= 80 ? 25000 : 22000;
+    // With the sums added up by gemm_reduce_kernel in 1 to 2 us less (more than 16 rows) the line lies lower, and between the rows of a block:
+    // 2560 x 5120 at 17 / 32 rows 11.2 / 11.1, 11.8 / 13.1; 2048 x 4096 at 32 10.1 / 9.9; 3072 x 4096 at 40 / 64 12.1 / 11.7, 13.8 / 14.7;
+    // 3584 x 8192 at 17 / 32 15.9 / 15.1, 16.8 / 18.0; 4096 x 6144 at 32 / 40 15.6 / 15.6, 16.8 / 17.7 (64 stripes leave no unit idle).  (Wider ones as before: 4608 x 4096 at 40 14.9 / 14.7.)
+    if (M > 16 && stripes <= 64 && (16 + M) * K > (stripes < 48 ? 224000 : stripes < 64 ? 320000 : 330000)) return false;
     return stripe_takes(M, stripes, K) && (stripes >= 96 || ((stripes > 64 ? 2 : 1) + (M + 15) / 16) * K <= most);
 }
 // A weight of fewer than 192 stripes: with a workspace, K slices bring the workgroups up to the chip's 256 compute units
@@ -198,10 +202,11 @@ inline GemmRoute gemm_route(int64_t M, int64_t N, int64_t K, bool nt, bool fast,
         if ((M <= 32 || N * K <= (INT64_C(1) << 25)) && !(fit > 1 && tile_plan(M, N, K, nt, kMostSlices, units()).slices > 1)) return {GemmKernel::skinny, 1, 0};
     }
     if (!nt && M <= kKnRows) {
-        // eight slices at most, 16 for rows of 80 K steps and more: further ones save less streaming than their sums cost (us, as many as fill
+        // eight slices at most, 16 for rows of 80 K steps and more, and for up to 1024 columns from 17 rows on (eight / 16: 512 x 4096 at 17 / 64 rows 9.4 / 9.2,
+        // 10.5 / 9.7; 1024 x 4096 9.7 / 9.4, 11.4 / 11.0; 2048 x 4096 at 40 10.9 / 11.6): further ones save less streaming than their sums cost (us, as many as fill
         // the chip / these: 1000 x 4096 at 1 / 9 / 16 rows 10.5 / 7.6, 13.5 / 8.7, 15.5 / 9.4; 2560 x 2560 at 12 10.0 / 8.1; 2048 x 4096 at 40 13.7 /
         // 11.9; 1024 x 14336 at 9 / 40 15.4 / 12.8, 19.4 / 17.2; 512 x 8192 at 9 17.0 / 9.6; minfer_gemm_workspace_bytes stays that of filling it)
-        const int most = std::min(kn_slices(M, N, K), K >= 80 * kBK ? 16 : 8);   // a smaller workspace: as many of these as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
+        const int most = std::min(kn_slices(M, N, K), K >= 80 * kBK || (M > 16 && N <= 1024) ? 16 : 8);   // a smaller workspace: as many of these as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
         return {GemmKernel::kn_rows, std::max((int)std::min<int64_t>(most, fit), 1), 0};
     }
     TilePlan plan = tile_plan(M, N, K, nt, kMostSlices, units());

@@ -567,6 +567,21 @@ def test_gemm_k_slices_of_stripes(gemm_plan, dtype, M, N, K, slices):
     assert_close(d, (2.0 * torch.mm(a.double(), b.T.contiguous().double()) + 3.0 * c.double()).cpu().numpy(), dtype)
 
 
+@pytest.mark.parametrize("layout,M,N,K,kernel,slices", [   # just past and just below where K slices are taken from 17 rows on
+    (NK, 28, 2560, 5120, rules.STRIPE_SLICES, 5), (NK, 24, 2560, 5120, rules.STRIPE, 1),
+    (NK, 63, 3080, 4096, rules.STRIPE_SLICES, 4), (NK, 62, 3072, 4096, rules.STRIPE, 1),
+    (NK, 40, 4096, 6144, rules.STRIPE_SLICES, 4), (NK, 37, 4096, 6144, rules.STRIPE, 1),
+    (KN, 17, 264, 4160, rules.KN_ROWS, 16), (KN, 64, 1024, 4096, rules.KN_ROWS, 16), (KN, 64, 1032, 4096, rules.KN_ROWS, 8),
+])
+def test_gemm_k_slices_beside_their_lines(gemm_plan, layout, M, N, K, kernel, slices):
+    assert gemm_plan(M, N, K, layout == NK, rules.MOST_SLICES)[:2] == (kernel, slices)
+    a, b, c = (x.to(DEV) for x in make(M, N, K, layout, torch.float16, M + N + K))
+    ws, d = sliced_call(a, b, c, layout, M, N, K)
+    assert written_slices(ws, M, N) == (slices if slices > 1 else 0)
+    exact = 2.0 * torch.mm(a.double(), (b if layout == KN else b.T.contiguous()).double()) + 3.0 * c.double()
+    assert_close(d, exact.cpu().numpy(), torch.float16)
+
+
 def test_gemm_workspace_bytes_is_zero_where_tiles_fill_the_chip():
     L = capi.lib()
     assert L.minfer_gemm_workspace_bytes(4096, 4096, 4096) == 0
