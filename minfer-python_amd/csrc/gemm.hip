@@ -45,20 +45,21 @@ MA_DEV f32x4 load_slice4(const GemmParams& p, int slice, int m, int n) {
     return __builtin_bit_cast(f32x4, u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)});
 }
 // Called by all THREADS threads of a slice's workgroup after their store_slice4: columns n0 .. n1 - 1 (multiples of 4, four
-// at least) of rows m0 .. m1 - 1; `flag`: a shared word.
-template <class T, int THREADS>
-MA_DEV void finish_slices(const GemmParams& p, int tile, int m0, int m1, int n0, int n1, int* flag) {
+// at least and COLS at most) of all the rows, one at least and kMeetRows at most (slices_meet); `flag`: a shared word.
+template <class T, int THREADS, int COLS>
+MA_DEV void finish_slices(const GemmParams& p, int tile, int n0, int n1, int* flag) {
+    static_assert(kMeetRows * COLS / 4 <= 2 * THREADS, "two pieces of four columns a thread");
     if (!p.done) return;
-    // C is requested before it is known who adds up, while the sums are on their way (slice_counters: up to 16 rows of 128 columns, so a
-    // thread has two pieces of four columns at most), and a thread without a piece reads nothing (us, before / after: 16 x 2560 x 2560 `[K, N]` 9.0 /
+    // C is requested before it is known who adds up, while the sums are on their way (pieces past the last one read that one's place), and a
+    // thread without a piece reads no sums (us, before / after: 16 x 2560 x 2560 `[K, N]` 9.0 /
     // 8.3, 4096 x 4096 at one row 9.7 / 9.4, 16 x 2048 x 8192 `[N, K]` 10.8 / 10.3, Q8_0 10.5 / 10.1; requested with the slices 8 x 1000 x 4096 was slower, 7.6 / 7.8, now 7.5)
-    const int n4 = (n1 - n0) >> 2, total = (m1 - m0) * n4;
+    const int n4 = (n1 - n0) >> 2, total = p.M * n4;
     int m[2], n[2];
     s16x4 c[2];
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
         const int i = min((int)threadIdx.x + e * THREADS, total - 1), r = i / n4;
-        m[e] = m0 + r; n[e] = n0 + 4 * (i - r * n4);
+        m[e] = r; n[e] = n0 + 4 * (i - r * n4);
         c[e] = load_c4(p, m[e], n[e]);
     }
     wait_vmcnt<0>();   // the thread's sums have arrived
@@ -201,7 +202,7 @@ __global__ __launch_bounds__(4 * 64) void gemm_kn_rows_kernel(const GemmParams p
     }
     if (p.splits > 1) {
         __shared__ int last_s;
-        finish_slices<T, 4 * 64>(p, tile, 0, p.M, n0, min(n0 + 128, p.N), &last_s);
+        finish_slices<T, 4 * 64, 128>(p, tile, n0, min(n0 + 128, p.N), &last_s);
     }
 }
 
@@ -603,7 +604,7 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_kernel(const GemmParams p)
     }
     if constexpr (SLICED) {
         __shared__ int last_s;
-        finish_slices<T, 4 * 64>(p, (int)blockIdx.x / p.splits, 0, p.M, 16 * blk_first, min(16 * blk_last, p.N), &last_s);
+        finish_slices<T, 4 * 64, 64>(p, (int)blockIdx.x / p.splits, 16 * blk_first, min(16 * blk_last, p.N), &last_s);
     }
 }
 // The smallest NB that goes through the `most` blocks of a workgroup in as few chunks as four would (five blocks as three and two: 18944 x 3584
@@ -1164,7 +1165,7 @@ __global__ __launch_bounds__(4 * 64) void gemm_stripe_q8_kernel(const GemmParams
     }
     if constexpr (SLICED) {
         __shared__ int last_s;
-        finish_slices<T, 4 * 64>(p, (int)blockIdx.x / p.splits, 0, p.M, 16 * blk_first, min(16 * blk_last, p.N), &last_s);
+        finish_slices<T, 4 * 64, 64>(p, (int)blockIdx.x / p.splits, 16 * blk_first, min(16 * blk_last, p.N), &last_s);
     }
 }
 template <int MB, bool SLICED>
@@ -1231,13 +1232,10 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmParams p) {
     }
 }
 
-// The counters of a sliced launch, when its workgroups are to add the slices up themselves: up to 16 rows and 2 MiB of sums.
-// Written through to where every XCD sees them they pass at about a microsecond per MiB, so larger ones are left to a second
-// launch (fused / two launches, the latter 1 us less since it reads its slices together: 1 MiB 12.2 / 13.4 us, 1.9 MiB 23.7 / 25.3, 2.4 MiB 18.0 / 15.0, 5 MiB 16.7 / 13.7), and so are
-// more rows, and so the slices of gemm_kernel, whose tiles' last workgroups add up what a second launch spreads over the chip (17 x 528 x 1152 9.5 / 8.7, 40 x
-// 808 x 1600 13.3 / 9.8, 24 x 3424 x 1408 11.3 / 9.7).  At most 256 tiles.
+// The counters of a sliced launch, when its workgroups are to add the slices up themselves.
 static uint32_t* slice_counters(const GemmParams& p, hipStream_t stream) {
-    return p.M <= 16 && (int64_t)p.splits * p.M * p.N * 4 <= (2 << 20) ? stream_counters(stream) : nullptr;
+    static_assert(kMeetTiles <= kStreamCounters, "a counter per tile");
+    return slices_meet(p.M, p.N, p.splits) ? stream_counters(stream) : nullptr;
 }
 
 // After a sliced launch: nothing where its workgroups have added the slices up themselves.

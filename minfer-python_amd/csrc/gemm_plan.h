@@ -58,7 +58,7 @@ inline bool stripe_blocks_pay(int64_t M, int64_t stripes, int64_t K) {
     return stripe_takes(M, stripes, K) && (stripes >= 96 || ((stripes > 64 ? 2 : 1) + (M + 15) / 16) * K <= most);
 }
 // A weight of fewer than 192 stripes: with a workspace, K slices bring the workgroups up to the chip's 256 compute units
-// (every slice four segments at least); the slices' sums are added up by finish_slices or gemm_reduce_kernel (slice_counters).
+// (every slice four segments at least); the slices' sums are added up by finish_slices or gemm_reduce_kernel (slices_meet).
 // 1 = no slices.
 inline int stripe_slices(int64_t M, int64_t N, int64_t K) {
     const int64_t stripes = (N + 63) / 64;
@@ -77,6 +77,16 @@ inline int kn_slices(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = (N + 127) / 128;
     return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(256 / tiles, K / kBK / (M <= 16 ? 2 : 4)), M <= 16 ? 64 : 32));
 }
+
+// ---- who adds the K slices up ----------------------------------------------------------------------------------
+// Whether the slices of stripe_slices or kn_slices meet inside the launch (finish_slices; where the stream has counters): up to kMeetRows
+// rows, which is what its threads have pieces for, and 2 MiB of sums.  Written through to where every XCD sees them they pass at about a
+// microsecond per MiB, so larger ones are left to a second launch (fused / two launches, the latter 1 us less since it reads its slices
+// together: 1 MiB 12.2 / 13.4 us, 1.9 MiB 23.7 / 25.3, 2.4 MiB 18.0 / 15.0, 5 MiB 16.7 / 13.7), and so are more rows, and so the slices of
+// gemm_kernel, whose tiles' last workgroups add up what a second launch spreads over the chip (17 x 528 x 1152 9.5 / 8.7, 40 x 808 x 1600
+// 13.3 / 9.8, 24 x 3424 x 1408 11.3 / 9.7).  Two slices and more are of at most kMeetTiles tiles: both size functions stay at 256 workgroups.
+constexpr int kMeetRows = 16, kMeetTiles = 128;
+inline bool slices_meet(int64_t M, int64_t N, int64_t slices) { return M <= kMeetRows && slices * M * N * 4 <= (2 << 20); }
 
 // ---- which tiles, how many K slices --------------------------------------------------------------------------
 inline int64_t tile_count(int64_t M, int64_t N, int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
