@@ -582,6 +582,54 @@ def test_gemm_k_slices_beside_their_lines(gemm_plan, layout, M, N, K, kernel, sl
     assert_close(d, exact.cpu().numpy(), torch.float16)
 
 
+Q8 = "q8_0"
+
+
+@pytest.mark.parametrize("dtype,weight,M,N,K,slices", [(dtype, *case) for case in [
+    (KN, 1, 4096, 4096, 8), (KN, 9, 1000, 4096, 8), (KN, 16, 264, 8192, 16),   # up to 16 rows: a tile's last workgroup adds the slices up
+    (NK, 9, 520, 6144, 6), (NK, 16, 2048, 8192, 8),
+    (Q8, 9, 1544, 8448, 8), (Q8, 2, 520, 8192, 8),
+    (KN, 17, 264, 4160, 16), (KN, 40, 4096, 4096, 8),                          # more: a second launch does
+    (NK, 17, 520, 8448, 8), (NK, 64, 3080, 6144, 5),
+    (Q8, 17, 2056, 6144, 6),
+    (KN, 130, 272, 5952, 31), (NK, 322, 5488, 4032, 3),                        # K slices of tiles
+] for dtype in (torch.float16, torch.bfloat16) if dtype == torch.float16 or case[0] != Q8])   # (a Q8_0 weight has float16 activations)
+def test_gemm_adds_c_in_place_over_k_slices(gemm_plan, dtype, weight, M, N, K, slices):
+    """The residual added in place over K slices, in rows of a wider buffer that start at multiples of 8 bytes only: bit-equal to the call
+    with C apart on the null stream and on one without counters, nothing else written."""
+    if weight == Q8:
+        a, b, c, w = make_q8(M, N, K, M + N + K)
+        assert gemm_plan.q8(M, N, K, True, rules.MOST_SLICES) == (rules.Q8_STRIPE_SLICES, slices)
+        w = w.T.contiguous()
+    else:
+        a, b, c = make(M, N, K, weight, dtype, M + N + K)
+        assert gemm_plan(M, N, K, weight == NK, rules.MOST_SLICES)[1] == slices
+        w = b if weight == KN else b.T.contiguous()
+    a, b, c = a.to(DEV), b.to(DEV), c.to(DEV)
+    ws = torch.empty(4 * M * N * slices, dtype=torch.uint8, device=DEV)
+
+    def call(c, d):
+        ws.fill_(0xFF)
+        rc = capi.gemm_q8_0(a, b, c, d, 2.0, 3.0, ws) if weight == Q8 else capi.gemm_ws(a, b, c, d, 2.0, 3.0, ws, weight)
+        assert rc == capi.OK, capi.last_error()
+        assert written_slices(ws, M, N) == slices
+
+    d = torch.full_like(c, float("nan"))
+    call(c, d)
+    assert_close(d, (2.0 * torch.mm(a.double(), w.to(DEV).double()) + 3.0 * c.double()).cpu().numpy(), dtype)
+    wide = torch.full((M + 2, N + 12), float("nan"), dtype=dtype, device=DEV)
+    view = wide[1:M + 1, 4:N + 4]
+    torch.cuda.synchronize()
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            view.copy_(c)
+            call(view, view)
+            assert torch.equal(view, d)
+            view.fill_(float("nan"))
+            assert torch.isnan(wide).all()
+        stream.synchronize()
+
+
 def test_gemm_workspace_bytes_is_zero_where_tiles_fill_the_chip():
     L = capi.lib()
     assert L.minfer_gemm_workspace_bytes(4096, 4096, 4096) == 0
