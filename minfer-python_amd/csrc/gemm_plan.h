@@ -32,30 +32,34 @@ inline bool rows_lds_takes(int64_t M, int64_t K) { return M <= 16 && K % (4 * kR
 // gemv_kernel: one to four rows that its LDS area holds.
 inline bool gemv_takes(int64_t M, int64_t K) { return M >= 1 && M <= 4 && K <= kGemvMaxKHalfs && (M == 1 || (K > kGemvSegHalfs && M * K <= 2 * kGemvMaxKHalfs)); }
 // gemm_stripe_kernel.  Which widths it takes (in stripes of 64 columns; weights coming from memory): from 96 on every row count that reaches
-// it (14336 x 4096 at 2-32 rows 22.8-23.7 us, the 16-column kernel 24.3-32.4); an output head from 5 rows on (128256 x 4096 at 8
-// rows 179 against 183, 57344 x 8192 166 against 185; up to 4 rows the kernels that keep more workgroups on a compute unit are
-// ahead); narrower ones down to 32 stripes from 5 rows on, up to 8 when their rows are long enough to matter, against the 16-column
-// and few-row kernels (us: 2048 x 4096 at 16 / 17 / 64 rows 9.1 / 7.2, 13.9 / 8.0, 21.3 / 12.2; 5120 x 5120 at 5 / 16 rows 14.1 / 10.9,
-// 13.4 / 11.0; 3072 x 8192 at 8 / 32 rows 14.9 / 10.8, 29.6 / 14.2; 4096 x 14336 at 8 / 64 rows 24.0 / 21.5, 54.9 / 44.9).
+// it (14336 x 4096 at 2-32 rows 21.6-22.4 us, the 16-column kernels 23.2-40.5); an output head from 5 rows on (128256 x 4096 at 8
+// rows 164 against 182, 57344 x 8192 160 against 186; at 2-4 rows the kernels that keep more workgroups on a compute unit
+// were ahead, 166-170 against 176-178, and on another box behind, 165-169 against 161-163); narrower ones down to 32 stripes from 5 rows on, up to 8 when their rows are long enough to matter, against the 16-column
+// and few-row kernels (us: 2048 x 4096 at 16 / 17 / 64 rows 9.6 / 7.8, 14.0 / 8.6, 21.5 / 14.0; 5120 x 5120 at 5 / 16 rows 14.9 / 12.9,
+// 20.4 / 14.5; 3072 x 8192 at 8 / 32 rows 14.9 / 12.8, 29.8 / 17.2; 4096 x 14336 at 8 / 64 rows 24.3 / 22.8, 70.8 / 44.1).
 inline bool stripe_takes(int64_t M, int64_t stripes, int64_t K) {
     if (M < 1 || M > 64 || K % kStripeSeg != 0) return false;
     if (stripes > 640) return M >= 5;
     return stripes >= 96 || (stripes >= 80 && M >= 8) || (stripes >= 32 && M >= 5 && (M > 8 || K >= 2560));
 }
-// Where it is also ahead of its K slices, whose workgroups copy less each but leave partial sums that a second launch adds up: by the rows
-// a unit copies, (NB + MB) x 16 of K values, the narrower the weight the fewer (us, slices / whole rows: 6144 x 4096 at 64 rows 15.9 /
-// 15.1, 5632 x 4096 15.5 / 15.1, 4608 x 4096 13.8 / 14.9 and at 33 rows 12.7 / 11.7; 4096 x 6144 at 33 / 64 rows 13.9 / 13.4, 15.2 /
-// 16.5; 3584 x 8192 at 32 / 48 rows 14.5 / 14.3, 16.1 / 18.2; 2560 x 5120 at 32 / 33 rows 10.7 / 10.1, 11.4 / 11.7; 2048 x 4096 at 32 /
-// 64 rows 9.3 / 8.4, 11.2 / 12.2; 2048 x 8192 at 5 rows 9.5 / 10.4; 4096 x 14336 at 16 / 24 rows 24.0 / 24.1, 24.8 / 27.8).
-// The lines lie between these: below 48 stripes a quarter of the units and more have no column block and whole rows pay less; from 65 to
-// 79 a few units have two blocks where the others have one.
+// Where it is also ahead of its K slices, whose workgroups copy less each but leave partial sums to be added up (us, slices / whole rows;
+// weights from memory: calls cycling over 640 MiB of copies, half of which and less the last-level cache would serve, 3584 x 8192 at 32 rows 17.7 or 13.5 for
+// whole rows; without C, which costs slices 0.1 and whole rows 0.3 up to 16 rows, 0.6 to 1.4 from 17 on).
+// By the rows a unit copies, (NB + MB) x 16 of K values, the narrower the weight the fewer, since below 48 stripes a quarter of the units and
+// more have no column block, and from 65 to 79 a few units have two where the others have one: 4096 x 14336 at 9 / 16 rows 23.6 / 22.9, 24.1 / 24.3; 3584 x 8192
+// at 16 15.1 / 13.9; 2560 x 5120 at 16 10.2 / 10.2; 2048 x 8192 at 5 10.2 / 12.0, 2048 x 4096 at 32 / 33 10.1 / 9.8, 10.4 / 10.5; 4608 x 4096 at 33 / 48 / 64
+// 14.3 / 13.8, 14.9 / 15.2, 15.7 / 17.2; 5632 x 4096 at 33 / 64 15.8 / 14.2, 18.1 / 17.7; 6144 x 4096 at 64 18.5 / 17.8.
+// From 17 rows on, where gemm_reduce_kernel adds up, the rows themselves count and up to 64 stripes the line is lower, in proportion to the units that have a
+// block: 2560 x 5120 at 28 / 32 rows 11.4 / 12.2, 11.7 / 13.1; 3072 x 4096 at 40 / 48 11.9 / 11.5, 12.2 / 12.3; 4096 x 4096 at 48 / 56 / 64 13.1 / 12.7, 13.5 / 14.1,
+// 13.8 / 14.6 (62 and 63 stripes alike); 4096 x 6144 at 32 / 36 15.2 / 14.9, 16.1 / 16.3; 3584 x 6144 at 28 / 32 14.1 / 13.9, 14.3 / 14.6.  Rows of 8192 values
+// keep whole rows longer: 4096 x 8192 at 24 / 28 / 32 17.7 / 16.2, 17.9 / 16.9, 17.9 / 18.0; 3584 x 8192 at 20 / 24 15.8 / 15.1, 15.8 / 16.0.
+// Over 1500 sizes of 32 to 64 stripes, 2560 to 14336 values and 17 to 64 rows the choice is 0.3 % behind the better one.
 inline bool stripe_blocks_pay(int64_t M, int64_t stripes, int64_t K) {
+    if (!stripe_takes(M, stripes, K)) return false;
+    if (stripes >= 96) return true;
+    if (M > 16 && stripes <= 64 && (16 + M) * K > std::max<int64_t>(224000, (K >= 8192 ? 5800 : 4800) * stripes)) return false;
     const int64_t most = stripes < 48 ? 16000 : stripes <= 64 || stripes >= 80 ? 25000 : 22000;
-    // With the sums added up by gemm_reduce_kernel in 1 to 2 us less (more than 16 rows) the line lies lower, and between the rows of a block:
-    // 2560 x 5120 at 17 / 32 rows 11.2 / 11.1, 11.8 / 13.1; 2048 x 4096 at 32 10.1 / 9.9; 3072 x 4096 at 40 / 64 12.1 / 11.7, 13.8 / 14.7;
-    // 3584 x 8192 at 17 / 32 15.9 / 15.1, 16.8 / 18.0; 4096 x 6144 at 32 / 40 15.6 / 15.6, 16.8 / 17.7 (64 stripes leave no unit idle).  (Wider ones as before: 4608 x 4096 at 40 14.9 / 14.7.)
-    if (M > 16 && stripes <= 64 && (16 + M) * K > (stripes < 48 ? 224000 : stripes < 64 ? 320000 : 330000)) return false;
-    return stripe_takes(M, stripes, K) && (stripes >= 96 || ((stripes > 64 ? 2 : 1) + (M + 15) / 16) * K <= most);
+    return ((stripes > 64 ? 2 : 1) + (M + 15) / 16) * K <= most;
 }
 // A weight of fewer than 192 stripes: with a workspace, K slices bring the workgroups up to the chip's 256 compute units
 // (every slice four segments at least); the slices' sums are added up by finish_slices or gemm_reduce_kernel (slices_meet).

@@ -70,7 +70,7 @@ def layout_slices(layout, M, N, K):
 def test_workspace_of_a_layout_is_what_its_route_uses(plan):
     """minfer_gemm_layout_workspace_bytes: no less than a call can use, and no more."""
     # whole rows of an [N, K] weight: from 96 stripes of 64 columns on always, and where stripe_blocks_pay says so
-    for M, N, K in ((40, 8192, 2048), (64, 6144, 4096), (9, 12280, 8192), (64, 4096, 4096), (24, 2048, 4096)):
+    for M, N, K in ((40, 8192, 2048), (64, 6144, 4096), (9, 12280, 8192), (59, 4096, 4096), (29, 4096, 8192), (24, 2048, 4096)):
         assert layout_slices(capi.GEMM_B_NK, M, N, K) == 0
     # a [K, N] weight: eight slices, or sixteen of long rows, however many would fill the chip
     assert layout_slices(capi.GEMM_B_KN, 9, 1000, 4096) == 8 and layout_slices(capi.GEMM_B_KN, 9, 1000, 8192) == 16

@@ -393,7 +393,7 @@ def test_qkv_op_and_reference_checks(kerns):
 @pytest.mark.parametrize("layout", [KN, NK])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K,alpha,beta", [
-    (64, 4096, 4096, 1.0, 0.0),      # [K, N]: 32 tiles of 128 columns, 8 slices of 8 steps; [N, K]: 256 blocks of 16 columns, no slices
+    (64, 4096, 4096, 1.0, 0.0),      # [K, N]: 32 tiles of 128 columns, 8 slices of 8 steps; [N, K]: four slices of 64 stripes
     (100, 1032, 2048, 2.0, 3.0),     # tiles of whole rows: the workspace is not needed
     (256, 2048, 1024, 0.5, 1.0),
     (40, 512, 1984, 1.0, 0.0),       # [K, N]: 31 K steps in 7 slices; [N, K]: whole rows
@@ -569,8 +569,10 @@ def test_gemm_k_slices_of_stripes(gemm_plan, dtype, M, N, K, slices):
 
 @pytest.mark.parametrize("layout,M,N,K,kernel,slices", [   # just past and just below where K slices are taken from 17 rows on
     (NK, 28, 2560, 5120, rules.STRIPE_SLICES, 5), (NK, 24, 2560, 5120, rules.STRIPE, 1),
-    (NK, 63, 3080, 4096, rules.STRIPE_SLICES, 4), (NK, 62, 3072, 4096, rules.STRIPE, 1),
-    (NK, 40, 4096, 6144, rules.STRIPE_SLICES, 4), (NK, 37, 4096, 6144, rules.STRIPE, 1),
+    (NK, 63, 3080, 4096, rules.STRIPE_SLICES, 4), (NK, 41, 3072, 4096, rules.STRIPE_SLICES, 4), (NK, 40, 3072, 4096, rules.STRIPE, 1),
+    (NK, 40, 4096, 6144, rules.STRIPE_SLICES, 4), (NK, 35, 4096, 6144, rules.STRIPE_SLICES, 4), (NK, 34, 4096, 6144, rules.STRIPE, 1),
+    (NK, 64, 4096, 4096, rules.STRIPE_SLICES, 4), (NK, 59, 4096, 4096, rules.STRIPE, 1),
+    (NK, 30, 4096, 8192, rules.STRIPE_SLICES, 4), (NK, 29, 4096, 8192, rules.STRIPE, 1),
     (KN, 17, 264, 4160, rules.KN_ROWS, 16), (KN, 64, 1024, 4096, rules.KN_ROWS, 16), (KN, 64, 1032, 4096, rules.KN_ROWS, 8),
 ])
 def test_gemm_k_slices_beside_their_lines(gemm_plan, layout, M, N, K, kernel, slices):
