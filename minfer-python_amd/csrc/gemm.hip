@@ -1235,7 +1235,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmParams p) {
 // The counters of a sliced launch, when its workgroups are to add the slices up themselves.
 static uint32_t* slice_counters(const GemmParams& p, hipStream_t stream) {
     static_assert(kMeetTiles <= kStreamCounters, "a counter per tile");
-    return slices_meet(p.M, p.N, p.splits) ? stream_counters(stream) : nullptr;
+    return slices_meet(p.M) ? stream_counters(stream) : nullptr;
 }
 
 // After a sliced launch: nothing where its workgroups have added the slices up themselves.

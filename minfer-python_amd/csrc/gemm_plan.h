@@ -84,13 +84,14 @@ inline int kn_slices(int64_t M, int64_t N, int64_t K) {
 
 // ---- who adds the K slices up ----------------------------------------------------------------------------------
 // Whether the slices of stripe_slices or kn_slices meet inside the launch (finish_slices; where the stream has counters): up to kMeetRows
-// rows, which is what its threads have pieces for, and 2 MiB of sums.  Written through to where every XCD sees them they pass at about a
-// microsecond per MiB, so larger ones are left to a second launch (fused / two launches, the latter 1 us less since it reads its slices
-// together: 1 MiB 12.2 / 13.4 us, 1.9 MiB 23.7 / 25.3, 2.4 MiB 18.0 / 15.0, 5 MiB 16.7 / 13.7), and so are more rows, and so the slices of
-// gemm_kernel, whose tiles' last workgroups add up what a second launch spreads over the chip (17 x 528 x 1152 9.5 / 8.7, 40 x 808 x 1600
-// 13.3 / 9.8, 24 x 3424 x 1408 11.3 / 9.7).  Two slices and more are of at most kMeetTiles tiles: both size functions stay at 256 workgroups.
+// rows, which is what its threads have pieces for.  Both rules stay at 256 workgroups, so two slices and more are of at most kMeetTiles tiles and
+// the sums are 2 MiB at most.  Written through to where every XCD sees them they are as fast as a second launch or faster up to 1 MiB, and level or behind
+// above it (us, weights from memory, in a loop of calls, inside / second launch: `[K, N]` 4 x 4096 x 4096, 0.5 MiB, 10.5 / 10.9; 8 x 4096 x 4096, 1 MiB, 11.0 / 11.0; 16 x 2048 x
+// 8192, 2 MiB in 16 slices, 12.9 / 12.2; 16 x 8192 x 4096, 2 MiB in four, 17.0 / 17.1; `[N, K]` 9 x 2048 x 8192 10.4 / 10.8, 16 x 1024 x 14336 in 14 slices 12.0 / 11.1; Q8_0 8 x
+// 8192 x 8192 18.3 / 18.8), but the launch is 2.7 us of the host's, which bounds the steps of so few rows.  The slices of gemm_kernel go to a second launch, which
+// spreads over the chip what its tiles' last workgroups would add up (17 x 528 x 1152 9.5 / 8.7, 40 x 808 x 1600 13.3 / 9.8, 24 x 3424 x 1408 11.3 / 9.7).
 constexpr int kMeetRows = 16, kMeetTiles = 128;
-inline bool slices_meet(int64_t M, int64_t N, int64_t slices) { return M <= kMeetRows && slices * M * N * 4 <= (2 << 20); }
+inline bool slices_meet(int64_t M) { return M <= kMeetRows; }
 
 // ---- which tiles, how many K slices --------------------------------------------------------------------------
 inline int64_t tile_count(int64_t M, int64_t N, int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }

@@ -36,7 +36,7 @@ extern "C" int64_t q8_rows_of_a_part(int64_t M, int64_t N, int64_t K, int aligne
 extern "C" void grouped(int64_t M, int64_t N, int64_t K, int* out) { tile_of(tile_plan(M, N, K, true, 1, 256).tile, out); }
 extern "C" int stripe_blocks_ahead(int64_t M, int64_t N, int64_t K) { return stripe_blocks_pay(M, (N + 63) / 64, K); }
 extern "C" int q8_blocks_ahead(int64_t M, int64_t N, int64_t K) { return q8_blocks_pay(M, N, K); }
-extern "C" int meet(int64_t M, int64_t N, int64_t slices) { return slices_meet(M, N, slices); }
+extern "C" int meet(int64_t M) { return slices_meet(M); }
 extern "C" int meet_rows() { return kMeetRows; }
 extern "C" int meet_tiles() { return kMeetTiles; }
 extern "C" long estimates_made() { return estimates; }
@@ -59,7 +59,7 @@ class GemmPlan:
         L.q8_rows_of_a_part.argtypes, L.q8_rows_of_a_part.restype = [i64, i64, i64, ctypes.c_int], i64
         L.grouped.argtypes = [i64, i64, i64, ints]
         L.stripe_blocks_ahead.argtypes = L.q8_blocks_ahead.argtypes = [i64, i64, i64]
-        L.meet.argtypes = [i64, i64, i64]
+        L.meet.argtypes = [i64]
         L.estimates_made.restype = ctypes.c_long
         self.lib = L
         self.estimates = L.estimates_made
