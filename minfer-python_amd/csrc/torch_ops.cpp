@@ -555,7 +555,7 @@ void qkv_hip(int64_t q_qtype_int, int64_t k_qtype_int, int64_t v_qtype_int, int6
             ws_max = need > ws_max ? need : ws_max;
         }
         const Workspace wsp(x, ws_max);
-            for (int i = 0; i < 3; ++i) {
+        for (int i = 0; i < 3; ++i) {
             const Tensor& w = *ws[i];
             Tensor& o = *outs[i];
             STD_TORCH_CHECK(on_gpu(w) && on_gpu(o) && type_of(o) == t, names[i], ": dtype or device mismatch");
