@@ -102,8 +102,11 @@ inline int64_t tile_count(int64_t M, int64_t N, int64_t bm, int64_t bn) { return
 // that in part: the three add up as their squares; past one round, where the clock has come down to what the power budget leaves, the
 // more the more a tile copies per flop (3072 x 8192 x 4096: 128 x 256 tiles 177.7 us, 192 x 256 167.1, without this estimated 171.7 and
 // 172.9; 4096 x 5120 x 4096 150.9 and 137.0); 3.6 us around it, 0.9 more for the launch that adds the slices up, and 0.29 us
-// per MB of sums.  Fitted to 4700 timed calls (150 shapes of 65 to 7000 rows, both layouts, up to 40 choices each): the choice it
-// makes is 1.0 % behind the best one on average, fixed rules for 128 x 128 and 128 x 256 slices and a table of rounds 6 %.
+// per MB of sums.  Fitted to 4700 timed calls (150 shapes of 65 to 7000 rows, both layouts, up to 40 choices each), whose sums were added up by
+// one load after the other: the choice it made was 1.0 % behind the best one on average, fixed rules for 128 x 128 and 128 x 256 slices and a
+// table of rounds 6 %.  With gemm_reduce_kernel as it is, 100 shapes for which slices and whole rows are estimated to be close (70 of them within 12 %), ten
+// choices each, weights from memory: 2.4 % behind the best one without C and 2.1 % with it, 10 of the 100 in slices where whole rows are faster and 9 the other way
+// round, so the line has no side that it leans to; the constants of the sums that would be best for these alone (1.7 us, 0.20 us per MB) are 1.8 % behind.
 inline double plan_cost(const GemmTile& t, int64_t tiles, int slices, int64_t M, int64_t N, int64_t K, int cus) {
     const double steps = (double)((K / kBK + slices - 1) / slices), area = t.m16 * t.n16;
     const double step = (0.0201 * area + 0.0738) * (t.occ == 2 ? 1.84 : 1.0) + (t.ns == 2 && t.occ == 1 ? 0.0147 + 0.0076 * (64 - area) : 0.0);
@@ -179,35 +182,35 @@ struct GemmRoute { GemmKernel kernel; int slices, tile; };
 // A decode step's few tokens against an [N, K] weight: stream the weight once.  Which kernel does that best was
 // measured with the calls cycling over copies of the weight, 640 MiB in all: a weight of up to 256 MiB called again
 // and again is served by the chip's last-level cache, where the order of the kernels is a different one (14336 x
-// 4096 at one row: stripes 18.0 us against 19.5 for whole rows per wave from the cache, 24.2 against 21.9 from memory).
+// 4096 at one row: stripes 18.0 us against 19.5 for whole rows per wave from the cache, 21.7-24.2 against 21.7-21.9 from memory).
 // These calls are bound by the host: no rule for up to 16 rows asks for a plan of tiles.
 inline GemmRoute gemm_route(int64_t M, int64_t N, int64_t K, bool nt, bool fast, int64_t fit, int (*units)()) {
     if (!fast) return {GemmKernel::plain, 1, 0};
     if (nt && M <= 64) {
         const int64_t stripes = (N + 63) / 64;
         const bool rows_takes = rows_lds_takes(M, K);
-        // one row: whole weight rows per wave (14336 x 4096: 21.9 us, the 16-column kernel 23.6, stripes 24.2; 28672 x 8192:
-        // 75.8 / 91 / 97); a weight under 32 M values goes to the 16-column kernel when it takes it (4096 x 4096: 8.5 against 10.5)
+        // one row: whole weight rows per wave (14336 x 4096: 21.7-21.9 us, the 16-column kernel 23.2-23.6, stripes 21.7-24.2; 28672 x 8192:
+        // 75-76 / 91 / 81-97); a weight under 32 M values goes to the 16-column kernel when it takes it (4096 x 4096: 8.4 against 10.6)
         if (M == 1 && K <= kGemvMaxKHalfs && (N * K >= (INT64_C(1) << 25) || !rows_takes)) return {GemmKernel::gemv, 1, 0};
         // two to four rows against long rows of a wide weight go the same way, every weight piece multiplied with the same
-        // piece of each activation row (28672 x 8192 at 2-4 rows: 78.6-82.6 us against 93-95 for the 16-column kernel, 10240 x
-        // 8192 at 2-3 rows 33.2-34.6 against 36.3; 8192 x 8192 30.5-33.9 against 29.2-29.6, and rows of 4096 values gain nothing)
+        // piece of each activation row (28672 x 8192 at 2-4 rows: 77.5-82.6 us against 92-95 for the 16-column kernel, 10240 x
+        // 8192 at 2-3 rows 32.1-34.6 against 36.3-38.8; 8192 x 8192 29.2-33.9 against 29.2-30.9, and rows of 4096 values gain nothing)
         if (M >= 2 && gemv_takes(M, K) && K >= 8192 && N >= 10240 && (M <= 3 || N >= 16384)) return {GemmKernel::gemv, 1, 0};
         // up to 4 rows (8 where stripe_takes says no) against fewer than 96 stripes, and up to 4 against an output head: the 16-column
-        // kernel (128256 x 4096 at 2-4 rows 166-170 against 176-178; 28672 x 4096 at 2-8 rows 42.2-44.5 against 41.5-41.7 and 14336 x
-        // 4096 24.3-25.8 against 22.8-23.0: those go on)
+        // kernel (128256 x 4096 at 2-4 rows 166-170 against 176-178, on another box 165-169 against 161-163; 28672 x 4096 at 2-8 rows 41.6-44.8 against 38.5-39.1 and 14336 x
+        // 4096 23.2-25.6 against 21.7-21.8: those go on)
         const bool rows_first = rows_takes && ((M <= 8 && stripes < 96 && !stripe_takes(M, stripes, K)) || (M <= 4 && stripes > 640));
         const int slices = stripe_slices(M, N, K);
         const bool sliceable = slices > 1 && fit >= slices;
         // ... except long rows of a narrow weight when a workspace allows K slices: one wave per 16 columns walks a whole row
-        // by itself (1024 x 14336 at 2-8 rows 16.5-20.8 us, in slices 13.1-14.1; 1536 x 8960 15.2-17.4 and 11.8-12.5; 2048 x
-        // 8192 at 5-8 rows 12.5-13.4 and 12.5-12.6, at 2-4 rows and for rows of 6144 values no gain)
+        // by itself (1024 x 14336 at 2-8 rows 16.5-20.8 us, in slices 10.5-10.9; 1536 x 8960 15.1-17.4 and 9.3-9.8; 2048 x
+        // 8192 at 5-8 rows 12.4-13.4 and 10.2-10.3.  The lines are those of slices that took a second launch; now that they meet inside it 2048 x 8192 at
+        // 2-4 rows, 11.4-12.0 and 10.1, and rows of 6144 values, 1536 x 6144 at 2-8 rows 8.8-10.4 and 8.4-8.8, would gain as well)
         const bool long_rows_few_stripes = K >= 8192 && ((M >= 5 && stripes <= 32) || (M >= 2 && stripes <= 24));
         if (rows_first && !(sliceable && long_rows_few_stripes)) return {GemmKernel::rows_lds, 1, 0};
-        // with a workspace, K slices of the stripes, from 9 rows on, where whole rows are not ahead (stripe_blocks_pay): two launches, 10.5
-        // us at least, where one launch over rows of 4096 values takes 8-10 at 9-16 rows: up to 16 rows only for 25 M weight values or
-        // rows of 6144 values and more (2048 x 8192 at 9-16 rows 12.7-13.0 against 13.9-16.5, 1024 x 14336 13.7-14.6 against 21.5-26.7),
-        // from 17 rows on for 8 M values (1536 x 5632 and the like: gemm_skinny_kernel is the other choice)
+        // with a workspace, K slices of the stripes, from 9 rows on, where whole rows are not ahead (stripe_blocks_pay): up to 16 rows only for 25 M
+        // weight values or rows of 6144 values and more (2048 x 8192 at 9-16 rows 10.5-11.0 against 13.9-16.7 for the 16-column kernel, 1024 x 14336 11.3-12.1 against
+        // 21.6-26.9), from 17 rows on for 8 M values (1536 x 5632 and the like: gemm_skinny_kernel is the other choice)
         const bool slices_pay = !stripe_blocks_pay(M, stripes, K) && (long_rows_few_stripes || (M >= 9 && (N * K >= INT64_C(25000000) || K >= 6144 || (M >= 17 && N * K >= (INT64_C(1) << 23)))));
         if (sliceable && slices_pay) return {GemmKernel::stripe_slices, slices, 0};
         if (stripe_takes(M, stripes, K)) return {GemmKernel::stripe, 1, 0};
@@ -217,11 +220,11 @@ inline GemmRoute gemm_route(int64_t M, int64_t N, int64_t K, bool nt, bool fast,
         if ((M <= 32 || N * K <= (INT64_C(1) << 25)) && !(fit > 1 && tile_plan(M, N, K, nt, kMostSlices, units()).slices > 1)) return {GemmKernel::skinny, 1, 0};
     }
     if (!nt && M <= kKnRows) {
-        // eight slices at most, 16 for rows of 80 K steps and more, and for up to 1024 columns from 17 rows on (eight / 16: 512 x 4096 at 17 / 64 rows 9.4 / 9.2,
-        // 10.5 / 9.7; 1024 x 4096 9.7 / 9.4, 11.4 / 11.0; 2048 x 4096 at 40 10.9 / 11.6): further ones save less streaming than their sums cost (us, as many as fill
-        // the chip / these: 1000 x 4096 at 1 / 9 / 16 rows 10.5 / 7.6, 13.5 / 8.7, 15.5 / 9.4; 2560 x 2560 at 12 10.0 / 8.1; 2048 x 4096 at 40 13.7 /
-        // 11.9; 1024 x 14336 at 9 / 40 15.4 / 12.8, 19.4 / 17.2; 512 x 8192 at 9 17.0 / 9.6; minfer_gemm_workspace_bytes stays that of filling it)
-        const int most = std::min(kn_slices(M, N, K), K >= 80 * kBK || (M > 16 && N <= 1024) ? 16 : 8);   // a smaller workspace: as many of these as it holds (40 x 4096 x 4096: none 30.4 us, two 18.9, four 12.9, all eight 12.6)
+        // eight slices at most, 16 for rows of 80 K steps and more, and for up to 1024 columns from 17 rows on (eight / 16: 512 x 4096 at 17 / 64 rows 8.9 / 7.8,
+        // 10.6 / 9.5; 1024 x 4096 9.2 / 8.5, 11.3 / 11.0; 1536 x 4096 at 17 / 64 9.5 / 9.0, 12.2 / 12.4; 2048 x 4096 at 40 11.1 / 11.8): further ones save less streaming than their sums
+        // cost (us, weights from memory, as many as fill the chip / these: 1000 x 4096 at 1 / 9 / 16 rows 10.4 / 7.7, 13.2 / 8.9, 15.1 / 9.6; 2560 x 2560 at 12 10.1 / 8.2;
+        // 1024 x 14336 at 9 / 40 15.2 / 12.8, 14.3 / 14.6; 512 x 8192 at 9 16.6 / 9.8; minfer_gemm_workspace_bytes stays that of filling it)
+        const int most = std::min(kn_slices(M, N, K), K >= 80 * kBK || (M > 16 && N <= 1024) ? 16 : 8);   // a smaller workspace: as many of these as it holds (40 x 4096 x 4096: none 31.7 us, two 20.9, four 14.6, all eight 12.6)
         return {GemmKernel::kn_rows, std::max((int)std::min<int64_t>(most, fit), 1), 0};
     }
     TilePlan plan = tile_plan(M, N, K, nt, kMostSlices, units());
