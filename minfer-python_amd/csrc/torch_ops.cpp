@@ -45,7 +45,8 @@ void* current_stream() {
 }
 
 // An operator looks at the type and device of up to nine tensors.  Asked for through the ABI's own numbers they take 3 ns each;
-// as ScalarType and Device they go through the translation of an argument (25 and 16 ns).
+// as ScalarType and Device they go through the translation of an argument (25 and 16 ns; of the 6 to 7 us that issuing an operator takes
+// 0.1 to 0.3).
 const int32_t kHalf = aoti_torch_dtype_float16(), kBFloat16 = aoti_torch_dtype_bfloat16(), kFloat = aoti_torch_dtype_float32(),
               kByte = aoti_torch_dtype_uint8(), kInt = aoti_torch_dtype_int32(), kBool = aoti_torch_dtype_bool();
 
@@ -72,7 +73,8 @@ int dtype_code(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& 
 }
 
 // Scratch memory on a tensor's device, from torch's allocator and so for the current stream; none at all for a call that needs
-// none.  (new_empty by the name of its operator, for every call, was 0.9 us of the 6 that issuing one took.)
+// none.  (With new_empty by the name of its operator, for every call, issuing one takes 0.3 us more: prefill of a short prompt 7.5 / 7.2, decode over
+// Q8_0 7.5 / 7.1, a projection 6.9 / 6.6.)
 class Workspace {
 public:
     Workspace(const Tensor& like, size_t nbytes) {
