@@ -29,33 +29,33 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 # same counter reads for a 1 GiB copy: x2.0 and x1.0), classify+main and split+combine respectively
 # These are figures from those earlier counter runs, not measured in the run that prints them.
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels_pmc.md (rocprofv3 --pmc runs of the same workloads; not re-measured by this run)"
-PREFILL_TRAFFIC_BYTES = 107316 * 1024
-DECODE_TRAFFIC_BYTES = 1092924 * 1024
+PREFILL_TRAFFIC_BYTES = 107314 * 1024
+DECODE_TRAFFIC_BYTES = 1092908 * 1024
 ROPE_TRAFFIC_BYTES = 393314 * 1024          # il_rope on [8,4096,48,128], rotary 64
 APPEND_TRAFFIC_BYTES = 786533 * 1024        # rope_kv_append, B=8 L=4096 Llama-3-8B heads
-NORM_TRAFFIC_BYTES = 786682 * 1024          # rmsnorm on [8,4096,6144]
-GEMM_TRAFFIC_BYTES = 229795 * 1024          # gemm 4096^3 (A and B panels are re-read by several XCDs)
-DECODE_Q8_TRAFFIC_BYTES = 598309 * 1024     # decode over Q8_0 caches (split + combine)
-APPEND_Q8_TRAFFIC_BYTES = 737593 * 1024     # rope_kv_append into Q8_0 caches
-APPEND_NORM_TRAFFIC_BYTES = 786638 * 1024   # rope_kv_append_norm, the same shape
-QKV_TRAFFIC_BYTES = 377984 * 1024           # qkv in one launch, M=K=4096, N=4096+1024+1024
-LONG_TRAFFIC_BYTES = 2721616 * 1024         # long-context prefill (classify + main), S=32768 bf16: the 1 GiB mask once, K/V re-fetched past the 4 MiB L2s
-RAGGED_TRAFFIC_BYTES = 748032 * 1024        # packed ragged prefill (T=20514, Hq=64)
-GEMM_Q8_TRAFFIC_BYTES = 61123 * 1024        # one token against a 14336 x 4096 weight of Q8_0 blocks
+NORM_TRAFFIC_BYTES = 786669 * 1024          # rmsnorm on [8,4096,6144]
+GEMM_TRAFFIC_BYTES = 229726 * 1024          # gemm 4096^3 (A and B panels are re-read by several XCDs)
+DECODE_Q8_TRAFFIC_BYTES = 597506 * 1024     # decode over Q8_0 caches (split + combine)
+APPEND_Q8_TRAFFIC_BYTES = 737591 * 1024     # rope_kv_append into Q8_0 caches
+APPEND_NORM_TRAFFIC_BYTES = 786611 * 1024   # rope_kv_append_norm, the same shape
+QKV_TRAFFIC_BYTES = 377747 * 1024           # qkv in one launch, M=K=4096, N=4096+1024+1024
+LONG_TRAFFIC_BYTES = 2721679 * 1024         # long-context prefill (classify + main), S=32768 bf16: the 1 GiB mask once, K/V re-fetched past the 4 MiB L2s
+RAGGED_TRAFFIC_BYTES = 747918 * 1024        # packed ragged prefill (T=20514, Hq=64)
+GEMM_Q8_TRAFFIC_BYTES = 61121 * 1024        # one token against a 14336 x 4096 weight of Q8_0 blocks
 GEMM_DECODE_TRAFFIC_BYTES = 120711 * 1024   # 64 tokens against the same weight in fp16, [N, K]
 # The kernel sources the counter runs were made against (first 12 hex digits of each file's sha1).  A row one of whose
 # sources has changed since carries "traffic_stale": true, so a constant that describes an earlier kernel says so.
 TRAFFIC_MEASURED_AGAINST = {
     "attn_common.h": "f00da2487c24",
     "attn_prefill.hip": "4aa50ccd63dd",
-    "attn_decode.hip": "322fe3fdb487",
+    "attn_decode.hip": "35cbde39fc19",
     "quant_q8.h": "4fea6a94e300",
-    "rope.hip": "f03d700b34e7",
+    "rope.hip": "50c43a5fa421",
     "rmsnorm.hip": "90740d99856e",
-    "gemm.hip": "106d5e4e5211",
-    "gemm_common.h": "608850fcbd9f",
-    "gemm_plan.h": "a390cbf53d12",
-    "gemm_tile.h": "f07b752e72ff",
+    "gemm.hip": "87632e517cc6",
+    "gemm_common.h": "efc44e77d7fe",
+    "gemm_plan.h": "1ffba093d146",
+    "gemm_tile.h": "9c625ec29d20",
     "gemm_tile_f16.hip": "969b3f4315b6",
     "gemm_tile_bf16.hip": "d2866de7d66d",
 }
