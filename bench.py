@@ -55,7 +55,7 @@ TRAFFIC_MEASURED_AGAINST = {
     "gemm.hip": "87632e517cc6",
     "gemm_common.h": "efc44e77d7fe",
     "gemm_plan.h": "1ffba093d146",
-    "gemm_tile.h": "9c625ec29d20",
+    "gemm_tile.h": "0509060bdf46",
     "gemm_tile_f16.hip": "969b3f4315b6",
     "gemm_tile_bf16.hip": "d2866de7d66d",
 }

@@ -283,10 +283,10 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
     int64_t i_ldd[IT];
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        const int idx = min(64 * it + lane, ITEMS - 1), g = idx % (2 * N16);   // (a lane without a piece: the last one's place)
+        const int idx = 64 * it + lane, g = idx % (2 * N16);
         i_row[it] = idx / (2 * N16);
         i_n[it] = n0 + 16 * N16 * wn + 8 * g;
-        i_on[it] = 64 * it + lane < ITEMS && i_n[it] < p.N;
+        i_on[it] = idx < ITEMS && i_n[it] < p.N;
         d_col[it] = (short*)p.D + i_n[it];
         i_ldd[it] = p.ldd;
         if (NT) {
@@ -297,7 +297,8 @@ __global__ __launch_bounds__(SH::WAVES * 64, SH::OCC) void gemm_kernel(const Gem
         }
     }
     typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
-    // A block row's pieces of C are requested CD block rows before they are added (rows and columns past the end, and lanes without a piece, read the last ones):
+    // A block row's pieces of C are requested CD block rows before they are added (rows and columns past the end read the last ones, and the
+    // lanes without a piece, an eighth of them with N16 = 7, the next rows'; giving those the last piece's place is 68 instructions more and no faster):
     // waited for as soon as requested, as they were, every one of a wave's 4 to 8 block rows costs the latency of memory, 3 to 12 us a
     // tile (with C, us, before / after: 4096^3 `[N, K]` 123.3 / 110.5, 8192 x 4096 x 4096 243.5 / 218.3, 600 x 14336 x 4096 75.1 / 67.6,
     // 1777 x 4096 x 4096 `[K, N]` 58.0 / 54.8, without C 51.4).
