@@ -54,7 +54,7 @@ TRAFFIC_MEASURED_AGAINST = {
     "rmsnorm.hip": "90740d99856e",
     "gemm.hip": "87632e517cc6",
     "gemm_common.h": "efc44e77d7fe",
-    "gemm_plan.h": "1ffba093d146",
+    "gemm_plan.h": "fa8c11000081",
     "gemm_tile.h": "0509060bdf46",
     "gemm_tile_f16.hip": "969b3f4315b6",
     "gemm_tile_bf16.hip": "d2866de7d66d",

@@ -34,7 +34,7 @@ inline bool gemv_takes(int64_t M, int64_t K) { return M >= 1 && M <= 4 && K <= k
 // gemm_stripe_kernel.  Which widths it takes (in stripes of 64 columns; weights coming from memory): from 96 on every row count that reaches
 // it (14336 x 4096 at 2-32 rows 21.6-22.4 us, the 16-column kernels 23.2-40.5); an output head from 5 rows on (128256 x 4096 at 8
 // rows 164 against 182, 57344 x 8192 160 against 186; at 2-4 rows the kernels that keep more workgroups on a compute unit
-// were ahead, 166-170 against 176-178, and on another box behind, 165-169 against 161-163); narrower ones down to 32 stripes from 5 rows on, up to 8 when their rows are long enough to matter, against the 16-column
+// were ahead, 166-170 against 176-178, and on another chip behind, 165-169 against 161-163); narrower ones down to 32 stripes from 5 rows on, up to 8 when their rows are long enough to matter, against the 16-column
 // and few-row kernels (us: 2048 x 4096 at 16 / 17 / 64 rows 9.6 / 7.8, 14.0 / 8.6, 21.5 / 14.0; 5120 x 5120 at 5 / 16 rows 14.9 / 12.9,
 // 20.4 / 14.5; 3072 x 8192 at 8 / 32 rows 14.9 / 12.8, 29.8 / 17.2; 4096 x 14336 at 8 / 64 rows 24.3 / 22.8, 70.8 / 44.1).
 inline bool stripe_takes(int64_t M, int64_t stripes, int64_t K) {
@@ -197,7 +197,7 @@ inline GemmRoute gemm_route(int64_t M, int64_t N, int64_t K, bool nt, bool fast,
         // 8192 at 2-3 rows 32.1-34.6 against 36.3-38.8; 8192 x 8192 29.2-33.9 against 29.2-30.9, and rows of 4096 values gain nothing)
         if (M >= 2 && gemv_takes(M, K) && K >= 8192 && N >= 10240 && (M <= 3 || N >= 16384)) return {GemmKernel::gemv, 1, 0};
         // up to 4 rows (8 where stripe_takes says no) against fewer than 96 stripes, and up to 4 against an output head: the 16-column
-        // kernel (128256 x 4096 at 2-4 rows 166-170 against 176-178, on another box 165-169 against 161-163; 28672 x 4096 at 2-8 rows 41.6-44.8 against 38.5-39.1 and 14336 x
+        // kernel (128256 x 4096 at 2-4 rows 166-170 against 176-178, on another chip 165-169 against 161-163; 28672 x 4096 at 2-8 rows 41.6-44.8 against 38.5-39.1 and 14336 x
         // 4096 23.2-25.6 against 21.7-21.8: those go on)
         const bool rows_first = rows_takes && ((M <= 8 && stripes < 96 && !stripe_takes(M, stripes, K)) || (M <= 4 && stripes > 640));
         const int slices = stripe_slices(M, N, K);
